@@ -340,11 +340,14 @@ __global__ __launch_bounds__(256) void spectral_reduce_kernel(const float* __res
 //   r[k, m] = (1/N) sum_n cos(theta k n) c[n, m] + sin(theta k n) c[N + n, m] = (1/N) Re sum_n e^{i theta k n} (c - i s)
 // is the compression GEMM with the roles of position and frequency exchanged: the rows are the positions k,
 // the "tokens" are the N coefficient indices.  A workgroup owns 128 positions, keeps their basis rows in
-// registers, and walks over every block of 64 columns: one pass over the cos coefficients (keeps the real part A_k),
+// registers, and walks over its blocks of 64 columns: one pass over the cos coefficients (keeps the real part A_k),
 // one over the sin coefficients (keeps the imaginary part B_k), then folds its positions into sum / max / min.
 // Position k gives r[k] = A_k + B_k and, because the period is a whole number of positions, also its mirror image
 // r[T - k] = A_k - B_k: only the positions up to T / 2 are computed, each standing for two where the sequence
 // reaches past T / 2.
+// The column blocks are dealt to the workgroups of a row block so that the launch fills the device (recon_col_share):
+// the matrix cores bound it, and with one workgroup per 128 positions four sequences of 1977 positions kept 64 of 256
+// compute units busy.
 // The coefficients travel as f16 scaled by a power of two per column (their range is not bounded).
 // ---------------------------------------------------------------------------------------------------------
 __global__ __launch_bounds__(1024) void coef_colscale_kernel(const float* __restrict__ c, float* __restrict__ scale,
@@ -382,6 +385,7 @@ struct ReconStatsParams {
   float* pmax;
   float* pmin;             // [B][RB][Mc]
   int B, N, Mc, CT, KS32, K, T, n_steps, RB;
+  int cb_per; // column blocks of a workgroup
   int Kd;     // positions computed directly: min(K, T / 2 + 1)
   int half;   // T / 2: mirror images beyond it count as positions of their own (a value no position exceeds
               // when the sequence is longer than the period and every position is computed directly)
@@ -398,11 +402,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int rt0 = (rb * 4 + w) * 4;
   const int n_rt = (p.Kd + 7) / 8;
   const int S = p.n_steps;
-  const int n_cb = (p.Mc + kWgCols - 1) / kWgCols;
+  const int cb0 = blockIdx.z * p.cb_per;
+  const int n_cb = min((p.Mc + kWgCols - 1) / kWgCols - cb0, p.cb_per);
   const int Q = n_cb * 2 * S;   // steps of this workgroup: column block, pass (cos, sin), step (last to first)
 
   auto issue = [&](int q, int stage) {
-    const int cb = q / (2 * S), rem = q - cb * 2 * S;
+    const int cb = cb0 + q / (2 * S), rem = q % (2 * S);
     const int pass = rem / S, s = S - 1 - (rem - pass * S);
     const int ct = min(cb * 4 + w, p.CT - 1);
     const _Float16* src = (const _Float16*)(p.packed[pass] + (((int64_t)b * p.CT + ct) * p.KS32) * 64) + lane * 8;
@@ -433,7 +438,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 
   const float inv_n = 1.0f / (float)p.N;
   for (int q = 0; q < Q; ++q) {
-    const int cb = q / (2 * S), rem = q - cb * 2 * S;
+    const int cb = cb0 + q / (2 * S), rem = q % (2 * S);
     const int pass = rem / S, it = rem - pass * S;
     const int stage = q % NST;
     if (q + NST - 2 < Q) wait_vmcnt<(NST - 2) * kStepK>();
@@ -709,6 +714,22 @@ ReconPlan recon_plan(int B, int N, int Mc, int K) {
 }
 }  // namespace
 
+namespace {
+// Column blocks per workgroup of the reconstruction statistics.  Two workgroups fit a compute unit, and a workgroup
+// pays about half a column block for its basis rows before the first product: take the share whose rounds over the
+// device, times the length of a round, come out shortest.
+int recon_col_share(int row_groups, int n_cb) {
+  int best = n_cb;
+  float best_cost = 1e30f;
+  for (int cs = 1; cs <= n_cb; ++cs) {
+    const int per = fa_cdiv(n_cb, cs);
+    const float cost = (float)fa_cdiv((int64_t)row_groups * fa_cdiv(n_cb, per), 512) * ((float)per + 0.5f);
+    if (cost < best_cost) { best_cost = cost; best = per; }
+  }
+  return best;
+}
+}  // namespace
+
 bool fa_recon_stats_mfma_ok(int N, int Mc, int K) { return N >= 32 && Mc >= 16 && K >= 1024; }
 
 size_t fa_recon_stats_mfma_workspace(int B, int N, int Mc, int K) { return recon_plan(B, N, Mc, K).total; }
@@ -743,6 +764,8 @@ int fa_recon_stats_mfma_launch(const float* c, int B, int N, int Mc, int K, int 
   rp.B = B; rp.N = N; rp.Mc = Mc; rp.CT = pl.CT; rp.KS32 = pl.KS32; rp.K = K; rp.T = T; rp.n_steps = pl.n_steps; rp.RB = RBd;
   rp.Kd = Kd;
   rp.half = mirror ? T / 2 : 0x7fffffff;
-  spectral_recon_stats_kernel<<<dim3(RBd, B), 256, 0, st>>>(rp);
+  const int n_cb = fa_cdiv(Mc, kWgCols);
+  rp.cb_per = recon_col_share(RBd * B, n_cb);
+  spectral_recon_stats_kernel<<<dim3(RBd, B, fa_cdiv(n_cb, rp.cb_per)), 256, 0, st>>>(rp);
   return RBd;
 }
