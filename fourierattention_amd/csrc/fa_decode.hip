@@ -323,7 +323,42 @@ __device__ __forceinline__ int64_t paged_offset(bool is_v, int dp, int64_t token
   return page * dp * 32 + (int64_t)(j >> 4) * 512 + ((t >> 3) * 16 + (j & 15)) * 8 + (t & 7);
 }
 
-template <typename E, bool PAGED>
+// eight consecutive elements of a row or page fragment as they are loaded
+template <typename E> struct Row8 { uint4 v[sizeof(E) / 2]; };
+template <typename E>
+__device__ __forceinline__ void row8_to_float(const Row8<E>& r, float (&f)[8]) {
+  const E* e = (const E*)&r;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) f[i] = fa_to_float(e[i]);
+}
+// sum of the eight products: pairs at a time for 16-bit elements
+template <typename E>
+__device__ __forceinline__ float dot8(const Row8<E>& a, const Row8<E>& b) {
+  if constexpr (sizeof(E) == 2) {
+    float s = fa_dot2<E>(a.v[0].x, b.v[0].x, 0.f);
+    s = fa_dot2<E>(a.v[0].y, b.v[0].y, s);
+    s = fa_dot2<E>(a.v[0].z, b.v[0].z, s);
+    return fa_dot2<E>(a.v[0].w, b.v[0].w, s);
+  } else {
+    float x[8], y[8], s = 0.f;
+    row8_to_float(a, x);
+    row8_to_float(b, y);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) s = fmaf(x[i], y[i], s);
+    return s;
+  }
+}
+
+// Any shape, fp32 arithmetic throughout; GM: query heads per KV head the instance holds (4 or 8).
+// Bound by the vector ALU and by the number of workgroups: a tile is 64 tokens shared by the four waves of a
+// workgroup - in the scores lane = token and each wave sums its quarter of the frequencies and of the stored dims, in
+// g = F^T p thread = (frequency, share of the tokens) - so that a short context still gives every compute unit a tile.
+// (One thread per token over all frequencies on tiles of 256 tokens took 137 us for 1532 mid rows of 24 / 8 heads and
+// 128 frequencies in fp32, 48 workgroups; this split KMID_US us.)  Weights and probabilities lie in LDS head by head, so a
+// thread fetches those of all heads with one broadcast read.
+constexpr int kMidTile = 64;   // tokens per tile
+
+template <typename E, bool PAGED, int GM>
 __global__ __launch_bounds__(256) void decode_mid_kernel(
     const E* __restrict__ q, const E* __restrict__ k_mn, int64_t k_bs, int64_t k_rs,
     const E* __restrict__ v_mn, int64_t v_bs, int64_t v_rs, int cap_pages, const int32_t* __restrict__ kpad_h,
@@ -332,43 +367,30 @@ __global__ __launch_bounds__(256) void decode_mid_kernel(
     const int32_t* __restrict__ vn_h, float* __restrict__ pm, float* __restrict__ pd,
     float* __restrict__ pg, float* __restrict__ pon, int Hq, int Hkv, int D, int N, int L_m, int T,
     int n_split, int tiles_per_split, float sm_log2e) {
-  extern __shared__ float smem[];
+  extern __shared__ __attribute__((aligned(16))) float smem[];
+  struct alignas(16) Heads { float v[GM]; };
   const int G = Hq / Hkv;
-  float* s_w = smem;                   // [G][2N]
-  float* s_qn = s_w + G * 2 * N;       // [G][D]
-  float* s_p = s_qn + G * D;           // [G][kTile]
-  float* s_red = s_p + G * kTile;      // [4][kGMax]
-  float* s_o = s_red + 4 * kGMax;      // [G][D]
+  Heads* s_w = (Heads*)smem;            // [N][cos, sin]
+  Heads* s_qn = s_w + 2 * N;            // [128]: stored query dims, zero past the head's
+  Heads* s_part = s_qn + 128;           // [4 waves][kMidTile]
+  Heads* s_p = s_part + 4 * kMidTile;   // [kMidTile]
+  float* s_alpha = (float*)(s_p + kMidTile);   // [GM]
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int split = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
   const int kn0 = kn_h[h], kn_len = kn_h[h + 1] - kn0;
   const int vn0 = vn_h[h], vn_len = vn_h[h + 1] - vn0;
 
-  for (int e = tid; e < G * 2 * N; e += 256) s_w[e] = W[((int64_t)b * Hq + h * G) * 2 * N + e];
-  for (int e = tid; e < G * D; e += 256) {
-    int g = e / D, j = e % D;
-    float v = 0.f;
-    if (j < kn_len) v = fa_to_float(q[((int64_t)b * Hq + h * G + g) * D + (kn_list[kn0 + j] - h * D)]) * sm_log2e;
-    s_qn[e] = v;
+  for (int e = tid; e < GM * 2 * N; e += 256) {
+    const int g = e / (2 * N), n = e - g * 2 * N;
+    const float x = g < G ? W[((int64_t)b * Hq + h * G + g) * 2 * N + n] : 0.f;
+    s_w[n < N ? 2 * n : 2 * (n - N) + 1].v[g] = x;
   }
-  float cz[kGMax], m_run[kGMax], d_run[kGMax];
-#pragma unroll
-  for (int g = 0; g < kGMax; ++g) {
-    cz[g] = g < G ? c0[(int64_t)b * Hq + h * G + g] : 0.f;
-    m_run[g] = -INFINITY;
-    d_run[g] = 0.f;
+  for (int e = tid; e < GM * 128; e += 256) {
+    const int g = e >> 7, j = e & 127;
+    s_qn[j].v[g] = g < G && j < kn_len ? fa_to_float(q[((int64_t)b * Hq + h * G + g) * D + (kn_list[kn0 + j] - h * D)]) * sm_log2e : 0.f;
   }
-  float gc[kFreqIters][kGMax], gs[kFreqIters][kGMax], on[kGMax];
-#pragma unroll
-  for (int i = 0; i < kFreqIters; ++i)
-#pragma unroll
-    for (int g = 0; g < kGMax; ++g) gc[i][g] = gs[i][g] = 0.f;
-#pragma unroll
-  for (int g = 0; g < kGMax; ++g) on[g] = 0.f;
-  __syncthreads();
-
-  const int l_beg = split * tiles_per_split * kTile;
-  const int l_end = min(L_m, l_beg + tiles_per_split * kTile);
+  const int l_beg = split * tiles_per_split * kMidTile;
+  const int l_end = min(L_m, l_beg + tiles_per_split * kMidTile);
   int dpk = 0, dpv = 0;
   const E* kb;
   const E* vb;
@@ -381,131 +403,195 @@ __global__ __launch_bounds__(256) void decode_mid_kernel(
     kb = k_mn + (int64_t)b * k_bs + kn0;
     vb = v_mn + (int64_t)b * v_bs + vn0;
   }
-  const int dim = tid % 128, half = tid / 128;
-
-  for (int l0 = l_beg; l0 < l_end; l0 += kTile) {
-    const int t_len = min(kTile, l_end - l0);
-    // ---- phase 1: scores, thread = token --------------------------------
-    const int l = l0 + tid;
-    const bool ok = tid < t_len;
-    float sc[kGMax];
+  // scores: this wave's frequencies
+  const int nq = (N + 3) / 4, n_lo = min(N, w * nq), n_hi = min(N, n_lo + nq);
+  // g: this thread's frequencies n_t + 256 i (up to 256 of them, the threads past N take another share of the tokens)
+  int ft = 256;
+  while (ft / 2 >= N && ft > 16) ft >>= 1;
+  const int n_t = tid & (ft - 1), tg = tid / ft, t_share = kMidTile * ft / 256;
+  float fr[kFreqIters], fi[kFreqIters];   // step of one token
 #pragma unroll
-    for (int g = 0; g < kGMax; ++g) sc[g] = cz[g];
-    if (ok) {
+  for (int i = 0; i < kFreqIters; ++i)
+    if (256 * i < N) fa_sincos_phase(min(n_t + 256 * i, N - 1), 1, T, &fi[i], &fr[i]);
+  float gc[kFreqIters][GM], gs[kFreqIters][GM], on[GM];
+#pragma unroll
+  for (int i = 0; i < kFreqIters; ++i)
+#pragma unroll
+    for (int g = 0; g < GM; ++g) gc[i][g] = gs[i][g] = 0.f;
+#pragma unroll
+  for (int g = 0; g < GM; ++g) on[g] = 0.f;
+  const int dim = tid & 127, half = tid >> 7;
+  // softmax: wave w keeps the running maximum and sum of heads w and w + 4
+  float m_run[GM / 4], d_run[GM / 4], cz[GM / 4];
+#pragma unroll
+  for (int i = 0; i < GM / 4; ++i) {
+    m_run[i] = -INFINITY;
+    d_run[i] = 0.f;
+    cz[i] = w + 4 * i < G ? c0[(int64_t)b * Hq + h * G + w + 4 * i] : 0.f;
+  }
+  __syncthreads();
+
+  for (int l0 = l_beg; l0 < l_end; l0 += kMidTile) {
+    const int t_len = min(kMidTile, l_end - l0);
+    // ---- phase 1: partial scores, lane = token -----------------------------
+    const int l = min(l0 + lane, L_m - 1);
+    float sc[GM];
+#pragma unroll
+    for (int g = 0; g < GM; ++g) sc[g] = 0.f;
+    {
       float sr, si, zr = 1.f, zi = 0.f;
       fa_sincos_phase(l, 1, T, &si, &sr);
-      for (int n = 0; n < N; ++n) {
-        if ((n & 63) == 0) fa_sincos_phase(l, n, T, &zi, &zr);
+      for (int n0 = n_lo; n0 < n_hi; n0 += 64) {
+        fa_sincos_phase(l, n0, T, &zi, &zr);
+        const int n1 = min(n_hi, n0 + 64);
+#pragma unroll 4
+        for (int n = n0; n < n1; ++n) {
+          const Heads wc = s_w[2 * n], ws = s_w[2 * n + 1];
 #pragma unroll
-        for (int g = 0; g < kGMax; ++g)
-          if (g < G) sc[g] = fmaf(zr, s_w[g * 2 * N + n], fmaf(zi, s_w[g * 2 * N + N + n], sc[g]));
-        float nr = zr * sr - zi * si;
-        float ni = zr * si + zi * sr;
-        zr = nr;
-        zi = ni;
+          for (int g = 0; g < GM; ++g) sc[g] = fmaf(zr, wc.v[g], fmaf(zi, ws.v[g], sc[g]));
+          const float nr = zr * sr - zi * si;
+          zi = zr * si + zi * sr;
+          zr = nr;
+        }
       }
-      for (int j = 0; j < kn_len; ++j) {
-        float kv = fa_to_float(PAGED ? kb[paged_offset(false, dpk, l, j)] : kb[(int64_t)l * k_rs + j]);
+      for (int j0 = 8 * w; j0 < kn_len; j0 += 32) {   // eight stored dims at a time
+        float kv[8];
+        if (PAGED) {
+          row8_to_float(*(const Row8<E>*)(kb + paged_offset(false, dpk, l, j0)), kv);
+        } else {
 #pragma unroll
-        for (int g = 0; g < kGMax; ++g)
-          if (g < G) sc[g] = fmaf(kv, s_qn[g * D + j], sc[g]);
+          for (int e = 0; e < 8; ++e) kv[e] = fa_to_float(kb[(int64_t)l * k_rs + min(j0 + e, kn_len - 1)]);
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const Heads qn = s_qn[j0 + e];
+#pragma unroll
+          for (int g = 0; g < GM; ++g) sc[g] = fmaf(kv[e], qn.v[g], sc[g]);
+        }
       }
     }
-    // ---- phase 2: online softmax over the tile --------------------------
+    {
+      Heads o;
 #pragma unroll
-    for (int g = 0; g < kGMax; ++g) {
-      float v = fa_wave_max(ok ? sc[g] : -INFINITY);
-      if (lane == 0) s_red[w * kGMax + g] = v;
+      for (int g = 0; g < GM; ++g) o.v[g] = sc[g];
+      s_part[w * kMidTile + lane] = o;
     }
     __syncthreads();
-    float alpha[kGMax];
+    // ---- phase 2: online softmax over the tile, head by head ----------------
 #pragma unroll
-    for (int g = 0; g < kGMax; ++g) {
-      float tm = fmaxf(fmaxf(s_red[g], s_red[kGMax + g]), fmaxf(s_red[2 * kGMax + g], s_red[3 * kGMax + g]));
-      float mn = fmaxf(m_run[g], tm);
-      alpha[g] = (m_run[g] == -INFINITY) ? 0.f : exp2f(m_run[g] - mn);
-      m_run[g] = mn;
+    for (int i = 0; i < GM / 4; ++i) {
+      const int g = w + 4 * i;
+      float x = cz[i];
+#pragma unroll
+      for (int ww = 0; ww < 4; ++ww) x += s_part[ww * kMidTile + lane].v[g];
+      const bool ok = lane < t_len && g < G;
+      const float m_new = fmaxf(m_run[i], fa_wave_max(ok ? x : -INFINITY));
+      const float p = ok ? exp2f(x - m_new) : 0.f;
+      const float alpha = m_run[i] == -INFINITY ? 0.f : exp2f(m_run[i] - m_new);
+      m_run[i] = m_new;
+      d_run[i] = d_run[i] * alpha + fa_wave_sum(p);
+      s_p[lane].v[g] = p;
+      if (lane == 0) s_alpha[g] = alpha;
     }
     __syncthreads();
+    float alpha[GM];
 #pragma unroll
-    for (int g = 0; g < kGMax; ++g) {
-      float p = (ok && g < G) ? exp2f(sc[g] - m_run[g]) : 0.f;
-      if (g < G) s_p[g * kTile + tid] = p;
-      float v = fa_wave_sum(p);
-      if (lane == 0) s_red[w * kGMax + g] = v;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int g = 0; g < kGMax; ++g)
-      d_run[g] = d_run[g] * alpha[g] + (s_red[g] + s_red[kGMax + g] + s_red[2 * kGMax + g] + s_red[3 * kGMax + g]);
-    // ---- phase 3: g[n] += sum_t p[t] e^{i theta n (l0 + t)}, thread = frequency
+    for (int g = 0; g < GM; ++g) alpha[g] = s_alpha[g];
+    // ---- phase 3: g[n] += sum_t p[t] e^{i theta n (l0 + t)} over this thread's share of the tokens
 #pragma unroll
     for (int i = 0; i < kFreqIters; ++i) {
-      const int n = tid + 256 * i;
+      const int n = n_t + 256 * i;
       if (n < N) {
 #pragma unroll
-        for (int g = 0; g < kGMax; ++g) {
+        for (int g = 0; g < GM; ++g) {
           gc[i][g] *= alpha[g];
           gs[i][g] *= alpha[g];
         }
-        float sr, si, zr, zi;
-        fa_sincos_phase(n, 1, T, &si, &sr);
-        for (int tt = 0; tt < t_len; ++tt) {
-          if ((tt & 63) == 0) fa_sincos_phase(n, l0 + tt, T, &zi, &zr);
+        const int t0 = tg * t_share, t1 = min(t_len, t0 + t_share);
+        float zr, zi;
+        fa_sincos_phase(n, l0 + t0, T, &zi, &zr);
+#pragma unroll 4
+        for (int t = t0; t < t1; ++t) {
+          const Heads p = s_p[t];
 #pragma unroll
-          for (int g = 0; g < kGMax; ++g)
-            if (g < G) {
-              float p = s_p[g * kTile + tt];
-              gc[i][g] = fmaf(p, zr, gc[i][g]);
-              gs[i][g] = fmaf(p, zi, gs[i][g]);
-            }
-          float nr = zr * sr - zi * si;
-          float ni = zr * si + zi * sr;
+          for (int g = 0; g < GM; ++g) {
+            gc[i][g] = fmaf(p.v[g], zr, gc[i][g]);
+            gs[i][g] = fmaf(p.v[g], zi, gs[i][g]);
+          }
+          const float nr = zr * fr[i] - zi * fi[i];
+          zi = zr * fi[i] + zi * fr[i];
           zr = nr;
-          zi = ni;
         }
       }
     }
-    // ---- phase 4: stored V dims, thread = (dim, tile half) ----------------
+    // ---- phase 4: stored V dims, thread = (dim, half of the tile), eight tokens at a time ----------------
 #pragma unroll
-    for (int g = 0; g < kGMax; ++g) on[g] *= alpha[g];
+    for (int g = 0; g < GM; ++g) on[g] *= alpha[g];
     if (dim < vn_len) {
-      for (int tt = half; tt < t_len; tt += 2) {
-        float vv = fa_to_float(PAGED ? vb[paged_offset(true, dpv, l0 + tt, dim)] : vb[(int64_t)(l0 + tt) * v_rs + dim]);
+      for (int t0 = half * (kMidTile / 2); t0 < min(t_len, (half + 1) * (kMidTile / 2)); t0 += 8) {
+        float vv[8];
+        if (PAGED) {   // (slots past the last row are zero, and their probabilities too)
+          row8_to_float(*(const Row8<E>*)(vb + paged_offset(true, dpv, l0 + t0, dim)), vv);
+        } else {
 #pragma unroll
-        for (int g = 0; g < kGMax; ++g)
-          if (g < G) on[g] = fmaf(s_p[g * kTile + tt], vv, on[g]);
+          for (int e = 0; e < 8; ++e) vv[e] = fa_to_float(vb[(int64_t)min(l0 + t0 + e, L_m - 1) * v_rs + dim]);
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const Heads p = s_p[t0 + e];
+#pragma unroll
+          for (int g = 0; g < GM; ++g) on[g] = fmaf(p.v[g], vv[e], on[g]);
+        }
       }
     }
-    __syncthreads();
+    __syncthreads();   // the probabilities are read; the next tile writes partial scores, then probabilities
   }
 
-  // ---- write the split's partials ---------------------------------------
-  if (half == 1 && dim < vn_len) {
+  // ---- write the split's partials (the weights are no longer needed: their place takes what has to be added up) -----
+  for (int other = 1; other < 256 / ft; ++other) {
+    if (tg == other && n_t < N)
 #pragma unroll
-    for (int g = 0; g < kGMax; ++g)
-      if (g < G) s_o[g * D + dim] = on[g];
+      for (int g = 0; g < GM; ++g) {
+        s_w[2 * n_t].v[g] = gc[0][g];
+        s_w[2 * n_t + 1].v[g] = gs[0][g];
+      }
+    __syncthreads();
+    if (tg == 0 && n_t < N)
+#pragma unroll
+      for (int g = 0; g < GM; ++g) {
+        gc[0][g] += s_w[2 * n_t].v[g];
+        gs[0][g] += s_w[2 * n_t + 1].v[g];
+      }
+    __syncthreads();
   }
+  if (half == 1)
+#pragma unroll
+    for (int g = 0; g < GM; ++g) s_qn[dim].v[g] = on[g];
   __syncthreads();
 #pragma unroll
-  for (int g = 0; g < kGMax; ++g) {
+  for (int g = 0; g < GM; ++g) {
     if (g >= G) continue;
     const int64_t r = ((int64_t)b * Hq + h * G + g) * n_split + split;
-    if (half == 0 && dim < vn_len) pon[r * D + dim] = on[g] + s_o[g * D + dim];
+    if (half == 0 && dim < vn_len) pon[r * D + dim] = on[g] + s_qn[dim].v[g];
+    if (tg == 0)
 #pragma unroll
-    for (int i = 0; i < kFreqIters; ++i) {
-      const int n = tid + 256 * i;
-      if (n < N) {
-        pg[r * 2 * N + n] = gc[i][g];
-        pg[r * 2 * N + N + n] = gs[i][g];
+      for (int i = 0; i < kFreqIters; ++i) {
+        const int n = n_t + 256 * i;
+        if (n < N) {
+          pg[r * 2 * N + n] = gc[i][g];
+          pg[r * 2 * N + N + n] = gs[i][g];
+        }
       }
-    }
-    if (tid == 0) {
-      pm[r] = m_run[g];
-      pd[r] = d_run[g];
+    if (w == (g & 3) && lane == 0) {
+      pm[r] = m_run[g / 4];
+      pd[r] = d_run[g / 4];
     }
   }
 }
+
+// dynamic LDS of the kernel above
+template <int GM>
+constexpr size_t decode_mid_lds(int N) { return ((size_t)2 * N + 128 + 5 * kMidTile + 1) * GM * sizeof(float); }
 
 // ---------------------------------------------------------------------------
 // merge: one block of 1024 threads per (b, KV head) combines, for the G query heads of that head,
@@ -1469,7 +1555,7 @@ __global__ __launch_bounds__(1024) void decode_merge_fast_kernel(const MergeRows
 
 
 // ---------------------------------------------------------------------------
-// sink + local window, vectorised (16-bit storage, head_dim 64 or 128, 16-byte aligned rows):
+// sink + local window, vectorised (head_dim 64 or 128, 16-byte aligned rows):
 // a block takes kIlFastTile rows; LPT = D/8 lanes share one row, each holding 8 dims; every wave
 // issues all of its loads first, then runs an online softmax of its own; the four waves of the
 // block are merged through LDS.
@@ -1516,21 +1602,21 @@ __device__ __forceinline__ void decode_il_fast_body(const IlArgs<E>& ia, int bx,
   const int split = bx, h = blockIdx.y, b = blockIdx.z;
   const int n_il = s0.rows + s1.rows;
   const int base = split * kIlFastTile + w * (kIlFastTile / 4);
-  uint4 kraw[ITERS], vraw[ITERS];
+  Row8<E> kraw[ITERS], vraw[ITERS];
 #pragma unroll
   for (int it = 0; it < ITERS; ++it) {
     const int i = base + it * TPW + tl;
     const int ii = i < n_il ? i : 0;
     const bool in0 = ii < s0.rows;
     const int64_t off = in0 ? (int64_t)b * s0.bs + (int64_t)ii * s0.rs : (int64_t)b * s1.bs + (int64_t)(ii - s0.rows) * s1.rs;
-    kraw[it] = *(const uint4*)((in0 ? (const E*)s0.k : (const E*)s1.k) + off + h * D + sub * 8);
-    vraw[it] = *(const uint4*)((in0 ? (const E*)s0.v : (const E*)s1.v) + off + h * D + sub * 8);
+    kraw[it] = *(const Row8<E>*)((in0 ? (const E*)s0.k : (const E*)s1.k) + off + h * D + sub * 8);
+    vraw[it] = *(const Row8<E>*)((in0 ? (const E*)s0.v : (const E*)s1.v) + off + h * D + sub * 8);
   }
   // the query slices: one unconditional 16-byte load per head (a head index past G repeats the last one)
-  uint4 qraw[GM];
+  Row8<E> qraw[GM];
 #pragma unroll
   for (int g = 0; g < GM; ++g)
-    qraw[g] = *(const uint4*)(q + ((int64_t)b * Hq + h * G + min(g, G - 1)) * D + sub * 8);
+    qraw[g] = *(const Row8<E>*)(q + ((int64_t)b * Hq + h * G + min(g, G - 1)) * D + sub * 8);
   // (the query stays packed: the scores are sums of pair products, v_dot2c, scaled once per score)
   // The wave holds only ITERS * TPW rows, so it takes one softmax block: all scores first, one maximum,
   // then the weighted sum (no running maximum, no rescaling).
@@ -1540,14 +1626,9 @@ __device__ __forceinline__ void decode_il_fast_body(const IlArgs<E>& ia, int bx,
 #pragma unroll
   for (int it = 0; it < ITERS; ++it) {
     const bool ok = base + it * TPW + tl < n_il;
-    const uint4 kr = kraw[it];
 #pragma unroll
     for (int g = 0; g < GM; ++g) {
-      float a = fa_dot2<E>(kr.x, qraw[g].x, 0.f);
-      a = fa_dot2<E>(kr.y, qraw[g].y, a);
-      a = fa_dot2<E>(kr.z, qraw[g].z, a);
-      a = fa_dot2<E>(kr.w, qraw[g].w, a);
-      a = fa_group_sum<LPT>(a) * sm_log2e;
+      const float a = fa_group_sum<LPT>(dot8(kraw[it], qraw[g])) * sm_log2e;
       sc[it][g] = (ok && g < G) ? a : -INFINITY;
       m[g] = fmaxf(m[g], sc[it][g]);
     }
@@ -1570,10 +1651,8 @@ __device__ __forceinline__ void decode_il_fast_body(const IlArgs<E>& ia, int bx,
       for (int e = 0; e < 8; ++e) o[gg][e] = 0.f;
 #pragma unroll
     for (int it = 0; it < ITERS; ++it) {
-      const E* ve = (const E*)&vraw[it];
       float vf[8];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) vf[e] = fa_to_float(ve[e]);
+      row8_to_float(vraw[it], vf);
 #pragma unroll
       for (int gg = 0; gg < 2; ++gg) {
         const int g = g0 + gg;
@@ -1640,8 +1719,11 @@ __global__ __launch_bounds__(256) void decode_il_fast_kernel(const IlArgs<E> ia)
 // The coefficient-domain query and the sink/window rows do not depend on each other and are both short,
 // latency-bound pieces of work: one launch runs them side by side (blocks [0, n_prep) prepare the query,
 // the rest attend over sink/window tiles).
+// waves per SIMD of that launch (rows of fp32 need twice the registers)
+template <typename E>
+constexpr int il_waves(int gm) { return (gm <= 4 ? 6 : 4) / (int)(sizeof(E) / 2); }
 template <typename E, int D, int GM, bool UPD>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(GM <= 4 ? 6 : 4, GM <= 4 ? 6 : 4)))
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(il_waves<E>(GM), il_waves<E>(GM))))
 void decode_prep_il_kernel(const PrepArgs<E> pa, const IlArgs<E> ia, int n_prep) {
   // one buffer for whichever piece the block runs: what a block holds in LDS decides how many run side by side
   constexpr int kLds = (int)sizeof(IlFastLds<D, GM>) > kPrepLdsBytes ? (int)sizeof(IlFastLds<D, GM>) : kPrepLdsBytes;
@@ -1798,7 +1880,7 @@ Plan make_plan(int B, int Hq, int Hkv, int D, int N, int n_il, int L_m, bool mfm
     p.n_mid_split = full_room && Hkv > 1 && Hkv <= fa_mfma::kSplitHeads ? room : largest;
     p.n_wg = p.st.first[Hkv <= fa_mfma::kSplitHeads ? Hkv : fa_mfma::kSplitHeads];
   } else {
-    const int tiles = fa_cdiv(L_m, kTile);
+    const int tiles = fa_cdiv(L_m, kMidTile);
     int want = fa_cdiv(1024, (int64_t)B * Hkv);
     if (want < 1) want = 1;
     int ns = tiles < want ? tiles : want;
@@ -1848,7 +1930,7 @@ Plan make_plan(int B, int Hq, int Hkv, int D, int N, int n_il, int L_m, bool mfm
 }
 
 bool il_fast_ok(const fa_decode_args& a) {
-  if (a.dtype == FA_FP32 || (a.D != 64 && a.D != 128)) return false;
+  if (a.D != 64 && a.D != 128) return false;
   if ((uintptr_t)a.q & 15) return false;   // query rows are read 16 bytes at a time
   for (int i = 0; i < 2; ++i) {
     if (a.il_rows[i] == 0) continue;
@@ -1992,7 +2074,7 @@ int launch_all(const fa_decode_args& a, const Plan& p, bool p_il_fast, float sm_
   Seg s1{a.k_il[1], a.v_il[1], a.il_rows[1], a.il_batch_stride[1], a.il_row_stride[1]};
   IlArgs<E> ia{(const E*)a.q, s0, s1, ilm, ild, ilo, a.Hq, a.Hkv, p.n_il_split, sm_log2e};
   // sink/window tiles ride in the query-preparation launch when both exist and the fast tile kernel applies
-  const bool fuse_il = sizeof(E) == 2 && p_il_fast && p.n_il_split > 0 && p.n_mid_split > 0;
+  const bool fuse_il = p_il_fast && p.n_il_split > 0 && p.n_mid_split > 0;
   uint16_t wg_map[fa_mfma::kFusedMaxWgs] = {};
   // (the sink/window tiles must be in front of the mid rows for the merge to run inside that launch)
   const bool fused = sizeof(E) == 2 && (fuse_il || p.n_il_split == 0) && fused_merge_plan(a, p, wg_map, st);
@@ -2023,19 +2105,17 @@ int launch_all(const fa_decode_args& a, const Plan& p, bool p_il_fast, float sm_
                    a.Ck > 0 ? (const E*)a.upd_k_row : nullptr, a.upd_batch_stride, a.upd_phase, a.upd_T};
     const int n_prep = fa_cdiv(2 * a.N, kPrepRows);
     if (fuse_il) {
-      if constexpr (sizeof(E) == 2) {
-        dim3 grid(n_prep + p.n_il_split, a.Hkv, a.B);
-        if (pa.upd_row) {
-          if (a.D == 128 && G <= 4) decode_prep_il_kernel<E, 128, 4, true><<<grid, 256, 0, st>>>(pa, ia, n_prep);
-          else if (a.D == 128) decode_prep_il_kernel<E, 128, kGMax, true><<<grid, 256, 0, st>>>(pa, ia, n_prep);
-          else if (G <= 4) decode_prep_il_kernel<E, 64, 4, true><<<grid, 256, 0, st>>>(pa, ia, n_prep);
-          else decode_prep_il_kernel<E, 64, kGMax, true><<<grid, 256, 0, st>>>(pa, ia, n_prep);
-        } else {
-          if (a.D == 128 && G <= 4) decode_prep_il_kernel<E, 128, 4, false><<<grid, 256, 0, st>>>(pa, ia, n_prep);
-          else if (a.D == 128) decode_prep_il_kernel<E, 128, kGMax, false><<<grid, 256, 0, st>>>(pa, ia, n_prep);
-          else if (G <= 4) decode_prep_il_kernel<E, 64, 4, false><<<grid, 256, 0, st>>>(pa, ia, n_prep);
-          else decode_prep_il_kernel<E, 64, kGMax, false><<<grid, 256, 0, st>>>(pa, ia, n_prep);
-        }
+      dim3 grid(n_prep + p.n_il_split, a.Hkv, a.B);
+      if (pa.upd_row) {
+        if (a.D == 128 && G <= 4) decode_prep_il_kernel<E, 128, 4, true><<<grid, 256, 0, st>>>(pa, ia, n_prep);
+        else if (a.D == 128) decode_prep_il_kernel<E, 128, kGMax, true><<<grid, 256, 0, st>>>(pa, ia, n_prep);
+        else if (G <= 4) decode_prep_il_kernel<E, 64, 4, true><<<grid, 256, 0, st>>>(pa, ia, n_prep);
+        else decode_prep_il_kernel<E, 64, kGMax, true><<<grid, 256, 0, st>>>(pa, ia, n_prep);
+      } else {
+        if (a.D == 128 && G <= 4) decode_prep_il_kernel<E, 128, 4, false><<<grid, 256, 0, st>>>(pa, ia, n_prep);
+        else if (a.D == 128) decode_prep_il_kernel<E, 128, kGMax, false><<<grid, 256, 0, st>>>(pa, ia, n_prep);
+        else if (G <= 4) decode_prep_il_kernel<E, 64, 4, false><<<grid, 256, 0, st>>>(pa, ia, n_prep);
+        else decode_prep_il_kernel<E, 64, kGMax, false><<<grid, 256, 0, st>>>(pa, ia, n_prep);
       }
     } else if (pa.upd_row) {
       decode_prep_kernel<E, true><<<dim3(n_prep, a.Hkv, a.B), 256, 0, st>>>(pa);
@@ -2084,25 +2164,28 @@ int launch_all(const fa_decode_args& a, const Plan& p, bool p_il_fast, float sm_
         launch_mid_rows<E>(mp, MidLaunch{p.n_wg, p.n_groups, KS, wide, NSL > 4, fused, sub}, st);
       }
     } else {
-      size_t lds = ((size_t)G * 2 * a.N + 2 * (size_t)G * a.D + (size_t)G * kTile + 4 * kGMax) * sizeof(float);
       const bool paged = a.mid_layout == FA_MID_PAGED;
-      const void* fn = paged ? reinterpret_cast<const void*>(&decode_mid_kernel<E, true>)
-                             : reinterpret_cast<const void*>(&decode_mid_kernel<E, false>);
-      if (lds > 64 * 1024) {
-        hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        FA_REQUIRE(e == hipSuccess, FA_ERR_UNSUPPORTED, "fa_decode_attn: %zu bytes of LDS refused", lds);
-      }
-      dim3 grid(p.n_mid_split, a.Hkv, a.B);
-      if (paged)
-        decode_mid_kernel<E, true><<<grid, 256, lds, st>>>(
-            (const E*)a.q, (const E*)a.k_mn, a.k_mn_batch_stride, 0, (const E*)a.v_mn, a.v_mn_batch_stride, 0,
-            a.mid_cap_pages, a.k_pad_h_list, a.v_pad_h_list, W, c0, a.kn_list, a.kn_h_list, a.vn_h_list, mm, md, mg,
-            mon, a.Hq, a.Hkv, a.D, a.N, a.L_m, a.T, p.n_mid_split, p.tiles_per_split, sm_log2e);
-      else
-        decode_mid_kernel<E, false><<<grid, 256, lds, st>>>(
-            (const E*)a.q, (const E*)a.k_mn, a.k_mn_batch_stride, a.k_mn_row_stride, (const E*)a.v_mn,
-            a.v_mn_batch_stride, a.v_mn_row_stride, 0, nullptr, nullptr, W, c0, a.kn_list, a.kn_h_list, a.vn_h_list,
-            mm, md, mg, mon, a.Hq, a.Hkv, a.D, a.N, a.L_m, a.T, p.n_mid_split, p.tiles_per_split, sm_log2e);
+      auto go = [&](auto paged_tag, auto gm_tag) -> int {
+        constexpr bool PG = decltype(paged_tag)::value;
+        constexpr int GM = decltype(gm_tag)::value;
+        const size_t lds = decode_mid_lds<GM>(a.N);
+        if (lds > 64 * 1024) {
+          hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&decode_mid_kernel<E, PG, GM>),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+          FA_REQUIRE(e == hipSuccess, FA_ERR_UNSUPPORTED, "fa_decode_attn: %zu bytes of LDS refused", lds);
+        }
+        decode_mid_kernel<E, PG, GM><<<dim3(p.n_mid_split, a.Hkv, a.B), 256, lds, st>>>(
+            (const E*)a.q, (const E*)a.k_mn, a.k_mn_batch_stride, PG ? 0 : a.k_mn_row_stride, (const E*)a.v_mn,
+            a.v_mn_batch_stride, PG ? 0 : a.v_mn_row_stride, PG ? a.mid_cap_pages : 0, PG ? a.k_pad_h_list : nullptr,
+            PG ? a.v_pad_h_list : nullptr, W, c0, a.kn_list, a.kn_h_list, a.vn_h_list, mm, md, mg, mon, a.Hq, a.Hkv, a.D, a.N,
+            a.L_m, a.T, p.n_mid_split, p.tiles_per_split, sm_log2e);
+        return FA_OK;
+      };
+      using G4 = std::integral_constant<int, 4>;
+      using G8 = std::integral_constant<int, kGMax>;
+      const int rc = paged ? (G <= 4 ? go(std::true_type{}, G4{}) : go(std::true_type{}, G8{}))
+                           : (G <= 4 ? go(std::false_type{}, G4{}) : go(std::false_type{}, G8{}));
+      if (rc != FA_OK) return rc;
     }
   }
   if (ev && (p.n_mid_split == 0 || p.path != Path::Mfma)) hipEventRecord(ev[1], st);
@@ -2116,17 +2199,12 @@ int launch_all(const fa_decode_args& a, const Plan& p, bool p_il_fast, float sm_
   }
   if (p.n_il_split > 0 && !fuse_il) {
     dim3 grid(p.n_il_split, a.Hkv, a.B);
-    bool launched = false;
-    if constexpr (sizeof(E) == 2) {
-      if (p_il_fast) {
-        launched = true;
-        if (a.D == 128 && G <= 4) decode_il_fast_kernel<E, 128, 4><<<grid, 256, 0, st>>>(ia);
-        else if (a.D == 128) decode_il_fast_kernel<E, 128, kGMax><<<grid, 256, 0, st>>>(ia);
-        else if (G <= 4) decode_il_fast_kernel<E, 64, 4><<<grid, 256, 0, st>>>(ia);
-        else decode_il_fast_kernel<E, 64, kGMax><<<grid, 256, 0, st>>>(ia);
-      }
-    }
-    if (!launched) {
+    if (p_il_fast) {
+      if (a.D == 128 && G <= 4) decode_il_fast_kernel<E, 128, 4><<<grid, 256, 0, st>>>(ia);
+      else if (a.D == 128) decode_il_fast_kernel<E, 128, kGMax><<<grid, 256, 0, st>>>(ia);
+      else if (G <= 4) decode_il_fast_kernel<E, 64, 4><<<grid, 256, 0, st>>>(ia);
+      else decode_il_fast_kernel<E, 64, kGMax><<<grid, 256, 0, st>>>(ia);
+    } else {
       size_t lds = (2 * (size_t)G * a.D + (size_t)G * kTile + 4 * kGMax) * sizeof(float);
       decode_il_kernel<E><<<grid, 256, lds, st>>>((const E*)a.q, s0, s1, ilm, ild, ilo, a.Hq, a.Hkv, a.D, p.n_il_split, sm_log2e);
     }

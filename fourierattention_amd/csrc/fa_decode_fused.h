@@ -43,8 +43,6 @@ template <>
 __device__ __forceinline__ float fa_dot2<f16_t>(unsigned a, unsigned b, float c) {
   return __builtin_amdgcn_fdot2(__builtin_bit_cast(fa_f16x2, a), __builtin_bit_cast(fa_f16x2, b), c, false);
 }
-template <>
-__device__ __forceinline__ float fa_dot2<float>(unsigned, unsigned, float c) { return c; }   // never run: 16-bit rows only
 
 namespace fa_mfma {
 

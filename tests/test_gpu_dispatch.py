@@ -24,3 +24,38 @@ def test_reconstruction_statistics_by_shares_of_column_blocks(B, L, C, N, T):
     size = (ref[0].abs() + ref[1].abs()).cpu().numpy()
     for a, b in zip(got, ref):
         assert np.max((a - b).abs().cpu().numpy() / size) <= 2e-3
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("B,Hq,Hkv,D,n_il,L,N,k_counts,v_counts", [
+    (1, 3, 1, 128, 5, 1, 5, [127], [1]),                        # one mid row; one stored K dim, one compressed V dim
+    (2, 8, 1, 64, 63, 64, 16, [3], [63]),                       # one whole tile, eight heads, sixteen frequencies
+    (1, 6, 2, 128, 65, 65, 100, [0, 57], [128, 0]),             # a tile and a row; a head that stores nothing and one that stores all
+    (1, 10, 2, 80, 10, 191, 129, [33, 80], [80, 40]),           # head dims without the vectorised window kernel, 129 frequencies
+    (2, 4, 2, 128, 130, 700, 300, [64, 64], [96, 17]),          # two rounds of frequencies per thread, several tiles per split
+    (1, 7, 1, 128, 64, 300, 600, [100], [31]),                  # three rounds, seven heads
+])
+def test_any_shape_decode_kernels(dtype, B, Hq, Hkv, D, n_il, L, N, k_counts, v_counts):
+    """The any-shape kernels on token-major and on paged mid rows against the float64 oracle.  Bound: the operands reach
+    the kernels exactly and the arithmetic is single precision, 2e-4 on outputs of order one as for the other
+    single-precision comparisons."""
+    from fourierattention_amd import ops
+    from fourierattention_amd.midstore import MidStore
+    from oracle import fourier_oracle as fo
+    from tests import helpers as H
+    case = H.attn_case(11, B, Hq, Hkv, D, n_il, L, N, 2 * L + 7, k_counts, v_counts, dtype)
+    want = fo.fourier_attn(**case)
+    g = H.attn_case_gpu(case, dtype)
+    lists = tuple(ops.as_i32(g[n]) for n in ("kc_list", "kc_h_list", "kn_list", "kn_h_list", "vc_list", "vc_h_list", "vn_list", "vn_h_list"))
+    f = lambda t: t.float().contiguous()
+    stats = [(f(g[f"avg_{t}_u"]), f(g[f"avg_{t}_d"]), f(g[f"scale_{t}"])) for t in "kv"]
+    stores = []
+    for t, n_h, is_v in ((g["k_mn"], lists[3], False), (g["v_mn"], lists[7], True)):
+        ident = torch.arange(t.shape[2], dtype=torch.int32, device="cuda")
+        st = MidStore(B, ident, n_h, n_h.tolist(), Hkv, D, L, dtype, "cuda", is_v)
+        st.pack(t, 0, L)
+        stores.append(st)
+    for k_mn, v_mn in ((g["k_mn"], g["v_mn"]), stores):
+        got = ops.decode_attn_raw(g["q"], [(g["k_il"], g["v_il"])], g["k_mc"], g["v_mc"], k_mn, v_mn, *stats, lists, Hq, Hkv, L,
+                                  case["T"], force_generic=True)
+        assert np.max(np.abs(got.cpu().numpy().astype(np.float64).reshape(want.shape) - want)) <= 2e-4
