@@ -164,6 +164,26 @@ def load():
     return lib
 
 
+_host = None
+
+
+def load_host():
+    """The CPython module that takes tensors and calls the library (``csrc/host/fa_host.cpp``), loaded once."""
+    global _host
+    if _host is None:
+        load()
+        import torch  # noqa: F401  (its libraries are the ones the module was linked against)
+        try:
+            from . import _fa_host
+        except ImportError as exc:
+            raise ImportError(f"{PKG_DIR}/_fa_host.so is missing or does not load ({exc}); run "
+                              "`python -m fourierattention_amd.build`") from exc
+        from . import ops
+        _fa_host.init(ops._raw_stream, check, ops.workspace)
+        _host = _fa_host
+    return _host
+
+
 def check(code: int) -> None:
     if code != 0:
         raise FourierAttnError(code, load().fa_last_error_string().decode("utf-8", "replace"))

@@ -61,6 +61,10 @@ def fourier_attention(query_states: torch.Tensor, key_states: torch.Tensor, valu
     Returns ``(B, q_len, Hq*D)`` in the query dtype (modeling_llama_fourier.py:618-663)."""
     bsz, _, q_len, head_dim = query_states.shape
     k_parts, v_parts = past_key_value.update(key_states, value_states, layer_idx, cache_kwargs)
+    if isinstance(k_parts, CacheParts):
+        # (B, Hq, 1, D) dense, rounded by the last kernel: the rows are those of (B, 1, Hq*D)
+        return past_key_value.decode_attention(query_states, layer_idx, num_heads, num_key_value_heads,
+                                               out_dtype=query_states.dtype).view(bsz, q_len, num_heads * head_dim)
     if k_parts["k_init"] is None and k_parts["k_compressed"] is None and k_parts["k_uncompressed"] is None:
         if q_len == 1 and query_states.is_cuda:
             o = past_key_value.decode_attention(query_states, layer_idx, num_heads, num_key_value_heads,
@@ -68,9 +72,6 @@ def fourier_attention(query_states: torch.Tensor, key_states: torch.Tensor, valu
             o = o.transpose(1, 2)
         else:
             o = _exact_attention(query_states, k_parts["k_local"], v_parts["v_local"], num_key_value_heads, head_dim)
-    elif isinstance(k_parts, CacheParts):
-        o = past_key_value.decode_attention(query_states, layer_idx, num_heads, num_key_value_heads,
-                                            out_dtype=query_states.dtype).transpose(1, 2)
     else:  # plain tensors in the reference's layout
         pkv = past_key_value
         o = ops.triton_fourier_attn(

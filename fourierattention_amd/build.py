@@ -16,6 +16,7 @@ PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(PKG_DIR, "csrc")
 LIB_NAME = "libfourier_attn_hip.so"
 LIB_PATH = os.path.join(PKG_DIR, LIB_NAME)
+HOST_PATH = os.path.join(PKG_DIR, "_fa_host.so")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
@@ -232,9 +233,27 @@ def build(verbose: bool = True, extra_flags=()) -> str:
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"link failed:\n{r.stdout}\n{r.stderr}")
+    build_host()
     if verbose:
         print(f"built {LIB_PATH} from {len(srcs)} sources")
     return LIB_PATH
+
+
+def build_host() -> str:
+    """The CPython module in front of the library (``csrc/host/fa_host.cpp``): host code only, against the headers of
+    the installed torch and linked to the library beside it."""
+    import sysconfig
+    import torch
+    root = os.path.dirname(torch.__file__)
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           f"-I{root}/include", f"-I{root}/include/torch/csrc/api/include", f"-I{sysconfig.get_paths()['include']}",
+           os.path.join(CSRC, "host", "fa_host.cpp"), "-o", HOST_PATH, f"-L{root}/lib", "-ltorch_python", "-ltorch_cpu",
+           "-lc10", f"-L{PKG_DIR}", f"-l:{LIB_NAME}", "-Wl,-rpath,$ORIGIN"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"g++ failed for the host module:\n{r.stdout}\n{r.stderr}")
+    return HOST_PATH
 
 
 if __name__ == "__main__":

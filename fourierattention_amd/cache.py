@@ -281,10 +281,9 @@ class DynamicCache(Cache):
         return [(layer.k.ring[:, : layer.n_local, :], layer.v.ring[:, : layer.n_local, :])]
 
     def _il_segments(self, layer: _Layer):
-        """Sink + window of a compressed layer as two views of the one buffer: the rows before and the rows
-        after the spare window slot."""
-        cut = self.numinittokens + layer.spare
-        return [(layer.k.il[:, :cut, :], layer.v.il[:, :cut, :]), (layer.k.il[:, cut + 1:, :], layer.v.il[:, cut + 1:, :])]
+        """Sink + window of a compressed layer: the one buffer of K and of V and the row of the spare window slot, which
+        separates the rows in front of it from those behind it."""
+        return (layer.k.il, layer.v.il, self.numinittokens + layer.spare)
 
     def _compress_tensor(self, t: _Tensor, states: torch.Tensor, c32: torch.Tensor, ch32: torch.Tensor, n32: torch.Tensor,
                          nh32: torch.Tensor, nh_host, is_v: bool, L: int, fft_rows: int, n_f: int):
@@ -323,12 +322,15 @@ class DynamicCache(Cache):
         ``*_compressed`` and ``*_uncompressed`` entries are ``None`` (exact attention over
         ``*_local``); otherwise ``CacheParts`` views of the four parts."""
         bsz, heads, q_len, head_dim = key_states.shape
-        self.heads, self.head_dim = heads, head_dim
-        step = self._book.step(layer_idx, bsz, q_len)
-        self._seen_tokens = self._book.seen_tokens
-        self.maxtokens = self._book.maxtokens
-        if self._book.prefilllen is not None:
-            self.prefilllen = self._book.prefilllen
+        book = self._book
+        step = book.step(layer_idx, bsz, q_len)
+        # (plain attributes, written past torch.nn.Module's own attribute handling: this runs once per layer and token)
+        own = self.__dict__
+        own["heads"], own["head_dim"], own["_seen_tokens"], own["maxtokens"] = heads, head_dim, book.seen_tokens, book.maxtokens
+        if book.prefilllen is not None:
+            own["prefilllen"] = book.prefilllen
+        if step.action is Action.STREAM:
+            return self._stream(key_states, value_states, layer_idx, step)
         k = key_states.permute(0, 2, 1, 3).reshape(bsz, q_len, heads * head_dim)
         v = value_states.permute(0, 2, 1, 3).reshape(bsz, q_len, heads * head_dim)
         layer = self._layers[layer_idx]
@@ -411,25 +413,31 @@ class DynamicCache(Cache):
                 "this call lands in the reference's late-compression branch (cache_utils_fourier.py:688-729), "
                 "which appends a new layer entry instead of updating this one; its result is undefined")
 
-        # ---- streaming: evict the oldest window row, then overwrite its slot with the new token
+    def _stream(self, key_states: torch.Tensor, value_states: torch.Tensor, layer_idx: int, step):
+        """One more token for a compressed layer: the oldest window row is evicted, then the spare slot takes the new
+        token."""
+        layer = self._layers[layer_idx]
+        self._settle_coefficients(layer_idx)        # the row they are owed sits in the window slot written next
         layer.version += 1
-        self.curr_tokennum[layer_idx] = lb.curr_tokennum
-        p = step.phase
+        self.curr_tokennum[layer_idx] = self._book.layers[layer_idx].curr_tokennum
+        bsz, heads, _, head_dim = key_states.shape
+        if not (key_states.stride(3) == 1 and key_states.stride(1) == head_dim and key_states.stride() == value_states.stride()):
+            key_states, value_states = (t.permute(0, 2, 1, 3).reshape(bsz, heads * head_dim) for t in (key_states, value_states))
         l32 = self._lists32[layer_idx]
-        slots = self.maxlocallen + 1
+        k, v = layer.k, layer.v
         sp = layer.spare
-        oldest = (sp + 1) % slots
-        for t in (layer.k, layer.v):
+        oldest = (sp + 1) % (self.maxlocallen + 1)
+        for t in (k, v):
             if layer.n_mid >= t.mid.cap_tokens:
                 t.mid.grow(layer.n_mid, 2 * t.mid.cap_tokens)
         # one launch: coefficients and page store take the oldest row, the new token takes the spare slot.  The
         # attention that follows streams the coefficients anyway: where it can, it is left to apply their rank-1
         # update on the way (the evicted row stays in its window slot until the next update of the layer writes there)
-        defer = bool(self.defer_coef_update and k.is_cuda and not torch.cuda.is_current_stream_capturing())
-        ops.stream_update(k[:, 0, :], v[:, 0, :], layer.k.ring, layer.v.ring, oldest, sp, layer.k.coef, layer.v.coef,
-                          l32[0], l32[4], p, self._book.t_c, layer.k.mid, layer.v.mid, layer.n_mid, skip_coef=defer)
+        defer = bool(self.defer_coef_update and key_states.is_cuda and not torch.cuda.is_current_stream_capturing())
+        ops.stream_update(key_states, value_states, k.ring, v.ring, oldest, sp, k.coef, v.coef, l32[0], l32[4], step.phase,
+                          self._book.t_c, k.mid, v.mid, layer.n_mid, skip_coef=defer)
         if defer:
-            layer.owed = (oldest, int(p), int(self._book.t_c))
+            layer.owed = (oldest, int(step.phase), int(self._book.t_c))
         layer.n_mid += 1
         layer.spare = oldest
         kview, vview = CacheParts(self, layer_idx, "k"), CacheParts(self, layer_idx, "v")
@@ -478,8 +486,10 @@ class DynamicCache(Cache):
         ``out_dtype = query_states.dtype`` the result comes back rounded to that type (the ``.to(dtype)`` of
         modeling_llama_fourier.py:663 done by the last kernel)."""
         layer = self._layers[layer_idx]
-        B, Hq, q_len, D = query_states.shape
-        q = query_states.transpose(1, 2).reshape(B, q_len, Hq * D).contiguous()
+        q = query_states
+        if q.shape[2] != 1 or not q.is_contiguous():
+            B, Hq, q_len, D = q.shape
+            q = q.transpose(1, 2).reshape(B, q_len, Hq * D).contiguous()
         l32 = self._lists32[layer_idx]
         if layer.window_only:
             return ops.decode_attn_raw(q, self._window_segments(layer), None, None, None, None, None, None, l32, num_heads,

@@ -1,0 +1,432 @@
+// The host side of the calls a decode step makes, as a CPython module on torch tensors (fourierattention_amd._fa_host).
+//
+// A decode step of one layer is three launches of a few microseconds each; filling the argument blocks of the C ABI
+// field by field from Python took longer than the launches (53 us of host work per layer for 35 us of kernels at 2600
+// tokens).  The functions below take the tensors themselves on every call, check them, fill the argument block and
+// launch on the caller's stream; they keep nothing between calls.
+#include <Python.h>
+
+#include <ATen/ATen.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include <vector>
+
+#include "../../../include/fourier_attn_hip.h"
+
+namespace {
+
+PyObject* g_stream_fn = nullptr;      // device index -> raw handle of torch's current stream
+PyObject* g_check_fn = nullptr;       // status -> raises the package's exception
+PyObject* g_workspace_fn = nullptr;   // (device, bytes, tag) -> uint8 tensor of at least that size
+
+// interned attribute names of a page store
+PyObject *s_data, *s_cap_pages, *s_batch_stride, *s_pad_h32, *s_max_pad, *s_pad_h_host, *s_n_list32, *s_n_h32, *s_Cn, *s_Hkv, *s_decode;
+
+struct PyError {};   // a Python exception is set
+
+[[noreturn]] void fail(PyObject* type, const char* msg) {
+  PyErr_SetString(type, msg);
+  throw PyError{};
+}
+#define CHECK(cond, msg) do { if (!(cond)) fail(PyExc_AssertionError, msg); } while (0)
+
+// owns one reference
+struct Ref {
+  PyObject* p;
+  explicit Ref(PyObject* o) : p(o) { if (!o) throw PyError{}; }
+  ~Ref() { Py_DECREF(p); }
+  Ref(const Ref&) = delete;
+};
+
+const at::Tensor& tensor(PyObject* o, const char* what) {
+  if (!THPVariable_Check(o)) {
+    PyErr_Format(PyExc_TypeError, "%s must be a tensor", what);
+    throw PyError{};
+  }
+  return THPVariable_Unpack(o);
+}
+const at::Tensor& gpu_tensor(PyObject* o, const char* what) {
+  const at::Tensor& t = tensor(o, what);
+  if (!t.is_cuda()) {
+    PyErr_Format(PyExc_RuntimeError, "%s must be a GPU tensor: the HIP kernels are the only implementation", what);
+    throw PyError{};
+  }
+  return t;
+}
+int64_t integer(PyObject* o) {
+  const long long v = PyLong_AsLongLong(o);
+  if (v == -1 && PyErr_Occurred()) throw PyError{};
+  return v;
+}
+double real(PyObject* o) {
+  const double v = PyFloat_AsDouble(o);
+  if (v == -1.0 && PyErr_Occurred()) throw PyError{};
+  return v;
+}
+bool truth(PyObject* o) {
+  const int v = PyObject_IsTrue(o);
+  if (v < 0) throw PyError{};
+  return v != 0;
+}
+int64_t int_attr(PyObject* o, PyObject* name) { return integer(Ref(PyObject_GetAttr(o, name)).p); }
+// (the store keeps its own reference to the tensor: it outlives the call)
+const at::Tensor& tensor_attr(PyObject* o, PyObject* name, const char* what) { return tensor(Ref(PyObject_GetAttr(o, name)).p, what); }
+
+int dtype_code(const at::Tensor& t) {
+  switch (t.scalar_type()) {
+    case at::kBFloat16: return FA_BF16;
+    case at::kHalf: return FA_FP16;
+    case at::kFloat: return FA_FP32;
+    default: fail(PyExc_TypeError, "unsupported dtype; expected bfloat16, float16 or float32");
+  }
+}
+template <typename T = void>
+T* ptr(const at::Tensor& t) { return t.numel() == 0 ? nullptr : static_cast<T*>(t.data_ptr()); }
+
+fa_stream_t stream_of(const at::Tensor& t) {
+  Ref idx(PyLong_FromLong(t.device().index()));
+  Ref s(PyObject_CallOneArg(g_stream_fn, idx.p));
+  return reinterpret_cast<fa_stream_t>(PyLong_AsVoidPtr(s.p));
+}
+void check_status(int rc) {
+  if (rc == FA_OK) return;
+  Ref code(PyLong_FromLong(rc));
+  Ref none(PyObject_CallOneArg(g_check_fn, code.p));
+  fail(PyExc_RuntimeError, "a HIP call failed");
+}
+
+#define FA_BEGIN HANDLE_TH_ERRORS try {
+#define FA_END } catch (const PyError&) { return nullptr; } END_HANDLE_TH_ERRORS
+
+// (B, width) rows, or the one new token (B, heads, 1, D) of a decode step whose heads lie side by side
+void token_rows(const at::Tensor& t, int64_t& batch, int64_t& width, int64_t& batch_stride) {
+  batch = t.size(0);
+  batch_stride = t.stride(0);
+  if (t.dim() == 2) {
+    CHECK(t.stride(1) == 1, "rows must be contiguous");
+    width = t.size(1);
+  } else {
+    CHECK(t.dim() == 4 && t.size(2) == 1 && t.stride(3) == 1 && t.stride(1) == t.size(3), "the heads of a token must lie side by side");
+    width = t.size(1) * t.size(3);
+  }
+}
+
+// stream_update(k_new, v_new, k_ring, v_ring, evict_slot, write_slot, k_coef, v_coef, kc_list, vc_list, phase, T,
+//               k_mid, v_mid, mid_pos, skip_coef)
+PyObject* stream_update(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  FA_BEGIN
+  CHECK(n == 16, "stream_update takes 16 arguments");
+  const at::Tensor &k_new = tensor(a[0], "k_new"), &v_new = tensor(a[1], "v_new");
+  const at::Tensor &k_ring = gpu_tensor(a[2], "k_ring"), &v_ring = gpu_tensor(a[3], "v_ring");
+  const at::Tensor &k_coef = tensor(a[6], "k_coef"), &v_coef = tensor(a[7], "v_coef");
+  const at::Tensor &kc = tensor(a[8], "kc_list"), &vc = tensor(a[9], "vc_list");
+  PyObject *k_mid = a[12], *v_mid = a[13];
+  fa_stream_args s{};
+  int64_t B, width, vB, v_width, v_stride;
+  token_rows(k_new, B, width, s.new_batch_stride);
+  token_rows(v_new, vB, v_width, v_stride);
+  CHECK(vB == B && v_width == width && v_stride == s.new_batch_stride, "k_new and v_new must share shape and strides");
+  CHECK(k_ring.dim() == 3 && k_ring.stride(2) == 1 && v_ring.strides() == k_ring.strides() && v_ring.sizes() == k_ring.sizes() &&
+        k_ring.size(0) == B && k_ring.size(2) == width, "k_ring and v_ring must share shape and strides");
+  CHECK(k_new.scalar_type() == k_ring.scalar_type() && v_new.scalar_type() == k_ring.scalar_type() && k_new.is_cuda() && v_new.is_cuda(),
+        "the new token must have the type of the window and be on the GPU");
+  CHECK(k_coef.scalar_type() == at::kFloat && v_coef.scalar_type() == at::kFloat && kc.scalar_type() == at::kInt && vc.scalar_type() == at::kInt,
+        "coefficients are float32, column lists int32");
+  s.k_new = k_new.data_ptr(); s.v_new = v_new.data_ptr();
+  s.k_ring = k_ring.data_ptr(); s.v_ring = v_ring.data_ptr();
+  s.ring_batch_stride = k_ring.stride(0); s.ring_row_stride = k_ring.stride(1);
+  s.evict_slot = (int32_t)integer(a[4]); s.write_slot = (int32_t)integer(a[5]);
+  CHECK(s.evict_slot != s.write_slot && s.evict_slot < k_ring.size(1) && s.write_slot < k_ring.size(1), "window slots");
+  s.k_coef = ptr<float>(k_coef); s.v_coef = ptr<float>(v_coef);
+  s.kc_list = ptr<int32_t>(kc); s.vc_list = ptr<int32_t>(vc);
+  s.Ck = (int32_t)kc.numel(); s.Cv = (int32_t)vc.numel();
+  s.N = (int32_t)(k_coef.size(1) / 2); s.phase = integer(a[10]); s.T = (int32_t)integer(a[11]);
+  s.k_mid = tensor_attr(k_mid, s_data, "k_mid.data").data_ptr(); s.v_mid = tensor_attr(v_mid, s_data, "v_mid.data").data_ptr();
+  s.k_mid_batch_stride = int_attr(k_mid, s_batch_stride); s.v_mid_batch_stride = int_attr(v_mid, s_batch_stride);
+  s.cap_pages = (int32_t)int_attr(k_mid, s_cap_pages); s.mid_pos = integer(a[14]);
+  CHECK(s.cap_pages == int_attr(v_mid, s_cap_pages), "the page stores of K and V must have the same capacity");
+  s.kn_list = ptr<int32_t>(tensor_attr(k_mid, s_n_list32, "n_list32")); s.vn_list = ptr<int32_t>(tensor_attr(v_mid, s_n_list32, "n_list32"));
+  s.kn_h_list = ptr<int32_t>(tensor_attr(k_mid, s_n_h32, "n_h32")); s.vn_h_list = ptr<int32_t>(tensor_attr(v_mid, s_n_h32, "n_h32"));
+  s.k_pad_h_list = ptr<int32_t>(tensor_attr(k_mid, s_pad_h32, "pad_h32")); s.v_pad_h_list = ptr<int32_t>(tensor_attr(v_mid, s_pad_h32, "pad_h32"));
+  s.Cnk = (int32_t)int_attr(k_mid, s_Cn); s.Cnv = (int32_t)int_attr(v_mid, s_Cn);
+  s.B = (int32_t)B; s.Hkv = (int32_t)int_attr(k_mid, s_Hkv); s.width = (int32_t)width; s.dtype = dtype_code(k_ring);
+  s.skip_coef = truth(a[15]);
+  check_status(fa_stream_update(&s, stream_of(k_ring)));
+  Py_RETURN_NONE;
+  FA_END
+}
+
+// one (rows, Hkv*D) segment of sink / window rows
+void il_segment(fa_decode_args& d, int i, const at::Tensor& k, const at::Tensor& v, int64_t row0, int64_t rows, at::ScalarType dt) {
+  if (rows <= 0) return;
+  CHECK(k.dim() == 3 && k.stride(2) == 1 && v.strides() == k.strides() && v.sizes() == k.sizes(), "sink/window rows of K and V must share shape and strides");
+  CHECK(k.scalar_type() == dt && v.scalar_type() == dt && k.is_cuda() && v.is_cuda(), "sink/window rows must have the type of q and be on the GPU");
+  const int64_t off = row0 * k.stride(1) * (int64_t)k.element_size();
+  d.k_il[i] = (const char*)k.data_ptr() + off; d.v_il[i] = (const char*)v.data_ptr() + off;
+  d.il_rows[i] = (int32_t)rows; d.il_batch_stride[i] = k.stride(0); d.il_row_stride[i] = k.stride(1);
+}
+
+const float* stat(PyObject* tuple, Py_ssize_t i) {
+  const at::Tensor& t = tensor(PyTuple_GET_ITEM(tuple, i), "statistics");
+  CHECK(t.scalar_type() == at::kFloat && t.is_contiguous(), "statistics must be contiguous float32");
+  return ptr<const float>(t);
+}
+
+// decode_attn(q, il, k_mc, v_mc, k_mn, v_mn, stats_k, stats_v, lists, Hq, Hkv, L_m, T, sm_scale, out, cast, tables,
+//             force_generic, balance_heads, no_fuse, pending, no_alloc, timings) -> out
+// q (B, 1, Hq*D) or (B, Hq, 1, D), contiguous.  il: a sequence of up to two (k, v) pairs of row views, or (k, v, r): the
+// rows of one buffer in front of and behind row r.
+PyObject* decode_attn(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  FA_BEGIN
+  CHECK(n == 23, "decode_attn takes 23 arguments");
+  const at::Tensor& q = gpu_tensor(a[0], "q");
+  fa_decode_args d{};
+  d.Hq = (int32_t)integer(a[9]); d.Hkv = (int32_t)integer(a[10]);
+  CHECK(q.is_contiguous() && (q.dim() == 3 || q.dim() == 4) && d.Hq > 0, "q must be contiguous, (B, 1, Hq*D) or (B, Hq, 1, D)");
+  const at::ScalarType dt = q.scalar_type();
+  d.B = (int32_t)q.size(0);
+  d.q_len = (int32_t)(q.dim() == 3 ? q.size(1) : q.size(2));
+  d.D = (int32_t)(q.dim() == 3 ? q.size(2) / d.Hq : q.size(3));
+  CHECK(q.dim() == 3 || q.size(1) == d.Hq, "q has another number of heads");
+  d.q = q.data_ptr();
+  d.dtype = dtype_code(q);
+  if (PyTuple_Check(a[1]) && PyTuple_GET_SIZE(a[1]) == 3) {
+    const at::Tensor &k = tensor(PyTuple_GET_ITEM(a[1], 0), "k"), &v = tensor(PyTuple_GET_ITEM(a[1], 1), "v");
+    const int64_t cut = integer(PyTuple_GET_ITEM(a[1], 2));
+    CHECK(k.dim() == 3 && cut >= 0 && cut < k.size(1), "row to leave out");
+    il_segment(d, 0, k, v, 0, cut, dt);
+    il_segment(d, 1, k, v, cut + 1, k.size(1) - cut - 1, dt);
+  } else {
+    Ref seq(PySequence_Fast(a[1], "il: (k, v) pairs"));
+    for (Py_ssize_t i = 0; i < 2 && i < PySequence_Fast_GET_SIZE(seq.p); ++i) {
+      PyObject* pair = PySequence_Fast_GET_ITEM(seq.p, i);
+      if (pair == Py_None) continue;
+      CHECK(PyTuple_Check(pair) && PyTuple_GET_SIZE(pair) == 2, "il: (k, v) pairs");
+      const at::Tensor& k = tensor(PyTuple_GET_ITEM(pair, 0), "k");
+      il_segment(d, (int)i, k, tensor(PyTuple_GET_ITEM(pair, 1), "v"), 0, k.dim() == 3 ? k.size(1) : 0, dt);
+    }
+  }
+  d.L_m = (int32_t)integer(a[11]); d.T = (int32_t)integer(a[12]);
+  CHECK(PyTuple_Check(a[8]) && PyTuple_GET_SIZE(a[8]) == 8, "lists: eight int32 tensors");
+  const int32_t* lp[8];
+  int32_t ln[8];
+  for (int i = 0; i < 8; ++i) {
+    const at::Tensor& t = tensor(PyTuple_GET_ITEM(a[8], i), "list");
+    CHECK(t.scalar_type() == at::kInt && t.is_contiguous(), "lists: contiguous int32 tensors");
+    lp[i] = static_cast<const int32_t*>(t.data_ptr());
+    ln[i] = (int32_t)t.numel();
+  }
+  d.kc_list = lp[0]; d.kc_h_list = lp[1]; d.kn_list = lp[2]; d.kn_h_list = lp[3];
+  d.vc_list = lp[4]; d.vc_h_list = lp[5]; d.vn_list = lp[6]; d.vn_h_list = lp[7];
+  d.Ck = ln[0]; d.Cnk = ln[2]; d.Cv = ln[4]; d.Cnv = ln[6];
+  std::vector<int32_t> kpad, vpad;
+  if (d.L_m > 0) {
+    const at::Tensor &k_mc = tensor(a[2], "k_mc"), &v_mc = tensor(a[3], "v_mc");
+    CHECK(k_mc.scalar_type() == at::kFloat && k_mc.is_contiguous() && v_mc.scalar_type() == at::kFloat && v_mc.is_contiguous() &&
+          k_mc.dim() == 3 && v_mc.dim() == 3, "coefficients must be contiguous float32");
+    d.N = (int32_t)((d.Ck ? k_mc : v_mc).size(1) / 2);
+    d.k_mc = ptr<const float>(k_mc); d.v_mc = ptr<const float>(v_mc);
+    if (THPVariable_Check(a[4])) {
+      const at::Tensor &k_mn = tensor(a[4], "k_mn"), &v_mn = tensor(a[5], "v_mn");
+      CHECK(k_mn.dim() == 3 && v_mn.dim() == 3 && k_mn.stride(2) == 1 && v_mn.stride(2) == 1 && k_mn.scalar_type() == dt && v_mn.scalar_type() == dt,
+            "stored dims must have contiguous rows of the type of q");
+      d.mid_layout = FA_MID_TOKEN_MAJOR;
+      d.k_mn = ptr<>(k_mn); d.v_mn = ptr<>(v_mn);
+      d.k_mn_batch_stride = k_mn.stride(0); d.k_mn_row_stride = k_mn.stride(1);
+      d.v_mn_batch_stride = v_mn.stride(0); d.v_mn_row_stride = v_mn.stride(1);
+    } else {
+      const at::Tensor &kd = tensor_attr(a[4], s_data, "k_mn.data"), &vd = tensor_attr(a[5], s_data, "v_mn.data");
+      CHECK(kd.scalar_type() == dt && vd.scalar_type() == dt && int_attr(a[4], s_cap_pages) == int_attr(a[5], s_cap_pages),
+            "the page stores must have the type of q and one capacity");
+      d.mid_layout = FA_MID_PAGED;
+      d.mid_cap_pages = (int32_t)int_attr(a[4], s_cap_pages);
+      d.k_mn = kd.data_ptr(); d.v_mn = vd.data_ptr();
+      d.k_mn_batch_stride = int_attr(a[4], s_batch_stride); d.v_mn_batch_stride = int_attr(a[5], s_batch_stride);
+      d.k_pad_h_list = ptr<const int32_t>(tensor_attr(a[4], s_pad_h32, "pad_h32"));
+      d.v_pad_h_list = ptr<const int32_t>(tensor_attr(a[5], s_pad_h32, "pad_h32"));
+      d.mid_max_k_pad = (int32_t)int_attr(a[4], s_max_pad); d.mid_max_v_pad = (int32_t)int_attr(a[5], s_max_pad);
+      if (truth(a[18])) {
+        auto host_list = [&](PyObject* store, std::vector<int32_t>& out) {
+          Ref attr(PyObject_GetAttr(store, s_pad_h_host));
+          Ref seq(PySequence_Fast(attr.p, "pad_h_host"));
+          const Py_ssize_t len = PySequence_Fast_GET_SIZE(seq.p);
+          CHECK(len == d.Hkv + 1, "pad_h_host: one entry per head and one more");
+          out.resize(len);
+          for (Py_ssize_t i = 0; i < len; ++i) out[i] = (int32_t)integer(PySequence_Fast_GET_ITEM(seq.p, i));
+        };
+        host_list(a[4], kpad);
+        host_list(a[5], vpad);
+        d.k_pad_h_host = kpad.data(); d.v_pad_h_host = vpad.data();
+      }
+    }
+    CHECK(PyTuple_Check(a[6]) && PyTuple_GET_SIZE(a[6]) == 3 && PyTuple_Check(a[7]) && PyTuple_GET_SIZE(a[7]) == 3, "statistics: (avg_u, avg_d, scale)");
+    d.avg_k_u = stat(a[6], 0); d.avg_k_d = stat(a[6], 1); d.scale_k = stat(a[6], 2);
+    d.avg_v_u = stat(a[7], 0); d.avg_v_d = stat(a[7], 1); d.scale_v = stat(a[7], 2);
+    if (a[16] != Py_None) d.tables = tensor(a[16], "tables").data_ptr();
+  }
+  if (a[20] != Py_None) {
+    CHECK(d.L_m > 0, "a layer without mid rows has no coefficients to update");
+    CHECK(PyTuple_Check(a[20]) && PyTuple_GET_SIZE(a[20]) == 4, "pending: (k_row, v_row, phase, T)");
+    const at::Tensor &uk = tensor(PyTuple_GET_ITEM(a[20], 0), "k_row"), &uv = tensor(PyTuple_GET_ITEM(a[20], 1), "v_row");
+    CHECK(uk.dim() == 2 && uk.stride(1) == 1 && uv.strides() == uk.strides() && uk.scalar_type() == dt && uv.scalar_type() == dt, "pending rows");
+    d.upd_k_row = uk.data_ptr(); d.upd_v_row = uv.data_ptr(); d.upd_batch_stride = uk.stride(0);
+    d.upd_phase = integer(PyTuple_GET_ITEM(a[20], 2)); d.upd_T = (int32_t)integer(PyTuple_GET_ITEM(a[20], 3));
+  }
+  d.sm_scale = (float)real(a[13]);
+  d.force_generic = truth(a[17]);
+  d.no_fuse = (int32_t)integer(a[19]);
+  at::Tensor out;
+  if (a[14] != Py_None) {
+    out = gpu_tensor(a[14], "out");
+    CHECK(out.is_contiguous() && out.numel() == q.numel(), "out must be contiguous and as large as q");
+  } else {
+    out = at::empty({d.B, d.Hq, 1, d.D}, q.options().dtype(truth(a[15]) ? dt : at::kFloat));
+  }
+  if (out.scalar_type() == at::kFloat) d.out = static_cast<float*>(out.data_ptr());
+  else {
+    CHECK(out.scalar_type() == dt, "out must be float32 or have the type of q");
+    d.out_cast = out.data_ptr();
+  }
+  const fa_stream_t st = stream_of(q);
+  if (truth(a[21])) {
+    check_status(fa_decode_attn_noalloc(&d, st));
+    return a[14] != Py_None ? (Py_INCREF(a[14]), a[14]) : THPVariable_Wrap(out);
+  }
+  const size_t need = fa_decode_attn_workspace_bytes(d.B, d.Hq, d.Hkv, d.D, d.N, d.il_rows[0] + d.il_rows[1], d.L_m);
+  Ref device(THPVariable_Check(a[0]) ? PyObject_GetAttrString(a[0], "device") : nullptr), bytes(PyLong_FromSize_t(need));
+  PyObject* wargs[3] = {device.p, bytes.p, s_decode};
+  Ref ws(PyObject_Vectorcall(g_workspace_fn, wargs, 3, nullptr));
+  const at::Tensor& w = gpu_tensor(ws.p, "workspace");
+  d.workspace = w.data_ptr(); d.workspace_bytes = (size_t)w.numel();
+  if (a[22] != Py_None) {
+    float ms[4];
+    check_status(fa_decode_attn_timed(&d, st, ms));
+    Ref list(PyList_New(4));
+    for (int i = 0; i < 4; ++i) PyList_SET_ITEM(list.p, i, PyFloat_FromDouble(ms[i]));
+    if (PyList_SetSlice(a[22], 0, PyList_GET_SIZE(a[22]), list.p) < 0) throw PyError{};
+  } else {
+    check_status(fa_decode_attn(&d, st));
+  }
+  return a[14] != Py_None ? (Py_INCREF(a[14]), a[14]) : THPVariable_Wrap(out);
+  FA_END
+}
+
+// add_rmsnorm(h, delta or None, weight, eps) -> y
+PyObject* add_rmsnorm(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  FA_BEGIN
+  CHECK(n == 4, "add_rmsnorm takes 4 arguments");
+  const at::Tensor &h = gpu_tensor(a[0], "h"), &w = tensor(a[2], "weight");
+  CHECK(h.is_contiguous() && w.is_contiguous() && w.scalar_type() == h.scalar_type() && h.dim() >= 1 && w.numel() == h.size(-1),
+        "add_rmsnorm: h and weight contiguous, of one type, weight as long as a row");
+  const void* delta = nullptr;
+  if (a[1] != Py_None) {
+    const at::Tensor& t = tensor(a[1], "delta");
+    CHECK(t.is_contiguous() && t.sizes() == h.sizes() && t.scalar_type() == h.scalar_type(), "add_rmsnorm: delta must match h");
+    delta = ptr<>(t);
+  }
+  at::Tensor y = at::empty_like(h);
+  const int64_t hidden = h.size(-1);
+  check_status(fa_add_rmsnorm(h.data_ptr(), delta, w.data_ptr(), y.data_ptr(), (int)(h.numel() / hidden), (int)hidden, (float)real(a[3]),
+                              dtype_code(h), stream_of(h)));
+  return THPVariable_Wrap(y);
+  FA_END
+}
+
+// distance of the rows of a (..., width) tensor whose rows are evenly spaced (the width for a single row, whatever its
+// view reports)
+int64_t row_stride(const at::Tensor& t) {
+  CHECK(t.stride(-1) == 1 || t.size(-1) == 1, "rows must be contiguous");
+  int64_t step = 0, span = 0;
+  for (int64_t i = t.dim() - 2; i >= 0; --i) {
+    if (t.size(i) == 1) continue;
+    if (step == 0) step = t.stride(i);
+    else CHECK(t.stride(i) == span, "rows are not evenly spaced");
+    span = t.stride(i) * t.size(i);
+  }
+  return step == 0 ? t.size(-1) : step;
+}
+
+// linear_packed(x, packed weight, k, n_out) -> (..., n_out)
+PyObject* linear_packed(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  FA_BEGIN
+  CHECK(n == 4, "linear_packed takes 4 arguments");
+  const at::Tensor &x = gpu_tensor(a[0], "x"), &w = gpu_tensor(a[1], "weight");
+  const int64_t k = integer(a[2]), n_out = integer(a[3]);
+  CHECK(x.scalar_type() == w.scalar_type() && x.dim() >= 1 && x.size(-1) == k && w.numel() == k * n_out, "linear_packed: x does not fit the weight");
+  at::DimVector shape(x.sizes().begin(), x.sizes().end());
+  shape.back() = n_out;
+  at::Tensor out = at::empty(shape, x.options());
+  check_status(fa_linear_packed(x.data_ptr(), row_stride(x), w.data_ptr(), out.data_ptr(), (int)(x.numel() / k), (int)k, (int)n_out,
+                                dtype_code(x), stream_of(x)));
+  return THPVariable_Wrap(out);
+  FA_END
+}
+
+// silu_mul(gate, up) -> dense
+PyObject* silu_mul(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  FA_BEGIN
+  CHECK(n == 2, "silu_mul takes 2 arguments");
+  const at::Tensor &g = gpu_tensor(a[0], "gate"), &u = gpu_tensor(a[1], "up");
+  CHECK(g.sizes() == u.sizes() && g.scalar_type() == u.scalar_type() && g.strides() == u.strides() && g.dim() >= 1 && g.stride(-1) == 1,
+        "silu_mul: gate and up must share shape, type and strides");
+  const int64_t cols = g.size(-1), rows = g.numel() / (cols > 0 ? cols : 1), stride = row_stride(g), es = g.element_size();
+  at::Tensor out = at::empty(g.sizes(), g.options().memory_format(at::MemoryFormat::Contiguous));
+  const fa_stream_t st = stream_of(g);
+  for (int64_t r0 = 0; r0 < rows; r0 += 65535)   // the row index is the launch's second grid dimension
+    check_status(fa_silu_mul((const char*)g.data_ptr() + r0 * stride * es, (const char*)u.data_ptr() + r0 * stride * es,
+                             (char*)out.data_ptr() + r0 * cols * es, (int)std::min<int64_t>(65535, rows - r0), (int)cols, stride,
+                             dtype_code(g), st));
+  return THPVariable_Wrap(out);
+  FA_END
+}
+
+// rope_qk(q, k, cos, sin, head_dim) -> q rotated, dense (q itself when it was dense); k in place.  cos, sin: one row per token
+PyObject* rope_qk(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  FA_BEGIN
+  CHECK(n == 5, "rope_qk takes 5 arguments");
+  const at::Tensor &q = gpu_tensor(a[0], "q"), &k = gpu_tensor(a[1], "k"), &cos = gpu_tensor(a[2], "cos"), &sin = gpu_tensor(a[3], "sin");
+  const int64_t D = integer(a[4]);
+  CHECK(q.dim() == 3 && k.dim() == 3 && q.scalar_type() == k.scalar_type() && q.size(0) == k.size(0) && q.size(1) == k.size(1) && D > 0,
+        "rope_qk: q and k (B, q_len, heads * D) of one type");
+  const int64_t rows = q.size(0) * q.size(1);
+  CHECK(cos.is_contiguous() && sin.is_contiguous() && cos.scalar_type() == q.scalar_type() && sin.scalar_type() == q.scalar_type() &&
+        cos.numel() == rows * D && sin.numel() == rows * D, "rope_qk: one row of cos and sin per token, of the type of q");
+  const bool dense = q.is_contiguous();
+  at::Tensor out = dense ? q : at::empty(q.sizes(), q.options().memory_format(at::MemoryFormat::Contiguous));
+  check_status(fa_rope_qk(q.data_ptr(), row_stride(q), out.data_ptr(), k.data_ptr(), row_stride(k), cos.data_ptr(), sin.data_ptr(), (int)rows,
+                          (int)(q.size(2) / D), (int)(k.size(2) / D), (int)D, dtype_code(q), stream_of(q)));
+  return dense ? (Py_INCREF(a[0]), a[0]) : THPVariable_Wrap(out);
+  FA_END
+}
+
+// init(stream_fn, check_fn, workspace_fn)
+PyObject* init(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  if (n != 3) {
+    PyErr_SetString(PyExc_TypeError, "init takes 3 arguments");
+    return nullptr;
+  }
+  PyObject** slots[3] = {&g_stream_fn, &g_check_fn, &g_workspace_fn};
+  for (int i = 0; i < 3; ++i) {
+    Py_INCREF(a[i]);
+    Py_XDECREF(*slots[i]);
+    *slots[i] = a[i];
+  }
+  Py_RETURN_NONE;
+}
+
+#define FN(name) {#name, (PyCFunction)(void*)name, METH_FASTCALL, nullptr}
+PyMethodDef methods[] = {FN(init), FN(stream_update), FN(decode_attn), FN(add_rmsnorm), FN(linear_packed), FN(silu_mul), FN(rope_qk),
+                         {nullptr, nullptr, 0, nullptr}};
+PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_fa_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__fa_host() {
+  struct { PyObject** at; const char* name; } names[] = {
+      {&s_data, "data"}, {&s_cap_pages, "cap_pages"}, {&s_batch_stride, "batch_stride"}, {&s_pad_h32, "pad_h32"}, {&s_max_pad, "max_pad"},
+      {&s_pad_h_host, "pad_h_host"}, {&s_n_list32, "n_list32"}, {&s_n_h32, "n_h32"}, {&s_Cn, "Cn"}, {&s_Hkv, "Hkv"}, {&s_decode, "decode"}};
+  for (auto& e : names)
+    if (!(*e.at = PyUnicode_InternFromString(e.name))) return nullptr;
+  return PyModule_Create(&module_def);
+}

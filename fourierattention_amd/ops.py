@@ -16,13 +16,12 @@ the current stream.
 """
 from __future__ import annotations
 
-import ctypes
 from typing import Dict, Optional, Tuple
 
 import torch
 
 from . import _lib
-from ._lib import FA_BF16, FA_FP16, FA_FP32, DecodeArgs, check
+from ._lib import FA_BF16, FA_FP16, FA_FP32, check
 
 _DTYPE_CODE = {torch.bfloat16: FA_BF16, torch.float16: FA_FP16, torch.float32: FA_FP32}
 
@@ -34,16 +33,20 @@ def dtype_code(dt: torch.dtype) -> int:
         raise TypeError(f"unsupported dtype {dt}; expected bfloat16, float16 or float32") from None
 
 
-_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+def _current_raw_stream(index: int) -> int:
+    return torch.cuda.current_stream(index).cuda_stream
+
+
+# device index -> handle of torch's current stream there (the bare handle where torch offers it, without building a
+# torch.cuda.Stream object around it)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or _current_raw_stream
 
 
 def _stream(device) -> int:
     """Handle of the stream the caller's tensor work is queued on (torch's current stream of ``device``).  Looked up
     on every call: the caller may switch streams, or capture into a graph, between two operators."""
-    if _raw_stream is not None:     # the bare handle, without building a torch.cuda.Stream object around it
-        idx = device.index
-        return _raw_stream(torch.cuda.current_device() if idx is None else idx)
-    return torch.cuda.current_stream(device).cuda_stream
+    idx = device.index
+    return _raw_stream(torch.cuda.current_device() if idx is None else idx)
 
 
 def _require_gpu(t: torch.Tensor, name: str) -> None:
@@ -202,71 +205,29 @@ def stream_update(k_new: torch.Tensor, v_new: torch.Tensor, k_ring: torch.Tensor
     """One streaming step of one layer in one launch (the body of cache_utils_fourier.py:731-748 for K and V):
     the rows in window slot ``evict_slot`` enter the coefficients (rank-1 update at ``phase``) and the page
     stores (at token ``mid_pos``); ``k_new, v_new (B, width)`` are written to window slot ``write_slot``.
-    ``k_ring, v_ring (B, slots, width)`` share their strides; ``k_mid, v_mid`` are ``MidStore`` objects.
+    ``k_ring, v_ring (B, slots, width)`` share their strides; ``k_mid, v_mid`` are ``MidStore`` objects.  The new rows
+    may also come as the token itself, ``(B, heads, 1, D)`` with the heads side by side.
     ``skip_coef``: leave the coefficients alone; the caller owes them the update (``coeff_update_``, or the
     ``pending`` argument of the layer's next ``decode_attn_raw``) before that window slot is written again."""
-    _require_gpu(k_ring, "k_ring")
-    assert k_new.dim() == 2 and k_new.stride(1) == 1 and v_new.stride() == k_new.stride()
-    assert k_ring.stride(2) == 1 and v_ring.stride() == k_ring.stride() and k_ring.shape == v_ring.shape
-    assert evict_slot != write_slot and k_mid.cap_pages == v_mid.cap_pages
-    a = _lib.StreamArgs()
-    a.k_new, a.v_new, a.new_batch_stride = k_new.data_ptr(), v_new.data_ptr(), k_new.stride(0)
-    a.k_ring, a.v_ring = k_ring.data_ptr(), v_ring.data_ptr()
-    a.ring_batch_stride, a.ring_row_stride = k_ring.stride(0), k_ring.stride(1)
-    a.evict_slot, a.write_slot = int(evict_slot), int(write_slot)
-    a.k_coef, a.v_coef = _ptr(k_coef), _ptr(v_coef)
-    a.kc_list, a.vc_list = _ptr(kc_list), _ptr(vc_list)
-    a.Ck, a.Cv = int(kc_list.numel()), int(vc_list.numel())
-    a.N, a.T, a.phase = int(k_coef.shape[1] // 2), int(T), int(phase)
-    a.k_mid, a.v_mid = k_mid.data.data_ptr(), v_mid.data.data_ptr()
-    a.k_mid_batch_stride, a.v_mid_batch_stride = int(k_mid.batch_stride), int(v_mid.batch_stride)
-    a.cap_pages, a.mid_pos = int(k_mid.cap_pages), int(mid_pos)
-    a.kn_list, a.kn_h_list, a.k_pad_h_list = _ptr(k_mid.n_list32), k_mid.n_h32.data_ptr(), k_mid.pad_h32.data_ptr()
-    a.vn_list, a.vn_h_list, a.v_pad_h_list = _ptr(v_mid.n_list32), v_mid.n_h32.data_ptr(), v_mid.pad_h32.data_ptr()
-    a.Cnk, a.Cnv = int(k_mid.Cn), int(v_mid.Cn)
-    a.B, a.Hkv, a.width, a.dtype = int(k_ring.shape[0]), int(k_mid.Hkv), int(k_ring.shape[2]), dtype_code(k_ring.dtype)
-    a.skip_coef = int(bool(skip_coef))
-    import ctypes
-    check(_lib.load().fa_stream_update(ctypes.byref(a), _stream(k_ring.device)))
+    _lib.load_host().stream_update(k_new, v_new, k_ring, v_ring, evict_slot, write_slot, k_coef, v_coef, kc_list, vc_list,
+                                   phase, T, k_mid, v_mid, mid_pos, skip_coef)
 
 
 def add_rmsnorm(h: torch.Tensor, delta: Optional[torch.Tensor], weight: torch.Tensor, eps: float) -> torch.Tensor:
     """``h += delta`` (when given, in place) and ``LlamaRMSNorm`` of the result in one launch
     (modeling_llama_fourier.py:735-750, 87-92).  ``h, delta (..., hidden)`` contiguous."""
-    _require_gpu(h, "h")
-    assert h.is_contiguous() and weight.is_contiguous() and weight.dtype == h.dtype
-    assert delta is None or (delta.is_contiguous() and delta.shape == h.shape and delta.dtype == h.dtype)
-    y = torch.empty_like(h)
-    hidden = h.shape[-1]
-    check(_lib.load().fa_add_rmsnorm(h.data_ptr(), _ptr(delta), weight.data_ptr(), y.data_ptr(), h.numel() // hidden, hidden,
-                                     float(eps), dtype_code(h.dtype), _stream(h.device)))
-    return y
-
-
-def _row_sliced(t: torch.Tensor) -> bool:
-    """(B, q_len, width) whose rows are evenly spaced slices of wider rows (or dense)."""
-    return t.dim() == 3 and t.stride(2) == 1 and (t.shape[1] == 1 or t.stride(0) == t.shape[1] * t.stride(1))
+    return _lib.load_host().add_rmsnorm(h, delta, weight, eps)
 
 
 def rope_qk(q: torch.Tensor, k: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, head_dim: int) -> torch.Tensor:
     """Rotary embedding of ``q (B, q_len, Hq*D)`` and ``k (B, q_len, Hkv*D)`` (the projection outputs, possibly
     column slices of one fused projection output); ``cos, sin (B or 1, q_len, D)`` (modeling_llama_fourier.py:213-244).
     ``k`` is rotated in place; the rotated ``q`` is returned densely packed (``q`` itself when it was dense)."""
-    _require_gpu(q, "q")
-    assert _row_sliced(q) and _row_sliced(k) and q.dtype == k.dtype
-    rows = q.shape[0] * q.shape[1]
     if cos.shape[0] != q.shape[0]:
         cos, sin = cos.expand(q.shape[0], -1, -1), sin.expand(q.shape[0], -1, -1)
-    cos, sin = cos.to(q.dtype).contiguous(), sin.to(q.dtype).contiguous()
-    q_out = q if q.is_contiguous() else torch.empty(q.shape, dtype=q.dtype, device=q.device)
-    qs = q.stride(1) if q.shape[1] > 1 else q.stride(0)
-    ks = k.stride(1) if k.shape[1] > 1 else k.stride(0)
-    if rows == 1:                      # a single row has no spacing, whatever its view reports
-        qs, ks = q.shape[2], k.shape[2]
-    check(_lib.load().fa_rope_qk(q.data_ptr(), qs, q_out.data_ptr(), k.data_ptr(), ks, cos.data_ptr(), sin.data_ptr(), rows,
-                                 q.shape[2] // head_dim, k.shape[2] // head_dim, head_dim, dtype_code(q.dtype),
-                                 _stream(q.device)))
-    return q_out
+    if cos.dtype != q.dtype or not (cos.is_contiguous() and sin.is_contiguous()):
+        cos, sin = cos.to(q.dtype).contiguous(), sin.to(q.dtype).contiguous()
+    return _lib.load_host().rope_qk(q, k, cos, sin, head_dim)
 
 
 def rope_qk_(q: torch.Tensor, k: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, head_dim: int) -> None:
@@ -278,20 +239,7 @@ def rope_qk_(q: torch.Tensor, k: torch.Tensor, cos: torch.Tensor, sin: torch.Ten
 def silu_mul(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
     """``silu(gate) * up`` in one launch (modeling_llama_fourier.py:277); ``gate, up (..., cols)`` dense or column
     slices of one fused projection output (rows evenly spaced, the same spacing for both); the result is dense."""
-    _require_gpu(gate, "gate")
-    assert gate.shape == up.shape and gate.dtype == up.dtype and gate.stride() == up.stride() and gate.stride(-1) == 1
-    cols = gate.shape[-1]
-    rows = gate.numel() // max(cols, 1)
-    stride = gate.stride(-2) if gate.dim() >= 2 and rows > 1 else cols
-    assert all(gate.shape[d] == 1 or gate.stride(d) == gate.stride(d + 1) * gate.shape[d + 1] for d in range(gate.dim() - 2)), \
-        "rows are not evenly spaced"
-    out = torch.empty(gate.shape, dtype=gate.dtype, device=gate.device)
-    es = gate.element_size()
-    for r0 in range(0, rows, 65535):   # the row index is the launch's second grid dimension
-        check(_lib.load().fa_silu_mul(gate.data_ptr() + r0 * stride * es, up.data_ptr() + r0 * stride * es,
-                                      out.data_ptr() + r0 * cols * es, min(65535, rows - r0), cols, stride,
-                                      dtype_code(gate.dtype), _stream(gate.device)))
-    return out
+    return _lib.load_host().silu_mul(gate, up)
 
 
 class WeightStamp:
@@ -338,15 +286,7 @@ class PackedLinearWeight:
 def linear_packed(x: torch.Tensor, w: PackedLinearWeight) -> torch.Tensor:
     """``F.linear(x, weight)`` for ``x (..., K)`` of at most 16 rows (fp32 accumulation, result in the storage type)
     on the packed weight; rows must be evenly spaced (dense, or slices of wider rows)."""
-    assert w.covers(x), "shape not covered: at most 16 rows, K a multiple of 1024, n_out of 16"
-    rows = x.numel() // w.k
-    stride = x.stride(-2) if x.dim() >= 2 and rows > 1 else w.k
-    assert all(x.shape[d] == 1 or x.stride(d) == x.stride(d + 1) * x.shape[d + 1] for d in range(x.dim() - 2)), \
-        "rows are not evenly spaced"
-    out = torch.empty(x.shape[:-1] + (w.n_out,), dtype=x.dtype, device=x.device)
-    check(_lib.load().fa_linear_packed(x.data_ptr(), stride, w.data.data_ptr(), out.data_ptr(), rows, w.k, w.n_out,
-                                       dtype_code(x.dtype), _stream(x.device)))
-    return out
+    return _lib.load_host().linear_packed(x, w.data, w.k, w.n_out)
 
 
 def prefill_attention_supported(q: torch.Tensor, k: torch.Tensor, head_dim: int) -> bool:
@@ -415,11 +355,13 @@ def decode_tables(n_f: int, period: int, device) -> Optional[torch.Tensor]:
 
 def decode_attn_raw(q, il_segments, k_mc, v_mc, k_mn, v_mn, stats_k, stats_v, lists, num_head_q, num_head_kv, seq_len_m,
                     T, sm_scale=-1.0, out=None, tables=None, force_generic=False, timings=None, out_dtype=None,
-                    no_alloc=False, balance_heads=True, no_fuse=False, pending=None):
+                    no_alloc=False, balance_heads=True, no_fuse=0, pending=None):
     """Thin call into ``fa_decode_attn``.  The result is float32 like the reference's (TRI:779) unless ``out_dtype``
     names the dtype of ``q``: then the merge launch rounds it to that type itself (the caller's ``.to(dtype)``).
 
-    ``il_segments``: up to two ``(k, v)`` pairs of ``(B, rows, Hkv*D)`` views (last dim contiguous).
+    ``q (B, 1, Hq*D)`` or ``(B, Hq, 1, D)``, contiguous.
+    ``il_segments``: up to two ``(k, v)`` pairs of ``(B, rows, Hkv*D)`` views (last dim contiguous), or ``(k, v, r)``: the
+    rows of one buffer in front of and behind row ``r``.
     ``k_mn`` / ``v_mn``: token-major ``(B, >=L_m, Cn)`` tensors or ``MidStore`` objects (paged).
     ``stats_*``: ``(avg_u, avg_d, scale)`` fp32 ``(B, C)``.  ``lists``: the eight int32 tensors
     ``kc, kc_h, kn, kn_h, vc, vc_h, vn, vn_h`` (``*_h`` with the leading 0).
@@ -433,106 +375,29 @@ def decode_attn_raw(q, il_segments, k_mc, v_mc, k_mn, v_mn, stats_k, stats_v, li
     ``pending``: ``(k_row, v_row, phase, T_c)``, a rank-1 update the coefficients are still owed (``stream_update``
     with ``skip_coef``): ``k_row, v_row (B, Hkv*D)`` are the rows that left the window (same strides).  The call
     applies it to ``k_mc`` / ``v_mc`` IN PLACE while it streams them, once; pass it to one call only."""
-    from .midstore import MidStore
-    _require_gpu(q, "q")
-    B, q_len, feat = q.shape
-    D = feat // num_head_q
-    a = DecodeArgs()
-    assert q.is_contiguous()
-    a.q = q.data_ptr()
-    total_il = 0
-    for i in range(2):
-        if i < len(il_segments) and il_segments[i] is not None and il_segments[i][0].shape[1] > 0:
-            k, v = il_segments[i]
-            assert k.stride(2) == 1 and v.stride(2) == 1 and k.stride() == v.stride() and k.shape == v.shape
-            assert k.dtype == q.dtype and v.dtype == q.dtype
-            a.k_il[i], a.v_il[i] = k.data_ptr(), v.data_ptr()
-            a.il_rows[i], a.il_batch_stride[i], a.il_row_stride[i] = k.shape[1], k.stride(0), k.stride(1)
-            total_il += k.shape[1]
-    kc, kc_h, kn, kn_h, vc, vc_h, vn, vn_h = lists
-    a.Ck, a.Cnk, a.Cv, a.Cnv = kc.numel(), kn.numel(), vc.numel(), vn.numel()
-    N = 0
-    if seq_len_m > 0:
-        N = (k_mc.shape[1] if a.Ck else v_mc.shape[1]) // 2
-        for t in (k_mc, v_mc):
-            assert t.dtype == torch.float32 and t.is_contiguous()
-        a.k_mc, a.v_mc = _ptr(k_mc), _ptr(v_mc)
-        if isinstance(k_mn, MidStore):
-            assert isinstance(v_mn, MidStore) and k_mn.dtype == q.dtype and k_mn.cap_pages == v_mn.cap_pages
-            a.mid_layout, a.mid_cap_pages = _lib.FA_MID_PAGED, k_mn.cap_pages
-            a.k_mn, a.v_mn = k_mn.data.data_ptr(), v_mn.data.data_ptr()
-            a.k_mn_batch_stride, a.v_mn_batch_stride = k_mn.batch_stride, v_mn.batch_stride
-            a.k_pad_h_list, a.v_pad_h_list = k_mn.pad_h32.data_ptr(), v_mn.pad_h32.data_ptr()
-            a.mid_max_k_pad, a.mid_max_v_pad = k_mn.max_pad, v_mn.max_pad
-            if balance_heads:
-                a.k_pad_h_host = ctypes.cast(k_mn.pad_h_c, ctypes.c_void_p)
-                a.v_pad_h_host = ctypes.cast(v_mn.pad_h_c, ctypes.c_void_p)
-        else:
-            for t in (k_mn, v_mn):
-                assert t.stride(2) == 1 and t.dtype == q.dtype
-            a.mid_layout = _lib.FA_MID_TOKEN_MAJOR
-            a.k_mn, a.v_mn = _ptr(k_mn), _ptr(v_mn)
-            a.k_mn_batch_stride, a.k_mn_row_stride = k_mn.stride(0), k_mn.stride(1)
-            a.v_mn_batch_stride, a.v_mn_row_stride = v_mn.stride(0), v_mn.stride(1)
-        a.avg_k_u, a.avg_k_d, a.scale_k = (_ptr(t) for t in stats_k)
-        a.avg_v_u, a.avg_v_d, a.scale_v = (_ptr(t) for t in stats_v)
-        for t in (*stats_k, *stats_v):
-            assert t.dtype == torch.float32 and t.is_contiguous()
-        if tables is not None:
-            a.tables = tables.data_ptr()
-    if pending is not None:
-        uk, uv, phase, t_c = pending
-        assert seq_len_m > 0, "a layer without mid rows has no coefficients to update"
-        assert uk.dim() == 2 and uk.stride(1) == 1 and uv.stride() == uk.stride() and uk.dtype == q.dtype == uv.dtype
-        a.upd_k_row, a.upd_v_row, a.upd_batch_stride = uk.data_ptr(), uv.data_ptr(), uk.stride(0)
-        a.upd_phase, a.upd_T = int(phase), int(t_c)
-    a.force_generic = int(bool(force_generic))
-    a.no_fuse = int(no_fuse)   # False / True, or the bits of fa_decode_args.no_fuse
     if seq_len_m >= _REPACK_MIN_ROWS and not force_generic:
-        _warn_if_off_the_matrix_cores(q.dtype, num_head_q, num_head_kv, D, N, isinstance(k_mn, MidStore))
-    a.kc_list, a.kc_h_list, a.kn_list, a.kn_h_list = kc.data_ptr(), kc_h.data_ptr(), kn.data_ptr(), kn_h.data_ptr()
-    a.vc_list, a.vc_h_list, a.vn_list, a.vn_h_list = vc.data_ptr(), vc_h.data_ptr(), vn.data_ptr(), vn_h.data_ptr()
-    if out is None:
-        cast = out_dtype is not None and out_dtype != torch.float32
-        assert not cast or out_dtype == q.dtype, "out_dtype must be float32 or the dtype of q"
-        out = torch.empty((B, num_head_q, 1, D), device=q.device, dtype=q.dtype if cast else torch.float32)
-    if out.dtype == torch.float32:
-        a.out = out.data_ptr()
-    else:
-        assert out.dtype == q.dtype and out.is_contiguous()
-        a.out_cast = out.data_ptr()
-    a.B, a.Hq, a.Hkv, a.D = B, num_head_q, num_head_kv, D
-    a.q_len, a.N, a.L_m, a.T = q_len, N, int(seq_len_m), int(T)
-    a.sm_scale = float(sm_scale)
-    a.dtype = dtype_code(q.dtype)
-    lib = _lib.load()
-    if no_alloc:
-        check(lib.fa_decode_attn_noalloc(ctypes.byref(a), _stream(q.device)))
-        return out
-    nbytes = lib.fa_decode_attn_workspace_bytes(B, num_head_q, num_head_kv, D, N, total_il, int(seq_len_m))
-    ws = workspace(q.device, nbytes, "decode")
-    a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel()
-    if timings is not None:   # list to receive [prep, mid, sink/window, merge] milliseconds
-        ms = (ctypes.c_float * 4)()
-        check(lib.fa_decode_attn_timed(ctypes.byref(a), _stream(q.device), ms))
-        timings[:] = list(ms)
-    else:
-        check(lib.fa_decode_attn(ctypes.byref(a), _stream(q.device)))
-    return out
+        _warn_if_off_the_matrix_cores(q.dtype, num_head_q, num_head_kv, q.numel() // (q.shape[0] * num_head_q),
+                                      (k_mc if lists[0].numel() else v_mc).shape[1] // 2, not isinstance(k_mn, torch.Tensor))
+    cast = out_dtype is not None and out_dtype != torch.float32
+    assert not cast or out_dtype == q.dtype, "out_dtype must be float32 or the dtype of q"
+    return _lib.load_host().decode_attn(q, il_segments, k_mc, v_mc, k_mn, v_mn, stats_k, stats_v, lists, num_head_q,
+                                        num_head_kv, seq_len_m, T, sm_scale, out, cast, tables, force_generic, balance_heads,
+                                        no_fuse, pending, no_alloc, timings)
 
 
 _warned_shapes = set()
+_SIXTEEN_BIT = (torch.bfloat16, torch.float16)
 
 
 def _warn_if_off_the_matrix_cores(dtype, num_head_q, num_head_kv, head_dim, n_f, paged):
     """Long contexts outside the shapes of the matrix-core kernels (16-bit paged storage, 128 / 256 / 512 / 1024
     frequencies, heads of at most 128 dims, at most 8 query heads per KV head) run on vector-ALU kernels that take any
-    shape and are far slower (16.2 ms against 0.31 ms per layer at B=4, 131072 tokens, 24 / 8 heads): say so once
-    per shape instead of being silently slow."""
-    g = num_head_q // max(num_head_kv, 1)
-    ok = (dtype in (torch.bfloat16, torch.float16) and paged and n_f in (128, 256, 512, 1024) and head_dim <= 128 and g <= 8)
+    shape and are far slower: say so once per shape instead of being silently slow."""
+    if (dtype in _SIXTEEN_BIT and paged and n_f in (128, 256, 512, 1024) and head_dim <= 128
+            and num_head_q // max(num_head_kv, 1) <= 8):
+        return
     key = (dtype, num_head_q, num_head_kv, head_dim, n_f, paged)
-    if ok or key in _warned_shapes:
+    if key in _warned_shapes:
         return
     _warned_shapes.add(key)
     import warnings
