@@ -12,6 +12,18 @@
 // slot order, is prepared once per call by a transposing pass over V (prefill_vt_kernel): 1 KiB fragments that
 // the main kernel streams into LDS unchanged.
 //
+// What bounds it: power, then issue.  On random operands the device runs this kernel at 1.8 - 1.9 GHz (the same launch on
+// zeros: 1538 TFLOP/s instead of 1131), so what counts is energy and instructions per score, not the order of the work.
+// Vector and matrix instructions of a SIMD overlap only in part (a 16x16x32 instruction holds the issue for half of its
+// 16 clocks).  The softmax of a tile therefore costs a lane one multiply-add, half a three-way maximum, one exponential,
+// half a conversion and half a dot product per score: distances from a reference that lags (kMaxLag), one vote per
+// tile on them without any lane exchange, denominators from the f16 probabilities by pairs.  Consecutive matrix
+// instructions change one operand at a time.  32768 tokens, 32 / 8 heads of 128 dims, bf16: 987 -> 1131 TFLOP/s.  Tried
+// and slower: 32x32x16 instructions (half the count, but twice the accumulator traffic per product: 1357 against 1939
+// TFLOP/s for bare products of random f16 operands; here 987 with this softmax), denominators on the matrix unit (1042),
+// two waves per SIMD (1102), a third stage (1116), twelve waves sharing the tiles of 96 keys (1134 against 1141 for a third of
+// the L2 traffic).
+//
 // Workgroup: one KV head, HW query heads of it (all that share its keys, up to four) times RW blocks of 32 query
 // rows, one wave each.  The key tiles travel HBM -> LDS once per workgroup (global_load_lds, two stages, one
 // meeting per tile) in fragment order, so every LDS read of a wave is one conflict-free 16 bytes per lane.
@@ -22,6 +34,10 @@ namespace {
 using namespace fa_mfma;
 
 constexpr int kTileKeys = 32;
+// a row's softmax reference moves only when a score exceeds it by more than this (base 2): the probabilities stay below
+// 2^8, exact to f16's eleven bits, and most tiles rescale nothing
+constexpr float kMaxLag = 8.f;
+constexpr float kNoReference = -1e30f;   // before a row's first key: finite, so that a masked score is -inf against it
 
 template <typename E>
 struct PrefillParams {
@@ -93,36 +109,30 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(3, 3
   const int wg_last_row = min(p.q_len, ((int)gridDim.x - (int)blockIdx.x) * p.RW * 32) - 1;
   const int n_t = min(p.n_tiles, (wg_last_row + offset) / kTileKeys + 1);
 
-  // this wave's share of a tile: fragments w, w + WAVES, ... (clamped to the last one: every wave issues OPS loads)
-  const E* kb_base = p.k + (int64_t)b * p.k_bs + (int64_t)kvh * D + 8 * lg;
-  const f16_t* vt_base = p.vt + ((int64_t)b * p.Hkv + kvh) * p.n_tiles * (int64_t)(kTileKeys * D) + lane * 8;
-  // The tiles are requested in order, so every load keeps a running pointer that moves on by one tile; only a last
-  // tile that reaches past the keys computes its (clamped) rows afresh.
-  const E* run[OPS];
-#pragma unroll
-  for (int i = 0; i < OPS; ++i) {
-    const int f = min(w + i * WAVES, NF - 1);
-    if (f < 2 * KS) run[i] = kb_base + (int64_t)(16 * (f / KS) + lc) * p.k_rs + 32 * (f % KS);
-    else run[i] = (const E*)(vt_base + (int64_t)(f - 2 * KS) * 512);   // (both 16-bit: the pointer only counts elements)
-  }
-  const int64_t k_step = (int64_t)kTileKeys * p.k_rs;
+  // this wave's share of a tile: fragments w, w + WAVES, ... (clamped to the last one: every wave issues OPS loads).
+  // Addresses are a wave-uniform base plus one 32-bit lane offset for K and one for V^T; only a last tile that reaches
+  // past the keys computes its (clamped) rows afresh.
+  const E* kb_base = p.k + (int64_t)b * p.k_bs + (int64_t)kvh * D;
+  const f16_t* vt_base = p.vt + ((int64_t)b * p.Hkv + kvh) * p.n_tiles * (int64_t)(kTileKeys * D);
+  const unsigned k_off = (unsigned)((lc * p.k_rs + 8 * lg) * (int64_t)sizeof(E)), vt_off = lane * 16;
   const bool ragged_keys = (p.S % kTileKeys) != 0;
   auto issue = [&](int t, int buf) {
     const bool clamp = ragged_keys && t == p.n_tiles - 1;   // wave-uniform
+    const E* k_tile = kb_base + (int64_t)t * kTileKeys * p.k_rs;
+    const f16_t* v_tile = vt_base + (int64_t)t * (kTileKeys * D);
 #pragma unroll
     for (int i = 0; i < OPS; ++i) {
       const int f = min(w + i * WAVES, NF - 1);
-      const E* src = run[i];
-      if (f < 2 * KS) {
-        if (clamp) {
-          const int key = min(t * kTileKeys + 16 * (f / KS) + lc, p.S - 1);
-          src = kb_base + (int64_t)key * p.k_rs + 32 * (f % KS);
-        }
-        run[i] += k_step;
-      } else {
-        run[i] += DG * 512;
+      const bool is_k = f < 2 * KS;
+      const char* base = is_k ? (const char*)(k_tile + (int64_t)(16 * (f / KS)) * p.k_rs + 32 * (f % KS))
+                              : (const char*)(v_tile + (f - 2 * KS) * 512);
+      unsigned off = is_k ? k_off : vt_off;
+      if (clamp && is_k) {
+        const int first = t * kTileKeys + 16 * (f / KS);   // (may itself lie past the keys: the base then moves back)
+        base = (const char*)(kb_base + 32 * (f % KS)) + (int64_t)min(first, p.S - 1) * p.k_rs * (int64_t)sizeof(E);
+        off = (unsigned)((max(min(first + lc, p.S - 1) - first, 0) * p.k_rs + 8 * lg) * (int64_t)sizeof(E));
       }
-      load_frag_to_lds(src, &s_tile[buf][f * 1024]);
+      load_frag_to_lds((const E*)(base + off), &s_tile[buf][f * 1024]);
     }
   };
   if (n_t > 0) issue(0, 0);
@@ -142,7 +152,7 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(3, 3
   float4v oacc[DG][2];
 #pragma unroll
   for (int dg = 0; dg < DG; ++dg) oacc[dg][0] = oacc[dg][1] = float4v{0.f, 0.f, 0.f, 0.f};
-  float m_run[2] = {-INFINITY, -INFINITY}, l_run[2] = {0.f, 0.f};
+  float m_run[2] = {kNoReference, kNoReference}, l_run[2] = {0.f, 0.f};
   // the query loads above must not be confused with the tile loads by the counted waits below
 #pragma unroll
   for (int rb = 0; rb < 2; ++rb)
@@ -164,11 +174,10 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(3, 3
     uint4v kf[4];
     constexpr int NFK = 2 * KS;
     auto s_pair = [&](uint4v& f0, uint4v& f1, int f) {   // fragments f, f + 1 (f is a constant after unrolling)
-#pragma unroll
-      for (int rb = 0; rb < 2; ++rb) {
-        sacc[f / KS][rb] = M::mma(__builtin_bit_cast(vec8, f0), Qf[rb][f % KS], sacc[f / KS][rb]);
-        sacc[(f + 1) / KS][rb] = M::mma(__builtin_bit_cast(vec8, f1), Qf[rb][(f + 1) % KS], sacc[(f + 1) / KS][rb]);
-      }
+      sacc[f / KS][0] = M::mma(__builtin_bit_cast(vec8, f0), Qf[0][f % KS], sacc[f / KS][0]);
+      sacc[f / KS][1] = M::mma(__builtin_bit_cast(vec8, f0), Qf[1][f % KS], sacc[f / KS][1]);
+      sacc[(f + 1) / KS][1] = M::mma(__builtin_bit_cast(vec8, f1), Qf[1][(f + 1) % KS], sacc[(f + 1) / KS][1]);
+      sacc[(f + 1) / KS][0] = M::mma(__builtin_bit_cast(vec8, f1), Qf[0][(f + 1) % KS], sacc[(f + 1) / KS][0]);
     };
     kf[0] = lds_read_b128_async_at<0 * 1024>(base);
     kf[1] = lds_read_b128_async_at<1 * 1024>(base);
@@ -202,52 +211,59 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(3, 3
     vf[2] = lds_read_b128_async_at<2048>(vbase);
     vf[3] = lds_read_b128_async_at<3072>(vbase);
     // ---- softmax of the tile (base 2), per row = per lane column
-    const bool edge = t * kTileKeys + 31 > r0 + offset || t * kTileKeys + 31 >= p.S;   // wave-uniform
-    half8 pb[2];   // probabilities as f16 operands
-    float alpha[2];
-#pragma unroll
-    for (int rb = 0; rb < 2; ++rb) {
-      float s[8];   // raw products: the softmax scale rides in the instruction that subtracts the reference
-#pragma unroll
-      for (int e = 0; e < 8; ++e) s[e] = sacc[e >> 2][rb][e & 3];
-      if (edge) {
-        asm volatile("");   // a real branch: as selects these masks would run on every tile
-        const int row_lim = r0 + 16 * rb + lc + offset;   // last key this row may see
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const int key = t * kTileKeys + slot_key(lg, e);
-          if (key > row_lim || key >= p.S) s[e] = -INFINITY;
-        }
-      }
-      float tmax = fa_fmax8(s);
-      tmax = fa_rows_max(tmax) * p.sm_log2e;   // (the scale is positive)
-      const float m_new = fa_fmax(m_run[rb], tmax);
-      const float m_use = m_new == -INFINITY ? 0.f : m_new;   // a row that has seen no key yet
-      alpha[rb] = __builtin_amdgcn_exp2f(m_run[rb] - m_use);   // 0 on the row's first tile
-      float psum = 0.f;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const float pv = __builtin_amdgcn_exp2f(__builtin_fmaf(s[e], p.sm_log2e, -m_use));
-        psum += pv;
-        pb[rb][e] = (_Float16)pv;
-      }
-      l_run[rb] = l_run[rb] * alpha[rb] + psum;
-      m_run[rb] = m_new;
-    }
-    if (__any(alpha[0] != 1.0f || alpha[1] != 1.0f)) {
-#pragma unroll
-      for (int dg = 0; dg < DG; ++dg) {
-        oacc[dg][0] *= alpha[0];
-        oacc[dg][1] *= alpha[1];
-      }
-    }
-    // ---- O^T += V^T . P^T (the fragments in pairs, like the K fragments above)
-    auto o_pair = [&](uint4v& f0, uint4v& f1, int dg) {
+    if (t * kTileKeys + 31 > r0 + offset || t * kTileKeys + 31 >= p.S) {   // wave-uniform
+      asm volatile("");   // a real branch: as selects these masks would run on every tile
 #pragma unroll
       for (int rb = 0; rb < 2; ++rb) {
-        oacc[dg][rb] = Mma<f16_t>::mma(__builtin_bit_cast(half8, f0), pb[rb], oacc[dg][rb]);
-        oacc[dg + 1][rb] = Mma<f16_t>::mma(__builtin_bit_cast(half8, f1), pb[rb], oacc[dg + 1][rb]);
+        const int lim = min(r0 + 16 * rb + lc + offset, p.S - 1) - t * kTileKeys;   // last key of the tile this row may see
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          if (slot_key(lg, e) > lim) sacc[e >> 2][rb][e & 3] = -INFINITY;
       }
+    }
+    // distance of every score from its row's reference (the scale of the softmax rides in the subtraction)
+    float x[2][8];
+    auto distances = [&]() {
+#pragma unroll
+      for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[rb][e] = __builtin_fmaf(sacc[e >> 2][rb][e & 3], p.sm_log2e, -m_run[rb]);
+    };
+    distances();
+    if (__any(fa_fmax(fa_fmax8(x[0]), fa_fmax8(x[1])) > kMaxLag)) {   // always on the first tile: every row sees its first key
+#pragma unroll
+      for (int rb = 0; rb < 2; ++rb) {
+        float s[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) s[e] = sacc[e >> 2][rb][e & 3];
+        const float m_new = fa_fmax(m_run[rb], fa_rows_max(fa_fmax8(s)) * p.sm_log2e);   // (the scale is positive)
+        const float alpha = __builtin_amdgcn_exp2f(m_run[rb] - m_new);
+        m_run[rb] = m_new;
+        l_run[rb] *= alpha;
+#pragma unroll
+        for (int dg = 0; dg < DG; ++dg) oacc[dg][rb] *= alpha;
+      }
+      distances();
+    }
+    half8 pb[2];   // probabilities as f16 operands
+    const half2v ones = {(_Float16)1.f, (_Float16)1.f};
+#pragma unroll
+    for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+      for (int e = 0; e < 8; e += 2) {
+        half2v pv;
+        pv[0] = (_Float16)__builtin_amdgcn_exp2f(x[rb][e]);
+        pv[1] = (_Float16)__builtin_amdgcn_exp2f(x[rb][e + 1]);
+        l_run[rb] = __builtin_amdgcn_fdot2(pv, ones, l_run[rb], false);   // (what the second product weighs the values with)
+        pb[rb][e] = pv[0];
+        pb[rb][e + 1] = pv[1];
+      }
+    // ---- O^T += V^T . P^T (the fragments in pairs, like the K fragments above)
+    auto o_pair = [&](uint4v& f0, uint4v& f1, int dg) {
+      oacc[dg][0] = Mma<f16_t>::mma(__builtin_bit_cast(half8, f0), pb[0], oacc[dg][0]);
+      oacc[dg][1] = Mma<f16_t>::mma(__builtin_bit_cast(half8, f0), pb[1], oacc[dg][1]);
+      oacc[dg + 1][1] = Mma<f16_t>::mma(__builtin_bit_cast(half8, f1), pb[1], oacc[dg + 1][1]);
+      oacc[dg + 1][0] = Mma<f16_t>::mma(__builtin_bit_cast(half8, f1), pb[0], oacc[dg + 1][0]);
     };
     if constexpr (DG == 8) {
       lds_wait_for2<2>(vf[0], vf[1]);

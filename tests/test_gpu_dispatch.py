@@ -59,3 +59,29 @@ def test_any_shape_decode_kernels(dtype, B, Hq, Hkv, D, n_il, L, N, k_counts, v_
         got = ops.decode_attn_raw(g["q"], [(g["k_il"], g["v_il"])], g["k_mc"], g["v_mc"], k_mn, v_mn, *stats, lists, Hq, Hkv, L,
                                   case["T"], force_generic=True)
         assert np.max(np.abs(got.cpu().numpy().astype(np.float64).reshape(want.shape) - want)) <= 2e-4
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("D,S,q_len,G", [(128, 31, 31, 1), (128, 161, 161, 4), (64, 200, 65, 3), (128, 97, 1, 2)])
+@pytest.mark.parametrize("climb", [0.0, 6.0, 40.0, -40.0])
+def test_prompt_attention_with_a_moving_reference(dtype, D, S, q_len, G, climb):
+    """Scores that climb (or fall) along the keys by ``climb`` per key tile, in units of log 2: the softmax reference of a
+    row lags by up to 8 before it moves, so 0 never moves it after the first tile, 6 moves it every other tile, 40
+    every tile.  Bound: f16 probabilities (2^-11 each, averaged) and the rounding of the result, as for the other shapes."""
+    from fourierattention_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(7)
+    q = torch.randn((1, 2 * G, q_len, D), generator=g, device="cuda")
+    k = torch.randn((1, S, 2, D), generator=g, device="cuda")
+    v = torch.randn((1, S, 2, D), generator=g, device="cuda")
+    # one dim of every head carries the climb: q there is 8, k there is the wanted score over q and the scale
+    q[..., 0] = 8.0
+    k[..., 0] = (climb * torch.arange(S, device="cuda") / 32 * np.log(2) * D ** 0.5 / 8.0)[None, :, None]
+    q, k, v = (t.to(dtype) for t in (q, k, v))
+    got = ops.prefill_attention(q, k.reshape(1, S, 2 * D), v.reshape(1, S, 2 * D), 2).double()
+    qd, kd, vd = q.double(), k.double().permute(0, 2, 1, 3).repeat_interleave(G, 1), v.double().permute(0, 2, 1, 3).repeat_interleave(G, 1)
+    s = qd.matmul(kd.transpose(2, 3).contiguous()) / D ** 0.5
+    seen = torch.arange(S, device="cuda")[None, :] <= torch.arange(q_len, device="cuda")[:, None] + S - q_len
+    want = s.masked_fill(~seen, float("-inf")).softmax(-1).matmul(vd).transpose(1, 2)
+    top = float(want.abs().max())
+    ulp = 2.0 ** (np.floor(np.log2(top)) - (7 if dtype == torch.bfloat16 else 10))
+    assert float((got - want).abs().max()) <= 0.5 * ulp + 1e-3
