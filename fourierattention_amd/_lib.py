@@ -15,7 +15,7 @@ LIB_PATH = os.path.join(PKG_DIR, "libfourier_attn_hip.so")
 FA_BF16, FA_FP16, FA_FP32 = 0, 1, 2
 FA_NO_ROUND = FA_FP32
 FA_MID_TOKEN_MAJOR, FA_MID_PAGED = 0, 1
-FA_COLS_ANY, FA_COLS_HEAD_DIMS = 0, 1
+FA_COLS_ANY, FA_COLS_HEAD_DIMS, FA_COLS_IN_ORDER = 0, 1, 2
 DECODE_NOALLOC_SCRATCH_BYTES = 32 << 20
 PAGE_TOKENS, K_DIM_PAD, V_DIM_PAD = 32, 32, 16
 
@@ -111,6 +111,7 @@ _SIGNATURES = {
     "fa_decode_tables_build": (c_int, [c_void_p, c_size_t, c_int, c_int, c_void_p]),
     "fa_mid_pack": (c_int, [c_void_p, c_int, c_int64, c_int64, c_int64, c_int, c_void_p, c_int64, c_int, c_void_p, c_void_p,
                             c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p]),
+    "fa_convert": (c_int, [c_void_p, c_int, c_void_p]),
     "fa_prefill_compress_ok": (c_int, [c_int, c_int, c_int, c_int, c_int, c_int]),
     "fa_prefill_compress_workspace_bytes": (c_size_t, [c_int, c_int, c_int, c_int, c_int]),
     "fa_prefill_compress": (c_int, [c_void_p, c_int, c_int64, c_int64, c_int64, c_int, c_int, c_void_p, c_int64, c_int,
@@ -132,7 +133,7 @@ _SIGNATURES = {
 EXPORTED = tuple(_SIGNATURES)
 
 # bumped with every change of a prototype or of an argument struct (fa_abi_version in the library)
-ABI_VERSION = 3
+ABI_VERSION = 4
 
 _lib = None
 

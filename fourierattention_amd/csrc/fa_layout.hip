@@ -134,6 +134,110 @@ __global__ __launch_bounds__(256) void mid_pack_rows_kernel(
   }
 }
 
+// Rows whose columns are the stored dims already, head by head (the reference's own k_uncompressed / v_uncompressed): head
+// h's run of n_h[h+1] - n_h[h] columns is read in pieces of eight, at whatever alignment the run has, and no index list is
+// involved.  A piece of a K fragment is eight neighbouring dims of one token, i.e. one piece of the source: it goes from
+// register to store.  V pieces hold eight tokens of one dim and turn round in LDS, kRunPages pages per block.
+// Bound by the chain of a block (offsets, rows, LDS, store) with eight blocks per compute unit: 15356 rows x 512 columns of
+// two sequences in 16 us (4 TB/s read and written), against 33 us through mid_pack_kernel's index list, whose loads
+// bring one element per lane.  Two pages per block let a thread have two pieces in flight.
+constexpr int kRunPages = 2;
+
+template <typename E, int MAXD>
+__global__ __launch_bounds__(256) void mid_pack_runs_kernel(
+    const E* __restrict__ src, int64_t src_bs, int64_t src_rs, int64_t row0, int L, E* __restrict__ store,
+    int64_t st_bs, int cap_pages, const int32_t* __restrict__ n_h, const int32_t* __restrict__ pad_h, int is_v) {
+  constexpr int kPitch = MAXD + 8;
+  struct alignas(sizeof(E) * 8) Piece { E v[8]; };
+  typedef uint64_t u64x2 __attribute__((ext_vector_type(2)));
+  __shared__ __attribute__((aligned(32))) E tile[kRunPages * 32][kPitch];
+  const int h = blockIdx.y, b = blockIdx.z, tid = threadIdx.x;
+  const int page0 = blockIdx.x * kRunPages;
+  const int n0 = n_h[h], n_len = n_h[h + 1] - n0;
+  const int p0 = pad_h[h], dp = pad_h[h + 1] - p0;
+  if (n_len <= 0) return;
+  const int n_pages = min(kRunPages, ((L + 31) >> 5) - page0);
+  const E* sb = src + (int64_t)b * src_bs + (row0 + (int64_t)page0 * 32) * src_rs + n0;
+  const int rows = min(n_pages * 32, L - page0 * 32);          // rows of the source behind this block's pages
+  // dims j0 .. j0 + 7 of row t; zeros past the head's dims and past the rows
+  auto fetch = [&](int t, int j0) {
+    const E* row = sb + (int64_t)min(t, rows - 1) * src_rs;
+    if constexpr (sizeof(E) == 2) if (n_len >= 8) {
+      // one load at whatever alignment the run has; the last piece of a run is read so that it ends with the run
+      const int s0 = min(j0, n_len - 8), past = t < rows ? j0 - s0 : 8;     // past: elements the load starts too early
+      u64x2 x;
+      __builtin_memcpy(&x, row + s0, 16);
+      const int by = past * 16;
+      const uint64_t lo = by == 0 ? x.x : by < 64 ? (x.x >> by) | (x.y << (64 - by)) : by < 128 ? x.y >> (by - 64) : 0;
+      const uint64_t hi = by < 64 ? x.y >> by : 0;
+      x.x = lo;
+      x.y = hi;
+      return __builtin_bit_cast(Piece, x);
+    }
+    Piece o;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const E x = row[min(j0 + e, n_len - 1)];
+      o.v[e] = (t < rows && j0 + e < n_len) ? x : E{};
+    }
+    return o;
+  };
+  Piece* out = (Piece*)(store + (int64_t)b * st_bs + (int64_t)p0 * 32 * cap_pages + (int64_t)page0 * dp * 32);
+  const int per_page = dp * 4;                                 // pieces of a page
+  const int n_pieces = n_pages * per_page;
+  if (!is_v) {
+    const int nks = dp >> 5;
+#pragma unroll 2
+    for (int q = tid; q < n_pieces; q += 256) {
+      const int f = q >> 6, lane = q & 63;                     // fragment (page, tb, s) of the block, lane of the fragment
+      const int ptb = f / nks, s_ = f - ptb * nks;
+      out[q] = fetch(ptb * 16 + (lane & 15), s_ * 32 + 8 * (lane >> 4));
+    }
+    return;
+  }
+  const int ppr = dp >> 3;                                     // pieces per row
+#pragma unroll 2
+  for (int q = tid; q < n_pages * 32 * ppr; q += 256) {
+    const int t = q / ppr, c = q - t * ppr;
+    *(Piece*)&tile[t][c * 8] = fetch(t, c * 8);
+  }
+  __syncthreads();
+  const int frags = dp >> 4;
+  for (int q = tid; q < n_pieces; q += 256) {
+    const int f = q >> 6, lane = q & 63;
+    const int pg = f / frags, dg = f - pg * frags;
+    Piece o;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) o.v[i] = tile[pg * 32 + 8 * (lane >> 4) + i][dg * 16 + (lane & 15)];
+    out[q] = o;
+  }
+}
+
+// Operands of a call in the types the kernels take, all in one launch: a grid row per item, items in the argument block.
+constexpr int kMaxConvert = 16;
+struct ConvertArgs { fa_convert_item item[kMaxConvert]; };
+
+__global__ __launch_bounds__(256) void convert_kernel(const ConvertArgs a) {
+  const fa_convert_item it = a.item[blockIdx.y];
+  const int64_t step = (int64_t)gridDim.x * 256;
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < it.count; i += step) {
+    switch (it.kind) {
+      case FA_CONVERT_I64_I32: ((int32_t*)it.dst)[i] = (int32_t)((const int64_t*)it.src)[i]; break;
+      case FA_CONVERT_BF16_F32: ((float*)it.dst)[i] = fa_to_float(((const bf16_t*)it.src)[i]); break;
+      case FA_CONVERT_F16_F32: ((float*)it.dst)[i] = fa_to_float(((const f16_t*)it.src)[i]); break;
+      default: {   // offsets of counts rounded up to whole units (at most a few dozen heads: every entry sums for itself)
+        int32_t sum = 0;
+        for (int64_t h = 0; h < i; ++h) {
+          const int32_t n = it.kind == FA_CONVERT_PAD_I64 ? (int32_t)(((const int64_t*)it.src)[h + 1] - ((const int64_t*)it.src)[h])
+                                                          : ((const int32_t*)it.src)[h + 1] - ((const int32_t*)it.src)[h];
+          sum += (n + it.unit - 1) / it.unit * it.unit;
+        }
+        ((int32_t*)it.dst)[i] = sum;
+      }
+    }
+  }
+}
+
 template <typename E>
 __global__ __launch_bounds__(256) void mid_append_kernel(
     const E* __restrict__ row, int64_t row_bs, int64_t pos, E* __restrict__ store, int64_t st_bs, int cap_pages,
@@ -182,8 +286,8 @@ extern "C" int fa_mid_pack(const void* src, int dtype, int64_t src_bs, int64_t s
                            void* store, int64_t st_bs, int cap_pages, const int32_t* n_list, const int32_t* n_h,
                            const int32_t* pad_h, int B, int Hkv, int D, int is_v, int cols_kind, fa_stream_t stream) {
   FA_REQUIRE(src && store && n_h && pad_h, FA_ERR_NULL_POINTER, "fa_mid_pack: null pointer");
-  FA_REQUIRE(cols_kind == FA_COLS_ANY || cols_kind == FA_COLS_HEAD_DIMS, FA_ERR_BAD_SHAPE, "fa_mid_pack: cols_kind %d",
-             cols_kind);
+  FA_REQUIRE(cols_kind == FA_COLS_ANY || cols_kind == FA_COLS_HEAD_DIMS || cols_kind == FA_COLS_IN_ORDER, FA_ERR_BAD_SHAPE,
+             "fa_mid_pack: cols_kind %d", cols_kind);
   FA_REQUIRE(B > 0 && Hkv > 0 && L >= 0 && cap_pages > 0 && row0 >= 0, FA_ERR_BAD_SHAPE, "fa_mid_pack: bad shape");
   FA_REQUIRE((int64_t)cap_pages * 32 >= L, FA_ERR_BAD_SHAPE, "fa_mid_pack: %d rows do not fit %d pages", L, cap_pages);
   if (L == 0) return FA_OK;
@@ -199,6 +303,16 @@ extern "C" int fa_mid_pack(const void* src, int dtype, int64_t src_bs, int64_t s
              "fa_mid_pack: rows of %lld elements cannot hold %d heads of %d dims", (long long)src_rs, Hkv, D);
   int rc = dispatch16(dtype, "fa_mid_pack", [&](auto tag) {
     using E = decltype(tag);
+    if (cols_kind == FA_COLS_IN_ORDER) {
+      const dim3 rgrid(fa_cdiv(fa_cdiv(L, 32), kRunPages), Hkv, B);
+      if (D <= 128)
+        mid_pack_runs_kernel<E, 128><<<rgrid, 256, 0, st>>>((const E*)src, src_bs, src_rs, row0, L, (E*)store, st_bs, cap_pages,
+                                                           n_h, pad_h, is_v);
+      else
+        mid_pack_runs_kernel<E, 256><<<rgrid, 256, 0, st>>>((const E*)src, src_bs, src_rs, row0, L, (E*)store, st_bs, cap_pages,
+                                                           n_h, pad_h, is_v);
+      return;
+    }
     if constexpr (sizeof(E) == 2) {
       if (rows16) {
         mid_pack_rows_kernel<E><<<grid, 256, 0, st>>>((const E*)src, src_bs, src_rs, row0, L, (E*)store, st_bs, cap_pages,
@@ -210,6 +324,25 @@ extern "C" int fa_mid_pack(const void* src, int dtype, int64_t src_bs, int64_t s
                                             n_h, pad_h, is_v);
   });
   return rc != FA_OK ? rc : fa_check_launch("fa_mid_pack");
+}
+
+extern "C" int fa_convert(const fa_convert_item* items, int n, fa_stream_t stream) {
+  FA_REQUIRE(items || n == 0, FA_ERR_NULL_POINTER, "fa_convert: null pointer");
+  FA_REQUIRE(n >= 0 && n <= kMaxConvert, FA_ERR_BAD_SHAPE, "fa_convert: %d items (at most %d)", n, kMaxConvert);
+  ConvertArgs a{};
+  int64_t most = 0;
+  for (int i = 0; i < n; ++i) {
+    const fa_convert_item& it = items[i];
+    FA_REQUIRE(it.count >= 0 && (it.count == 0 || (it.src && it.dst)), FA_ERR_NULL_POINTER, "fa_convert: item %d", i);
+    FA_REQUIRE(it.kind >= FA_CONVERT_I64_I32 && it.kind <= FA_CONVERT_PAD_I32, FA_ERR_BAD_DTYPE, "fa_convert: kind %d", it.kind);
+    FA_REQUIRE(it.kind < FA_CONVERT_PAD_I64 || it.unit > 0, FA_ERR_BAD_SHAPE, "fa_convert: unit %d", it.unit);
+    a.item[i] = it;
+    if (it.count > most) most = it.count;
+  }
+  if (most == 0) return FA_OK;
+  const int64_t blocks = (most + 255) / 256;
+  convert_kernel<<<dim3((unsigned)(blocks < 64 ? blocks : 64), n), 256, 0, fa_hip_stream(stream)>>>(a);
+  return fa_check_launch("fa_convert");
 }
 
 extern "C" int fa_mid_append(const void* row, int dtype, int64_t row_bs, int64_t pos, void* store, int64_t st_bs,

@@ -400,6 +400,109 @@ PyObject* rope_qk(PyObject*, PyObject* const* a, Py_ssize_t n) {
   FA_END
 }
 
+// operands(lists, stats, k_unit, v_unit) -> (lists, stats, paging)
+// The index lists (a tuple of eight: kc, kc_h, kn, kn_h, vc, vc_h, vn, vn_h) as int32 and the statistics (a tuple) as
+// contiguous float32, those that are not of these types already in one launch and one allocation.  With k_unit > 0 also
+// what a page store of the stored dims needs: paging = (kn_h, vn_h on the host, padded offsets of K and V on the device),
+// one copy and one wait for it; None otherwise.
+PyObject* operands(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  FA_BEGIN
+  CHECK(n == 4 && PyTuple_Check(a[0]) && PyTuple_GET_SIZE(a[0]) == 8 && PyTuple_Check(a[1]), "operands takes 4 arguments");
+  const Py_ssize_t n_st = PyTuple_GET_SIZE(a[1]);
+  CHECK(n_st <= 6, "operands: at most six statistics");
+  const int32_t k_unit = (int32_t)integer(a[2]), v_unit = (int32_t)integer(a[3]);
+  const at::Tensor& first = gpu_tensor(PyTuple_GET_ITEM(a[0], 0), "list");
+  const at::Device dev = first.device();
+  at::Tensor lists[8], stats[6];
+  fa_convert_item items[16];
+  int64_t at_item[16];
+  int n_items = 0;
+  int64_t used = 0;                                      // in 4-byte elements, every piece at a multiple of 16 bytes
+  auto add = [&](const at::Tensor& src, int64_t count, int kind, int unit) {
+    items[n_items] = fa_convert_item{src.numel() ? src.data_ptr() : nullptr, nullptr, count, kind, unit};
+    at_item[n_items] = used;
+    used += (count + 3) / 4 * 4;
+    return n_items++;
+  };
+  int list_item[8], stat_item[6], pad_item[2] = {-1, -1};
+  // (the per-head offsets first: they go to the host in one piece)
+  static const int order[8] = {3, 7, 0, 1, 2, 4, 5, 6};
+  for (int o : order) {
+    const at::Tensor& t = tensor(PyTuple_GET_ITEM(a[0], o), "list");
+    list_item[o] = -1;
+    if (t.scalar_type() == at::kInt) lists[o] = t;
+    else if (t.scalar_type() == at::kLong && t.is_contiguous() && t.device() == dev) list_item[o] = add(t, t.numel(), FA_CONVERT_I64_I32, 1);
+    else lists[o] = t.to(at::kInt);
+  }
+  for (Py_ssize_t i = 0; i < n_st; ++i) {
+    const at::Tensor& t = tensor(PyTuple_GET_ITEM(a[1], i), "statistics");
+    stat_item[i] = -1;
+    const bool here = t.is_contiguous() && t.device() == dev;
+    if (here && t.scalar_type() == at::kBFloat16) stat_item[i] = add(t, t.numel(), FA_CONVERT_BF16_F32, 1);
+    else if (here && t.scalar_type() == at::kHalf) stat_item[i] = add(t, t.numel(), FA_CONVERT_F16_F32, 1);
+    else stats[i] = t.to(at::kFloat).contiguous();
+  }
+  if (k_unit > 0) {
+    for (int i = 0; i < 2; ++i) {
+      const int o = i ? 7 : 3;
+      const at::Tensor& t = tensor(PyTuple_GET_ITEM(a[0], o), "list");
+      const bool wide = list_item[o] >= 0;
+      const at::Tensor& src = wide ? t : lists[o];
+      CHECK(src.is_contiguous() && src.device() == dev && src.numel() >= 1, "per-head offsets: contiguous, on the GPU");
+      pad_item[i] = add(src, src.numel(), wide ? FA_CONVERT_PAD_I64 : FA_CONVERT_PAD_I32, i ? v_unit : k_unit);
+    }
+  }
+  at::Tensor arena;
+  if (used > 0) {
+    arena = at::empty({used}, at::TensorOptions().dtype(at::kInt).device(dev));
+    for (int i = 0; i < n_items; ++i) items[i].dst = static_cast<int32_t*>(arena.data_ptr()) + at_item[i];
+    check_status(fa_convert(items, n_items, stream_of(arena)));
+  }
+  auto part = [&](int item) { return arena.narrow(0, at_item[item], items[item].count); };
+  Ref out(PyTuple_New(3));
+  PyObject* ls = PyTuple_New(8);
+  PyTuple_SET_ITEM(out.p, 0, ls);
+  for (int o = 0; o < 8; ++o) {
+    if (list_item[o] >= 0) lists[o] = part(list_item[o]);
+    PyTuple_SET_ITEM(ls, o, THPVariable_Wrap(lists[o]));
+  }
+  PyObject* ss = PyTuple_New(n_st);
+  PyTuple_SET_ITEM(out.p, 1, ss);
+  for (Py_ssize_t i = 0; i < n_st; ++i) {
+    const at::Tensor& t = tensor(PyTuple_GET_ITEM(a[1], i), "statistics");
+    if (stat_item[i] >= 0) stats[i] = part(stat_item[i]).view(at::kFloat).view(t.sizes());
+    PyTuple_SET_ITEM(ss, i, THPVariable_Wrap(stats[i]));
+  }
+  if (k_unit <= 0) {
+    Py_INCREF(Py_None);
+    PyTuple_SET_ITEM(out.p, 2, Py_None);
+    Py_INCREF(out.p);
+    return out.p;
+  }
+  PyObject* paging = PyTuple_New(4);
+  PyTuple_SET_ITEM(out.p, 2, paging);
+  const bool one = list_item[3] == 0 && list_item[7] == 1;
+  at::Tensor host[2];
+  if (one) {
+    const at::Tensor both = arena.narrow(0, 0, at_item[1] + items[1].count).cpu();
+    for (int i = 0; i < 2; ++i) host[i] = both.narrow(0, at_item[i], items[i].count);
+  } else {
+    host[0] = lists[3].cpu();
+    host[1] = lists[7].cpu();
+  }
+  for (int i = 0; i < 2; ++i) {
+    const int64_t len = host[i].numel();
+    PyObject* l = PyList_New(len);
+    PyTuple_SET_ITEM(paging, i, l);
+    const int32_t* v = static_cast<const int32_t*>(host[i].data_ptr());
+    for (int64_t j = 0; j < len; ++j) PyList_SET_ITEM(l, j, PyLong_FromLong(v[j]));
+    PyTuple_SET_ITEM(paging, 2 + i, THPVariable_Wrap(part(pad_item[i])));
+  }
+  Py_INCREF(out.p);
+  return out.p;
+  FA_END
+}
+
 // init(stream_fn, check_fn, workspace_fn)
 PyObject* init(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (n != 3) {
@@ -416,7 +519,7 @@ PyObject* init(PyObject*, PyObject* const* a, Py_ssize_t n) {
 }
 
 #define FN(name) {#name, (PyCFunction)(void*)name, METH_FASTCALL, nullptr}
-PyMethodDef methods[] = {FN(init), FN(stream_update), FN(decode_attn), FN(add_rmsnorm), FN(linear_packed), FN(silu_mul), FN(rope_qk),
+PyMethodDef methods[] = {FN(init), FN(stream_update), FN(decode_attn), FN(add_rmsnorm), FN(linear_packed), FN(silu_mul), FN(rope_qk), FN(operands),
                          {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_fa_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 

@@ -15,7 +15,10 @@ from .ops import _stream, dtype_code
 
 class MidStore:
     def __init__(self, batch: int, n_list32: torch.Tensor, n_h32: torch.Tensor, n_h_host: List[int], num_kv_heads: int,
-                 head_dim: int, cap_tokens: int, dtype: torch.dtype, device, is_v: bool):
+                 head_dim: int, cap_tokens: int, dtype: torch.dtype, device, is_v: bool, pad_h32=None, zeroed: bool = True):
+        """``pad_h32``: the padded per-head offsets where the caller has them on the device already.  ``zeroed=False``: the
+        caller packs rows for every page of the store right away (``pack`` writes its pages whole).  ``n_list32`` may be
+        ``None`` for a store that only ever packs rows whose columns are the stored dims in order."""
         self.B, self.Hkv, self.D, self.is_v = batch, num_kv_heads, head_dim, bool(is_v)
         self.n_list32, self.n_h32 = n_list32, n_h32
         self.Cn = int(n_h_host[-1])
@@ -26,32 +29,35 @@ class MidStore:
             pad.append(pad[-1] + (n + unit - 1) // unit * unit)
         self.pad_h_host = pad
         self.max_pad = max([pad[h + 1] - pad[h] for h in range(num_kv_heads)] + [0])
-        self.pad_h32 = torch.tensor(pad, dtype=torch.int32, device=device)
+        self.pad_h32 = torch.tensor(pad, dtype=torch.int32, device=device) if pad_h32 is None else pad_h32
         self.dtype, self.device = dtype, torch.device(device)
-        self._alloc(cap_tokens)
+        self._alloc(cap_tokens, zeroed)
 
-    def _alloc(self, cap_tokens: int):
+    def _alloc(self, cap_tokens: int, zeroed: bool = True):
         self.cap_pages = max(1, (int(cap_tokens) + PAGE_TOKENS - 1) // PAGE_TOKENS)
         self.batch_stride = self.pad_h_host[-1] * PAGE_TOKENS * self.cap_pages
         # zero-filled: padded dims and unused token slots must read as zero
-        self.data = torch.zeros(max(self.B * self.batch_stride, 8), dtype=self.dtype, device=self.device)
+        self.data = (torch.zeros if zeroed else torch.empty)(max(self.B * self.batch_stride, 8), dtype=self.dtype, device=self.device)
 
     @property
     def cap_tokens(self) -> int:
         return self.cap_pages * PAGE_TOKENS
 
-    def pack(self, src: torch.Tensor, row0: int, rows: int, n_list32=None, head_dims: bool = False) -> None:
+    def pack(self, src: torch.Tensor, row0: int, rows: int, n_list32=None, head_dims: bool = False, in_order: bool = False) -> None:
         """Store ``src[:, row0:row0+rows, n_list]`` (``src (B, S, width)``, last dim contiguous) from token 0.
         ``head_dims``: ``src`` holds full K/V rows and the list is the reference's ``kn_list`` / ``vn_list`` (flat
-        ``h*D + d`` entries, head by head); otherwise the entries are plain column numbers of ``src``."""
+        ``h*D + d`` entries, head by head); ``in_order``: the columns of ``src`` are the stored dims already and no list
+        is read; otherwise the entries are plain column numbers of ``src``."""
         assert src.dim() == 3 and src.stride(2) == 1 and src.dtype == self.dtype and rows <= self.cap_tokens
+        assert not in_order or (src.shape[2] >= self.Cn and self.max_pad <= (self.D + 31) // 32 * 32)
         if rows == 0 or self.Cn == 0:
             return
         nl = self.n_list32 if n_list32 is None else n_list32
+        kind = _lib.FA_COLS_IN_ORDER if in_order else _lib.FA_COLS_HEAD_DIMS if head_dims else _lib.FA_COLS_ANY
         check(_lib.load().fa_mid_pack(src.data_ptr(), dtype_code(src.dtype), src.stride(0), src.stride(1), int(row0), int(rows),
-                                      self.data.data_ptr(), self.batch_stride, self.cap_pages, nl.data_ptr(),
+                                      self.data.data_ptr(), self.batch_stride, self.cap_pages, None if in_order else nl.data_ptr(),
                                       self.n_h32.data_ptr(), self.pad_h32.data_ptr(), self.B, self.Hkv, self.D,
-                                      int(self.is_v), _lib.FA_COLS_HEAD_DIMS if head_dims else _lib.FA_COLS_ANY,
+                                      int(self.is_v), kind,
                                       _stream(self.device)))
 
     def pack_and_compress(self, src: torch.Tensor, row0: int, rows: int, fft_rows: int, c_list32: torch.Tensor,
@@ -105,5 +111,4 @@ class MidStore:
         """Re-page into a larger store (the head regions move when the capacity changes)."""
         dense = self.dense(rows_in_use)
         self._alloc(new_cap_tokens)
-        ident = torch.arange(self.Cn, dtype=torch.int32, device=self.device)
-        self.pack(dense, 0, rows_in_use, n_list32=ident)
+        self.pack(dense, 0, rows_in_use, in_order=True)

@@ -270,18 +270,39 @@ enum fa_mid_layout { FA_MID_TOKEN_MAJOR = 0, FA_MID_PAGED = 1 };
 #define FA_COLS_HEAD_DIMS 1 /* the source rows are full K/V rows of Hkv*D elements and the entries of head h
                                lie in [h*D, (h+1)*D): the reference's kn_list / vn_list (CACHE:445-447) */
 
+#define FA_COLS_IN_ORDER 2  /* the source rows hold the stored dims already, in order: column n_h[h] + j is stored dim j
+                               of head h (the reference's k_uncompressed / v_uncompressed).  No list is read */
+
 /* Scatter rows [row0, row0 + L) of src (B, S, width), taking for each head the
  * columns n_list[n_h[h] .. n_h[h+1]) (the gather x[:, :, kn] of CACHE:560, 578),
  * into pages starting at token 0.  is_v selects the V fragment order.  With
  * cols_kind == FA_COLS_HEAD_DIMS (and 16-bit, 16-byte aligned rows) the head's
  * slice of every row is read whole and the stored dims are picked from it, which
  * is faster; entries outside the head's range then read a clamped dim.  With
- * FA_COLS_ANY (e.g. an identity list over rows that are gathered already) every
- * element is fetched by its own column number. */
+ * FA_COLS_ANY every element is fetched by its own column number.  With
+ * FA_COLS_IN_ORDER (n_list may be null) the head's columns are read as a run.
+ * Every page of the rows is written whole, padded dims and token slots past L as zeros. */
 int fa_mid_pack(const void* src, int dtype, int64_t src_batch_stride, int64_t src_row_stride, int64_t row0,
                 int L, void* store, int64_t store_batch_stride, int cap_pages, const int32_t* n_list,
                 const int32_t* n_h_list, const int32_t* pad_h_list, int B, int Hkv, int D, int is_v,
                 int cols_kind, fa_stream_t stream);
+
+/* Small operands of a call (index lists, statistics) in the types the kernels take, all in one launch of at most 16
+ * items: dst[i] = src[i] converted, for i < count; with the FA_CONVERT_PAD kinds src holds per-head offsets with the
+ * leading 0 and dst[h] = sum over g < h of (src[g+1] - src[g]) rounded up to whole units (the pad_h list of a page
+ * store).  Items must not overlap. */
+#define FA_CONVERT_I64_I32 0
+#define FA_CONVERT_BF16_F32 1
+#define FA_CONVERT_F16_F32 2
+#define FA_CONVERT_PAD_I64 3
+#define FA_CONVERT_PAD_I32 4
+typedef struct fa_convert_item {
+  const void* src;
+  void* dst;
+  int64_t count;
+  int32_t kind, unit;
+} fa_convert_item;
+int fa_convert(const fa_convert_item* items, int n, fa_stream_t stream);
 
 /* The prompt's mid rows of K (or V) in one pass: what the cache's prefill does with them in CACHE:560-565 (K) and
  * CACHE:578-587 (V) -- keep the stored dims (fa_mid_pack with FA_COLS_HEAD_DIMS), transform the first K_fft rows of

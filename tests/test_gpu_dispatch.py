@@ -85,3 +85,49 @@ def test_prompt_attention_with_a_moving_reference(dtype, D, S, q_len, G, climb):
     top = float(want.abs().max())
     ulp = 2.0 ** (np.floor(np.log2(top)) - (7 if dtype == torch.bfloat16 else 10))
     assert float((got - want).abs().max()) <= 0.5 * ulp + 1e-3
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("B,D,rows,extra,counts", [
+    (1, 128, 1, 0, [128, 1]),                 # one row; a full head and a single dim
+    (2, 128, 65, 3, [7, 0, 120, 33]),         # a page of one row in the second block; runs at odd columns, odd row length
+    (1, 64, 2080, 0, [64, 9, 17]),            # whole pages, an odd number of them
+    (3, 200, 96, 5, [200, 150]),              # heads above 128 dims
+])
+def test_pages_of_rows_in_order(dtype, B, D, rows, extra, counts):
+    """Columns that are the stored dims already against the same pack through an index list into a zero-filled store: the
+    pages bit for bit, in a store that held NaN, from rows that are slices of wider rows."""
+    from fourierattention_amd.midstore import MidStore
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    cn = sum(counts)
+    src = torch.randn((B, rows, cn + extra), generator=g, device="cuda").to(dtype)[:, :, extra:]
+    n_h_host = [sum(counts[:i]) for i in range(len(counts) + 1)]
+    n_h = torch.tensor(n_h_host, dtype=torch.int32, device="cuda")
+    ident = torch.arange(cn, dtype=torch.int32, device="cuda")
+    for is_v in (False, True):
+        want, got = (MidStore(B, ident, n_h, n_h_host, len(counts), D, rows, dtype, "cuda", is_v) for _ in range(2))
+        want.pack(src, 0, rows)
+        got.data.fill_(float("nan"))
+        got.pack(src, 0, rows, in_order=True)
+        assert torch.equal(got.data, want.data)
+        assert torch.equal(got.dense(rows), src)
+
+
+@pytest.mark.parametrize("list_dtype", [torch.int64, torch.int32])
+@pytest.mark.parametrize("stat_dtype", [torch.bfloat16, torch.float16, torch.float32, torch.float64])
+def test_operands_in_the_types_the_kernels_take(list_dtype, stat_dtype):
+    """Lists, statistics (empty and strided ones among them) and padded offsets against the tensor operations."""
+    from fourierattention_amd import _lib
+    g = torch.Generator(device="cuda").manual_seed(5)
+    lists = tuple(torch.randint(0, 1000, (n,), generator=g, device="cuda").to(list_dtype) for n in (0, 9, 1023, 9, 257, 9, 1, 9))
+    heads = [torch.tensor([0] + [int(x) for x in torch.randint(0, 129, (8,)).cumsum(0)], device="cuda", dtype=list_dtype) for _ in range(2)]
+    lists = lists[:3] + (heads[0],) + lists[4:7] + (heads[1],)
+    stats = tuple(torch.randn((2, 2 * n), generator=g, device="cuda").to(stat_dtype)[:, ::s] for n, s in ((0, 1), (1, 2), (300, 1), (17, 2), (4, 1), (1023, 1)))
+    l32, s32, paging = _lib.load_host().operands(lists, stats, 32, 16)
+    assert all(a.dtype == torch.int32 and torch.equal(a, b.to(torch.int32)) for a, b in zip(l32, lists))
+    assert all(a.dtype == torch.float32 and a.is_contiguous() and torch.equal(a, b.float()) for a, b in zip(s32, stats))
+    for i, unit in enumerate((32, 16)):
+        n = heads[i].cpu().diff()
+        pad = torch.cat([torch.zeros(1, dtype=n.dtype), ((n + unit - 1) // unit * unit).cumsum(0)])
+        assert paging[i] == heads[i].tolist() and paging[2 + i].tolist() == pad.tolist()
+    assert _lib.load_host().operands(lists, stats, 0, 0)[2] is None
