@@ -26,33 +26,41 @@ constexpr int kWgCols = 64;                    // columns per workgroup (four co
 
 // ---- basis table: A operands E[row tile rt][kstep][lane] x half8, row r of a tile = frequency rt*8 + r/2,
 // cos (r even) or sin (r odd); lane l holds row l % 16, tokens 8 * (l / 16) + e of the kstep ----------------
-__global__ __launch_bounds__(256) void spectral_table_kernel(half8* __restrict__ tab, int N, int T) {
+// A thread takes two tokens of a frequency and writes both rows: one evaluation per phase (a thread per row would
+// evaluate every phase twice), short chains (7.4 -> 5.6 us for 512 frequencies).
+constexpr int kTableThreads = kStepK * 128;    // per row tile
+__global__ __launch_bounds__(256) void spectral_table_kernel(half2v* __restrict__ tab, int N, int T) {
   const int idx = blockIdx.x * 256 + threadIdx.x;
-  const int total = (N / 8) * kStepK * 64;
-  if (idx >= total) return;
-  const int lane = idx & 63, ks = (idx >> 6) % kStepK, rt = idx / (64 * kStepK);
-  const int r = lane & 15, lg = lane >> 4;
-  const int n = rt * 8 + (r >> 1);
-  half8 v;
+  if (idx >= (N / 8) * kTableThreads) return;
+  const int ep = idx & 3, f = (idx >> 2) & 7, lg = (idx >> 5) & 3, frag = idx >> 7;   // frag = rt * kStepK + ks
+  const int n = frag / kStepK * 8 + f, token = frag % kStepK * 32 + 8 * lg + 2 * ep;
+  half2v c, s;
 #pragma unroll
-  for (int e = 0; e < 8; ++e) {
+  for (int e = 0; e < 2; ++e) {
     float sn, co;
-    fa_sincos_phase(n, ks * 32 + 8 * lg + e, T, &sn, &co);
-    v[e] = (_Float16)((r & 1) ? sn : co);
+    fa_sincos_phase(n, token + e, T, &sn, &co);
+    c[e] = (_Float16)co;
+    s[e] = (_Float16)sn;
   }
-  tab[idx] = v;
+  half2v* out = tab + ((int64_t)frag * 64 + lg * 16 + 2 * f) * 4 + ep;
+  out[0] = c;
+  out[4] = s;
 }
 
 // ---- pack: block = 32 tokens x 256 columns; lanes run along the columns for the gather, the transposition to
-// token-contiguous fragments goes through LDS ----------------------------------------------------------------
+// token-contiguous fragments goes through LDS.  grid (ksteps, column blocks, parts * B): part p of the input starts
+// p * a_part elements behind the first and its fragments p * out_part behind the first's ------------------------
 template <typename E>
 __global__ __launch_bounds__(256) void spectral_pack_kernel(
     const E* __restrict__ a, int64_t a_bs, int64_t a_rs, const int32_t* __restrict__ cols,
-    const float* __restrict__ col_inv_scale, half8* __restrict__ out, int K, int Mc, int CT, int KS32) {
+    const float* __restrict__ col_inv_scale, half8* __restrict__ out, int K, int Mc, int CT, int KS32, int B, int64_t a_part,
+    int64_t out_part) {
   constexpr int kPitch = 256 + 4;   // f16 elements per LDS row: 8 rows apart = 16 banks apart
   __shared__ _Float16 tile[32][kPitch];
   const int tid = threadIdx.x;
-  const int ks = blockIdx.x, m0 = blockIdx.y * 256, b = blockIdx.z;
+  const int ks = blockIdx.x, m0 = blockIdx.y * 256, part = blockIdx.z / B, b = blockIdx.z - part * B;
+  a += part * a_part;
+  out += part * out_part;
   const int m = m0 + tid;
   const bool mok = m < Mc;
   const int col = mok ? (cols ? cols[m] : m) : 0;
@@ -207,6 +215,53 @@ __global__ __launch_bounds__(256) void prefill_pack_kernel(const PrefillPackPara
   }
 }
 
+// One step of the Horner walk: acc <- E * (the step's four column tiles in LDS) + rotation * acc.  The tiles of a kstep
+// ((j, ks) at lds + (4 j + ks) KiB) are requested one kstep ahead of the products that take them, the first ones in
+// front of the rotation, which has 128 vector instructions to cover them: a wave that read and then waited spent longer
+// on LDS latency than on its matrix instructions.  No branch between a request and its wait (accumulators start as
+// zeros, which rotate to zeros).  32768 rows x 512 columns, 512 frequencies: 37.8 -> 34.8 us (990 TFLOP/s), reconstruction
+// statistics of the same size 56 -> 48 us together with the scales kept in LDS.
+__device__ __forceinline__ void spectral_step(float4v (&acc)[4][4], const half8 (&Ea)[4][kStepK], const float (&rc)[4][2],
+                                              const float (&rs)[4][2], unsigned lds) {
+  uint4v b0[4], b1[4];
+#define FA_STEP_READ(B, ks)                                   \
+  B[0] = lds_read_b128_async_at<(0 * kStepK + (ks)) * 1024>(lds); \
+  B[1] = lds_read_b128_async_at<(1 * kStepK + (ks)) * 1024>(lds); \
+  B[2] = lds_read_b128_async_at<(2 * kStepK + (ks)) * 1024>(lds); \
+  B[3] = lds_read_b128_async_at<(3 * kStepK + (ks)) * 1024>(lds)
+  auto products = [&](const uint4v (&b)[4], int ks) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Ea[i][ks], __builtin_bit_cast(half8, b[j]), acc[i][j], 0, 0, 0);
+  };
+  static_assert(kStepK == 4, "four ksteps, two register sets");
+  FA_STEP_READ(b0, 0);
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int f2 = 0; f2 < 2; ++f2) {
+        const float c = acc[i][j][2 * f2], sn = acc[i][j][2 * f2 + 1];
+        acc[i][j][2 * f2] = rc[i][f2] * c - rs[i][f2] * sn;
+        acc[i][j][2 * f2 + 1] = rs[i][f2] * c + rc[i][f2] * sn;
+      }
+  FA_STEP_READ(b1, 1);
+  lds_wait_for4<4>(b0);
+  products(b0, 0);
+  FA_STEP_READ(b0, 2);
+  lds_wait_for4<4>(b1);
+  products(b1, 1);
+  FA_STEP_READ(b1, 3);
+  lds_wait_for4<4>(b0);
+  products(b0, 2);
+  lds_wait_for4<0>(b1);
+  products(b1, 3);
+#undef FA_STEP_READ
+}
+
 struct SpectralGemmParams {
   const half8* tab;      // basis table
   const half8* packed;   // [B][CT][KS32][64] fragments
@@ -270,30 +325,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     else wait_vmcnt<0>();
     barrier_lds_only();   // every wave's share of step s has landed; nobody still reads the stage refilled next
     if (it + NST - 1 < n_it) issue(s - (NST - 1), (it + NST - 1) % NST);
-    if (it > 0) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-          for (int f2 = 0; f2 < 2; ++f2) {
-            const float c = acc[i][j][2 * f2], sn = acc[i][j][2 * f2 + 1];
-            acc[i][j][2 * f2] = rc[i][f2] * c - rs[i][f2] * sn;
-            acc[i][j][2 * f2 + 1] = rs[i][f2] * c + rc[i][f2] * sn;
-          }
-    }
-#pragma unroll
-    for (int ks = 0; ks < kStepK; ++ks) {
-      uint4v braw[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) braw[j] = lds_read_b128_async(&s_stage[stage][j][ks][lane * 16]);
-      lds_wait_for4<0>(braw);
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Ea[i][ks], __builtin_bit_cast(half8, braw[j]), acc[i][j], 0, 0, 0);
-    }
+    spectral_step(acc, Ea, rc, rs, lds_addr_of(&s_stage[stage][0][0][lane * 16]));
   }
 
   // into the common frame (phase of the chunk's first token) and out
@@ -352,16 +384,17 @@ __global__ __launch_bounds__(256) void spectral_reduce_kernel(const float* __res
 // ---------------------------------------------------------------------------------------------------------
 __global__ __launch_bounds__(1024) void coef_colscale_kernel(const float* __restrict__ c, float* __restrict__ scale,
                                                              float* __restrict__ inv_scale, int N2, int Mc) {
-  __shared__ float s_mx[16][64];
-  const int lane = threadIdx.x & 63, g = threadIdx.x >> 6;   // 64 columns x 16 row classes
-  const int m = blockIdx.x * 64 + lane, b = blockIdx.y;
+  // 16 columns x 64 row classes: 64 bytes of a row per access, and four times the blocks of whole waves of columns
+  __shared__ float s_mx[64][16];
+  const int lane = threadIdx.x & 15, g = threadIdx.x >> 4;
+  const int m = blockIdx.x * 16 + lane, b = blockIdx.y;
   float mx = 0.f;
   if (m < Mc) {
     const float* cp = c + (int64_t)b * N2 * Mc + m;
-    for (int n0 = g; n0 < N2; n0 += 16 * 8) {
+    for (int n0 = g; n0 < N2; n0 += 64 * 8) {
       float v[8];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) v[u] = cp[(int64_t)min(n0 + 16 * u, N2 - 1) * Mc];
+      for (int u = 0; u < 8; ++u) v[u] = cp[(int64_t)min(n0 + 64 * u, N2 - 1) * Mc];
 #pragma unroll
       for (int u = 0; u < 8; ++u) mx = fmaxf(mx, fabsf(v[u]));
     }
@@ -370,12 +403,14 @@ __global__ __launch_bounds__(1024) void coef_colscale_kernel(const float* __rest
   __syncthreads();
   if (g == 0 && m < Mc) {
 #pragma unroll
-    for (int i = 1; i < 16; ++i) mx = fmaxf(mx, s_mx[i][lane]);
+    for (int i = 1; i < 64; ++i) mx = fmaxf(mx, s_mx[i][lane]);
     const float sc = mx > 0.f ? exp2f(ceilf(log2f(mx))) : 1.f;   // power of two: scaling is exact
     scale[(int64_t)b * Mc + m] = sc;
     inv_scale[(int64_t)b * Mc + m] = 1.0f / sc;
   }
 }
+
+constexpr int kMaxColShare = 16;   // column blocks of a workgroup at most
 
 struct ReconStatsParams {
   const half8* tab;        // basis rows of the positions: [ceil(K/8)][kStepK][64]
@@ -396,6 +431,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   constexpr int NST = 4;
   __shared__ __attribute__((aligned(16))) unsigned char s_stage[NST][4][kStepK][1024];
   __shared__ float s_red[3][4][kWgCols];
+  __shared__ float s_scale[kMaxColShare * kWgCols];   // scale / N of this workgroup's columns
   const int tid = threadIdx.x, lane = tid & 63, lg = lane >> 4, lc = lane & 15;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int rb = blockIdx.x, b = blockIdx.y;
@@ -406,18 +442,23 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int n_cb = min((p.Mc + kWgCols - 1) / kWgCols - cb0, p.cb_per);
   const int Q = n_cb * 2 * S;   // steps of this workgroup: column block, pass (cos, sin), step (last to first)
 
-  auto issue = [&](int q, int stage) {
-    const int cb = cb0 + q / (2 * S), rem = q % (2 * S);
-    const int pass = rem / S, s = S - 1 - (rem - pass * S);
-    const int ct = min(cb * 4 + w, p.CT - 1);
-    const _Float16* src = (const _Float16*)(p.packed[pass] + (((int64_t)b * p.CT + ct) * p.KS32) * 64) + lane * 8;
+  int next_cb = cb0, next_pass = 0, next_s = S - 1;   // the step requested next (walked, not divided out of a step number)
+  auto issue = [&](int stage) {
+    const int ct = min(next_cb * 4 + w, p.CT - 1);
+    const half8* frags = next_pass ? p.packed[1] : p.packed[0];
+    const _Float16* src = (const _Float16*)(frags + (((int64_t)b * p.CT + ct) * p.KS32) * 64) + lane * 8;
 #pragma unroll
     for (int ks = 0; ks < kStepK; ++ks)
-      load_frag_to_lds(src + (int64_t)(s * kStepK + ks) * 512, &s_stage[stage][w][ks][0]);
+      load_frag_to_lds(src + (int64_t)(next_s * kStepK + ks) * 512, &s_stage[stage][w][ks][0]);
+    if (--next_s < 0) {
+      next_s = S - 1;
+      next_cb += next_pass;
+      next_pass ^= 1;
+    }
   };
 #pragma unroll
   for (int i = 0; i < NST - 1; ++i)
-    if (i < Q) issue(i, i);
+    if (i < Q) issue(i);
 
   half8 Ea[4][kStepK];
 #pragma unroll
@@ -434,46 +475,31 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
   for (int i = 0; i < 4; ++i)
 #pragma unroll
+    for (int j = 0; j < 4; ++j) acc[i][j] = float4v{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
     for (int ks = 0; ks < kStepK; ++ks) asm volatile("" ::"v"(Ea[i][ks]));
 
+  // (read here once: a load behind the walk of a column block would wait for every tile on its way)
   const float inv_n = 1.0f / (float)p.N;
+  for (int i = tid; i < n_cb * kWgCols; i += 256) {
+    const int m = cb0 * kWgCols + i;
+    s_scale[i] = m < p.Mc ? p.scale[(int64_t)b * p.Mc + m] * inv_n : 0.f;
+  }
+  int cb = cb0, pass = 0, it = -1;
   for (int q = 0; q < Q; ++q) {
-    const int cb = cb0 + q / (2 * S), rem = q % (2 * S);
-    const int pass = rem / S, it = rem - pass * S;
+    if (++it == S) {
+      it = 0;
+      cb += pass;
+      pass ^= 1;
+    }
     const int stage = q % NST;
     if (q + NST - 2 < Q) wait_vmcnt<(NST - 2) * kStepK>();
     else wait_vmcnt<0>();
     barrier_lds_only();
-    if (q + NST - 1 < Q) issue(q + NST - 1, (q + NST - 1) % NST);
-    if (it == 0) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = float4v{0.f, 0.f, 0.f, 0.f};
-    } else {
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-          for (int f2 = 0; f2 < 2; ++f2) {
-            const float c = acc[i][j][2 * f2], sn = acc[i][j][2 * f2 + 1];
-            acc[i][j][2 * f2] = rc[i][f2] * c - rs[i][f2] * sn;
-            acc[i][j][2 * f2 + 1] = rs[i][f2] * c + rc[i][f2] * sn;
-          }
-    }
-#pragma unroll
-    for (int ks = 0; ks < kStepK; ++ks) {
-      uint4v braw[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) braw[j] = lds_read_b128_async(&s_stage[stage][j][ks][lane * 16]);
-      lds_wait_for4<0>(braw);
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Ea[i][ks], __builtin_bit_cast(half8, braw[j]), acc[i][j], 0, 0, 0);
-    }
+    if (q + NST - 1 < Q) issue((q + NST - 1) % NST);
+    spectral_step(acc, Ea, rc, rs, lds_addr_of(&s_stage[stage][0][0][lane * 16]));
     if (it != S - 1) continue;
     if (pass == 0) {
 #pragma unroll
@@ -482,6 +508,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         for (int j = 0; j < 4; ++j) {
           re[i][j][0] = acc[i][j][0];
           re[i][j][1] = acc[i][j][2];
+          acc[i][j] = float4v{0.f, 0.f, 0.f, 0.f};
         }
       continue;
     }
@@ -490,8 +517,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const int half = p.half;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const int m = (cb * 4 + j) * 16 + lc;
-      const float sc = m < p.Mc ? p.scale[(int64_t)b * p.Mc + m] * inv_n : 0.f;
+      const float sc = s_scale[((cb - cb0) * 4 + j) * 16 + lc];
       float sum = 0.f, mx = -INFINITY, mn = INFINITY;
 #pragma unroll
       for (int i = 0; i < 4; ++i)
@@ -532,6 +558,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       }
     }
     // the next barrier (top of the loop) orders these reads before s_red is written again
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc[i][j] = float4v{0.f, 0.f, 0.f, 0.f};
   }
 }
 
@@ -585,9 +615,9 @@ int fa_spectral_mfma_launch(const void* a, int a_dtype, int64_t a_bs, int64_t a_
   half8* packed = (half8*)((char*)workspace + pl.off_packed);
   dim3 pgrid(pl.KS32, fa_cdiv(Mc, 256), B);
   if (a_dtype == FA_BF16)
-    spectral_pack_kernel<bf16_t><<<pgrid, 256, 0, st>>>((const bf16_t*)a, a_bs, a_rs, cols, nullptr, packed, K, Mc, pl.CT, pl.KS32);
+    spectral_pack_kernel<bf16_t><<<pgrid, 256, 0, st>>>((const bf16_t*)a, a_bs, a_rs, cols, nullptr, packed, K, Mc, pl.CT, pl.KS32, B, 0, 0);
   else
-    spectral_pack_kernel<f16_t><<<pgrid, 256, 0, st>>>((const f16_t*)a, a_bs, a_rs, cols, nullptr, packed, K, Mc, pl.CT, pl.KS32);
+    spectral_pack_kernel<f16_t><<<pgrid, 256, 0, st>>>((const f16_t*)a, a_bs, a_rs, cols, nullptr, packed, K, Mc, pl.CT, pl.KS32, B, 0, 0);
   return spectral_after_pack(pl, c, B, Mc, N, T, k_start, accumulate, workspace, st);
 }
 
@@ -599,7 +629,7 @@ int spectral_after_pack(const SpectralPlan& pl, float* c, int B, int Mc, int N, 
   half8* tab = (half8*)(ws + pl.off_tab);
   half8* packed = (half8*)(ws + pl.off_packed);
   float* part = (float*)(ws + pl.off_part);
-  spectral_table_kernel<<<fa_cdiv((N / 8) * kStepK * 64, 256), 256, 0, st>>>(tab, N, T);
+  spectral_table_kernel<<<fa_cdiv((int64_t)(N / 8) * kTableThreads, 256), 256, 0, st>>>((half2v*)tab, N, T);
   SpectralGemmParams gp{};
   const bool direct = pl.n_chunks == 1;   // nothing to sum: the GEMM writes (or adds to) c itself
   gp.tab = tab; gp.packed = packed; gp.part = direct ? c : part;
@@ -719,10 +749,11 @@ namespace {
 // pays about half a column block for its basis rows before the first product: take the share whose rounds over the
 // device, times the length of a round, come out shortest.
 int recon_col_share(int row_groups, int n_cb) {
-  int best = n_cb;
+  int best = n_cb < fa_mfma::kMaxColShare ? n_cb : fa_mfma::kMaxColShare;
   float best_cost = 1e30f;
   for (int cs = 1; cs <= n_cb; ++cs) {
     const int per = fa_cdiv(n_cb, cs);
+    if (per > fa_mfma::kMaxColShare) continue;
     const float cost = (float)fa_cdiv((int64_t)row_groups * fa_cdiv(n_cb, per), 512) * ((float)per + 0.5f);
     if (cost < best_cost) { best_cost = cost; best = per; }
   }
@@ -752,12 +783,11 @@ int fa_recon_stats_mfma_launch(const float* c, int B, int N, int Mc, int K, int 
   const int Kd = mirror && T / 2 + 1 < K ? T / 2 + 1 : K;
   const int RBd = fa_cdiv(Kd, kWgFreqs);
   const int kp8 = fa_cdiv(Kd, 8) * 8;
-  spectral_table_kernel<<<fa_cdiv((kp8 / 8) * kStepK * 64, 256), 256, 0, st>>>(tab, kp8, T);
-  coef_colscale_kernel<<<dim3(fa_cdiv(Mc, 64), B), 1024, 0, st>>>(c, scale, inv, 2 * N, Mc);
-  dim3 pgrid(pl.KS32, fa_cdiv(Mc, 256), B);
-  spectral_pack_kernel<float><<<pgrid, 256, 0, st>>>(c, (int64_t)2 * N * Mc, Mc, nullptr, inv, pc, N, Mc, pl.CT, pl.KS32);
-  spectral_pack_kernel<float><<<pgrid, 256, 0, st>>>(c + (int64_t)N * Mc, (int64_t)2 * N * Mc, Mc, nullptr, inv, ps, N, Mc,
-                                                     pl.CT, pl.KS32);
+  spectral_table_kernel<<<fa_cdiv((int64_t)(kp8 / 8) * kTableThreads, 256), 256, 0, st>>>((half2v*)tab, kp8, T);
+  coef_colscale_kernel<<<dim3(fa_cdiv(Mc, 16), B), 1024, 0, st>>>(c, scale, inv, 2 * N, Mc);
+  // the cosine rows and, behind them, the sine rows
+  spectral_pack_kernel<float><<<dim3(pl.KS32, fa_cdiv(Mc, 256), 2 * B), 256, 0, st>>>(c, (int64_t)2 * N * Mc, Mc, nullptr, inv, pc, N, Mc,
+                                                                                     pl.CT, pl.KS32, B, (int64_t)N * Mc, ps - pc);
   ReconStatsParams rp{};
   rp.tab = tab; rp.packed[0] = pc; rp.packed[1] = ps; rp.scale = scale;
   rp.psum = *psum; rp.pmax = *pmax; rp.pmin = *pmin;

@@ -131,3 +131,30 @@ def test_operands_in_the_types_the_kernels_take(list_dtype, stat_dtype):
         pad = torch.cat([torch.zeros(1, dtype=n.dtype), ((n + unit - 1) // unit * unit).cumsum(0)])
         assert paging[i] == heads[i].tolist() and paging[2 + i].tolist() == pad.tolist()
     assert _lib.load_host().operands(lists, stats, 0, 0)[2] is None
+
+
+@pytest.mark.parametrize("L,C,N,T", [
+    (512, 1, 8, 700),           # one row tile of frequencies, one column, one chunk of four steps
+    (1300, 70, 136, 1301),      # a row tile past a whole workgroup, two column blocks, a ragged last step
+    (33000, 1100, 24, 40000),   # more than 128 splits of the statistics; eighteen column blocks, shares at their limit
+])
+def test_spectral_operators_at_the_edges_of_their_tiles(L, C, N, T):
+    """Coefficients and both statistics against the fp32 vector kernels.  Bounds: the basis is rounded to f16 (2^-11 per
+    entry, errors of both signs over L rows: well below 5e-4 of the column's norm); statistics as above."""
+    from fourierattention_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(L)
+    a = torch.randn((2, L, C), generator=g, device="cuda").to(torch.bfloat16)
+    got, ref = (ops.mat_fourier(a, N, T, matrix_cores=m) for m in (True, False))
+    assert float(((got - ref).norm(dim=1) / ref.norm(dim=1)).max()) <= 5e-4
+    if L >= 1024 and C >= 16 and N >= 32 or C > 1000:
+        c = torch.randn((2, 2 * max(N, 32), C), generator=g, device="cuda")
+        st, sr = (ops.mat_fourier_avg_std(c, L, T, torch.float16, matrix_cores=m) for m in (True, False))
+        size = sr[0].abs() + sr[1].abs()
+        assert all(float(((x - y).abs() / size).max()) <= 2e-3 for x, y in zip(st, sr))
+    avg, dev = ops.mat_avg_std_triton(a)
+    want = a.double().mean(1)
+    # float32 sums of L values of order one, then one rounding to bf16: eight significant bits, so half a unit in the last
+    # place is up to 2^-8 of the value
+    assert float((avg.double() - want).abs().max()) <= 2.0 ** -8 * float(want.abs().max()) + 1e-5
+    spread = torch.maximum(a.double().amax(1) - want, want - a.double().amin(1))
+    assert float(((dev.double() - spread) / spread).abs().max()) <= 2.0 ** -8
