@@ -106,6 +106,9 @@ _SIGNATURES = {
     "fa_linear_pack": (c_int, [c_void_p, c_void_p, c_int, c_int, c_int, c_void_p]),
     "fa_linear_packed_ok": (c_int, [c_int, c_int, c_int]),
     "fa_linear_packed": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p]),
+    "fa_linear_packed_norm_ok": (c_int, [c_int, c_int]),
+    "fa_linear_packed_step": (c_int, [c_void_p, c_int64, c_void_p, c_float, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int,
+                                      c_void_p]),
     "fa_decode_split_plan": (c_int, [c_int] * 7 + [c_void_p, c_void_p, c_void_p, c_void_p]),
     "fa_decode_tables_bytes": (c_size_t, [c_int]),
     "fa_decode_tables_build": (c_int, [c_void_p, c_size_t, c_int, c_int, c_void_p]),
@@ -133,7 +136,7 @@ _SIGNATURES = {
 EXPORTED = tuple(_SIGNATURES)
 
 # bumped with every change of a prototype or of an argument struct (fa_abi_version in the library)
-ABI_VERSION = 4
+ABI_VERSION = 5
 
 _lib = None
 

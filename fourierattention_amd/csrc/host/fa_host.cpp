@@ -347,18 +347,41 @@ int64_t row_stride(const at::Tensor& t) {
   return step == 0 ? t.size(-1) : step;
 }
 
-// linear_packed(x, packed weight, k, n_out) -> (..., n_out)
+// linear_packed(x, packed weight, k, n_out[, norm weight or None, eps, residual or None, gated]) -> (..., n_out), or
+// (..., n_out / 2) when gated, or the residual, added to in place
 PyObject* linear_packed(PyObject*, PyObject* const* a, Py_ssize_t n) {
   FA_BEGIN
-  CHECK(n == 4, "linear_packed takes 4 arguments");
+  CHECK(n == 4 || n == 8, "linear_packed takes 4 or 8 arguments");
   const at::Tensor &x = gpu_tensor(a[0], "x"), &w = gpu_tensor(a[1], "weight");
   const int64_t k = integer(a[2]), n_out = integer(a[3]);
   CHECK(x.scalar_type() == w.scalar_type() && x.dim() >= 1 && x.size(-1) == k && w.numel() == k * n_out, "linear_packed: x does not fit the weight");
+  const void* norm = nullptr;
+  float eps = 0.f;
+  bool gated = false;
   at::DimVector shape(x.sizes().begin(), x.sizes().end());
   shape.back() = n_out;
+  if (n == 8) {
+    if (a[4] != Py_None) {
+      const at::Tensor& nw = gpu_tensor(a[4], "norm weight");
+      CHECK(nw.scalar_type() == x.scalar_type() && nw.is_contiguous() && nw.numel() == k, "linear_packed: the norm weight must match the rows of x");
+      norm = nw.data_ptr();
+      eps = (float)real(a[5]);
+    }
+    gated = truth(a[7]);
+    if (a[6] != Py_None) {
+      const at::Tensor& res = gpu_tensor(a[6], "residual");
+      CHECK(!gated && res.is_contiguous() && res.scalar_type() == x.scalar_type() && res.sizes() == at::IntArrayRef(shape),
+            "linear_packed: the residual must be contiguous and have the type and shape of the result");
+      check_status(fa_linear_packed_step(x.data_ptr(), row_stride(x), norm, eps, w.data_ptr(), res.data_ptr(), (int)(x.numel() / k), (int)k,
+                                         (int)n_out, 1, dtype_code(x), stream_of(x)));
+      Py_INCREF(a[6]);
+      return a[6];
+    }
+  }
+  if (gated) shape.back() = n_out / 2;
   at::Tensor out = at::empty(shape, x.options());
-  check_status(fa_linear_packed(x.data_ptr(), row_stride(x), w.data_ptr(), out.data_ptr(), (int)(x.numel() / k), (int)k, (int)n_out,
-                                dtype_code(x), stream_of(x)));
+  check_status(fa_linear_packed_step(x.data_ptr(), row_stride(x), norm, eps, w.data_ptr(), out.data_ptr(), (int)(x.numel() / k), (int)k,
+                                     (int)n_out, gated ? 2 : 0, dtype_code(x), stream_of(x)));
   return THPVariable_Wrap(out);
   FA_END
 }

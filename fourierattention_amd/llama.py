@@ -115,9 +115,16 @@ class LlamaDecoderLayer(nn.Module):
             return None
         return w
 
-    def _linear(self, name, x, fallback):
+    def _linear(self, name, x, fallback, onto=None):
+        """A projection on its packed copy where that covers ``x``.  ``onto``: the residual stream its output belongs to;
+        the packed projection adds it in its own launch and leaves nothing to add (``None``)."""
         w = self._packed_weight(name)
-        return ops.linear_packed(x, w) if w is not None and w.covers(x) else fallback(x)
+        if w is None or not w.covers(x):
+            return fallback(x)
+        if onto is None:
+            return ops.linear_packed(x, w)
+        ops.linear_packed_step(x, w, residual=onto)
+        return None
 
     def fuse_projections(self, max_rows: int = 16384):
         """Moves the q/k/v weights into one tensor and the gate/up weights into another; the five modules keep
@@ -149,34 +156,46 @@ class LlamaDecoderLayer(nn.Module):
     def forward_fused(self, h, delta, position_embeddings, past_key_value, cache_position=None):
         """The same layer on the GPU with its elementwise chains in single launches.  ``h`` is the residual
         stream, updated in place; ``delta`` the branch output not yet added to it (``None`` for the first layer).
-        Returns this layer's MLP output, to be added by whoever normalises next."""
+        Returns this layer's MLP output, to be added by whoever normalises next (``None``: ``h`` has it already)."""
         at = self.self_attn
-        y = ops.add_rmsnorm(h, delta, self.input_layernorm.weight, self.input_layernorm.variance_epsilon)
-        bsz, q_len, _ = y.shape
+        bsz, q_len, _ = h.shape
         nq, nk = at.num_heads * at.head_dim, at.num_key_value_heads * at.head_dim
         pk = self._packed_weight("qkv")
-        if pk is not None and pk.covers(y):
-            q, k, v = ops.linear_packed(y, pk).split((nq, nk, nk), dim=-1)
-        elif self._qkv_weight is not None:
-            q, k, v = F.linear(y, self._qkv_weight).split((nq, nk, nk), dim=-1)
+        norm = self.input_layernorm
+        if pk is not None and delta is None and pk.covers(h) and pk.normalises(h, norm.weight):
+            q, k, v = ops.linear_packed_step(h, pk, norm.weight, norm.variance_epsilon).split((nq, nk, nk), dim=-1)
         else:
-            q, k, v = at.q_proj(y), at.k_proj(y), at.v_proj(y)
+            y = ops.add_rmsnorm(h, delta, norm.weight, norm.variance_epsilon)
+            if pk is not None and pk.covers(y):
+                q, k, v = ops.linear_packed(y, pk).split((nq, nk, nk), dim=-1)
+            elif self._qkv_weight is not None:
+                q, k, v = F.linear(y, self._qkv_weight).split((nq, nk, nk), dim=-1)
+            else:
+                q, k, v = at.q_proj(y), at.k_proj(y), at.v_proj(y)
         cos, sin = position_embeddings
         q = ops.rope_qk(q, k, cos, sin, at.head_dim)
         split = lambda t, n: t.view(bsz, q_len, n, at.head_dim).transpose(1, 2)
         o = fourier_attention(split(q, at.num_heads), split(k, at.num_key_value_heads), split(v, at.num_key_value_heads),
                               past_key_value, at.layer_idx, at.num_heads, at.num_key_value_heads,
                               {"sin": sin, "cos": cos, "cache_position": cache_position})
-        y = ops.add_rmsnorm(h, self._linear("o", o, at.o_proj), self.post_attention_layernorm.weight,
-                            self.post_attention_layernorm.variance_epsilon)
+        delta = self._linear("o", o, at.o_proj, onto=h)
         pk = self._packed_weight("gate_up")
-        if pk is not None and pk.covers(y):
-            gate, up = ops.linear_packed(y, pk).chunk(2, dim=-1)
-        elif self._gate_up_weight is not None:
-            gate, up = F.linear(y, self._gate_up_weight).chunk(2, dim=-1)
+        norm = self.post_attention_layernorm
+        if pk is not None and pk.covers(h):
+            gated = pk.n_out % 32 == 0      # whole tiles of gate rows, then whole tiles of up rows
+            if delta is None and gated and pk.normalises(h, norm.weight):
+                act = ops.linear_packed_step(h, pk, norm.weight, norm.variance_epsilon, gated=True)
+            else:
+                y = ops.add_rmsnorm(h, delta, norm.weight, norm.variance_epsilon)
+                act = ops.linear_packed_step(y, pk, gated=True) if gated else ops.silu_mul(*ops.linear_packed(y, pk).chunk(2, dim=-1))
         else:
-            gate, up = self.mlp.gate_proj(y), self.mlp.up_proj(y)
-        return self._linear("down", ops.silu_mul(gate, up), self.mlp.down_proj)
+            y = ops.add_rmsnorm(h, delta, norm.weight, norm.variance_epsilon)
+            if self._gate_up_weight is not None:
+                gate, up = F.linear(y, self._gate_up_weight).chunk(2, dim=-1)
+            else:
+                gate, up = self.mlp.gate_proj(y), self.mlp.up_proj(y)
+            act = ops.silu_mul(gate, up)
+        return self._linear("down", act, self.mlp.down_proj, onto=h)
 
 
 class LlamaModel(nn.Module):

@@ -274,6 +274,7 @@ class PackedLinearWeight:
         self.n_out, self.k = int(weight.shape[0]), int(weight.shape[1])
         self.dtype = weight.dtype
         self._rows_ok = {}     # row count -> whether the kernel takes it (asked once per count)
+        self._norm_ok = {}     # ... and an RMSNorm in front of it
         self.data = torch.empty_like(weight)
         check(_lib.load().fa_linear_pack(weight.data_ptr(), self.data.data_ptr(), self.n_out, self.k, dtype_code(weight.dtype),
                                          _stream(weight.device)))
@@ -289,6 +290,26 @@ class PackedLinearWeight:
         if ok is None:
             ok = self._rows_ok[rows] = bool(_lib.load().fa_linear_packed_ok(rows, self.k, self.n_out))
         return ok
+
+    def normalises(self, x: torch.Tensor, norm: torch.Tensor) -> bool:
+        """Whether ``linear_packed_step`` takes an RMSNorm of the rows of ``x`` into its launch: rows that a workgroup
+        normalises for itself, 16-byte aligned like the norm's weight."""
+        if (x.data_ptr() | norm.data_ptr()) % 16:
+            return False
+        rows = x.numel() // max(self.k, 1)
+        ok = self._norm_ok.get(rows)
+        if ok is None:
+            ok = self._norm_ok[rows] = bool(_lib.load().fa_linear_packed_norm_ok(rows, self.k))
+        return ok
+
+
+def linear_packed_step(x: torch.Tensor, w: PackedLinearWeight, norm: Optional[torch.Tensor] = None, eps: float = 0.0,
+                       residual: Optional[torch.Tensor] = None, gated: bool = False) -> torch.Tensor:
+    """``linear_packed`` with the decoder's elementwise steps in the same launch, rounded where ``add_rmsnorm`` and
+    ``silu_mul`` round: ``norm``, the weight of an RMSNorm of the rows of ``x`` in front (``w.normalises(x, norm)``);
+    ``residual (..., n_out)``, which the product is added to in place (and which is returned); ``gated``, a weight of gate
+    and then up rows (``n_out`` a multiple of 32), ``silu(gate) * up`` is returned (modeling_llama_fourier.py:87-92, 277, 735-750)."""
+    return _lib.load_host().linear_packed(x, w.data, w.k, w.n_out, norm, eps, residual, gated)
 
 
 def linear_packed(x: torch.Tensor, w: PackedLinearWeight) -> torch.Tensor:

@@ -449,6 +449,14 @@ int fa_linear_pack(const void* w, void* packed, int n_out, int K, int dtype, fa_
 int fa_linear_packed_ok(int rows, int K, int n_out);
 int fa_linear_packed(const void* x, int64_t x_row_stride, const void* w_packed, void* out, int rows, int K,
                      int n_out, int dtype, fa_stream_t stream);
+/* The same with the steps either side of it in the launch, rounded where fa_add_rmsnorm and fa_silu_mul round:
+ * norm_weight (K elements, may be null): the rows of x go through RMSNorm first (fa_linear_packed_norm_ok: the rows a
+ * workgroup can normalise for itself).  epilogue 0: out = product.  1: out (rows, n_out) += product in place; x must be
+ * another tensor.  2: the weight holds n_out / 2 gate rows and then as many up rows (n_out a multiple of 32), out
+ * (rows, n_out / 2) = silu(gate) * up. */
+int fa_linear_packed_norm_ok(int rows, int K);
+int fa_linear_packed_step(const void* x, int64_t x_row_stride, const void* norm_weight, float eps, const void* w_packed,
+                          void* out, int rows, int K, int n_out, int epilogue, int dtype, fa_stream_t stream);
 
 #ifdef __cplusplus
 }

@@ -158,3 +158,37 @@ def test_spectral_operators_at_the_edges_of_their_tiles(L, C, N, T):
     assert float((avg.double() - want).abs().max()) <= 2.0 ** -8 * float(want.abs().max()) + 1e-5
     spread = torch.maximum(a.double().amax(1) - want, want - a.double().amin(1))
     assert float(((dev.double() - spread) / spread).abs().max()) <= 2.0 ** -8
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows,K,n_out", [(1, 1024, 32), (16, 1024, 96), (5, 3072, 64), (4, 4096, 160), (2, 8192, 32), (3, 8192, 32)])
+def test_projections_with_the_steps_beside_them(dtype, rows, K, n_out):
+    """RMSNorm, gate and residual in the projection's launch against the launches of their own: the same bits without the
+    norm (same sums, same rounding); with it the sum of squares is taken in another order, which moves the scale of a row
+    by a place of float32 and with it single operands by a place of ``dtype`` (2^-8 / 2^-11 relative)."""
+    from fourierattention_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(rows + K)
+    rn = lambda *s: torch.randn(s, generator=g, device="cuda")
+    pw = ops.PackedLinearWeight((rn(n_out, K) * 0.05).to(dtype))
+    x, h = (rn(rows, 1, K) * 3).to(dtype), rn(rows, 1, n_out).to(dtype)
+    norm = (1 + 0.1 * rn(K)).to(dtype)
+    plain = ops.linear_packed(x, pw)
+    kept = h.clone()
+    assert ops.linear_packed_step(x, pw, residual=kept) is kept and torch.equal(kept, h + plain)
+    assert torch.equal(ops.linear_packed_step(x, pw, gated=True), ops.silu_mul(*plain.chunk(2, dim=-1)))
+    assert pw.normalises(x, norm) == (rows * K <= 16384) and not pw.normalises(x, torch.cat([norm, norm])[1:K + 1])
+    if rows * K > 16384:
+        with pytest.raises(RuntimeError):
+            ops.linear_packed_step(x, pw, norm, 1e-5)
+        return
+    before = x.clone()
+    got = ops.linear_packed_step(x, pw, norm, 1e-5)
+    y = ops.add_rmsnorm(x, None, norm, 1e-5)
+    want = ops.linear_packed(y, pw)
+    ulp = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    bound = 2 * ulp * float(want.abs().max()) + ulp * float(y.abs().max()) * 0.2 * 4
+    assert torch.equal(x, before) and float((got.float() - want.float()).abs().max()) <= bound
+    gate = ops.linear_packed_step(x, pw, norm, 1e-5, gated=True)
+    assert torch.equal(gate, ops.silu_mul(*got.chunk(2, dim=-1)))
+    kept = h.clone()
+    assert torch.equal(ops.linear_packed_step(x, pw, norm, 1e-5, residual=kept), h + got)
