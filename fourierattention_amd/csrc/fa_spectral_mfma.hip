@@ -245,8 +245,9 @@ __device__ __forceinline__ void spectral_step(float4v (&acc)[4][4], const half8 
 #pragma unroll
       for (int f2 = 0; f2 < 2; ++f2) {
         const float c = acc[i][j][2 * f2], sn = acc[i][j][2 * f2 + 1];
-        acc[i][j][2 * f2] = rc[i][f2] * c - rs[i][f2] * sn;
-        acc[i][j][2 * f2 + 1] = rs[i][f2] * c + rc[i][f2] * sn;
+        // (spelled out: left to itself the compiler rounds the one product for some tiles and the other for the rest)
+        acc[i][j][2 * f2] = __builtin_fmaf(rc[i][f2], c, -(rs[i][f2] * sn));
+        acc[i][j][2 * f2 + 1] = __builtin_fmaf(rc[i][f2], sn, rs[i][f2] * c);
       }
   FA_STEP_READ(b1, 1);
   lds_wait_for4<4>(b0);
