@@ -100,6 +100,7 @@ _SIGNATURES = {
                                 c_void_p]),
     "fa_decode_attn_workspace_bytes": (c_size_t, [c_int, c_int, c_int, c_int, c_int, c_int, c_int]),
     "fa_decode_attn": (c_int, [POINTER(DecodeArgs), c_void_p]),
+    "fa_decode_step": (c_int, [POINTER(StreamArgs), POINTER(DecodeArgs), c_void_p]),
     "fa_decode_attn_noalloc": (c_int, [POINTER(DecodeArgs), c_void_p]),
     "fa_decode_attn_timed": (c_int, [POINTER(DecodeArgs), c_void_p, POINTER(c_float)]),
     "fa_decode_attn_last_fused": (c_int, []),
@@ -136,7 +137,7 @@ _SIGNATURES = {
 EXPORTED = tuple(_SIGNATURES)
 
 # bumped with every change of a prototype or of an argument struct (fa_abi_version in the library)
-ABI_VERSION = 5
+ABI_VERSION = 6
 
 _lib = None
 

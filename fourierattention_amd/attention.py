@@ -60,7 +60,13 @@ def fourier_attention(query_states: torch.Tensor, key_states: torch.Tensor, valu
     """``query_states (B, Hq, q_len, D)``, ``key_states / value_states (B, Hkv, q_len, D)`` after RoPE.
     Returns ``(B, q_len, Hq*D)`` in the query dtype (modeling_llama_fourier.py:618-663)."""
     bsz, _, q_len, head_dim = query_states.shape
-    k_parts, v_parts = past_key_value.update(key_states, value_states, layer_idx, cache_kwargs)
+    if q_len == 1 and type(past_key_value) is DynamicCache:   # (a subclass may do more in update or decode_attention)
+        k_parts, v_parts, o = past_key_value.update_and_attend(query_states, key_states, value_states, layer_idx, num_heads,
+                                                               num_key_value_heads, query_states.dtype)
+        if o is not None:
+            return o.view(bsz, q_len, num_heads * head_dim)
+    else:
+        k_parts, v_parts = past_key_value.update(key_states, value_states, layer_idx, cache_kwargs)
     if isinstance(k_parts, CacheParts):
         # (B, Hq, 1, D) dense, rounded by the last kernel: the rows are those of (B, 1, Hq*D)
         return past_key_value.decode_attention(query_states, layer_idx, num_heads, num_key_value_heads,

@@ -321,6 +321,10 @@ class DynamicCache(Cache):
         prefill call and for layers that only keep a window, plain dicts whose ``*_init``,
         ``*_compressed`` and ``*_uncompressed`` entries are ``None`` (exact attention over
         ``*_local``); otherwise ``CacheParts`` views of the four parts."""
+        return self._apply(self._begin(key_states, layer_idx), key_states, value_states, layer_idx)
+
+    def _begin(self, key_states: torch.Tensor, layer_idx: int):
+        """What the next rows of a layer are for (the bookkeeping of ``update``)."""
         bsz, heads, q_len, head_dim = key_states.shape
         book = self._book
         step = book.step(layer_idx, bsz, q_len)
@@ -329,6 +333,10 @@ class DynamicCache(Cache):
         own["heads"], own["head_dim"], own["_seen_tokens"], own["maxtokens"] = heads, head_dim, book.seen_tokens, book.maxtokens
         if book.prefilllen is not None:
             own["prefilllen"] = book.prefilllen
+        return step
+
+    def _apply(self, step, key_states: torch.Tensor, value_states: torch.Tensor, layer_idx: int):
+        bsz, heads, q_len, head_dim = key_states.shape
         if step.action is Action.STREAM:
             return self._stream(key_states, value_states, layer_idx, step)
         k = key_states.permute(0, 2, 1, 3).reshape(bsz, q_len, heads * head_dim)
@@ -413,9 +421,22 @@ class DynamicCache(Cache):
                 "this call lands in the reference's late-compression branch (cache_utils_fourier.py:688-729), "
                 "which appends a new layer entry instead of updating this one; its result is undefined")
 
-    def _stream(self, key_states: torch.Tensor, value_states: torch.Tensor, layer_idx: int, step):
+    def update_and_attend(self, query_states: torch.Tensor, key_states: torch.Tensor, value_states: torch.Tensor, layer_idx: int,
+                          num_heads: int, num_kv_heads: int, out_dtype=None):
+        """``update``, then ``decode_attention`` of one new token where the layer streams: ``(k_parts, v_parts, out)`` with the
+        same results, the update in the attention's first launch where the shapes allow it.  In every other case
+        ``update`` alone, and ``None`` for ``out``."""
+        step = self._begin(key_states, layer_idx)
+        if (step.action is not Action.STREAM or self._layers[layer_idx].window_only or self.defer_coef_update
+                or not query_states.is_cuda):
+            return (*self._apply(step, key_states, value_states, layer_idx), None)
+        args = []
+        parts = self._stream(key_states, value_states, layer_idx, step, args)
+        return (*parts, self.decode_attention(query_states, layer_idx, num_heads, num_kv_heads, out_dtype=out_dtype, step=args[0]))
+
+    def _stream(self, key_states: torch.Tensor, value_states: torch.Tensor, layer_idx: int, step, joined: Optional[list] = None):
         """One more token for a compressed layer: the oldest window row is evicted, then the spare slot takes the new
-        token."""
+        token.  ``joined``: the launch is left to the caller, who finds its arguments there."""
         layer = self._layers[layer_idx]
         self._settle_coefficients(layer_idx)        # the row they are owed sits in the window slot written next
         layer.version += 1
@@ -433,9 +454,13 @@ class DynamicCache(Cache):
         # one launch: coefficients and page store take the oldest row, the new token takes the spare slot.  The
         # attention that follows streams the coefficients anyway: where it can, it is left to apply their rank-1
         # update on the way (the evicted row stays in its window slot until the next update of the layer writes there)
-        defer = bool(self.defer_coef_update and key_states.is_cuda and not torch.cuda.is_current_stream_capturing())
-        ops.stream_update(key_states, value_states, k.ring, v.ring, oldest, sp, k.coef, v.coef, l32[0], l32[4], step.phase,
-                          self._book.t_c, k.mid, v.mid, layer.n_mid, skip_coef=defer)
+        defer = bool(joined is None and self.defer_coef_update and key_states.is_cuda and not torch.cuda.is_current_stream_capturing())
+        args = (key_states, value_states, k.ring, v.ring, oldest, sp, k.coef, v.coef, l32[0], l32[4], step.phase, self._book.t_c,
+                k.mid, v.mid, layer.n_mid, defer)
+        if joined is None:
+            ops.stream_update(*args)
+        else:
+            joined.append(args)
         if defer:
             layer.owed = (oldest, int(step.phase), int(self._book.t_c))
         layer.n_mid += 1
@@ -480,11 +505,11 @@ class DynamicCache(Cache):
 
     # -- attention over the cache's own buffers --------------------------------------
     def decode_attention(self, query_states: torch.Tensor, layer_idx: int, num_heads: int, num_kv_heads: int,
-                         sm_scale: float = -1.0, timings=None, out_dtype=None, out=None, no_alloc=False) -> torch.Tensor:
+                         sm_scale: float = -1.0, timings=None, out_dtype=None, out=None, no_alloc=False, step=None) -> torch.Tensor:
         """``query_states (B, Hq, 1, D)`` -> ``(B, Hq, 1, D)`` float32 over the current state of
         ``layer_idx`` (what modeling_llama_fourier.py:641-660 computes from the returned parts); with
         ``out_dtype = query_states.dtype`` the result comes back rounded to that type (the ``.to(dtype)`` of
-        modeling_llama_fourier.py:663 done by the last kernel)."""
+        modeling_llama_fourier.py:663 done by the last kernel).  ``step``: see ``ops.decode_attn_raw``."""
         layer = self._layers[layer_idx]
         q = query_states
         if q.shape[2] != 1 or not q.is_contiguous():
@@ -508,4 +533,4 @@ class DynamicCache(Cache):
                                    layer.v.stats32, l32, num_heads, num_kv_heads, layer.n_mid, self.period_reconstruct,
                                    sm_scale, tables=self._tables, force_generic=self.force_generic, timings=timings,
                                    out_dtype=out_dtype, out=out, no_alloc=no_alloc, balance_heads=self.balance_heads,
-                                   no_fuse=(0 if self.fuse_decode else 1) | (0 if self.sub_splits else 2), pending=pending)
+                                   no_fuse=(0 if self.fuse_decode else 1) | (0 if self.sub_splits else 2), pending=pending, step=step)

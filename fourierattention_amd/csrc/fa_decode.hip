@@ -8,6 +8,7 @@
 // so one pass over the coefficients before (prep) and one after (merge) replace the
 // per-token reconstruction, and the token loop only touches the stored dims.
 // All exponentials are base 2 (scores carry log2(e)).
+#include "fa_stream.h"
 #include <stdlib.h>
 #include <string.h>
 
@@ -35,9 +36,10 @@ struct Seg {
 // ---------------------------------------------------------------------------
 // prep: W[b, hq, n] = (sm*log2e/N) sum_j coef[b, n, kc0 + j] q[b, hq, d_j] s[b, kc0 + j]
 //       c0[b, hq]   = sm*log2e * sum_j q[b, hq, d_j] (avg_u - avg_d s)[b, kc0 + j]
-// block = 64 coefficient rows of one (b, KV head); thread = (row, one of 4 column classes):
-// a thread reads every 4th compressed dim of its row (up to 32 independent loads in flight),
-// four neighbouring lanes finish the dot product.
+// block = 64 coefficient rows of one (b, KV head); thread = (four rows, one of 16 column classes): a thread reads every
+// 16th compressed dim of its rows (up to 32 independent loads in flight), sixteen neighbouring lanes finish the dot
+// products.  Four lanes to a row would touch four times the cache lines per access, which the write-back of a pending
+// update pays twice: eight sequences of 32k tokens, update included, 30.4 -> 26.9 us.
 // ---------------------------------------------------------------------------
 constexpr int kPrepRows = 64;
 
@@ -82,7 +84,7 @@ struct PrepArgs {
 
 // LDS of the query preparation: the gathered query dims times the scale / the mean terms, per query head; the
 // compressed dims of a row the coefficients are still owed
-constexpr int kPrepLdsBytes = (2 * kGMax * 128 + 128) * (int)sizeof(float);
+constexpr int kPrepLdsBytes = (2 * kGMax * 128 + 128 + kPrepRows) * (int)sizeof(float);
 
 // bx: block index along x (row chunk of kPrepRows coefficient rows); y, z come from blockIdx; lds: kPrepLdsBytes
 // UPD: a rank-1 update of the K coefficients is pending (an instance of its own: the code for it costs the launch
@@ -103,6 +105,7 @@ __device__ __forceinline__ void decode_prep_body(const PrepArgs<E>& pa, int bx, 
   float (&s_qs)[kGMax][128] = *reinterpret_cast<float (*)[kGMax][128]>(lds);
   float (&s_qa)[kGMax][128] = *reinterpret_cast<float (*)[kGMax][128]>((float*)lds + kGMax * 128);
   float* s_ue = (float*)lds + 2 * kGMax * 128;
+  float* s_uf = s_ue + 128;   // a pending update's factor of every row of the block
   const int tid = threadIdx.x;
   const int h = blockIdx.y, b = blockIdx.z;
   const int G = Hq / Hkv;
@@ -122,6 +125,14 @@ __device__ __forceinline__ void decode_prep_body(const PrepArgs<E>& pa, int bx, 
     s_qa[g][j] = qa;
     if constexpr (UPD)
       if (g == 0) s_ue[j] = j < kc_len ? fa_to_float(pa.upd_row[(int64_t)b * pa.upd_bs + kc_list[kc0 + j]]) : 0.f;
+  }
+  if constexpr (UPD) {
+    if (tid < kPrepRows) {
+      const int n = min(bx * kPrepRows + tid, 2 * N - 1);
+      float sn, co;
+      fa_sincos_phase(n >= N ? n - N : n, pa.upd_phase, pa.upd_T, &sn, &co);
+      s_uf[tid] = n >= N ? sn : co;
+    }
   }
   __syncthreads();
   if (bx == 0 && tid < 2 && pa.team_cnt && b % pa.nbpg == 0) pa.team_cnt[((int64_t)(b / pa.nbpg) * Hkv + h) * 2 + tid] = 0u;
@@ -150,27 +161,33 @@ __device__ __forceinline__ void decode_prep_body(const PrepArgs<E>& pa, int bx, 
       *(uint4*)(pa.q_stored + ((((int64_t)(grp * Hkv + h) * 4 + sl) * 4 + s) * 64 + lane) * 8) = o.raw;
     }
   }
-  const int n = bx * kPrepRows + (tid >> 2), jq = tid & 3;
-  if (n >= 2 * N) return;
-  const float* row = k_mc + ((int64_t)b * 2 * N + n) * Ck + kc0;
-  float v[32];
+  // sixteen lanes share a row (64 bytes of it per access), a thread four rows.  (Requested ahead of the query's list and gather instead: 17.3 us where this takes
+  // 14.6 at one sequence of 32k tokens, 27.9 against 26.9 at eight: the loads the rest of the chain waits for queue behind them.)
+  const int lr = tid & 15, r0 = tid >> 4;
+  const float* rows = k_mc + ((int64_t)b * 2 * N + bx * kPrepRows) * Ck + kc0;
+  const int n_left = 2 * N - bx * kPrepRows;      // rows from here to the end
+  float v[4][8];
 #pragma unroll
-  for (int i = 0; i < 32; ++i) {
-    const int j = jq + 4 * i;
-    v[i] = j < kc_len ? row[j] : 0.f;
-  }
+  for (int r = 0; r < 4; ++r)
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int rr = r0 + 16 * r, j = lr + 16 * i;
+      v[r][i] = rr < n_left && j < kc_len ? rows[(int64_t)rr * Ck + j] : 0.f;
+    }
   if constexpr (UPD) {
-    // the pending rank-1 update of this row (the arithmetic of fa_stream_update / fa_coeff_update)
-    float sn, co;
-    fa_sincos_phase(n >= N ? n - N : n, pa.upd_phase, pa.upd_T, &sn, &co);
-    const float f = n >= N ? sn : co;
-    float* wrow = const_cast<float*>(row);
+    // the pending rank-1 update of these rows (the arithmetic of fa_stream_update / fa_coeff_update)
+    float* wrows = const_cast<float*>(rows);
 #pragma unroll
-    for (int i = 0; i < 32; ++i) {
-      const int j = jq + 4 * i;
-      if (j < kc_len) {
-        v[i] = v[i] + f * s_ue[j];
-        wrow[j] = v[i];
+    for (int r = 0; r < 4; ++r) {
+      const int rr = r0 + 16 * r;
+      const float f = s_uf[rr];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int j = lr + 16 * i;
+        if (rr < n_left && j < kc_len) {
+          v[r][i] = v[r][i] + f * s_ue[j];
+          wrows[(int64_t)rr * Ck + j] = v[r][i];
+        }
       }
     }
   }
@@ -178,20 +195,28 @@ __device__ __forceinline__ void decode_prep_body(const PrepArgs<E>& pa, int bx, 
 #pragma unroll
   for (int g = 0; g < kGMax; ++g) {
     if (g >= G) break;
-    float a = 0.f;
+    float a[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int i = 0; i < 32; ++i) a = fmaf(v[i], s_qs[g][jq + 4 * i], a);
-    a = fa_group_sum<4>(a);
-    if (jq == 0) {
+    for (int i = 0; i < 8; ++i) {
+      const float w = s_qs[g][lr + 16 * i];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) a[r] = fmaf(v[r][i], w, a[r]);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) a[r] = fa_group_sum<16>(a[r]);
+    // lane r of a row group writes row r0 + 16 r
+    const float out = lr == 0 ? a[0] : lr == 1 ? a[1] : lr == 2 ? a[2] : a[3];
+    const int n = bx * kPrepRows + r0 + 16 * lr;
+    if (lr < 4 && n < 2 * N) {
       if (pa.W_lane) {
         const int cs = n >= N, nn = n - cs * N;
         const int per = 16 * pa.ks, sl = nn / per, r = nn - sl * per;
         const int grp = b / pa.nbpg, lc = (b - grp * pa.nbpg) * G + g;
         const int lane = lc * 4 + ((r & 7) >> 1);
         const int64_t tile = ((int64_t)(grp * Hkv + h) * pa.n_slices + sl) * 2 * pa.ks + (r >> 3);
-        pa.W_lane[((tile * 2 + cs) * 64 + lane) * 2 + (r & 1)] = a * mul;
+        pa.W_lane[((tile * 2 + cs) * 64 + lane) * 2 + (r & 1)] = out * mul;
       } else {
-        W[((int64_t)b * Hq + h * G + g) * 2 * N + n] = a * mul;
+        W[((int64_t)b * Hq + h * G + g) * 2 * N + n] = out * mul;
       }
     }
   }
@@ -1571,6 +1596,12 @@ struct IlArgs {
   float* po;
   int Hq, Hkv, n_split;
   float sm_log2e;
+  // a step that also takes the new token (STEP): row `fresh` of the segments is being written by another block of this
+  // launch and is read from the token itself
+  int fresh;
+  const E* k_new;
+  const E* v_new;
+  int64_t new_bs;
 };
 
 // LDS of a sink/window block: the four waves' maxima, denominators and outputs meet here
@@ -1582,7 +1613,7 @@ struct IlFastLds {
 };
 
 // bx: block index along x (tile of kIlFastTile rows); y, z come from blockIdx; lds: an IlFastLds<D, GM>
-template <typename E, int D, int GM>
+template <typename E, int D, int GM, bool STEP>
 __device__ __forceinline__ void decode_il_fast_body(const IlArgs<E>& ia, int bx, void* lds) {
   const E* __restrict__ q = ia.q;
   const Seg s0 = ia.s0, s1 = ia.s1;
@@ -1609,8 +1640,15 @@ __device__ __forceinline__ void decode_il_fast_body(const IlArgs<E>& ia, int bx,
     const int ii = i < n_il ? i : 0;
     const bool in0 = ii < s0.rows;
     const int64_t off = in0 ? (int64_t)b * s0.bs + (int64_t)ii * s0.rs : (int64_t)b * s1.bs + (int64_t)(ii - s0.rows) * s1.rs;
-    kraw[it] = *(const Row8<E>*)((in0 ? (const E*)s0.k : (const E*)s1.k) + off + h * D + sub * 8);
-    vraw[it] = *(const Row8<E>*)((in0 ? (const E*)s0.v : (const E*)s1.v) + off + h * D + sub * 8);
+    const E* kr = (in0 ? (const E*)s0.k : (const E*)s1.k) + off;
+    const E* vr = (in0 ? (const E*)s0.v : (const E*)s1.v) + off;
+    if constexpr (STEP) {
+      const bool fresh = ii == ia.fresh;
+      kr = fresh ? ia.k_new + b * ia.new_bs : kr;
+      vr = fresh ? ia.v_new + b * ia.new_bs : vr;
+    }
+    kraw[it] = *(const Row8<E>*)(kr + h * D + sub * 8);
+    vraw[it] = *(const Row8<E>*)(vr + h * D + sub * 8);
   }
   // the query slices: one unconditional 16-byte load per head (a head index past G repeats the last one)
   Row8<E> qraw[GM];
@@ -1713,7 +1751,7 @@ __device__ __forceinline__ void decode_il_fast_body(const IlArgs<E>& ia, int bx,
 template <typename E, int D, int GM>
 __global__ __launch_bounds__(256) void decode_il_fast_kernel(const IlArgs<E> ia) {
   __shared__ __attribute__((aligned(16))) unsigned char lds[sizeof(IlFastLds<D, GM>)];
-  decode_il_fast_body<E, D, GM>(ia, blockIdx.x, lds);
+  decode_il_fast_body<E, D, GM, false>(ia, blockIdx.x, lds);
 }
 
 // The coefficient-domain query and the sink/window rows do not depend on each other and are both short,
@@ -1722,14 +1760,26 @@ __global__ __launch_bounds__(256) void decode_il_fast_kernel(const IlArgs<E> ia)
 // waves per SIMD of that launch (rows of fp32 need twice the registers)
 template <typename E>
 constexpr int il_waves(int gm) { return (gm <= 4 ? 6 : 4) / (int)(sizeof(E) / 2); }
+// UPD: a rank-1 update of the K coefficients rides along and, with sp.total > 0, the rest of the layer's streaming update
+// (a decode step of the cache): its blocks lie behind the others, Hkv of them to an x.  Launch and update, the launch of
+// the update before it -> together: eight sequences of 32k tokens (half mask) 18.3 + 13.5 -> 26.9 us, three of 12k 8.5 + 8.6
+// -> 15.4, fp32 at 2k 6.2 + 4.2 -> 8.4, one of 32k 8.6 + 5.5 -> 14.6 and the gap between two launches less.
 template <typename E, int D, int GM, bool UPD>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(il_waves<E>(GM), il_waves<E>(GM))))
-void decode_prep_il_kernel(const PrepArgs<E> pa, const IlArgs<E> ia, int n_prep) {
+void decode_prep_il_kernel(const PrepArgs<E> pa, const IlArgs<E> ia, int n_prep, const fa_stream::StreamParams sp) {
   // one buffer for whichever piece the block runs: what a block holds in LDS decides how many run side by side
   constexpr int kLds = (int)sizeof(IlFastLds<D, GM>) > kPrepLdsBytes ? (int)sizeof(IlFastLds<D, GM>) : kPrepLdsBytes;
   __shared__ __attribute__((aligned(16))) unsigned char lds[kLds];
+  if constexpr (UPD) {
+    const int rest = (int)blockIdx.x - n_prep - ia.n_split;
+    if (rest >= 0) {
+      const int bx = rest * gridDim.y + blockIdx.y;
+      if (bx < sp.total) fa_stream::stream_update_body<E>(sp, bx, blockIdx.z, (float2*)lds);
+      return;
+    }
+  }
   if ((int)blockIdx.x < n_prep) decode_prep_body<E, UPD>(pa, blockIdx.x, lds);
-  else decode_il_fast_body<E, D, GM>(ia, blockIdx.x - n_prep, lds);
+  else decode_il_fast_body<E, D, GM, UPD>(ia, blockIdx.x - n_prep, lds);
 }
 
 // ---------------------------------------------------------------------------
@@ -2053,10 +2103,22 @@ static size_t merge_fast_lds(const fa_decode_args& a, const Plan& p, int G) {
   return lds <= 64 * 1024 ? lds : 0;
 }
 
+// the streaming update that rides in the first launch of a decode call (fa_decode_step), and where the token's row lies
+// among the sink/window rows
+struct JoinedStep {
+  fa_stream::StreamParams sp;
+  const void* k_new;
+  const void* v_new;
+  int64_t new_bs;
+  int fresh;
+  bool* launched;   // set once the launch that carries the update is out
+};
+
 // ev (optional): five events recorded before the first kernel and after each of prep (+ tables),
 // mid, sink/window and merge
 template <typename E>
-int launch_all(const fa_decode_args& a, const Plan& p, bool p_il_fast, float sm_scale, hipStream_t st, hipEvent_t* ev) {
+int launch_all(const fa_decode_args& a, const Plan& p, bool p_il_fast, float sm_scale, hipStream_t st, hipEvent_t* ev,
+               const JoinedStep* step) {
   if (ev) hipEventRecord(ev[0], st);
   char* ws = (char*)a.workspace;
   float* W = (float*)(ws + p.off_W);
@@ -2072,7 +2134,12 @@ int launch_all(const fa_decode_args& a, const Plan& p, bool p_il_fast, float sm_
   const float sm_log2e = sm_scale * kLog2e;
   Seg s0{a.k_il[0], a.v_il[0], a.il_rows[0], a.il_batch_stride[0], a.il_row_stride[0]};
   Seg s1{a.k_il[1], a.v_il[1], a.il_rows[1], a.il_batch_stride[1], a.il_row_stride[1]};
-  IlArgs<E> ia{(const E*)a.q, s0, s1, ilm, ild, ilo, a.Hq, a.Hkv, p.n_il_split, sm_log2e};
+  IlArgs<E> ia{(const E*)a.q, s0, s1, ilm, ild, ilo, a.Hq, a.Hkv, p.n_il_split, sm_log2e, -1, nullptr, nullptr, 0};
+  fa_stream::StreamParams sp{};
+  if (step) {
+    sp = step->sp;
+    ia.fresh = step->fresh; ia.k_new = (const E*)step->k_new; ia.v_new = (const E*)step->v_new; ia.new_bs = step->new_bs;
+  }
   // sink/window tiles ride in the query-preparation launch when both exist and the fast tile kernel applies
   const bool fuse_il = p_il_fast && p.n_il_split > 0 && p.n_mid_split > 0;
   uint16_t wg_map[fa_mfma::kFusedMaxWgs] = {};
@@ -2105,18 +2172,19 @@ int launch_all(const fa_decode_args& a, const Plan& p, bool p_il_fast, float sm_
                    a.Ck > 0 ? (const E*)a.upd_k_row : nullptr, a.upd_batch_stride, a.upd_phase, a.upd_T};
     const int n_prep = fa_cdiv(2 * a.N, kPrepRows);
     if (fuse_il) {
-      dim3 grid(n_prep + p.n_il_split, a.Hkv, a.B);
-      if (pa.upd_row) {
-        if (a.D == 128 && G <= 4) decode_prep_il_kernel<E, 128, 4, true><<<grid, 256, 0, st>>>(pa, ia, n_prep);
-        else if (a.D == 128) decode_prep_il_kernel<E, 128, kGMax, true><<<grid, 256, 0, st>>>(pa, ia, n_prep);
-        else if (G <= 4) decode_prep_il_kernel<E, 64, 4, true><<<grid, 256, 0, st>>>(pa, ia, n_prep);
-        else decode_prep_il_kernel<E, 64, kGMax, true><<<grid, 256, 0, st>>>(pa, ia, n_prep);
+      dim3 grid(n_prep + p.n_il_split + fa_cdiv(sp.total, a.Hkv), a.Hkv, a.B);
+      if (pa.upd_row || step) {
+        if (a.D == 128 && G <= 4) decode_prep_il_kernel<E, 128, 4, true><<<grid, 256, 0, st>>>(pa, ia, n_prep, sp);
+        else if (a.D == 128) decode_prep_il_kernel<E, 128, kGMax, true><<<grid, 256, 0, st>>>(pa, ia, n_prep, sp);
+        else if (G <= 4) decode_prep_il_kernel<E, 64, 4, true><<<grid, 256, 0, st>>>(pa, ia, n_prep, sp);
+        else decode_prep_il_kernel<E, 64, kGMax, true><<<grid, 256, 0, st>>>(pa, ia, n_prep, sp);
       } else {
-        if (a.D == 128 && G <= 4) decode_prep_il_kernel<E, 128, 4, false><<<grid, 256, 0, st>>>(pa, ia, n_prep);
-        else if (a.D == 128) decode_prep_il_kernel<E, 128, kGMax, false><<<grid, 256, 0, st>>>(pa, ia, n_prep);
-        else if (G <= 4) decode_prep_il_kernel<E, 64, 4, false><<<grid, 256, 0, st>>>(pa, ia, n_prep);
-        else decode_prep_il_kernel<E, 64, kGMax, false><<<grid, 256, 0, st>>>(pa, ia, n_prep);
+        if (a.D == 128 && G <= 4) decode_prep_il_kernel<E, 128, 4, false><<<grid, 256, 0, st>>>(pa, ia, n_prep, sp);
+        else if (a.D == 128) decode_prep_il_kernel<E, 128, kGMax, false><<<grid, 256, 0, st>>>(pa, ia, n_prep, sp);
+        else if (G <= 4) decode_prep_il_kernel<E, 64, 4, false><<<grid, 256, 0, st>>>(pa, ia, n_prep, sp);
+        else decode_prep_il_kernel<E, 64, kGMax, false><<<grid, 256, 0, st>>>(pa, ia, n_prep, sp);
       }
+      if (step) *step->launched = true;
     } else if (pa.upd_row) {
       decode_prep_kernel<E, true><<<dim3(n_prep, a.Hkv, a.B), 256, 0, st>>>(pa);
     } else {
@@ -2312,7 +2380,7 @@ extern "C" int fa_decode_tables_build(void* tables, size_t tables_bytes, int N, 
   return fa_check_launch("fa_decode_tables_build");
 }
 
-static int decode_attn_impl(const fa_decode_args* a, fa_stream_t stream, hipEvent_t* ev) {
+static int decode_attn_impl(const fa_decode_args* a, fa_stream_t stream, hipEvent_t* ev, const JoinedStep* step = nullptr) {
   FA_REQUIRE(a, FA_ERR_NULL_POINTER, "fa_decode_attn: null argument block");
   FA_REQUIRE(a->q_len == 1, FA_ERR_BAD_SHAPE, "fa_decode_attn: q_len = %d, decode needs exactly one query row", a->q_len);
   FA_REQUIRE(a->B > 0 && a->Hq > 0 && a->Hkv > 0 && a->D > 0, FA_ERR_BAD_SHAPE, "fa_decode_attn: bad B/Hq/Hkv/D");
@@ -2369,13 +2437,60 @@ static int decode_attn_impl(const fa_decode_args* a, fa_stream_t stream, hipEven
   const float sm = a->sm_scale > 0.f ? a->sm_scale : 1.0f / sqrtf((float)a->D);
   hipStream_t st = fa_hip_stream(stream);
   switch (a->dtype) {
-    case FA_BF16: return launch_all<bf16_t>(*a, p, il_fast, sm, st, ev);
-    case FA_FP16: return launch_all<f16_t>(*a, p, il_fast, sm, st, ev);
-    default: return launch_all<float>(*a, p, il_fast, sm, st, ev);
+    case FA_BF16: return launch_all<bf16_t>(*a, p, il_fast, sm, st, ev, step);
+    case FA_FP16: return launch_all<f16_t>(*a, p, il_fast, sm, st, ev, step);
+    default: return launch_all<float>(*a, p, il_fast, sm, st, ev, step);
   }
 }
 
 extern "C" int fa_decode_attn(const fa_decode_args* a, fa_stream_t stream) { return decode_attn_impl(a, stream, nullptr); }
+
+// Whether the update `s` can ride in the first launch of the attention `a`: that launch exists (vectorised sink/window rows
+// in front of mid rows), the attention reads the state the update leaves (the sink/window rows are one buffer around the
+// evicted slot, the new token's slot among them), and the token can be read like a row of the window.
+static bool step_joins(const fa_stream_args* s, const fa_decode_args* a, JoinedStep& j) {
+  if (!s || !a || s->skip_coef || a->upd_k_row || a->upd_v_row || a->L_m <= 0 || a->B != s->B || a->Hkv != s->Hkv ||
+      a->dtype != s->dtype || a->N != s->N || a->D <= 0 || s->width != a->Hkv * a->D || a->q_len != 1)
+    return false;
+  if (a->dtype != FA_BF16 && a->dtype != FA_FP16 && a->dtype != FA_FP32) return false;
+  if (a->k_mc != s->k_coef || a->v_mc != s->v_coef || a->Ck != s->Ck || a->Cv != s->Cv || a->kc_list != s->kc_list ||
+      a->il_rows[0] <= 0 || a->il_rows[1] < 0 || !il_fast_ok(*a))
+    return false;
+  const int64_t es = a->dtype == FA_FP32 ? 4 : 2, rs = a->il_row_stride[0] * es;
+  if (rs <= 0 || a->il_row_stride[0] != s->ring_row_stride || a->il_batch_stride[0] != s->ring_batch_stride) return false;
+  const int64_t at = (const char*)s->k_ring - (const char*)a->k_il[0], gap = a->il_rows[0];
+  if (at < 0 || at % rs || (const char*)s->v_ring - (const char*)a->v_il[0] != at) return false;
+  if (a->il_rows[1] > 0 && (a->il_row_stride[1] != s->ring_row_stride || a->il_batch_stride[1] != s->ring_batch_stride ||
+                            (const char*)a->k_il[1] - (const char*)a->k_il[0] != (gap + 1) * rs ||
+                            (const char*)a->v_il[1] - (const char*)a->v_il[0] != (gap + 1) * rs))
+    return false;
+  const int64_t fresh = at / rs + s->write_slot, evicted = at / rs + s->evict_slot;
+  if (evicted != gap || fresh == gap || fresh - (fresh > gap) >= gap + a->il_rows[1]) return false;
+  if ((((uintptr_t)s->k_new | (uintptr_t)s->v_new | (uintptr_t)(s->new_batch_stride * es)) & 15) != 0 || !s->k_new || !s->v_new) return false;
+  if (fa_stream::stream_params(s, true, j.sp) != FA_OK) return false;
+  j.k_new = s->k_new; j.v_new = s->v_new; j.new_bs = s->new_batch_stride;
+  j.fresh = (int)(fresh - (fresh > gap));
+  return true;
+}
+
+extern "C" int fa_decode_step(const fa_stream_args* s, const fa_decode_args* a, fa_stream_t stream) {
+  JoinedStep j{};
+  if (!step_joins(s, a, j)) {
+    const int rc = fa_stream_update(s, stream);
+    return rc != FA_OK ? rc : decode_attn_impl(a, stream, nullptr);
+  }
+  bool launched = false;
+  j.launched = &launched;
+  fa_decode_args b = *a;
+  b.upd_k_row = (const char*)s->k_ring + (int64_t)s->evict_slot * s->ring_row_stride * (a->dtype == FA_FP32 ? 4 : 2);
+  b.upd_batch_stride = s->ring_batch_stride; b.upd_phase = s->phase; b.upd_T = s->T;
+  const int rc = decode_attn_impl(&b, stream, nullptr, &j);
+  if (!launched) {   // the attention was refused: the update happens all the same, as it does with a call of its own
+    const int up = fa_stream_update(s, stream);
+    return rc != FA_OK ? rc : up;
+  }
+  return rc;
+}
 
 // ---- the entry point that allocates nothing -------------------------------------------------------------------
 // Device memory for the partial results of one decode call (what `workspace` brings in for fa_decode_attn), held

@@ -114,15 +114,13 @@ void token_rows(const at::Tensor& t, int64_t& batch, int64_t& width, int64_t& ba
 
 // stream_update(k_new, v_new, k_ring, v_ring, evict_slot, write_slot, k_coef, v_coef, kc_list, vc_list, phase, T,
 //               k_mid, v_mid, mid_pos, skip_coef)
-PyObject* stream_update(PyObject*, PyObject* const* a, Py_ssize_t n) {
-  FA_BEGIN
-  CHECK(n == 16, "stream_update takes 16 arguments");
+// fills `s` from them and returns the window buffer of K
+const at::Tensor& stream_args(PyObject* const* a, fa_stream_args& s) {
   const at::Tensor &k_new = tensor(a[0], "k_new"), &v_new = tensor(a[1], "v_new");
   const at::Tensor &k_ring = gpu_tensor(a[2], "k_ring"), &v_ring = gpu_tensor(a[3], "v_ring");
   const at::Tensor &k_coef = tensor(a[6], "k_coef"), &v_coef = tensor(a[7], "v_coef");
   const at::Tensor &kc = tensor(a[8], "kc_list"), &vc = tensor(a[9], "vc_list");
   PyObject *k_mid = a[12], *v_mid = a[13];
-  fa_stream_args s{};
   int64_t B, width, vB, v_width, v_stride;
   token_rows(k_new, B, width, s.new_batch_stride);
   token_rows(v_new, vB, v_width, v_stride);
@@ -152,6 +150,14 @@ PyObject* stream_update(PyObject*, PyObject* const* a, Py_ssize_t n) {
   s.Cnk = (int32_t)int_attr(k_mid, s_Cn); s.Cnv = (int32_t)int_attr(v_mid, s_Cn);
   s.B = (int32_t)B; s.Hkv = (int32_t)int_attr(k_mid, s_Hkv); s.width = (int32_t)width; s.dtype = dtype_code(k_ring);
   s.skip_coef = truth(a[15]);
+  return k_ring;
+}
+
+PyObject* stream_update(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  FA_BEGIN
+  CHECK(n == 16, "stream_update takes 16 arguments");
+  fa_stream_args s{};
+  const at::Tensor& k_ring = stream_args(a, s);
   check_status(fa_stream_update(&s, stream_of(k_ring)));
   Py_RETURN_NONE;
   FA_END
@@ -174,12 +180,18 @@ const float* stat(PyObject* tuple, Py_ssize_t i) {
 }
 
 // decode_attn(q, il, k_mc, v_mc, k_mn, v_mn, stats_k, stats_v, lists, Hq, Hkv, L_m, T, sm_scale, out, cast, tables,
-//             force_generic, balance_heads, no_fuse, pending, no_alloc, timings) -> out
+//             force_generic, balance_heads, no_fuse, pending, no_alloc, timings[, step]) -> out
+// step: the arguments of stream_update as a tuple; the update comes in front of the attention
 // q (B, 1, Hq*D) or (B, Hq, 1, D), contiguous.  il: a sequence of up to two (k, v) pairs of row views, or (k, v, r): the
 // rows of one buffer in front of and behind row r.
 PyObject* decode_attn(PyObject*, PyObject* const* a, Py_ssize_t n) {
   FA_BEGIN
-  CHECK(n == 23, "decode_attn takes 23 arguments");
+  CHECK(n == 23 || n == 24, "decode_attn takes 23 or 24 arguments");
+  PyObject* step = n == 24 && a[23] != Py_None ? a[23] : nullptr;
+  CHECK(!step || (PyTuple_Check(step) && PyTuple_GET_SIZE(step) == 16 && a[20] == Py_None && !truth(a[21]) && a[22] == Py_None),
+        "step: the 16 arguments of stream_update, with a workspace, no pending update and no timings");
+  fa_stream_args su{};
+  if (step) stream_args(&PyTuple_GET_ITEM(step, 0), su);
   const at::Tensor& q = gpu_tensor(a[0], "q");
   fa_decode_args d{};
   d.Hq = (int32_t)integer(a[9]); d.Hkv = (int32_t)integer(a[10]);
@@ -305,6 +317,8 @@ PyObject* decode_attn(PyObject*, PyObject* const* a, Py_ssize_t n) {
     Ref list(PyList_New(4));
     for (int i = 0; i < 4; ++i) PyList_SET_ITEM(list.p, i, PyFloat_FromDouble(ms[i]));
     if (PyList_SetSlice(a[22], 0, PyList_GET_SIZE(a[22]), list.p) < 0) throw PyError{};
+  } else if (step) {
+    check_status(fa_decode_step(&su, &d, st));
   } else {
     check_status(fa_decode_attn(&d, st));
   }

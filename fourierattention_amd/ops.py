@@ -384,7 +384,7 @@ def decode_tables(n_f: int, period: int, device) -> Optional[torch.Tensor]:
 
 def decode_attn_raw(q, il_segments, k_mc, v_mc, k_mn, v_mn, stats_k, stats_v, lists, num_head_q, num_head_kv, seq_len_m,
                     T, sm_scale=-1.0, out=None, tables=None, force_generic=False, timings=None, out_dtype=None,
-                    no_alloc=False, balance_heads=True, no_fuse=0, pending=None):
+                    no_alloc=False, balance_heads=True, no_fuse=0, pending=None, step=None):
     """Thin call into ``fa_decode_attn``.  The result is float32 like the reference's (TRI:779) unless ``out_dtype``
     names the dtype of ``q``: then the merge launch rounds it to that type itself (the caller's ``.to(dtype)``).
 
@@ -403,7 +403,9 @@ def decode_attn_raw(q, il_segments, k_mc, v_mc, k_mn, v_mn, stats_k, stats_v, li
     but without the four sub-splits per workgroup that a batch of one sequence otherwise runs).
     ``pending``: ``(k_row, v_row, phase, T_c)``, a rank-1 update the coefficients are still owed (``stream_update``
     with ``skip_coef``): ``k_row, v_row (B, Hkv*D)`` are the rows that left the window (same strides).  The call
-    applies it to ``k_mc`` / ``v_mc`` IN PLACE while it streams them, once; pass it to one call only."""
+    applies it to ``k_mc`` / ``v_mc`` IN PLACE while it streams them, once; pass it to one call only.
+    ``step``: the arguments of ``stream_update`` as a tuple: that update, then the attention over the state it leaves
+    (which the other arguments describe), in one launch less where the shapes allow it."""
     if seq_len_m >= _REPACK_MIN_ROWS and not force_generic:
         _warn_if_off_the_matrix_cores(q.dtype, num_head_q, num_head_kv, q.numel() // (q.shape[0] * num_head_q),
                                       (k_mc if lists[0].numel() else v_mc).shape[1] // 2, not isinstance(k_mn, torch.Tensor))
@@ -411,7 +413,7 @@ def decode_attn_raw(q, il_segments, k_mc, v_mc, k_mn, v_mn, stats_k, stats_v, li
     assert not cast or out_dtype == q.dtype, "out_dtype must be float32 or the dtype of q"
     return _lib.load_host().decode_attn(q, il_segments, k_mc, v_mc, k_mn, v_mn, stats_k, stats_v, lists, num_head_q,
                                         num_head_kv, seq_len_m, T, sm_scale, out, cast, tables, force_generic, balance_heads,
-                                        no_fuse, pending, no_alloc, timings)
+                                        no_fuse, pending, no_alloc, timings, step)
 
 
 _warned_shapes = set()

@@ -386,6 +386,10 @@ int fa_decode_attn_last_fused(void);
  * milliseconds spent in (0) the coefficient-domain query kernel (plus the operand tables when
  * they are built in the workspace), (1) the mid-row kernel, (2) the sink/window kernel and
  * (3) the merge kernel.  A measurement aid for benchmarks (the reference has no timers). */
+/* fa_stream_update(s) followed by fa_decode_attn(a), whose arguments describe the state the update leaves: the same results,
+ * in one launch less where the update can ride in the attention's first launch (16- or 32-bit rows with vectorised
+ * sink/window kernels, the window as one buffer around the evicted slot, a 16-byte aligned token). */
+int fa_decode_step(const fa_stream_args* s, const fa_decode_args* a, fa_stream_t stream);
 int fa_decode_attn_timed(const fa_decode_args* args, fa_stream_t stream, float* ms_out);
 
 /* ---------------------------------------------------------------------------

@@ -192,3 +192,40 @@ def test_projections_with_the_steps_beside_them(dtype, rows, K, n_out):
     assert torch.equal(gate, ops.silu_mul(*got.chunk(2, dim=-1)))
     kept = h.clone()
     assert torch.equal(ops.linear_packed_step(x, pw, norm, 1e-5, residual=kept), h + got)
+
+
+@pytest.mark.parametrize("dtype,B,Hq,Hkv,D,states,init,W,counts,wide", [
+    (torch.bfloat16, 1, 8, 2, 128, 256, 4, 100, [64, 64], False),     # matrix cores, merge in the launch, sub-splits
+    (torch.bfloat16, 3, 12, 4, 128, 256, 4, 61, [128, 0, 77, 1], True),   # a head without compressed K, tokens as slices of wider rows
+    (torch.float16, 2, 16, 2, 64, 512, 1, 64, [40, 13], False),       # heads of 64 dims, eight query heads
+    (torch.float32, 1, 6, 2, 128, 64, 4, 33, [100, 128], False),      # single precision
+    (torch.bfloat16, 2, 8, 2, 128, 64, 0, 40, [64, 100], False),      # no sink rows
+    (torch.bfloat16, 1, 4, 2, 80, 64, 4, 40, [30, 50], False),        # head dims without the vectorised window kernel
+])
+def test_update_in_the_attention_launch(dtype, B, Hq, Hkv, D, states, init, W, counts, wide):
+    """A decode step through ``fourier_attention`` (the update in the attention's first launch, or in front of it where it
+    cannot be) against ``update`` and ``decode_attention`` as calls of their own, on two caches with the same prompt:
+    the same window, pages and attention arithmetic, bit for bit, over enough steps for the ring to come round."""
+    from fourierattention_amd import DynamicCache, ExtraConfig, masks
+    from fourierattention_amd.attention import fourier_attention
+    g = torch.Generator(device="cuda").manual_seed(W)
+    rn = lambda *s: torch.randn(s, generator=g, device="cuda").to(dtype)
+    m = masks.synthetic_masks(1, Hkv, D, counts, counts[::-1], seed=3)
+    cfg = ExtraConfig(numinittokens=init, maxlocallen=W, maxmidstates=states, non_critical_dims=m, non_critical_dims_path=None,
+                      max_position_embeddings=8192, num_key_value_heads=Hkv, max_new_tokens=8, model_type="llama")
+    S = init + W + states + 700
+    prompt = rn(B, Hkv, S, D), rn(B, Hkv, S, D)
+    one, two = DynamicCache(cfg), DynamicCache(cfg)
+    one.update(*prompt, 0)
+    two.update(*prompt, 0)
+    for t in range(W + 5):
+        q = rn(B, Hq, 1, D)
+        k, v = rn(B, 1, 2 * Hkv * D).split(Hkv * D, dim=-1)
+        k, v = (x.view(B, 1, Hkv, D).transpose(1, 2) if wide else x.reshape(B, Hkv, 1, D).contiguous() for x in (k, v))
+        got = fourier_attention(q, k, v, one, 0, Hq, Hkv)
+        two.update(k, v, 0)
+        want = two.decode_attention(q, 0, Hq, Hkv, out_dtype=dtype).view(B, 1, Hq * D)
+        assert torch.equal(got, want), t
+    for a, b in zip((one.key_cache[0], one.value_cache[0]), (two.key_cache[0], two.value_cache[0])):
+        assert all(torch.equal(a[n], b[n]) for n in a)
+    assert one.get_seq_length() == two.get_seq_length() == S + W + 5
