@@ -115,6 +115,8 @@ _SIGNATURES = {
     "fa_decode_tables_build": (c_int, [c_void_p, c_size_t, c_int, c_int, c_void_p]),
     "fa_mid_pack": (c_int, [c_void_p, c_int, c_int64, c_int64, c_int64, c_int, c_void_p, c_int64, c_int, c_void_p, c_void_p,
                             c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p]),
+    "fa_append_rows": (c_int, [c_void_p, c_void_p, c_int64, c_int64, c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int, c_int,
+                               c_int, c_int, c_void_p]),
     "fa_convert": (c_int, [c_void_p, c_int, c_void_p]),
     "fa_prefill_compress_ok": (c_int, [c_int, c_int, c_int, c_int, c_int, c_int]),
     "fa_prefill_compress_workspace_bytes": (c_size_t, [c_int, c_int, c_int, c_int, c_int]),
@@ -137,7 +139,7 @@ _SIGNATURES = {
 EXPORTED = tuple(_SIGNATURES)
 
 # bumped with every change of a prototype or of an argument struct (fa_abi_version in the library)
-ABI_VERSION = 6
+ABI_VERSION = 7
 
 _lib = None
 

@@ -213,6 +213,18 @@ __global__ __launch_bounds__(256) void mid_pack_runs_kernel(
   }
 }
 
+// New rows of K and of V behind those a window buffer holds, both in one launch; U: the unit that strides and widths allow.
+template <typename U>
+__global__ __launch_bounds__(256) void append_rows_kernel(const U* __restrict__ k, const U* __restrict__ v, int64_t src_bs,
+                                                          int64_t src_rs, U* __restrict__ k_dst, U* __restrict__ v_dst,
+                                                          int64_t dst_bs, int64_t dst_rs, int width, int B) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= width) return;
+  const bool is_v = (int)blockIdx.z >= B;
+  const int64_t b = is_v ? blockIdx.z - B : blockIdx.z, t = blockIdx.y;
+  (is_v ? v_dst : k_dst)[b * dst_bs + t * dst_rs + i] = (is_v ? v : k)[b * src_bs + t * src_rs + i];
+}
+
 // Operands of a call in the types the kernels take, all in one launch: a grid row per item, items in the argument block.
 constexpr int kMaxConvert = 16;
 struct ConvertArgs { fa_convert_item item[kMaxConvert]; };
@@ -324,6 +336,30 @@ extern "C" int fa_mid_pack(const void* src, int dtype, int64_t src_bs, int64_t s
                                             n_h, pad_h, is_v);
   });
   return rc != FA_OK ? rc : fa_check_launch("fa_mid_pack");
+}
+
+extern "C" int fa_append_rows(const void* k, const void* v, int64_t src_bs, int64_t src_rs, void* k_dst, void* v_dst, int64_t dst_bs,
+                              int64_t dst_rs, int64_t pos, int B, int rows, int width, int dtype, fa_stream_t stream) {
+  FA_REQUIRE(k && v && k_dst && v_dst, FA_ERR_NULL_POINTER, "fa_append_rows: null pointer");
+  FA_REQUIRE(B > 0 && B <= 32767 && rows >= 0 && rows <= 65535 && width > 0 && pos >= 0, FA_ERR_BAD_SHAPE,
+             "fa_append_rows: B=%d rows=%d width=%d", B, rows, width);
+  FA_REQUIRE(dtype == FA_BF16 || dtype == FA_FP16 || dtype == FA_FP32, FA_ERR_BAD_DTYPE, "fa_append_rows: dtype %d", dtype);
+  if (rows == 0) return FA_OK;
+  hipStream_t st = fa_hip_stream(stream);
+  const int es = dtype == FA_FP32 ? 4 : 2;
+  char *kd = (char*)k_dst + pos * dst_rs * es, *vd = (char*)v_dst + pos * dst_rs * es;
+  auto go = [&](auto tag) {
+    using U = decltype(tag);
+    const int per = (int)sizeof(U) / es;
+    append_rows_kernel<U><<<dim3(fa_cdiv(width / per, 256), rows, 2 * B), 256, 0, st>>>(
+        (const U*)k, (const U*)v, src_bs / per, src_rs / per, (U*)kd, (U*)vd, dst_bs / per, dst_rs / per, width / per, B);
+  };
+  const uintptr_t ptrs = (uintptr_t)k | (uintptr_t)v | (uintptr_t)kd | (uintptr_t)vd;
+  const uint64_t steps = (uint64_t)((src_bs | src_rs | dst_bs | dst_rs | (int64_t)width) * es);
+  if (((ptrs | steps) & 15) == 0) go(uint4{});
+  else if (es == 4) go(uint32_t{});
+  else go(uint16_t{});
+  return fa_check_launch("fa_append_rows");
 }
 
 extern "C" int fa_convert(const fa_convert_item* items, int n, fa_stream_t stream) {

@@ -437,6 +437,22 @@ PyObject* rope_qk(PyObject*, PyObject* const* a, Py_ssize_t n) {
   FA_END
 }
 
+// append_rows(k, v, k_dst, v_dst, pos): rows of K and V (B, rows, width) to row pos of the buffers
+PyObject* append_rows(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  FA_BEGIN
+  CHECK(n == 5, "append_rows takes 5 arguments");
+  const at::Tensor &k = gpu_tensor(a[0], "k"), &v = gpu_tensor(a[1], "v"), &kd = gpu_tensor(a[2], "k_dst"), &vd = gpu_tensor(a[3], "v_dst");
+  const int64_t pos = integer(a[4]);
+  CHECK(k.dim() == 3 && k.sizes() == v.sizes() && k.strides() == v.strides() && k.stride(2) == 1 && kd.dim() == 3 && kd.sizes() == vd.sizes() &&
+        kd.strides() == vd.strides() && kd.stride(2) == 1 && kd.size(0) == k.size(0) && kd.size(2) == k.size(2), "append_rows: shapes and strides");
+  CHECK(v.scalar_type() == k.scalar_type() && kd.scalar_type() == k.scalar_type() && vd.scalar_type() == k.scalar_type() && pos >= 0 &&
+        pos + k.size(1) <= kd.size(1), "append_rows: types, rows past the end");
+  check_status(fa_append_rows(k.data_ptr(), v.data_ptr(), k.stride(0), k.stride(1), kd.data_ptr(), vd.data_ptr(), kd.stride(0), kd.stride(1),
+                              pos, (int)k.size(0), (int)k.size(1), (int)k.size(2), dtype_code(k), stream_of(kd)));
+  Py_RETURN_NONE;
+  FA_END
+}
+
 // operands(lists, stats, k_unit, v_unit) -> (lists, stats, paging)
 // The index lists (a tuple of eight: kc, kc_h, kn, kn_h, vc, vc_h, vn, vn_h) as int32 and the statistics (a tuple) as
 // contiguous float32, those that are not of these types already in one launch and one allocation.  With k_unit > 0 also
@@ -556,7 +572,7 @@ PyObject* init(PyObject*, PyObject* const* a, Py_ssize_t n) {
 }
 
 #define FN(name) {#name, (PyCFunction)(void*)name, METH_FASTCALL, nullptr}
-PyMethodDef methods[] = {FN(init), FN(stream_update), FN(decode_attn), FN(add_rmsnorm), FN(linear_packed), FN(silu_mul), FN(rope_qk), FN(operands),
+PyMethodDef methods[] = {FN(init), FN(stream_update), FN(decode_attn), FN(add_rmsnorm), FN(linear_packed), FN(silu_mul), FN(rope_qk), FN(operands), FN(append_rows),
                          {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_fa_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 

@@ -221,6 +221,11 @@ def stream_update(k_new: torch.Tensor, v_new: torch.Tensor, k_ring: torch.Tensor
                                    phase, T, k_mid, v_mid, mid_pos, skip_coef)
 
 
+def append_rows(k: torch.Tensor, v: torch.Tensor, k_dst: torch.Tensor, v_dst: torch.Tensor, pos: int) -> None:
+    """Rows of K and V ``(B, rows, width)`` to rows ``pos ..`` of two buffers, in one launch."""
+    _lib.load_host().append_rows(k, v, k_dst, v_dst, pos)
+
+
 def add_rmsnorm(h: torch.Tensor, delta: Optional[torch.Tensor], weight: torch.Tensor, eps: float) -> torch.Tensor:
     """``h += delta`` (when given, in place) and ``LlamaRMSNorm`` of the result in one launch
     (modeling_llama_fourier.py:735-750, 87-92).  ``h, delta (..., hidden)`` contiguous."""

@@ -287,6 +287,12 @@ int fa_mid_pack(const void* src, int dtype, int64_t src_batch_stride, int64_t sr
                 const int32_t* n_h_list, const int32_t* pad_h_list, int B, int Hkv, int D, int is_v,
                 int cols_kind, fa_stream_t stream);
 
+/* rows new rows of K and V, (B, rows, width) with common strides in elements, copied to rows pos .. of two buffers with common
+ * strides (the growing window of a layer that keeps nothing else), in one launch */
+int fa_append_rows(const void* k, const void* v, int64_t src_batch_stride, int64_t src_row_stride, void* k_dst, void* v_dst,
+                   int64_t dst_batch_stride, int64_t dst_row_stride, int64_t pos, int B, int rows, int width, int dtype,
+                   fa_stream_t stream);
+
 /* Small operands of a call (index lists, statistics) in the types the kernels take, all in one launch of at most 16
  * items: dst[i] = src[i] converted, for i < count; with the FA_CONVERT_PAD kinds src holds per-head offsets with the
  * leading 0 and dst[h] = sum over g < h of (src[g+1] - src[g]) rounded up to whole units (the pad_h list of a page

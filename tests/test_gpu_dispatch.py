@@ -229,3 +229,41 @@ def test_update_in_the_attention_launch(dtype, B, Hq, Hkv, D, states, init, W, c
     for a, b in zip((one.key_cache[0], one.value_cache[0]), (two.key_cache[0], two.value_cache[0])):
         assert all(torch.equal(a[n], b[n]) for n in a)
     assert one.get_seq_length() == two.get_seq_length() == S + W + 5
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("B,Hq,Hkv,D,rows", [(1, 2, 1, 128, 1), (2, 6, 2, 64, 64), (3, 8, 2, 80, 65), (1, 16, 2, 128, 4161), (2, 4, 4, 8, 1100)])
+def test_window_only_decode(dtype, B, Hq, Hkv, D, rows):
+    """A layer that keeps only a window, one tile to more tiles than a wave has lanes, against float64.  Bound: single
+    precision over ``rows`` keys of order one, then the rounding of the result to ``dtype``."""
+    from fourierattention_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    q, k, v = (torch.randn(s, generator=g, device="cuda").to(dtype) for s in ((B, Hq, 1, D), (B, rows, Hkv * D), (B, rows, Hkv * D)))
+    lists = (torch.zeros(Hkv + 1, dtype=torch.int32, device="cuda"),) * 8
+    qd = q.double().view(B, Hkv, Hq // Hkv, D)
+    kd, vd = (t.double().view(B, rows, Hkv, D).permute(0, 2, 1, 3).contiguous() for t in (k, v))
+    p = (qd.matmul(kd.transpose(2, 3).contiguous()) / D ** 0.5).softmax(-1)
+    want = p.matmul(vd).view(B, Hq, 1, D)
+    for cast in (None, dtype):
+        got = ops.decode_attn_raw(q, [(k, v)], None, None, None, None, None, None, lists, Hq, Hkv, 0, 1, out_dtype=cast)
+        ulp = 2.0 ** -8 if got.dtype == torch.bfloat16 else 0.0
+        assert got.dtype == (cast or torch.float32)
+        assert bool(((got.double() - want).abs() <= 2e-5 + ulp * want.abs()).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("width,rows,slice_", [(256, 1, False), (1023, 3, False), (1024, 16, True), (7, 2, True)])
+def test_append_rows(dtype, width, rows, slice_):
+    """New rows behind a window, dense or slices of wider rows, aligned and not: the rows and nothing beside them."""
+    from fourierattention_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(width)
+    wide = torch.randn((2, rows, 2 * width), generator=g, device="cuda").to(dtype)
+    k, v = wide.split(width, dim=-1) if slice_ else (x.contiguous() for x in wide.split(width, dim=-1))
+    bufs = [torch.randn((2, 40, width), generator=g, device="cuda").to(dtype) for _ in range(2)]
+    want = [b.clone() for b in bufs]
+    for b, x in zip(want, (k, v)):
+        b[:, 5:5 + rows] = x
+    ops.append_rows(k, v, *bufs, 5)
+    assert torch.equal(bufs[0], want[0]) and torch.equal(bufs[1], want[1])
+    with pytest.raises(AssertionError):
+        ops.append_rows(k, v, *bufs, 41 - rows)
