@@ -230,7 +230,9 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(3, 3
         for (int e = 0; e < 8; ++e) x[rb][e] = __builtin_fmaf(sacc[e >> 2][rb][e & 3], p.sm_log2e, -m_run[rb]);
     };
     distances();
-    if (__any(fa_fmax(fa_fmax8(x[0]), fa_fmax8(x[1])) > kMaxLag)) {   // always on the first tile: every row sees its first key
+    // always on the first tile: every row sees its first key.  (Not "> kMaxLag": a lane votes for two rows, and the maximum
+    // hands a NaN on, so a row of NaN would withhold the vote of the other.)
+    if (__any(!(fa_fmax(fa_fmax8(x[0]), fa_fmax8(x[1])) <= kMaxLag))) {
 #pragma unroll
       for (int rb = 0; rb < 2; ++rb) {
         float s[8];

@@ -87,6 +87,38 @@ def test_prompt_attention_with_a_moving_reference(dtype, D, S, q_len, G, climb):
     assert float((got - want).abs().max()) <= 0.5 * ulp + 1e-3
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("D,G", [(128, 4), (128, 3), (64, 1)])
+@pytest.mark.parametrize("first,last,keys", [(16, 32, False), (5, 161, False), (5, 161, True), (37, 38, False), (1, 17, True)])
+@pytest.mark.parametrize("climb", [0.0, 40.0])
+def test_prompt_rows_beside_rows_that_are_not_numbers(dtype, D, G, first, last, keys, climb):
+    """Query rows ``first .. last`` (and, with ``keys``, their keys) are NaN: every other row that sees no such key is what it
+    is without them, and the NaN rows stay NaN.  Scores climb as above, so a vote withheld would overflow f16.  Bound: as
+    above."""
+    from fourierattention_amd import ops
+    S = 161
+    g = torch.Generator(device="cuda").manual_seed(11)
+    q = torch.randn((1, 2 * G, S, D), generator=g, device="cuda")
+    k = torch.randn((1, S, 2, D), generator=g, device="cuda")
+    v = torch.randn((1, S, 2, D), generator=g, device="cuda")
+    q[..., 0] = 8.0
+    k[..., 0] = (climb * torch.arange(S, device="cuda") / 32 * np.log(2) * D ** 0.5 / 8.0)[None, :, None]
+    q, k, v = (t.to(dtype) for t in (q, k, v))
+    qd, kd, vd = q.double(), k.double().permute(0, 2, 1, 3).repeat_interleave(G, 1), v.double().permute(0, 2, 1, 3).repeat_interleave(G, 1)
+    s = qd.matmul(kd.transpose(2, 3).contiguous()) / D ** 0.5
+    rows = torch.arange(S, device="cuda")
+    want = s.masked_fill(rows[None, :] > rows[:, None], float("-inf")).softmax(-1).matmul(vd).transpose(1, 2)
+    q[:, :, first:last] = float("nan")
+    if keys:
+        k[:, first:last] = float("nan")
+    got = ops.prefill_attention(q, k.reshape(1, S, 2 * D), v.reshape(1, S, 2 * D), 2).double()
+    bad = (rows >= first) if keys else (rows >= first) & (rows < last)
+    assert bool(got[:, bad].isnan().all())
+    top = float(want.abs().max())
+    ulp = 2.0 ** (np.floor(np.log2(top)) - (7 if dtype == torch.bfloat16 else 10))
+    assert float((got - want)[:, ~bad].abs().max()) <= 0.5 * ulp + 1e-3
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("B,D,rows,extra,counts", [
     (1, 128, 1, 0, [128, 1]),                 # one row; a full head and a single dim
