@@ -12,17 +12,17 @@
 // slot order, is prepared once per call by a transposing pass over V (prefill_vt_kernel): 1 KiB fragments that
 // the main kernel streams into LDS unchanged.
 //
-// What bounds it: power, then issue.  On random operands the device runs this kernel at 1.8 - 1.9 GHz (the same launch on
-// zeros: 1538 TFLOP/s instead of 1131), so what counts is energy and instructions per score, not the order of the work.
-// Vector and matrix instructions of a SIMD overlap only in part (a 16x16x32 instruction holds the issue for half of its
-// 16 clocks).  The softmax of a tile therefore costs a lane one multiply-add, half a three-way maximum, one exponential,
-// half a conversion and half a dot product per score: distances from a reference that lags (kMaxLag), one vote per
-// tile on them without any lane exchange, denominators from the f16 probabilities by pairs.  Consecutive matrix
-// instructions change one operand at a time.  32768 tokens, 32 / 8 heads of 128 dims, bf16: 987 -> 1131 TFLOP/s.  Tried
-// and slower: 32x32x16 instructions (half the count, but twice the accumulator traffic per product: 1357 against 1939
-// TFLOP/s for bare products of random f16 operands; here 987 with this softmax), denominators on the matrix unit (1042),
-// two waves per SIMD (1102), a third stage (1116), twelve waves sharing the tiles of 96 keys (1134 against 1141 for a third of
-// the L2 traffic).
+// What bounds it: power, then issue.  On random operands the device runs this kernel at 1.8 - 1.9 GHz, so what counts is
+// energy and instructions per score, not the order of the work.  Vector and matrix instructions of a SIMD overlap only in
+// part (a 16x16x32 instruction holds the issue for half of its 16 clocks).  The softmax of a tile therefore costs a lane one
+// multiply-add, half a three-way maximum, one exponential, half a conversion and one addition per score, and one vote per
+// sixteen rows: only where a row's maximum rises do lanes exchange it and rescale.  Consecutive matrix instructions change one
+// operand at a time.  32768 tokens, 32 / 8 heads of 128 dims, bf16, behind the other kernels of a prompt: 9.47 ms (an exchange on
+// every tile) -> 8.70 ms, 1011 TFLOP/s; four sequences of 3001 tokens, 24 / 8 heads: 344 -> 329 us, where maxima still rise
+// on most tiles.  A reference that lags behind the maximum by up to 8 would rescale next to nothing (8.27 ms), but rounds
+// the largest weights, which are exact against the maximum: the error of peaked rows against 64 bits rose by a fifth; so did
+// denominators from the f16 weights.  Slower: 32x32x16 instructions (half the count, but twice the accumulator traffic per
+// product), denominators on the matrix unit, two waves per SIMD, a third stage.
 //
 // Workgroup: one KV head, HW query heads of it (all that share its keys, up to four) times RW blocks of 32 query
 // rows, one wave each.  The key tiles travel HBM -> LDS once per workgroup (global_load_lds, two stages, one
@@ -36,7 +36,7 @@ using namespace fa_mfma;
 constexpr int kTileKeys = 32;
 // a row's softmax reference moves only when a score exceeds it by more than this (base 2): the probabilities stay below
 // 2^8, exact to f16's eleven bits, and most tiles rescale nothing
-constexpr float kMaxLag = 8.f;
+constexpr float kMaxLag = 0.f;
 constexpr float kNoReference = -1e30f;   // before a row's first key: finite, so that a masked score is -inf against it
 
 template <typename E>
@@ -221,20 +221,18 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(3, 3
           if (slot_key(lg, e) > lim) sacc[e >> 2][rb][e & 3] = -INFINITY;
       }
     }
-    // distance of every score from its row's reference (the scale of the softmax rides in the subtraction)
+    // distance of every score from its row's reference, the running maximum (the scale of the softmax rides in the
+    // subtraction).  Most tiles raise no row's maximum: a vote per sixteen rows finds that out without a lane exchange.
     float x[2][8];
-    auto distances = [&]() {
+    auto distances = [&](int rb) {
 #pragma unroll
-      for (int rb = 0; rb < 2; ++rb)
-#pragma unroll
-        for (int e = 0; e < 8; ++e) x[rb][e] = __builtin_fmaf(sacc[e >> 2][rb][e & 3], p.sm_log2e, -m_run[rb]);
+      for (int e = 0; e < 8; ++e) x[rb][e] = __builtin_fmaf(sacc[e >> 2][rb][e & 3], p.sm_log2e, -m_run[rb]);
     };
-    distances();
-    // always on the first tile: every row sees its first key.  (Not "> kMaxLag": a lane votes for two rows, and the maximum
-    // hands a NaN on, so a row of NaN would withhold the vote of the other.)
-    if (__any(!(fa_fmax(fa_fmax8(x[0]), fa_fmax8(x[1])) <= kMaxLag))) {
 #pragma unroll
-      for (int rb = 0; rb < 2; ++rb) {
+    for (int rb = 0; rb < 2; ++rb) {
+      distances(rb);
+      // always on the first tile: every row sees its first key.  (Not "> 0": the maximum hands a NaN on)
+      if (__any(!(fa_fmax8(x[rb]) <= 0.f))) {
         float s[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) s[e] = sacc[e >> 2][rb][e & 3];
@@ -244,22 +242,21 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(3, 3
         l_run[rb] *= alpha;
 #pragma unroll
         for (int dg = 0; dg < DG; ++dg) oacc[dg][rb] *= alpha;
+        distances(rb);
       }
-      distances();
     }
-    half8 pb[2];   // probabilities as f16 operands
-    const half2v ones = {(_Float16)1.f, (_Float16)1.f};
+    half8 pb[2];   // probabilities as f16 operands; the denominators add the exponentials themselves
 #pragma unroll
-    for (int rb = 0; rb < 2; ++rb)
+    for (int rb = 0; rb < 2; ++rb) {
+      float psum = 0.f;
 #pragma unroll
-      for (int e = 0; e < 8; e += 2) {
-        half2v pv;
-        pv[0] = (_Float16)__builtin_amdgcn_exp2f(x[rb][e]);
-        pv[1] = (_Float16)__builtin_amdgcn_exp2f(x[rb][e + 1]);
-        l_run[rb] = __builtin_amdgcn_fdot2(pv, ones, l_run[rb], false);   // (what the second product weighs the values with)
-        pb[rb][e] = pv[0];
-        pb[rb][e + 1] = pv[1];
+      for (int e = 0; e < 8; ++e) {
+        const float pv = __builtin_amdgcn_exp2f(x[rb][e]);
+        psum += pv;
+        pb[rb][e] = (_Float16)pv;
       }
+      l_run[rb] += psum;
+    }
     // ---- O^T += V^T . P^T (the fragments in pairs, like the K fragments above)
     auto o_pair = [&](uint4v& f0, uint4v& f1, int dg) {
       oacc[dg][0] = Mma<f16_t>::mma(__builtin_bit_cast(half8, f0), pb[0], oacc[dg][0]);

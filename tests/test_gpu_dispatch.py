@@ -66,8 +66,8 @@ def test_any_shape_decode_kernels(dtype, B, Hq, Hkv, D, n_il, L, N, k_counts, v_
 @pytest.mark.parametrize("climb", [0.0, 6.0, 40.0, -40.0])
 def test_prompt_attention_with_a_moving_reference(dtype, D, S, q_len, G, climb):
     """Scores that climb (or fall) along the keys by ``climb`` per key tile, in units of log 2: the softmax reference of a
-    row lags by up to 8 before it moves, so 0 never moves it after the first tile, 6 moves it every other tile, 40
-    every tile.  Bound: f16 probabilities (2^-11 each, averaged) and the rounding of the result, as for the other shapes."""
+    row moves with its maximum, so -40 never moves it after the first tile, 0 here and there, 6 and 40 on every
+    tile.  Bound: f16 probabilities (2^-11 each, averaged) and the rounding of the result, as for the other shapes."""
     from fourierattention_amd import ops
     g = torch.Generator(device="cuda").manual_seed(7)
     q = torch.randn((1, 2 * G, q_len, D), generator=g, device="cuda")
@@ -299,3 +299,47 @@ def test_append_rows(dtype, width, rows, slice_):
     assert torch.equal(bufs[0], want[0]) and torch.equal(bufs[1], want[1])
     with pytest.raises(AssertionError):
         ops.append_rows(k, v, *bufs, 41 - rows)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_prompt_rows_whose_denominator_is_many_small_weights(dtype):
+    """One key of weight 1 and 32767 keys of about 1.4 * 2^-24, where f16 holds multiples of 2^-24 only: together they are
+    0.27% of the denominator.  The values of the many are zero, so the result is the denominator's inverse: it has to
+    come from the weights in single precision.  Bound: the rounding of the result (of values just below 1), and single precision
+    over 32768 weights."""
+    from fourierattention_amd import ops
+    S, D = 32768, 128
+    q = torch.zeros((1, 4, 40, D), device="cuda", dtype=dtype)
+    k = torch.zeros((1, S, D), device="cuda", dtype=dtype)
+    v = torch.zeros((1, S, D), device="cuda", dtype=dtype)
+    q[..., 0] = 16.0
+    k[:, 0, 0] = float(np.log(2) * (24 - np.log2(1.4)) * D ** 0.5 / 16.0)
+    v[:, 0] = 1.0
+    score = float(k[0, 0, 0]) * 16.0 / D ** 0.5
+    got = ops.prefill_attention(q, k, v, 1)[0].double()                  # row i sees keys 0 .. S - 40 + i
+    seen = torch.arange(S - 40, S, device="cuda", dtype=torch.float64)
+    want = (1.0 / (1.0 + seen * np.exp(-score)))[:, None, None].expand_as(got)
+    assert float((got - want).abs().max()) <= 2.0 ** (-9 if dtype == torch.bfloat16 else -12) + 2e-5
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_prompt_rows_whose_largest_weight_comes_late(dtype):
+    """Two keys, the second one (a tile later) ahead by up to six units of log 2, and only it has a value: its weight against
+    the row's maximum is exactly one, so the result is the denominator's inverse to the rounding of the result itself (a weight
+    of, say, 2^0.4 against the first key would already be rounded to f16).  Bound as above."""
+    from fourierattention_amd import ops
+    S, D, q_len = 64, 128, 24
+    g = torch.Generator(device="cuda").manual_seed(2)
+    q = torch.zeros((128, 4, q_len, D), device="cuda")
+    q[..., 0] = 6 * np.log(2) * D ** 0.5 * torch.rand((128, 4, q_len), generator=g, device="cuda")
+    q[..., 1] = 64.0
+    k = torch.zeros((128, S, D), device="cuda")
+    k[:, :, 1] = -64.0                       # every other key is out of reach
+    k[:, (0, 40), 1] = 0.0
+    k[:, 40, 0] = 1.0
+    v = torch.zeros((128, S, D), device="cuda")
+    v[:, 40] = 1.0
+    q, k, v = (t.to(dtype) for t in (q, k, v))
+    got = ops.prefill_attention(q, k, v, 1).double()
+    want = torch.sigmoid(q[..., 0].double() / D ** 0.5).transpose(1, 2)[..., None].expand_as(got)
+    assert float((got - want).abs().max()) <= 2.0 ** (-9 if dtype == torch.bfloat16 else -12) + 2e-5
