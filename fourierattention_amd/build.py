@@ -158,6 +158,20 @@ def kernels_with_atomics_outside(asm_text: str, kernels=HANDOVER_KERNELS):
     return out
 
 
+def kernels_with_scratch(asm_text: str):
+    """Kernels of a listing that keep registers in scratch memory (``name: bytes per lane``)."""
+    out, kernel = [], None
+    for line in asm_text.split("\n"):
+        m = re.match(r"\s*\.amdhsa_(kernel|private_segment_fixed_size)\s+(\S+)", line)
+        if m and m.group(1) == "kernel":
+            kernel = m.group(2)
+        elif m and int(m.group(2)) > 0:
+            out.append(f"{kernel}: {m.group(2)} bytes of scratch per lane")
+    return out
+
+
+# sources whose kernels are written to fit their registers at the occupancy they ask for
+NO_SCRATCH_SOURCES = ("fa_prefill",)
 ASYNC_LDS_SOURCES = ("fa_decode_mid_bf16", "fa_decode_mid_f16", "fa_prefill", "fa_spectral_mfma")
 HANDOVER_SOURCES = ("fa_decode", "fa_decode_mid_bf16", "fa_decode_mid_f16")
 
@@ -189,6 +203,9 @@ def audit_listings(base: str, listings) -> list:
     if base in ASYNC_LDS_SOURCES and reads == 0:
         found.append(f"{base}: no inline-asm LDS read found in the assembly of a source that issues them "
                      "(markers or spellings the scan relies on have changed)")
+    if base in NO_SCRATCH_SOURCES:
+        for text in listings:
+            found += kernels_with_scratch(text)
     if base in HANDOVER_SOURCES:
         atomics = 0
         for text in listings:

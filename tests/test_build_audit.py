@@ -114,6 +114,14 @@ def test_audit_fails_closed():
     assert audit_listings("fa_stream", [BAD_COPY]) != []       # but a violation is reported wherever it shows up
 
 
+def test_spilled_registers_are_reported_where_none_are_expected():
+    from fourierattention_amd.build import audit_listings
+    text = GOOD + "\t.amdhsa_kernel _Zkernel_a\n\t\t.amdhsa_private_segment_fixed_size %d\n\t.end_amdhsa_kernel\n"
+    assert audit_listings("fa_prefill", [text % 0]) == []
+    assert audit_listings("fa_prefill", [text % 12]) == ["_Zkernel_a: 12 bytes of scratch per lane"]
+    assert audit_listings("fa_stream", [text % 12]) == []
+
+
 # ---- hand-over between workgroups: stores, wait, counting atomic ----------------------------------------------------
 HANDOVER_GOOD = """
 _Z24decode_merge_rows_kernel13MergeRowsArgs:
