@@ -490,8 +490,9 @@ __global__ __launch_bounds__(256) void decode_mid_kernel(
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
           const Heads qn = s_qn[j0 + e];
+          const float x = j0 + e < kn_len ? kv[e] : 0.f;   // (zero query dims do not silence an infinity past the head's dims)
 #pragma unroll
-          for (int g = 0; g < GM; ++g) sc[g] = fmaf(kv[e], qn.v[g], sc[g]);
+          for (int g = 0; g < GM; ++g) sc[g] = fmaf(x, qn.v[g], sc[g]);
         }
       }
     }
@@ -555,7 +556,7 @@ __global__ __launch_bounds__(256) void decode_mid_kernel(
     if (dim < vn_len) {
       for (int t0 = half * (kMidTile / 2); t0 < min(t_len, (half + 1) * (kMidTile / 2)); t0 += 8) {
         float vv[8];
-        if (PAGED) {   // (slots past the last row are zero, and their probabilities too)
+        if (PAGED) {
           row8_to_float(*(const Row8<E>*)(vb + paged_offset(true, dpv, l0 + t0, dim)), vv);
         } else {
 #pragma unroll
@@ -564,8 +565,9 @@ __global__ __launch_bounds__(256) void decode_mid_kernel(
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
           const Heads p = s_p[t0 + e];
+          const float x = t0 + e < t_len ? vv[e] : 0.f;   // (nor do zero probabilities past the rows)
 #pragma unroll
-          for (int g = 0; g < GM; ++g) on[g] = fmaf(p.v[g], vv[e], on[g]);
+          for (int g = 0; g < GM; ++g) on[g] = fmaf(p.v[g], x, on[g]);
         }
       }
     }

@@ -343,3 +343,40 @@ def test_prompt_rows_whose_largest_weight_comes_late(dtype):
     got = ops.prefill_attention(q, k, v, 1).double()
     want = torch.sigmoid(q[..., 0].double() / D ** 0.5).transpose(1, 2)[..., None].expand_as(got)
     assert float((got - want).abs().max()) <= 2.0 ** (-9 if dtype == torch.bfloat16 else -12) + 2e-5
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("L,k_counts,v_counts", [(70, [33, 122], [100, 121]), (1, [127, 128], [1, 127]), (130, [97, 60], [64, 128])])
+def test_any_shape_decode_kernels_beside_infinities(dtype, L, k_counts, v_counts):
+    """The last stored K dim of a head is -inf in some rows (their weight is zero) and the last row's first stored V dim is
+    +inf (so is the result): what a kernel reads past a head's dims or past the rows must not reach a sum.  Bound as
+    above."""
+    from fourierattention_amd import ops
+    from fourierattention_amd.midstore import MidStore
+    from oracle import fourier_oracle as fo
+    from tests import helpers as H
+    Hq, Hkv, D = 4, 2, 128
+    case = H.attn_case(13, 1, Hq, Hkv, D, 9, L, 40, 2 * L + 9, k_counts, v_counts, dtype)
+    case["q"] = np.abs(case["q"]) + 0.25     # (a key of -inf scores -inf for every query head)
+    case["q"] = H.to_dtype_np(case["q"], dtype)
+    for h in range(Hkv):
+        if case["kn_h_list"][h + 1] > case["kn_h_list"][h]:
+            case["k_mn"][:, : L - 1 : 3, case["kn_h_list"][h + 1] - 1] = -np.inf
+    case["v_mn"][:, L - 1, 0] = np.inf
+    want = fo.fourier_attn(**case)
+    g = H.attn_case_gpu(case, dtype)
+    lists = tuple(ops.as_i32(g[n]) for n in ("kc_list", "kc_h_list", "kn_list", "kn_h_list", "vc_list", "vc_h_list", "vn_list", "vn_h_list"))
+    f = lambda t: t.float().contiguous()
+    stats = [(f(g[f"avg_{t}_u"]), f(g[f"avg_{t}_d"]), f(g[f"scale_{t}"])) for t in "kv"]
+    stores = []
+    for t, n_h, is_v in ((g["k_mn"], lists[3], False), (g["v_mn"], lists[7], True)):
+        ident = torch.arange(t.shape[2], dtype=torch.int32, device="cuda")
+        st = MidStore(1, ident, n_h, n_h.tolist(), Hkv, D, L, dtype, "cuda", is_v)
+        st.pack(t, 0, L)
+        stores.append(st)
+    for k_mn, v_mn in ((g["k_mn"], g["v_mn"]), stores):
+        got = ops.decode_attn_raw(g["q"], [(g["k_il"], g["v_il"])], g["k_mc"], g["v_mc"], k_mn, v_mn, *stats, lists, Hq, Hkv, L,
+                                  case["T"], force_generic=True).cpu().numpy().astype(np.float64).reshape(want.shape)
+        finite = np.isfinite(want)
+        assert np.array_equal(got[~finite], want[~finite]) and (~finite).any()
+        assert np.max(np.abs(got[finite] - want[finite])) <= 2e-4
