@@ -1712,6 +1712,10 @@ __device__ __forceinline__ void decode_il_fast_body(const IlArgs<E>& ia, int bx,
     if (LPT == 8) m[g] = fmaxf(m[g], fa_dpp<FA_DPP_ROR8>(m[g]));
     m[g] = fa_rows_max(m[g]);
   }
+  // rows past the last one read the first, whose values a weight of zero does not silence if they are infinite
+#pragma unroll
+  for (int it = 0; it < ITERS; ++it)
+    if (base + it * TPW + tl >= n_il) vraw[it] = Row8<E>{};
   // The weighted sums take the query heads two at a time (the rows' V values are converted once per pair): sixteen
   // accumulators live instead of eight per head, which is what lets six waves share a SIMD.
   // Rows held side by side in the wave: lanes i and i + 32 meet in registers, the rest in LDS together with the

@@ -380,3 +380,24 @@ def test_any_shape_decode_kernels_beside_infinities(dtype, L, k_counts, v_counts
         finite = np.isfinite(want)
         assert np.array_equal(got[~finite], want[~finite]) and (~finite).any()
         assert np.max(np.abs(got[finite] - want[finite])) <= 2e-4
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rows", [1, 63, 65, 200])
+def test_window_rows_with_an_infinite_value(dtype, rows):
+    """The first row holds infinite values: they are the result in those dims and touch no other, however far the last
+    tile reaches past the rows.  Bound: as for the window above."""
+    from fourierattention_amd import ops
+    B, Hq, Hkv, D = 2, 6, 2, 128
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    q, k, v = (torch.randn(s, generator=g, device="cuda").to(dtype) for s in ((B, Hq, 1, D), (B, rows, Hkv * D), (B, rows, Hkv * D)))
+    v[:, 0, 5] = float("inf")
+    v[:, 0, 200] = -float("inf")
+    lists = (torch.zeros(Hkv + 1, dtype=torch.int32, device="cuda"),) * 8
+    kd, vd = (t.double().view(B, rows, Hkv, D).permute(0, 2, 1, 3).contiguous() for t in (k, v))
+    p = (q.double().view(B, Hkv, Hq // Hkv, D).matmul(kd.transpose(2, 3).contiguous()) / D ** 0.5).softmax(-1)
+    want = p.matmul(vd).view(B, Hq, 1, D)
+    got = ops.decode_attn_raw(q, [(k, v)], None, None, None, None, None, None, lists, Hq, Hkv, 0, 1).double()
+    inf = want.isinf()
+    assert int(inf.sum()) == B * Hq and torch.equal(got[inf], want[inf])
+    assert float((got - want)[~inf].abs().max()) <= 2e-5
