@@ -438,13 +438,25 @@ class DynamicCache(Cache):
         if (step.action is not Action.STREAM or self._layers[layer_idx].window_only or self.defer_coef_update
                 or not query_states.is_cuda):
             return (*self._apply(step, key_states, value_states, layer_idx), None)
-        args = []
-        parts = self._stream(key_states, value_states, layer_idx, step, args)
-        return (*parts, self.decode_attention(query_states, layer_idx, num_heads, num_kv_heads, out_dtype=out_dtype, step=args[0]))
+        layer = self._layers[layer_idx]
+        spare, joined = layer.spare, []
+        parts = self._stream(key_states, value_states, layer_idx, step, joined)
+        try:
+            out = self.decode_attention(query_states, layer_idx, num_heads, num_kv_heads, out_dtype=out_dtype, step=joined)
+        except BaseException:
+            if joined:     # the attention was refused on the way to the launch: the update happens all the same ...
+                try:
+                    ops.stream_update(*joined[0])
+                except BaseException:      # ... unless it is refused too: then the layer holds what it held
+                    layer.n_mid -= 1
+                    layer.spare = spare
+                    raise
+            raise
+        return (*parts, out)
 
     def _stream(self, key_states: torch.Tensor, value_states: torch.Tensor, layer_idx: int, step, joined: Optional[list] = None):
         """One more token for a compressed layer: the oldest window row is evicted, then the spare slot takes the new
-        token.  ``joined``: the launch is left to the caller, who finds its arguments there."""
+        token.  ``joined``: the launch is left to the caller, who finds its arguments there until they are launched."""
         layer = self._layers[layer_idx]
         self._settle_coefficients(layer_idx)        # the row they are owed sits in the window slot written next
         layer.version += 1

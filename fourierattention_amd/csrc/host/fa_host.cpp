@@ -181,13 +181,20 @@ const float* stat(PyObject* tuple, Py_ssize_t i) {
 
 // decode_attn(q, il, k_mc, v_mc, k_mn, v_mn, stats_k, stats_v, lists, Hq, Hkv, L_m, T, sm_scale, out, cast, tables,
 //             force_generic, balance_heads, no_fuse, pending, no_alloc, timings[, step]) -> out
-// step: the arguments of stream_update as a tuple; the update comes in front of the attention
+// step: the arguments of stream_update as a tuple, or that in a list, which loses it when the update is launched; the update
+// comes in front of the attention
 // q (B, 1, Hq*D) or (B, Hq, 1, D), contiguous.  il: a sequence of up to two (k, v) pairs of row views, or (k, v, r): the
 // rows of one buffer in front of and behind row r.
 PyObject* decode_attn(PyObject*, PyObject* const* a, Py_ssize_t n) {
   FA_BEGIN
   CHECK(n == 23 || n == 24, "decode_attn takes 23 or 24 arguments");
   PyObject* step = n == 24 && a[23] != Py_None ? a[23] : nullptr;
+  PyObject* step_list = step && PyList_Check(step) ? step : nullptr;
+  if (step_list) {
+    CHECK(PyList_GET_SIZE(step_list) == 1, "step: a list of one tuple");
+    step = PyList_GET_ITEM(step_list, 0);
+  }
+  Ref step_held(step ? (Py_INCREF(step), step) : (Py_INCREF(Py_None), Py_None));
   CHECK(!step || (PyTuple_Check(step) && PyTuple_GET_SIZE(step) == 16 && a[20] == Py_None && !truth(a[21]) && a[22] == Py_None),
         "step: the 16 arguments of stream_update, with a workspace, no pending update and no timings");
   fa_stream_args su{};
@@ -318,6 +325,8 @@ PyObject* decode_attn(PyObject*, PyObject* const* a, Py_ssize_t n) {
     for (int i = 0; i < 4; ++i) PyList_SET_ITEM(list.p, i, PyFloat_FromDouble(ms[i]));
     if (PyList_SetSlice(a[22], 0, PyList_GET_SIZE(a[22]), list.p) < 0) throw PyError{};
   } else if (step) {
+    // (the library launches the update even where it refuses the attention)
+    if (step_list && PyList_SetSlice(step_list, 0, 1, nullptr) < 0) throw PyError{};
     check_status(fa_decode_step(&su, &d, st));
   } else {
     check_status(fa_decode_attn(&d, st));

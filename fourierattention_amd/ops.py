@@ -410,7 +410,8 @@ def decode_attn_raw(q, il_segments, k_mc, v_mc, k_mn, v_mn, stats_k, stats_v, li
     with ``skip_coef``): ``k_row, v_row (B, Hkv*D)`` are the rows that left the window (same strides).  The call
     applies it to ``k_mc`` / ``v_mc`` IN PLACE while it streams them, once; pass it to one call only.
     ``step``: the arguments of ``stream_update`` as a tuple: that update, then the attention over the state it leaves
-    (which the other arguments describe), in one launch less where the shapes allow it."""
+    (which the other arguments describe), in one launch less where the shapes allow it.  In a list of their own they are
+    taken out of it when the update is launched: what raises before leaves them there."""
     if seq_len_m >= _REPACK_MIN_ROWS and not force_generic:
         _warn_if_off_the_matrix_cores(q.dtype, num_head_q, num_head_kv, q.numel() // (q.shape[0] * num_head_q),
                                       (k_mc if lists[0].numel() else v_mc).shape[1] // 2, not isinstance(k_mn, torch.Tensor))

@@ -401,3 +401,73 @@ def test_window_rows_with_an_infinite_value(dtype, rows):
     inf = want.isinf()
     assert int(inf.sum()) == B * Hq and torch.equal(got[inf], want[inf])
     assert float((got - want)[~inf].abs().max()) <= 2e-5
+
+
+def _two_caches(dtype, B=2, Hkv=2, D=128, W=40, states=128):
+    """Two caches with the same prompt, and a source of new tokens."""
+    from fourierattention_amd import DynamicCache, ExtraConfig, masks
+    g = torch.Generator(device="cuda").manual_seed(21)
+    rn = lambda *s: torch.randn(s, generator=g, device="cuda").to(dtype)
+    m = masks.synthetic_masks(1, Hkv, D, [64, 40], [30, 64], seed=3)
+    cfg = ExtraConfig(numinittokens=4, maxlocallen=W, maxmidstates=states, non_critical_dims=m, non_critical_dims_path=None,
+                      max_position_embeddings=8192, num_key_value_heads=Hkv, max_new_tokens=8, model_type="llama")
+    one, two = DynamicCache(cfg), DynamicCache(cfg)
+    prompt = rn(B, Hkv, 4 + W + states + 300, D), rn(B, Hkv, 4 + W + states + 300, D)
+    one.update(*prompt, 0)
+    two.update(*prompt, 0)
+    return one, two, rn
+
+
+def _same_state(one, two):
+    a, b = one._layers[0], two._layers[0]
+    parts = zip((one.key_cache[0], one.value_cache[0]), (two.key_cache[0], two.value_cache[0]))
+    return (a.n_mid, a.spare) == (b.n_mid, b.spare) and all(torch.equal(x[n], y[n]) for x, y in parts for n in x)
+
+
+@pytest.mark.parametrize("refusal", ["type of q", "heads of q", "warning as an error"])
+def test_a_refused_attention_leaves_the_update(refusal):
+    """A decode step whose attention is refused on the way to the launch: the token is in the cache all the same, as with
+    ``update`` alone, and the next step is what it is there."""
+    import warnings
+    from fourierattention_amd import ops
+    from fourierattention_amd.attention import fourier_attention
+    B, Hq, Hkv, D, dtype = 2, 8, 2, 128, torch.float16
+    one, two, rn = _two_caches(dtype)
+    for _ in range(2):
+        q, k, v = rn(B, Hq, 1, D), rn(B, Hkv, 1, D), rn(B, Hkv, 1, D)
+        two.update(k, v, 0)
+        if refusal == "warning as an error":
+            old = ops._REPACK_MIN_ROWS
+            ops._REPACK_MIN_ROWS = 1
+            ops._warned_shapes.clear()
+            warn = ops._warn_if_off_the_matrix_cores
+            ops._warn_if_off_the_matrix_cores = lambda *a: warnings.warn("off the matrix cores", RuntimeWarning)
+            try:
+                with warnings.catch_warnings(), pytest.raises(RuntimeWarning):
+                    warnings.simplefilter("error")
+                    fourier_attention(q, k, v, one, 0, Hq, Hkv)
+            finally:
+                ops._REPACK_MIN_ROWS, ops._warn_if_off_the_matrix_cores = old, warn
+        else:
+            with pytest.raises((AssertionError, RuntimeError)):
+                fourier_attention(q.float() if refusal == "type of q" else rn(B, 9, 1, D), k, v, one, 0, Hq if refusal == "type of q" else 9, Hkv)
+        assert _same_state(one, two)
+        q, k, v = rn(B, Hq, 1, D), rn(B, Hkv, 1, D), rn(B, Hkv, 1, D)
+        got = fourier_attention(q, k, v, one, 0, Hq, Hkv)
+        two.update(k, v, 0)
+        assert torch.equal(got, two.decode_attention(q, 0, Hq, Hkv, out_dtype=dtype).view(B, 1, Hq * D)) and _same_state(one, two)
+
+
+def test_a_refused_update_leaves_the_layer():
+    """A token of another type than the window: neither call counts a row that was never written."""
+    from fourierattention_amd.attention import fourier_attention
+    one, two, rn = _two_caches(torch.bfloat16)
+    q, k, v = rn(2, 8, 1, 128), rn(2, 2, 1, 128), rn(2, 2, 1, 128)
+    with pytest.raises(AssertionError):
+        fourier_attention(q, k.float(), v.float(), one, 0, 8, 2)
+    with pytest.raises(AssertionError):
+        two.update(k.float(), v.float(), 0)
+    a, b = one._layers[0], two._layers[0]       # (the views of the parts are of the state before, on either side)
+    assert (a.n_mid, a.spare, a.version) == (b.n_mid, b.spare, b.version)
+    for x, y in ((a.k, b.k), (a.v, b.v)):
+        assert torch.equal(x.ring[:, :40], y.ring[:, :40]) and torch.equal(x.coef, y.coef) and torch.equal(x.mid.data, y.mid.data)
