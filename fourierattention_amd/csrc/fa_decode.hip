@@ -1935,9 +1935,11 @@ int share_out_splits(fa_mfma::SplitTable& st, int Hkv, int tiles, int ns, int ro
 
 // kpad / vpad: see share_out_splits.  full_room: size the partial buffers for the most uneven share a call with those
 // lists could ask for (the workspace query, which does not see them).
+// max_splits: splits of the mid rows on the any-shape path at most
+constexpr int kAnyShapeSplits = 64;
 Plan make_plan(int B, int Hq, int Hkv, int D, int N, int n_il, int L_m, bool mfma, bool il_fast,
                const int32_t* kpad = nullptr, const int32_t* vpad = nullptr, bool full_room = false,
-               bool fill_dies = true) {
+               bool fill_dies = true, int max_splits = kAnyShapeSplits) {
   Plan p{};
   p.path = mfma ? Path::Mfma : Path::Generic;
   p.n_il_split = fa_cdiv(n_il, il_fast ? kIlFastTile : kTile);
@@ -1974,7 +1976,7 @@ Plan make_plan(int B, int Hq, int Hkv, int D, int N, int n_il, int L_m, bool mfm
     int want = fa_cdiv(1024, (int64_t)B * Hkv);
     if (want < 1) want = 1;
     int ns = tiles < want ? tiles : want;
-    if (ns > 64) ns = 64;
+    if (ns > max_splits) ns = max_splits;
     p.tiles_per_split = ns > 0 ? fa_cdiv(tiles, ns) : 0;
     p.n_mid_split = ns > 0 ? fa_cdiv(tiles, p.tiles_per_split) : 0;
     for (int h = 0; h < fa_mfma::kSplitHeads; ++h) p.st.n[h] = p.n_mid_split;
@@ -2376,14 +2378,22 @@ bool use_mfma(const fa_decode_args& a) {
 
 }  // namespace
 
-// full_room: room for the uneven shares that a call with the per-head lists on the host side may ask for
+// full_room: room for the uneven shares that a call with the per-head lists on the host side may ask for, and for as many
+// splits as the any-shape path takes where nothing limits it (without: one per 256 rows or more, which it gets by with)
 static size_t workspace_bytes_for(int B, int Hq, int Hkv, int D, int N, int il_rows_total, int L_m, bool full_room) {
   if (B <= 0 || Hq <= 0 || Hkv <= 0 || D <= 0 || N < 0 || il_rows_total < 0 || L_m < 0 || Hq % Hkv) return 0;
   const int n = N > 0 ? N : 1;
   // large enough for either path
+  int coarse = kAnyShapeSplits;
+  if (!full_room && L_m > 0) {
+    const int tiles = fa_cdiv(L_m, 256), want = fa_cdiv(1024, (int64_t)B * Hkv);
+    const int ns = tiles < want ? tiles : want;
+    coarse = fa_cdiv(tiles, fa_cdiv(tiles, ns < kAnyShapeSplits ? ns : kAnyShapeSplits));
+  }
   size_t a = 0;
   for (int il_fast = 0; il_fast < 2; ++il_fast) {
-    size_t b = make_plan(B, Hq, Hkv, D, n, il_rows_total, L_m, false, il_fast != 0).total;
+    size_t b = make_plan(B, Hq, Hkv, D, n, il_rows_total, L_m, false, il_fast != 0, nullptr, nullptr, false, true,
+                         coarse).total;
     if (b > a) a = b;
     if (mfma_shape_ok(Hq, Hkv, D, n, FA_BF16, FA_MID_PAGED)) {
       b = make_plan(B, Hq, Hkv, D, n, il_rows_total, L_m, true, il_fast != 0, nullptr, nullptr, full_room).total;
@@ -2471,8 +2481,13 @@ static int decode_attn_impl(const fa_decode_args* a, fa_stream_t stream, hipEven
   }
   const bool mfma = use_mfma(*a);
   const bool il_fast = il_fast_ok(*a);
-  const Plan p = make_plan(a->B, a->Hq, a->Hkv, a->D, a->N > 0 ? a->N : 1, a->il_rows[0] + a->il_rows[1], a->L_m, mfma,
-                           il_fast, a->k_pad_h_host, a->v_pad_h_host, false, !(a->no_fuse & 1));
+  auto plan = [&](int max_splits) {
+    return make_plan(a->B, a->Hq, a->Hkv, a->D, a->N > 0 ? a->N : 1, a->il_rows[0] + a->il_rows[1], a->L_m, mfma,
+                     il_fast, a->k_pad_h_host, a->v_pad_h_host, false, !(a->no_fuse & 1), max_splits);
+  };
+  Plan p = plan(kAnyShapeSplits);
+  // (the any-shape path does with fewer splits where the workspace holds no more)
+  while (!mfma && p.total > a->workspace_bytes && p.n_mid_split > 1) p = plan(p.n_mid_split - 1);
   FA_REQUIRE(a->workspace && a->workspace_bytes >= p.total, FA_ERR_WORKSPACE, "fa_decode_attn: workspace %zu < %zu",
              a->workspace_bytes, p.total);
   FA_REQUIRE(((uintptr_t)a->workspace & 255) == 0, FA_ERR_MISALIGNED, "fa_decode_attn: workspace not 256-byte aligned");

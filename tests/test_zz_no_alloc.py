@@ -168,3 +168,39 @@ def test_captured_in_a_graph_and_replayed():
             graph.replay()
             torch.cuda.synchronize()
             assert torch.equal(out, eager)
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,N,L_m,near", [(2, 64, 8, 512, 4096, 1028), (2, 32, 8, 1000, 4096, 1028), (1, 64, 8, 1000, 4096, 100),
+                                                  (8, 64, 8, 1000, 1500, 100), (16, 16, 2, 1000, 2048, 1028)])
+def test_middle_contexts_fit_the_buffer(B, Hq, Hkv, N, L_m, near):
+    """Shapes with a few thousand mid rows, on either path: the any-shape kernels cut them into as many splits as fit.
+    Needs no GPU: the call ends at its null pointers, behind the check of the size."""
+    from fourierattention_amd import _lib
+    lib = _lib.load()
+    a = _lib.DecodeArgs()
+    a.B, a.Hq, a.Hkv, a.D, a.N, a.L_m, a.q_len, a.T = B, Hq, Hkv, 128, N, L_m, 1, 131072
+    a.il_rows[0] = near
+    for a.mid_layout in (0, 1):
+        assert lib.fa_decode_attn_noalloc(ctypes.byref(a), None) != -4, lib.fa_last_error_string()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_any_shape_kernels_with_fewer_splits_than_a_workspace_allows(dtype):
+    """1000 frequencies: the any-shape kernels, whose partial results for every 64 rows are more than the buffer holds.  The
+    call cuts the rows into fewer splits; the same sums in another order (single precision over 4096 rows of order one)."""
+    from fourierattention_amd import _lib, ops
+    B, Hq, Hkv, D, N, L = 2, 32, 8, 128, 1000, 4096
+    g = torch.Generator(device="cuda").manual_seed(9)
+    rn = lambda *s: torch.randn(s, generator=g, device="cuda")
+    flat = lambda lo, hi: torch.cat([torch.arange(h * D + lo, h * D + hi) for h in range(Hkv)]).int().cuda()
+    offs = (torch.arange(Hkv + 1) * 64).int().cuda()
+    lists = (flat(0, 64), offs, flat(64, 128), offs) * 2
+    C = Hkv * 64
+    stats = [(rn(B, C), rn(B, C), rn(B, C).abs()) for _ in range(2)]
+    args = (rn(B, 1, Hq * D).to(dtype), [(rn(B, 200, Hkv * D).to(dtype), rn(B, 200, Hkv * D).to(dtype))], rn(B, 2 * N, C), rn(B, 2 * N, C),
+            rn(B, L, C).to(dtype), rn(B, L, C).to(dtype), *stats, lists, Hq, Hkv, L, 131072)
+    assert _lib.load().fa_decode_attn_workspace_bytes(B, Hq, Hkv, D, N, 200, L) > _lib.DECODE_NOALLOC_SCRATCH_BYTES
+    want = ops.decode_attn_raw(*args, force_generic=True)
+    got = ops.decode_attn_raw(*args, force_generic=True, no_alloc=True)
+    assert float((got - want).abs().max()) <= 2e-5 * max(1.0, float(want.abs().max()))
