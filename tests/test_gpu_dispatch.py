@@ -471,3 +471,30 @@ def test_a_refused_update_leaves_the_layer():
     assert (a.n_mid, a.spare, a.version) == (b.n_mid, b.spare, b.version)
     for x, y in ((a.k, b.k), (a.v, b.v)):
         assert torch.equal(x.ring[:, :40], y.ring[:, :40]) and torch.equal(x.coef, y.coef) and torch.equal(x.mid.data, y.mid.data)
+
+
+@pytest.mark.parametrize("rows,launches", [(1, 1), (3, 1), (4, 3), (16, 3)])
+def test_where_the_norms_of_a_decoder_step_run(rows, launches, monkeypatch):
+    """Up to 6144 elements the two norms of a layer ride in its projections and only the final one is a launch; above, all
+    three are.  The logits against the chain of tensor ops, which rounds between them: bf16 through one layer, 2^-8 of the
+    largest, a few times over."""
+    from fourierattention_amd import DynamicCache, ExtraConfig, masks, ops
+    from fourierattention_amd.llama import LlamaConfig, random_init
+    llama = LlamaConfig(hidden_size=2048, intermediate_size=2048, num_hidden_layers=1, num_attention_heads=16, num_key_value_heads=8,
+                        head_dim=128, vocab_size=512)
+    model = random_init(llama, torch.bfloat16, "cuda:0", seed=1)
+    model.model.pack_projections()
+    cfg = ExtraConfig(numinittokens=4, maxlocallen=64, maxmidstates=64, non_critical_dims=masks.synthetic_masks(1, 8, 128, [64] * 8, [64] * 8, seed=1),
+                      non_critical_dims_path=None, max_position_embeddings=4096, num_key_value_heads=8, max_new_tokens=8, model_type="llama")
+    ids = torch.randint(0, 512, (rows, 21), device="cuda")
+    own, calls, logits = ops.add_rmsnorm, [], []
+    monkeypatch.setattr(ops, "add_rmsnorm", lambda *a: (calls.append(1), own(*a))[1])
+    with torch.no_grad():
+        for fused in (True, False):
+            model.model.fused_elementwise = fused
+            cache = DynamicCache(cfg)
+            model(ids[:, :20], cache)
+            calls.clear()
+            logits.append(model(ids[:, 20:], cache).logits)
+            assert len(calls) == (launches if fused else 0)
+    assert float((logits[0] - logits[1]).abs().max()) <= 4 * 2.0 ** -8 * float(logits[1].abs().max())
