@@ -672,7 +672,9 @@ __device__ __forceinline__ float weighted_sum(const float* __restrict__ ptr, int
 
 // The merge of a layer without mid rows: partial results of sink/window tiles only, one block per query head and a thread
 // per dim.  A chain of two loads (maxima, then nothing but the outputs requested with them) and one barrier; the general merge
-// below runs its seven phases with 1024 threads for it (23 tiles of two sequences: 7.1 us against 3.9).
+// below runs its seven phases with 1024 threads for it (23 tiles of two sequences: 7.1 us against 3.9).  With many tiles the
+// 1024 threads win: call and all, 256 tiles 38.6 us here and 39.3 there, 320 46.0 / 46.8, 384 54.4 / 54.1, 1024 132.9 / 129.2.
+constexpr int kIlMergeTiles = 320;
 __global__ __launch_bounds__(128) void decode_il_merge_kernel(const float* __restrict__ il_m, const float* __restrict__ il_d,
                                                               const float* __restrict__ il_o, int n, float* __restrict__ out,
                                                               void* __restrict__ out_cast, int cast_dtype, int Hq, int D) {
@@ -2351,7 +2353,7 @@ int launch_all(const fa_decode_args& a, const Plan& p, bool p_il_fast, float sm_
     // (with few splits the registers go to more rows of the V coefficients per thread instead)
     if (p.n_mid_split <= 8) decode_merge_fast_kernel<8, 8><<<grid, 1024, lds, st>>>(ma);
     else decode_merge_fast_kernel<16, 4><<<grid, 1024, lds, st>>>(ma);
-  } else if (p.n_mid_split == 0 && p.n_il_split <= 16384) {   // (their weights fit 64 KB of LDS)
+  } else if (p.n_mid_split == 0 && p.n_il_split <= kIlMergeTiles) {
     decode_il_merge_kernel<<<dim3(a.Hq, a.B), 128, (size_t)p.n_il_split * sizeof(float), st>>>(
         ilm, ild, ilo, p.n_il_split, a.out, a.out_cast, a.dtype, a.Hq, a.D);
   } else {

@@ -264,9 +264,10 @@ def test_update_in_the_attention_launch(dtype, B, Hq, Hkv, D, states, init, W, c
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("B,Hq,Hkv,D,rows", [(1, 2, 1, 128, 1), (2, 6, 2, 64, 64), (3, 8, 2, 80, 65), (1, 16, 2, 128, 4161), (2, 4, 4, 8, 1100)])
+@pytest.mark.parametrize("B,Hq,Hkv,D,rows", [(1, 2, 1, 128, 1), (2, 6, 2, 64, 64), (3, 8, 2, 80, 65), (1, 16, 2, 128, 4161), (2, 4, 4, 8, 1100),
+                                             (1, 4, 1, 128, 20480), (1, 4, 1, 128, 20481)])
 def test_window_only_decode(dtype, B, Hq, Hkv, D, rows):
-    """A layer that keeps only a window, one tile to more tiles than a wave has lanes, against float64.  Bound: single
+    """A layer that keeps only a window, one tile to more tiles than the merge for it takes, against float64.  Bound: single
     precision over ``rows`` keys of order one, then the rounding of the result to ``dtype``."""
     from fourierattention_amd import ops
     g = torch.Generator(device="cuda").manual_seed(rows)
