@@ -436,8 +436,10 @@ PyObject* rope_qk(PyObject*, PyObject* const* a, Py_ssize_t n) {
   CHECK(q.dim() == 3 && k.dim() == 3 && q.scalar_type() == k.scalar_type() && q.size(0) == k.size(0) && q.size(1) == k.size(1) && D > 0,
         "rope_qk: q and k (B, q_len, heads * D) of one type");
   const int64_t rows = q.size(0) * q.size(1);
+  // (one sequence may bring longer tables, of which the first rows are its own)
+  auto fits = [&](const at::Tensor& t) { return q.size(0) == 1 ? t.numel() >= rows * D : t.numel() == rows * D; };
   CHECK(cos.is_contiguous() && sin.is_contiguous() && cos.scalar_type() == q.scalar_type() && sin.scalar_type() == q.scalar_type() &&
-        cos.numel() == rows * D && sin.numel() == rows * D, "rope_qk: one row of cos and sin per token, of the type of q");
+        fits(cos) && fits(sin), "rope_qk: one row of cos and sin per token, of the type of q");
   const bool dense = q.is_contiguous();
   at::Tensor out = dense ? q : at::empty(q.sizes(), q.options().memory_format(at::MemoryFormat::Contiguous));
   check_status(fa_rope_qk(q.data_ptr(), row_stride(q), out.data_ptr(), k.data_ptr(), row_stride(k), cos.data_ptr(), sin.data_ptr(), (int)rows,

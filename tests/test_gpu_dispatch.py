@@ -499,3 +499,33 @@ def test_where_the_norms_of_a_decoder_step_run(rows, launches, monkeypatch):
             logits.append(model(ids[:, 20:], cache).logits)
             assert len(calls) == (launches if fused else 0)
     assert float((logits[0] - logits[1]).abs().max()) <= 4 * 2.0 ** -8 * float(logits[1].abs().max())
+
+
+def test_argument_forms_of_the_decode_call():
+    """Lists instead of tuples, whole numbers that are not ints, timings in any mutable sequence; the sine table alone in another
+    type, tables with rows to spare."""
+    from collections import UserList
+    from fourierattention_amd import ops
+    from tests import helpers as H
+    dtype = torch.float32
+    case = H.attn_case(3, 1, 4, 2, 128, 9, 70, 16, 300, [64, 40], [30, 64], dtype)
+    g = H.attn_case_gpu(case, dtype)
+    lists = [ops.as_i32(g[n]) for n in ("kc_list", "kc_h_list", "kn_list", "kn_h_list", "vc_list", "vc_h_list", "vn_list", "vn_h_list")]
+    f = lambda t: t.float().contiguous()
+    stats = [[f(g[f"avg_{t}_u"]), f(g[f"avg_{t}_d"]), f(g[f"scale_{t}"])] for t in "kv"]
+    args = (g["k_mc"], g["v_mc"], g["k_mn"], g["v_mn"])
+    pair = [g["k_il"], g["v_il"]]
+    want = ops.decode_attn_raw(g["q"], [tuple(pair)], *args, *map(tuple, stats), tuple(lists), 4, 2, 70, 300)
+    got = ops.decode_attn_raw(g["q"], (pair, None), *args, *stats, lists, 4, 2, np.int64(70), 300.0, no_fuse=np.bool_(False))
+    assert torch.equal(got, want)
+    ms = UserList()
+    assert torch.equal(ops.decode_attn_raw(g["q"], [pair], *args, *stats, lists, 4, 2, torch.tensor(70), 300, timings=ms), want)
+    assert len(ms) == 4 and all(isinstance(x, float) for x in ms)
+    q, k = (torch.randn((2, 3, n * 128), device="cuda").bfloat16() for n in (4, 2))
+    cos, sin = torch.randn((2, 2, 3, 128), device="cuda").bfloat16().unbind(0)
+    k1, k2 = k.clone(), k.clone()
+    a, b = ops.rope_qk(q.clone(), k1, cos, sin, 128), ops.rope_qk(q.clone(), k2, cos, sin.float(), 128)
+    assert torch.equal(a, b) and torch.equal(k1, k2)
+    k1, k2 = k[:1].clone(), k[:1].clone()      # one sequence, tables with rows to spare
+    a, b = ops.rope_qk(q[:1].clone(), k1, cos[:1], sin[:1], 128), ops.rope_qk(q[:1].clone(), k2, *(t.reshape(1, 6, 128) for t in (cos, sin)), 128)
+    assert torch.equal(a, b) and torch.equal(k1, k2)
