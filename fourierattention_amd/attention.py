@@ -54,13 +54,22 @@ def _exact_attention(query_states, k_local, v_local, num_kv_heads, head_dim):
     return o.transpose(1, 2)  # (B, q_len, Hq, D)
 
 
+# what update_and_attend stands for: a cache (a subclass, an instance, a patched class) with others of its own goes through them
+_OWN = (DynamicCache.update, DynamicCache.decode_attention)
+
+
+def _takes_a_step(cache) -> bool:
+    return (type(cache) is DynamicCache and "update" not in cache.__dict__ and "decode_attention" not in cache.__dict__
+            and DynamicCache.update is _OWN[0] and DynamicCache.decode_attention is _OWN[1])
+
+
 def fourier_attention(query_states: torch.Tensor, key_states: torch.Tensor, value_states: torch.Tensor,
                       past_key_value: DynamicCache, layer_idx: int, num_heads: int, num_key_value_heads: int,
                       cache_kwargs=None) -> torch.Tensor:
     """``query_states (B, Hq, q_len, D)``, ``key_states / value_states (B, Hkv, q_len, D)`` after RoPE.
     Returns ``(B, q_len, Hq*D)`` in the query dtype (modeling_llama_fourier.py:618-663)."""
     bsz, _, q_len, head_dim = query_states.shape
-    if q_len == 1 and type(past_key_value) is DynamicCache:   # (a subclass may do more in update or decode_attention)
+    if q_len == 1 and _takes_a_step(past_key_value):
         k_parts, v_parts, o = past_key_value.update_and_attend(query_states, key_states, value_states, layer_idx, num_heads,
                                                                num_key_value_heads, query_states.dtype)
         if o is not None:

@@ -39,3 +39,31 @@ def test_row_slices_of_wider_rows(B, q_len, dtype):
         w = torch.randn((48, 1024), generator=g, device="cuda").to(dtype)
         packed = ops.PackedLinearWeight(w)
         assert torch.equal(ops.linear_packed(gate, packed), ops.linear_packed(gate.contiguous(), packed))
+
+
+@pytest.mark.parametrize("how", ["instance", "class", "subclass"])
+def test_a_replaced_update_is_what_the_attention_calls(how, monkeypatch):
+    """``fourier_attention`` goes through ``update`` of the cache it is given, for one token as for many."""
+    from fourierattention_amd import DynamicCache, ExtraConfig, masks
+    from fourierattention_amd.attention import fourier_attention
+    m = masks.synthetic_masks(1, 2, 16, [8, 8], [8, 8], seed=3)
+    cfg = ExtraConfig(numinittokens=4, maxlocallen=16, maxmidstates=16, non_critical_dims=m, non_critical_dims_path=None,
+                      max_position_embeddings=512, num_key_value_heads=2, max_new_tokens=8, model_type="llama")
+    calls = []
+
+    def update(key_states, value_states, layer_idx, cache_kwargs=None):
+        calls.append(layer_idx)
+        k, v = (t.transpose(1, 2).reshape(1, 1, 32) for t in (key_states, value_states))
+        return ({"k_init": None, "k_compressed": None, "k_uncompressed": None, "k_local": k},
+                {"v_init": None, "v_compressed": None, "v_uncompressed": None, "v_local": v})
+    if how == "subclass":
+        cache = type("Own", (DynamicCache,), {"update": lambda self, *a, **k: update(*a, **k)})(cfg, device="cpu")
+    else:
+        cache = DynamicCache(cfg, device="cpu")
+        if how == "instance":
+            cache.update = update
+        else:
+            monkeypatch.setattr(DynamicCache, "update", lambda self, *a, **k: update(*a, **k))
+    q, k, v = torch.randn(1, 4, 1, 16), torch.randn(1, 2, 1, 16), torch.randn(1, 2, 1, 16)
+    out = fourier_attention(q, k, v, cache, 0, 4, 2)
+    assert calls == [0] and torch.allclose(out.view(1, 2, 2, 16), v.transpose(1, 2).reshape(1, 2, 1, 16).expand(1, 2, 2, 16))
