@@ -96,6 +96,19 @@ void check_status(int rc) {
   fail(PyExc_RuntimeError, "a HIP call failed");
 }
 
+// Runs f without the interpreter lock: a launch waits where the queue is full, an allocation or a copy to the host may wait for
+// everything queued, and other Python threads go on meanwhile.  Whatever f needs of Python is taken beforehand, and the
+// tensors behind its pointers are held.
+template <typename F>
+auto unlocked(F&& f) {
+  struct Guard {
+    PyThreadState* state = PyEval_SaveThread();
+    ~Guard() { PyEval_RestoreThread(state); }
+  } guard;
+  return f();
+}
+#define LAUNCH(call) check_status(unlocked([&] { return call; }))
+
 #define FA_BEGIN HANDLE_TH_ERRORS try {
 #define FA_END } catch (const PyError&) { return nullptr; } END_HANDLE_TH_ERRORS
 
@@ -114,8 +127,8 @@ void token_rows(const at::Tensor& t, int64_t& batch, int64_t& width, int64_t& ba
 
 // stream_update(k_new, v_new, k_ring, v_ring, evict_slot, write_slot, k_coef, v_coef, kc_list, vc_list, phase, T,
 //               k_mid, v_mid, mid_pos, skip_coef)
-// fills `s` from them and returns the window buffer of K
-const at::Tensor& stream_args(PyObject* const* a, fa_stream_args& s) {
+// fills `s` from them and returns the window buffer of K; held: the memory of the page stores, which grow by replacing it
+const at::Tensor& stream_args(PyObject* const* a, fa_stream_args& s, at::Tensor (&held)[2]) {
   const at::Tensor &k_new = tensor(a[0], "k_new"), &v_new = tensor(a[1], "v_new");
   const at::Tensor &k_ring = gpu_tensor(a[2], "k_ring"), &v_ring = gpu_tensor(a[3], "v_ring");
   const at::Tensor &k_coef = tensor(a[6], "k_coef"), &v_coef = tensor(a[7], "v_coef");
@@ -140,7 +153,8 @@ const at::Tensor& stream_args(PyObject* const* a, fa_stream_args& s) {
   s.kc_list = ptr<int32_t>(kc); s.vc_list = ptr<int32_t>(vc);
   s.Ck = (int32_t)kc.numel(); s.Cv = (int32_t)vc.numel();
   s.N = (int32_t)(k_coef.size(1) / 2); s.phase = integer(a[10]); s.T = (int32_t)integer(a[11]);
-  s.k_mid = tensor_attr(k_mid, s_data, "k_mid.data").data_ptr(); s.v_mid = tensor_attr(v_mid, s_data, "v_mid.data").data_ptr();
+  held[0] = tensor_attr(k_mid, s_data, "k_mid.data"); held[1] = tensor_attr(v_mid, s_data, "v_mid.data");
+  s.k_mid = held[0].data_ptr(); s.v_mid = held[1].data_ptr();
   s.k_mid_batch_stride = int_attr(k_mid, s_batch_stride); s.v_mid_batch_stride = int_attr(v_mid, s_batch_stride);
   s.cap_pages = (int32_t)int_attr(k_mid, s_cap_pages); s.mid_pos = integer(a[14]);
   CHECK(s.cap_pages == int_attr(v_mid, s_cap_pages), "the page stores of K and V must have the same capacity");
@@ -157,8 +171,10 @@ PyObject* stream_update(PyObject*, PyObject* const* a, Py_ssize_t n) {
   FA_BEGIN
   CHECK(n == 16, "stream_update takes 16 arguments");
   fa_stream_args s{};
-  const at::Tensor& k_ring = stream_args(a, s);
-  check_status(fa_stream_update(&s, stream_of(k_ring)));
+  at::Tensor held[2];
+  const at::Tensor& k_ring = stream_args(a, s, held);
+  const fa_stream_t st = stream_of(k_ring);
+  LAUNCH(fa_stream_update(&s, st));
   Py_RETURN_NONE;
   FA_END
 }
@@ -198,7 +214,8 @@ PyObject* decode_attn(PyObject*, PyObject* const* a, Py_ssize_t n) {
   CHECK(!step || (PyTuple_Check(step) && PyTuple_GET_SIZE(step) == 16 && a[20] == Py_None && !truth(a[21]) && a[22] == Py_None),
         "step: the 16 arguments of stream_update, with a workspace, no pending update and no timings");
   fa_stream_args su{};
-  if (step) stream_args(&PyTuple_GET_ITEM(step, 0), su);
+  at::Tensor held[2], step_mem[2];
+  if (step) stream_args(&PyTuple_GET_ITEM(step, 0), su, step_mem);
   const at::Tensor& q = gpu_tensor(a[0], "q");
   fa_decode_args d{};
   d.Hq = (int32_t)integer(a[9]); d.Hkv = (int32_t)integer(a[10]);
@@ -255,7 +272,7 @@ PyObject* decode_attn(PyObject*, PyObject* const* a, Py_ssize_t n) {
       d.k_mn_batch_stride = k_mn.stride(0); d.k_mn_row_stride = k_mn.stride(1);
       d.v_mn_batch_stride = v_mn.stride(0); d.v_mn_row_stride = v_mn.stride(1);
     } else {
-      const at::Tensor &kd = tensor_attr(a[4], s_data, "k_mn.data"), &vd = tensor_attr(a[5], s_data, "v_mn.data");
+      const at::Tensor &kd = held[0] = tensor_attr(a[4], s_data, "k_mn.data"), &vd = held[1] = tensor_attr(a[5], s_data, "v_mn.data");
       CHECK(kd.scalar_type() == dt && vd.scalar_type() == dt && int_attr(a[4], s_cap_pages) == int_attr(a[5], s_cap_pages),
             "the page stores must have the type of q and one capacity");
       d.mid_layout = FA_MID_PAGED;
@@ -300,7 +317,8 @@ PyObject* decode_attn(PyObject*, PyObject* const* a, Py_ssize_t n) {
     out = gpu_tensor(a[14], "out");
     CHECK(out.is_contiguous() && out.numel() == q.numel(), "out must be contiguous and as large as q");
   } else {
-    out = at::empty({d.B, d.Hq, 1, d.D}, q.options().dtype(truth(a[15]) ? dt : at::kFloat));
+    const auto options = q.options().dtype(truth(a[15]) ? dt : at::kFloat);
+    out = unlocked([&] { return at::empty({d.B, d.Hq, 1, d.D}, options); });
   }
   if (out.scalar_type() == at::kFloat) d.out = static_cast<float*>(out.data_ptr());
   else {
@@ -309,7 +327,7 @@ PyObject* decode_attn(PyObject*, PyObject* const* a, Py_ssize_t n) {
   }
   const fa_stream_t st = stream_of(q);
   if (truth(a[21])) {
-    check_status(fa_decode_attn_noalloc(&d, st));
+    LAUNCH(fa_decode_attn_noalloc(&d, st));
     return a[14] != Py_None ? (Py_INCREF(a[14]), a[14]) : THPVariable_Wrap(out);
   }
   const size_t need = fa_decode_attn_workspace_bytes(d.B, d.Hq, d.Hkv, d.D, d.N, d.il_rows[0] + d.il_rows[1], d.L_m);
@@ -320,16 +338,16 @@ PyObject* decode_attn(PyObject*, PyObject* const* a, Py_ssize_t n) {
   d.workspace = w.data_ptr(); d.workspace_bytes = (size_t)w.numel();
   if (a[22] != Py_None) {
     float ms[4];
-    check_status(fa_decode_attn_timed(&d, st, ms));
+    LAUNCH(fa_decode_attn_timed(&d, st, ms));
     Ref list(PyList_New(4));
     for (int i = 0; i < 4; ++i) PyList_SET_ITEM(list.p, i, PyFloat_FromDouble(ms[i]));
     if (PyList_SetSlice(a[22], 0, PyList_GET_SIZE(a[22]), list.p) < 0) throw PyError{};
   } else if (step) {
     // (the library launches the update even where it refuses the attention)
     if (step_list && PyList_SetSlice(step_list, 0, 1, nullptr) < 0) throw PyError{};
-    check_status(fa_decode_step(&su, &d, st));
+    LAUNCH(fa_decode_step(&su, &d, st));
   } else {
-    check_status(fa_decode_attn(&d, st));
+    LAUNCH(fa_decode_attn(&d, st));
   }
   return a[14] != Py_None ? (Py_INCREF(a[14]), a[14]) : THPVariable_Wrap(out);
   FA_END
@@ -348,10 +366,12 @@ PyObject* add_rmsnorm(PyObject*, PyObject* const* a, Py_ssize_t n) {
     CHECK(t.is_contiguous() && t.sizes() == h.sizes() && t.scalar_type() == h.scalar_type(), "add_rmsnorm: delta must match h");
     delta = ptr<>(t);
   }
-  at::Tensor y = at::empty_like(h);
+  at::Tensor y = unlocked([&] { return at::empty_like(h); });
   const int64_t hidden = h.size(-1);
-  check_status(fa_add_rmsnorm(h.data_ptr(), delta, w.data_ptr(), y.data_ptr(), (int)(h.numel() / hidden), (int)hidden, (float)real(a[3]),
-                              dtype_code(h), stream_of(h)));
+  const float eps = (float)real(a[3]);
+  const int dtype = dtype_code(h);
+  const fa_stream_t st = stream_of(h);
+  LAUNCH(fa_add_rmsnorm(h.data_ptr(), delta, w.data_ptr(), y.data_ptr(), (int)(h.numel() / hidden), (int)hidden, eps, dtype, st));
   return THPVariable_Wrap(y);
   FA_END
 }
@@ -378,6 +398,9 @@ PyObject* linear_packed(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const at::Tensor &x = gpu_tensor(a[0], "x"), &w = gpu_tensor(a[1], "weight");
   const int64_t k = integer(a[2]), n_out = integer(a[3]);
   CHECK(x.scalar_type() == w.scalar_type() && x.dim() >= 1 && x.size(-1) == k && w.numel() == k * n_out, "linear_packed: x does not fit the weight");
+  const int rows = (int)(x.numel() / k), dtype = dtype_code(x);
+  const int64_t stride = row_stride(x);
+  const fa_stream_t st = stream_of(x);
   const void* norm = nullptr;
   float eps = 0.f;
   bool gated = false;
@@ -395,16 +418,14 @@ PyObject* linear_packed(PyObject*, PyObject* const* a, Py_ssize_t n) {
       const at::Tensor& res = gpu_tensor(a[6], "residual");
       CHECK(!gated && res.is_contiguous() && res.scalar_type() == x.scalar_type() && res.sizes() == at::IntArrayRef(shape),
             "linear_packed: the residual must be contiguous and have the type and shape of the result");
-      check_status(fa_linear_packed_step(x.data_ptr(), row_stride(x), norm, eps, w.data_ptr(), res.data_ptr(), (int)(x.numel() / k), (int)k,
-                                         (int)n_out, 1, dtype_code(x), stream_of(x)));
+      LAUNCH(fa_linear_packed_step(x.data_ptr(), stride, norm, eps, w.data_ptr(), res.data_ptr(), rows, (int)k, (int)n_out, 1, dtype, st));
       Py_INCREF(a[6]);
       return a[6];
     }
   }
   if (gated) shape.back() = n_out / 2;
-  at::Tensor out = at::empty(shape, x.options());
-  check_status(fa_linear_packed_step(x.data_ptr(), row_stride(x), norm, eps, w.data_ptr(), out.data_ptr(), (int)(x.numel() / k), (int)k,
-                                     (int)n_out, gated ? 2 : 0, dtype_code(x), stream_of(x)));
+  at::Tensor out = unlocked([&] { return at::empty(shape, x.options()); });
+  LAUNCH(fa_linear_packed_step(x.data_ptr(), stride, norm, eps, w.data_ptr(), out.data_ptr(), rows, (int)k, (int)n_out, gated ? 2 : 0, dtype, st));
   return THPVariable_Wrap(out);
   FA_END
 }
@@ -417,12 +438,13 @@ PyObject* silu_mul(PyObject*, PyObject* const* a, Py_ssize_t n) {
   CHECK(g.sizes() == u.sizes() && g.scalar_type() == u.scalar_type() && g.strides() == u.strides() && g.dim() >= 1 && g.stride(-1) == 1,
         "silu_mul: gate and up must share shape, type and strides");
   const int64_t cols = g.size(-1), rows = g.numel() / (cols > 0 ? cols : 1), stride = row_stride(g), es = g.element_size();
-  at::Tensor out = at::empty(g.sizes(), g.options().memory_format(at::MemoryFormat::Contiguous));
+  const auto options = g.options().memory_format(at::MemoryFormat::Contiguous);
+  at::Tensor out = unlocked([&] { return at::empty(g.sizes(), options); });
   const fa_stream_t st = stream_of(g);
+  const int dtype = dtype_code(g);
   for (int64_t r0 = 0; r0 < rows; r0 += 65535)   // the row index is the launch's second grid dimension
-    check_status(fa_silu_mul((const char*)g.data_ptr() + r0 * stride * es, (const char*)u.data_ptr() + r0 * stride * es,
-                             (char*)out.data_ptr() + r0 * cols * es, (int)std::min<int64_t>(65535, rows - r0), (int)cols, stride,
-                             dtype_code(g), st));
+    LAUNCH(fa_silu_mul((const char*)g.data_ptr() + r0 * stride * es, (const char*)u.data_ptr() + r0 * stride * es,
+                       (char*)out.data_ptr() + r0 * cols * es, (int)std::min<int64_t>(65535, rows - r0), (int)cols, stride, dtype, st));
   return THPVariable_Wrap(out);
   FA_END
 }
@@ -441,9 +463,13 @@ PyObject* rope_qk(PyObject*, PyObject* const* a, Py_ssize_t n) {
   CHECK(cos.is_contiguous() && sin.is_contiguous() && cos.scalar_type() == q.scalar_type() && sin.scalar_type() == q.scalar_type() &&
         fits(cos) && fits(sin), "rope_qk: one row of cos and sin per token, of the type of q");
   const bool dense = q.is_contiguous();
-  at::Tensor out = dense ? q : at::empty(q.sizes(), q.options().memory_format(at::MemoryFormat::Contiguous));
-  check_status(fa_rope_qk(q.data_ptr(), row_stride(q), out.data_ptr(), k.data_ptr(), row_stride(k), cos.data_ptr(), sin.data_ptr(), (int)rows,
-                          (int)(q.size(2) / D), (int)(k.size(2) / D), (int)D, dtype_code(q), stream_of(q)));
+  const auto options = q.options().memory_format(at::MemoryFormat::Contiguous);
+  at::Tensor out = dense ? q : unlocked([&] { return at::empty(q.sizes(), options); });
+  const int64_t q_stride = row_stride(q), k_stride = row_stride(k);
+  const int dtype = dtype_code(q);
+  const fa_stream_t st = stream_of(q);
+  LAUNCH(fa_rope_qk(q.data_ptr(), q_stride, out.data_ptr(), k.data_ptr(), k_stride, cos.data_ptr(), sin.data_ptr(), (int)rows,
+                    (int)(q.size(2) / D), (int)(k.size(2) / D), (int)D, dtype, st));
   return dense ? (Py_INCREF(a[0]), a[0]) : THPVariable_Wrap(out);
   FA_END
 }
@@ -458,8 +484,10 @@ PyObject* append_rows(PyObject*, PyObject* const* a, Py_ssize_t n) {
         kd.strides() == vd.strides() && kd.stride(2) == 1 && kd.size(0) == k.size(0) && kd.size(2) == k.size(2), "append_rows: shapes and strides");
   CHECK(v.scalar_type() == k.scalar_type() && kd.scalar_type() == k.scalar_type() && vd.scalar_type() == k.scalar_type() && pos >= 0 &&
         pos + k.size(1) <= kd.size(1), "append_rows: types, rows past the end");
-  check_status(fa_append_rows(k.data_ptr(), v.data_ptr(), k.stride(0), k.stride(1), kd.data_ptr(), vd.data_ptr(), kd.stride(0), kd.stride(1),
-                              pos, (int)k.size(0), (int)k.size(1), (int)k.size(2), dtype_code(k), stream_of(kd)));
+  const int dtype = dtype_code(k);
+  const fa_stream_t st = stream_of(kd);
+  LAUNCH(fa_append_rows(k.data_ptr(), v.data_ptr(), k.stride(0), k.stride(1), kd.data_ptr(), vd.data_ptr(), kd.stride(0), kd.stride(1),
+                        pos, (int)k.size(0), (int)k.size(1), (int)k.size(2), dtype, st));
   Py_RETURN_NONE;
   FA_END
 }
@@ -496,7 +524,7 @@ PyObject* operands(PyObject*, PyObject* const* a, Py_ssize_t n) {
     list_item[o] = -1;
     if (t.scalar_type() == at::kInt) lists[o] = t;
     else if (t.scalar_type() == at::kLong && t.is_contiguous() && t.device() == dev) list_item[o] = add(t, t.numel(), FA_CONVERT_I64_I32, 1);
-    else lists[o] = t.to(at::kInt);
+    else lists[o] = unlocked([&] { return t.to(at::kInt); });
   }
   for (Py_ssize_t i = 0; i < n_st; ++i) {
     const at::Tensor& t = tensor(PyTuple_GET_ITEM(a[1], i), "statistics");
@@ -504,7 +532,7 @@ PyObject* operands(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const bool here = t.is_contiguous() && t.device() == dev;
     if (here && t.scalar_type() == at::kBFloat16) stat_item[i] = add(t, t.numel(), FA_CONVERT_BF16_F32, 1);
     else if (here && t.scalar_type() == at::kHalf) stat_item[i] = add(t, t.numel(), FA_CONVERT_F16_F32, 1);
-    else stats[i] = t.to(at::kFloat).contiguous();
+    else stats[i] = unlocked([&] { return t.to(at::kFloat).contiguous(); });
   }
   if (k_unit > 0) {
     for (int i = 0; i < 2; ++i) {
@@ -518,9 +546,10 @@ PyObject* operands(PyObject*, PyObject* const* a, Py_ssize_t n) {
   }
   at::Tensor arena;
   if (used > 0) {
-    arena = at::empty({used}, at::TensorOptions().dtype(at::kInt).device(dev));
+    arena = unlocked([&] { return at::empty({used}, at::TensorOptions().dtype(at::kInt).device(dev)); });
     for (int i = 0; i < n_items; ++i) items[i].dst = static_cast<int32_t*>(arena.data_ptr()) + at_item[i];
-    check_status(fa_convert(items, n_items, stream_of(arena)));
+    const fa_stream_t st = stream_of(arena);
+    LAUNCH(fa_convert(items, n_items, st));
   }
   auto part = [&](int item) { return arena.narrow(0, at_item[item], items[item].count); };
   Ref out(PyTuple_New(3));
@@ -548,11 +577,13 @@ PyObject* operands(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const bool one = list_item[3] == 0 && list_item[7] == 1;
   at::Tensor host[2];
   if (one) {
-    const at::Tensor both = arena.narrow(0, 0, at_item[1] + items[1].count).cpu();
+    const at::Tensor both = unlocked([&] { return arena.narrow(0, 0, at_item[1] + items[1].count).cpu(); });
     for (int i = 0; i < 2; ++i) host[i] = both.narrow(0, at_item[i], items[i].count);
   } else {
-    host[0] = lists[3].cpu();
-    host[1] = lists[7].cpu();
+    unlocked([&] {
+      host[0] = lists[3].cpu();
+      host[1] = lists[7].cpu();
+    });
   }
   for (int i = 0; i < 2; ++i) {
     const int64_t len = host[i].numel();

@@ -67,3 +67,31 @@ def test_a_replaced_update_is_what_the_attention_calls(how, monkeypatch):
     q, k, v = torch.randn(1, 4, 1, 16), torch.randn(1, 2, 1, 16), torch.randn(1, 2, 1, 16)
     out = fourier_attention(q, k, v, cache, 0, 4, 2)
     assert calls == [0] and torch.allclose(out.view(1, 2, 2, 16), v.transpose(1, 2).reshape(1, 2, 1, 16).expand(1, 2, 2, 16))
+
+
+@pytest.mark.gpu
+def test_other_threads_run_while_a_call_waits_for_the_gpu():
+    """The offsets of ``operands`` are waited for behind whatever the stream holds; another Python thread goes on meanwhile."""
+    import threading
+    import time
+    from fourierattention_amd import _lib
+    host = _lib.load_host()
+    lists = tuple(torch.tensor([0, 5, 9], device="cuda") for _ in range(8))
+    host.operands(lists, (), 32, 16)
+    ticks, stop = [0], threading.Event()
+
+    def tick():
+        while not stop.is_set():
+            ticks[0] += 1
+            time.sleep(0.001)
+    t = threading.Thread(target=tick)
+    t.start()
+    try:
+        torch.cuda._sleep(int(4e8))        # a few tenths of a second
+        before, t0 = ticks[0], time.perf_counter()
+        paging = host.operands(lists, (), 32, 16)[2]
+        waited, seen = time.perf_counter() - t0, ticks[0] - before
+    finally:
+        stop.set()
+        t.join()
+    assert paging[0] == [0, 5, 9] and waited > 0.05 and seen >= 10, (waited, seen)
