@@ -39,6 +39,21 @@ struct Ref {
   Ref(const Ref&) = delete;
 };
 
+// a sequence of any kind, held as a list or tuple
+struct Items : Ref {
+  Items(PyObject* o, const char* msg) : Ref(sequence(o, msg)) {}
+  Py_ssize_t size() const { return PySequence_Fast_GET_SIZE(p); }
+  PyObject* operator[](Py_ssize_t i) const { return PySequence_Fast_GET_ITEM(p, i); }
+  static PyObject* sequence(PyObject* o, const char* msg) {
+    PyObject* r = PySequence_Fast(o, msg);
+    if (!r) {   // (what is no sequence is refused like every other operand)
+      PyErr_Clear();
+      fail(PyExc_AssertionError, msg);
+    }
+    return r;
+  }
+};
+
 const at::Tensor& tensor(PyObject* o, const char* what) {
   if (!THPVariable_Check(o)) {
     PyErr_Format(PyExc_TypeError, "%s must be a tensor", what);
@@ -58,6 +73,11 @@ int64_t integer(PyObject* o) {
   const long long v = PyLong_AsLongLong(o);
   if (v == -1 && PyErr_Occurred()) throw PyError{};
   return v;
+}
+// what int() makes of it
+int64_t whole(PyObject* o) {
+  if (PyLong_CheckExact(o)) return integer(o);
+  return integer(Ref(PyNumber_Long(o)).p);
 }
 double real(PyObject* o) {
   const double v = PyFloat_AsDouble(o);
@@ -147,16 +167,16 @@ const at::Tensor& stream_args(PyObject* const* a, fa_stream_args& s, at::Tensor 
   s.k_new = k_new.data_ptr(); s.v_new = v_new.data_ptr();
   s.k_ring = k_ring.data_ptr(); s.v_ring = v_ring.data_ptr();
   s.ring_batch_stride = k_ring.stride(0); s.ring_row_stride = k_ring.stride(1);
-  s.evict_slot = (int32_t)integer(a[4]); s.write_slot = (int32_t)integer(a[5]);
+  s.evict_slot = (int32_t)whole(a[4]); s.write_slot = (int32_t)whole(a[5]);
   CHECK(s.evict_slot != s.write_slot && s.evict_slot < k_ring.size(1) && s.write_slot < k_ring.size(1), "window slots");
   s.k_coef = ptr<float>(k_coef); s.v_coef = ptr<float>(v_coef);
   s.kc_list = ptr<int32_t>(kc); s.vc_list = ptr<int32_t>(vc);
   s.Ck = (int32_t)kc.numel(); s.Cv = (int32_t)vc.numel();
-  s.N = (int32_t)(k_coef.size(1) / 2); s.phase = integer(a[10]); s.T = (int32_t)integer(a[11]);
+  s.N = (int32_t)(k_coef.size(1) / 2); s.phase = whole(a[10]); s.T = (int32_t)whole(a[11]);
   held[0] = tensor_attr(k_mid, s_data, "k_mid.data"); held[1] = tensor_attr(v_mid, s_data, "v_mid.data");
   s.k_mid = held[0].data_ptr(); s.v_mid = held[1].data_ptr();
   s.k_mid_batch_stride = int_attr(k_mid, s_batch_stride); s.v_mid_batch_stride = int_attr(v_mid, s_batch_stride);
-  s.cap_pages = (int32_t)int_attr(k_mid, s_cap_pages); s.mid_pos = integer(a[14]);
+  s.cap_pages = (int32_t)int_attr(k_mid, s_cap_pages); s.mid_pos = whole(a[14]);
   CHECK(s.cap_pages == int_attr(v_mid, s_cap_pages), "the page stores of K and V must have the same capacity");
   s.kn_list = ptr<int32_t>(tensor_attr(k_mid, s_n_list32, "n_list32")); s.vn_list = ptr<int32_t>(tensor_attr(v_mid, s_n_list32, "n_list32"));
   s.kn_h_list = ptr<int32_t>(tensor_attr(k_mid, s_n_h32, "n_h32")); s.vn_h_list = ptr<int32_t>(tensor_attr(v_mid, s_n_h32, "n_h32"));
@@ -189,8 +209,8 @@ void il_segment(fa_decode_args& d, int i, const at::Tensor& k, const at::Tensor&
   d.il_rows[i] = (int32_t)rows; d.il_batch_stride[i] = k.stride(0); d.il_row_stride[i] = k.stride(1);
 }
 
-const float* stat(PyObject* tuple, Py_ssize_t i) {
-  const at::Tensor& t = tensor(PyTuple_GET_ITEM(tuple, i), "statistics");
+const float* stat(const Items& stats, Py_ssize_t i) {
+  const at::Tensor& t = tensor(stats[i], "statistics");
   CHECK(t.scalar_type() == at::kFloat && t.is_contiguous(), "statistics must be contiguous float32");
   return ptr<const float>(t);
 }
@@ -200,7 +220,7 @@ const float* stat(PyObject* tuple, Py_ssize_t i) {
 // step: the arguments of stream_update as a tuple, or that in a list, which loses it when the update is launched; the update
 // comes in front of the attention
 // q (B, 1, Hq*D) or (B, Hq, 1, D), contiguous.  il: a sequence of up to two (k, v) pairs of row views, or (k, v, r): the
-// rows of one buffer in front of and behind row r.
+// rows of one buffer in front of and behind row r.  Sequences of any kind; whole numbers as int() takes them.
 PyObject* decode_attn(PyObject*, PyObject* const* a, Py_ssize_t n) {
   FA_BEGIN
   CHECK(n == 23 || n == 24, "decode_attn takes 23 or 24 arguments");
@@ -227,28 +247,29 @@ PyObject* decode_attn(PyObject*, PyObject* const* a, Py_ssize_t n) {
   CHECK(q.dim() == 3 || q.size(1) == d.Hq, "q has another number of heads");
   d.q = q.data_ptr();
   d.dtype = dtype_code(q);
-  if (PyTuple_Check(a[1]) && PyTuple_GET_SIZE(a[1]) == 3) {
-    const at::Tensor &k = tensor(PyTuple_GET_ITEM(a[1], 0), "k"), &v = tensor(PyTuple_GET_ITEM(a[1], 1), "v");
-    const int64_t cut = integer(PyTuple_GET_ITEM(a[1], 2));
+  const Items il(a[1], "il: (k, v) pairs");
+  if (il.size() == 3 && THPVariable_Check(il[0])) {
+    const at::Tensor &k = tensor(il[0], "k"), &v = tensor(il[1], "v");
+    const int64_t cut = integer(il[2]);
     CHECK(k.dim() == 3 && cut >= 0 && cut < k.size(1), "row to leave out");
     il_segment(d, 0, k, v, 0, cut, dt);
     il_segment(d, 1, k, v, cut + 1, k.size(1) - cut - 1, dt);
   } else {
-    Ref seq(PySequence_Fast(a[1], "il: (k, v) pairs"));
-    for (Py_ssize_t i = 0; i < 2 && i < PySequence_Fast_GET_SIZE(seq.p); ++i) {
-      PyObject* pair = PySequence_Fast_GET_ITEM(seq.p, i);
-      if (pair == Py_None) continue;
-      CHECK(PyTuple_Check(pair) && PyTuple_GET_SIZE(pair) == 2, "il: (k, v) pairs");
-      const at::Tensor& k = tensor(PyTuple_GET_ITEM(pair, 0), "k");
-      il_segment(d, (int)i, k, tensor(PyTuple_GET_ITEM(pair, 1), "v"), 0, k.dim() == 3 ? k.size(1) : 0, dt);
+    for (Py_ssize_t i = 0; i < 2 && i < il.size(); ++i) {
+      if (il[i] == Py_None) continue;
+      const Items pair(il[i], "il: (k, v) pairs");
+      CHECK(pair.size() == 2, "il: (k, v) pairs");
+      const at::Tensor& k = tensor(pair[0], "k");
+      il_segment(d, (int)i, k, tensor(pair[1], "v"), 0, k.dim() == 3 ? k.size(1) : 0, dt);
     }
   }
-  d.L_m = (int32_t)integer(a[11]); d.T = (int32_t)integer(a[12]);
-  CHECK(PyTuple_Check(a[8]) && PyTuple_GET_SIZE(a[8]) == 8, "lists: eight int32 tensors");
+  d.L_m = (int32_t)whole(a[11]); d.T = (int32_t)whole(a[12]);
+  const Items lists(a[8], "lists: eight int32 tensors");
+  CHECK(lists.size() == 8, "lists: eight int32 tensors");
   const int32_t* lp[8];
   int32_t ln[8];
   for (int i = 0; i < 8; ++i) {
-    const at::Tensor& t = tensor(PyTuple_GET_ITEM(a[8], i), "list");
+    const at::Tensor& t = tensor(lists[i], "list");
     CHECK(t.scalar_type() == at::kInt && t.is_contiguous(), "lists: contiguous int32 tensors");
     lp[i] = static_cast<const int32_t*>(t.data_ptr());
     ln[i] = (int32_t)t.numel();
@@ -296,22 +317,24 @@ PyObject* decode_attn(PyObject*, PyObject* const* a, Py_ssize_t n) {
         d.k_pad_h_host = kpad.data(); d.v_pad_h_host = vpad.data();
       }
     }
-    CHECK(PyTuple_Check(a[6]) && PyTuple_GET_SIZE(a[6]) == 3 && PyTuple_Check(a[7]) && PyTuple_GET_SIZE(a[7]) == 3, "statistics: (avg_u, avg_d, scale)");
-    d.avg_k_u = stat(a[6], 0); d.avg_k_d = stat(a[6], 1); d.scale_k = stat(a[6], 2);
-    d.avg_v_u = stat(a[7], 0); d.avg_v_d = stat(a[7], 1); d.scale_v = stat(a[7], 2);
+    const Items stats_k(a[6], "statistics: (avg_u, avg_d, scale)"), stats_v(a[7], "statistics: (avg_u, avg_d, scale)");
+    CHECK(stats_k.size() == 3 && stats_v.size() == 3, "statistics: (avg_u, avg_d, scale)");
+    d.avg_k_u = stat(stats_k, 0); d.avg_k_d = stat(stats_k, 1); d.scale_k = stat(stats_k, 2);
+    d.avg_v_u = stat(stats_v, 0); d.avg_v_d = stat(stats_v, 1); d.scale_v = stat(stats_v, 2);
     if (a[16] != Py_None) d.tables = tensor(a[16], "tables").data_ptr();
   }
   if (a[20] != Py_None) {
     CHECK(d.L_m > 0, "a layer without mid rows has no coefficients to update");
-    CHECK(PyTuple_Check(a[20]) && PyTuple_GET_SIZE(a[20]) == 4, "pending: (k_row, v_row, phase, T)");
-    const at::Tensor &uk = tensor(PyTuple_GET_ITEM(a[20], 0), "k_row"), &uv = tensor(PyTuple_GET_ITEM(a[20], 1), "v_row");
+    const Items pending(a[20], "pending: (k_row, v_row, phase, T)");
+    CHECK(pending.size() == 4, "pending: (k_row, v_row, phase, T)");
+    const at::Tensor &uk = tensor(pending[0], "k_row"), &uv = tensor(pending[1], "v_row");
     CHECK(uk.dim() == 2 && uk.stride(1) == 1 && uv.strides() == uk.strides() && uk.scalar_type() == dt && uv.scalar_type() == dt, "pending rows");
     d.upd_k_row = uk.data_ptr(); d.upd_v_row = uv.data_ptr(); d.upd_batch_stride = uk.stride(0);
-    d.upd_phase = integer(PyTuple_GET_ITEM(a[20], 2)); d.upd_T = (int32_t)integer(PyTuple_GET_ITEM(a[20], 3));
+    d.upd_phase = whole(pending[2]); d.upd_T = (int32_t)whole(pending[3]);
   }
   d.sm_scale = (float)real(a[13]);
   d.force_generic = truth(a[17]);
-  d.no_fuse = (int32_t)integer(a[19]);
+  d.no_fuse = (int32_t)whole(a[19]);
   at::Tensor out;
   if (a[14] != Py_None) {
     out = gpu_tensor(a[14], "out");
@@ -341,7 +364,8 @@ PyObject* decode_attn(PyObject*, PyObject* const* a, Py_ssize_t n) {
     LAUNCH(fa_decode_attn_timed(&d, st, ms));
     Ref list(PyList_New(4));
     for (int i = 0; i < 4; ++i) PyList_SET_ITEM(list.p, i, PyFloat_FromDouble(ms[i]));
-    if (PyList_SetSlice(a[22], 0, PyList_GET_SIZE(a[22]), list.p) < 0) throw PyError{};
+    Ref all(PySlice_New(nullptr, nullptr, nullptr));
+    if (PyObject_SetItem(a[22], all.p, list.p) < 0) throw PyError{};   // timings[:] = list
   } else if (step) {
     // (the library launches the update even where it refuses the attention)
     if (step_list && PyList_SetSlice(step_list, 0, 1, nullptr) < 0) throw PyError{};

@@ -133,10 +133,6 @@ class LlamaDecoderLayer(nn.Module):
         ops.linear_packed_step(x, w, residual=onto)
         return None
 
-    @staticmethod
-    def _normalises(w, h, norm):
-        return h.numel() <= _NORM_IN_PROJECTION and w.normalises(h, norm.weight)
-
     def fuse_projections(self, max_rows: int = 16384):
         """Moves the q/k/v weights into one tensor and the gate/up weights into another; the five modules keep
         views of them (same values, same state dict), ``forward_fused`` runs one GEMM per group.  A decode step
@@ -169,11 +165,12 @@ class LlamaDecoderLayer(nn.Module):
         stream, updated in place; ``delta`` the branch output not yet added to it (``None`` for the first layer).
         Returns this layer's MLP output, to be added by whoever normalises next (``None``: ``h`` has it already)."""
         at = self.self_attn
-        bsz, q_len, _ = h.shape
+        bsz, q_len, width = h.shape
+        norm_rides = bsz * q_len * width <= _NORM_IN_PROJECTION
         nq, nk = at.num_heads * at.head_dim, at.num_key_value_heads * at.head_dim
         pk = self._packed_weight("qkv")
         norm = self.input_layernorm
-        if pk is not None and delta is None and pk.covers(h) and self._normalises(pk, h, norm):
+        if norm_rides and delta is None and pk is not None and pk.covers(h) and pk.normalises(h, norm.weight):
             q, k, v = ops.linear_packed_step(h, pk, norm.weight, norm.variance_epsilon).split((nq, nk, nk), dim=-1)
         else:
             y = ops.add_rmsnorm(h, delta, norm.weight, norm.variance_epsilon)
@@ -194,7 +191,7 @@ class LlamaDecoderLayer(nn.Module):
         norm = self.post_attention_layernorm
         if pk is not None and pk.covers(h):
             gated = pk.n_out % 32 == 0      # whole tiles of gate rows, then whole tiles of up rows
-            if delta is None and gated and self._normalises(pk, h, norm):
+            if norm_rides and delta is None and gated and pk.normalises(h, norm.weight):
                 act = ops.linear_packed_step(h, pk, norm.weight, norm.variance_epsilon, gated=True)
             else:
                 y = ops.add_rmsnorm(h, delta, norm.weight, norm.variance_epsilon)

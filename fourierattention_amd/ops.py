@@ -217,8 +217,8 @@ def stream_update(k_new: torch.Tensor, v_new: torch.Tensor, k_ring: torch.Tensor
     may also come as the token itself, ``(B, heads, 1, D)`` with the heads side by side.
     ``skip_coef``: leave the coefficients alone; the caller owes them the update (``coeff_update_``, or the
     ``pending`` argument of the layer's next ``decode_attn_raw``) before that window slot is written again."""
-    _lib.load_host().stream_update(k_new, v_new, k_ring, v_ring, int(evict_slot), int(write_slot), k_coef, v_coef, kc_list, vc_list,
-                                   int(phase), int(T), k_mid, v_mid, int(mid_pos), skip_coef)
+    _lib.load_host().stream_update(k_new, v_new, k_ring, v_ring, evict_slot, write_slot, k_coef, v_coef, kc_list, vc_list,
+                                   phase, T, k_mid, v_mid, mid_pos, skip_coef)
 
 
 def append_rows(k: torch.Tensor, v: torch.Tensor, k_dst: torch.Tensor, v_dst: torch.Tensor, pos: int) -> None:
@@ -412,26 +412,14 @@ def decode_attn_raw(q, il_segments, k_mc, v_mc, k_mn, v_mn, stats_k, stats_v, li
     ``step``: the arguments of ``stream_update`` as a tuple: that update, then the attention over the state it leaves
     (which the other arguments describe), in one launch less where the shapes allow it.  In a list of their own they are
     taken out of it when the update is launched: what raises before leaves them there."""
-    # (the forms the host module reads; what the cache hands over has them already)
-    lists = lists if type(lists) is tuple else tuple(lists)
-    stats_k = stats_k if stats_k is None or type(stats_k) is tuple else tuple(stats_k)
-    stats_v = stats_v if stats_v is None or type(stats_v) is tuple else tuple(stats_v)
-    if not (type(il_segments) is tuple and len(il_segments) == 3 and isinstance(il_segments[0], torch.Tensor)):
-        il_segments = [p if p is None or type(p) is tuple else tuple(p) for p in il_segments[:2]]
-    if pending is not None:
-        pending = (pending[0], pending[1], int(pending[2]), int(pending[3]))
-    seq_len_m, ms = int(seq_len_m), None if timings is None else []
     if seq_len_m >= _REPACK_MIN_ROWS and not force_generic:
         _warn_if_off_the_matrix_cores(q.dtype, num_head_q, num_head_kv, q.numel() // (q.shape[0] * num_head_q),
                                       (k_mc if lists[0].numel() else v_mc).shape[1] // 2, not isinstance(k_mn, torch.Tensor))
     cast = out_dtype is not None and out_dtype != torch.float32
     assert not cast or out_dtype == q.dtype, "out_dtype must be float32 or the dtype of q"
-    out = _lib.load_host().decode_attn(q, il_segments, k_mc, v_mc, k_mn, v_mn, stats_k, stats_v, lists, num_head_q,
-                                       num_head_kv, seq_len_m, int(T), sm_scale, out, cast, tables, force_generic, balance_heads,
-                                       int(no_fuse), pending, no_alloc, ms, step)
-    if timings is not None:
-        timings[:] = ms
-    return out
+    return _lib.load_host().decode_attn(q, il_segments, k_mc, v_mc, k_mn, v_mn, stats_k, stats_v, lists, num_head_q,
+                                        num_head_kv, seq_len_m, T, sm_scale, out, cast, tables, force_generic, balance_heads,
+                                        no_fuse, pending, no_alloc, timings, step)
 
 
 _warned_shapes = set()
