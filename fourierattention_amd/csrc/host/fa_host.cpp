@@ -569,7 +569,7 @@ PyObject* operands(PyObject*, PyObject* const* a, Py_ssize_t n) {
     }
   }
   at::Tensor arena;
-  if (used > 0) {
+  if (n_items > 0) {   // (empty items are views of it too)
     arena = unlocked([&] { return at::empty({used}, at::TensorOptions().dtype(at::kInt).device(dev)); });
     for (int i = 0; i < n_items; ++i) items[i].dst = static_cast<int32_t*>(arena.data_ptr()) + at_item[i];
     const fa_stream_t st = stream_of(arena);

@@ -529,3 +529,17 @@ def test_argument_forms_of_the_decode_call():
     k1, k2 = k[:1].clone(), k[:1].clone()      # one sequence, tables with rows to spare
     a, b = ops.rope_qk(q[:1].clone(), k1, cos[:1], sin[:1], 128), ops.rope_qk(q[:1].clone(), k2, *(t.reshape(1, 6, 128) for t in (cos, sin)), 128)
     assert torch.equal(a, b) and torch.equal(k1, k2)
+
+
+def test_operands_when_only_empty_lists_need_a_conversion():
+    """Empty 64-bit lists beside 32-bit ones and single-precision statistics: nothing to convert, and nothing lost."""
+    from fourierattention_amd import _lib
+    i = lambda *v: torch.tensor(v, dtype=torch.int32, device="cuda")
+    none = torch.empty(0, dtype=torch.int64, device="cuda")
+    lists = (none, i(0, 0, 0), i(3, 4), i(0, 1, 2), none, i(0, 0, 0), i(7), i(0, 1, 1))
+    stats = (torch.ones((1, 0), device="cuda", dtype=torch.bfloat16),) + tuple(torch.ones((1, 2), device="cuda") for _ in range(5))
+    for units in ((0, 0), (32, 16)):
+        l32, s32, paging = _lib.load_host().operands(lists, stats, *units)
+        assert all(a.dtype == torch.int32 and a.tolist() == b.tolist() for a, b in zip(l32, lists))
+        assert all(a.dtype == torch.float32 and torch.equal(a, b.float()) for a, b in zip(s32, stats))
+        assert paging is None or (paging[0], paging[1], paging[2].tolist(), paging[3].tolist()) == ([0, 1, 2], [0, 1, 1], [0, 32, 64], [0, 16, 16])
