@@ -382,7 +382,7 @@ PyObject* add_rmsnorm(PyObject*, PyObject* const* a, Py_ssize_t n) {
   FA_BEGIN
   CHECK(n == 4, "add_rmsnorm takes 4 arguments");
   const at::Tensor &h = gpu_tensor(a[0], "h"), &w = tensor(a[2], "weight");
-  CHECK(h.is_contiguous() && w.is_contiguous() && w.scalar_type() == h.scalar_type() && h.dim() >= 1 && w.numel() == h.size(-1),
+  CHECK(h.is_contiguous() && w.is_contiguous() && w.scalar_type() == h.scalar_type() && h.dim() >= 1 && w.numel() == h.size(-1) && h.size(-1) > 0,
         "add_rmsnorm: h and weight contiguous, of one type, weight as long as a row");
   const void* delta = nullptr;
   if (a[1] != Py_None) {
@@ -421,7 +421,7 @@ PyObject* linear_packed(PyObject*, PyObject* const* a, Py_ssize_t n) {
   CHECK(n == 4 || n == 8, "linear_packed takes 4 or 8 arguments");
   const at::Tensor &x = gpu_tensor(a[0], "x"), &w = gpu_tensor(a[1], "weight");
   const int64_t k = integer(a[2]), n_out = integer(a[3]);
-  CHECK(x.scalar_type() == w.scalar_type() && x.dim() >= 1 && x.size(-1) == k && w.numel() == k * n_out, "linear_packed: x does not fit the weight");
+  CHECK(x.scalar_type() == w.scalar_type() && x.dim() >= 1 && k > 0 && x.size(-1) == k && w.numel() == k * n_out, "linear_packed: x does not fit the weight");
   const int rows = (int)(x.numel() / k), dtype = dtype_code(x);
   const int64_t stride = row_stride(x);
   const fa_stream_t st = stream_of(x);

@@ -95,3 +95,15 @@ def test_other_threads_run_while_a_call_waits_for_the_gpu():
         stop.set()
         t.join()
     assert paging[0] == [0, 5, 9] and waited > 0.05 and seen >= 10, (waited, seen)
+
+
+@pytest.mark.gpu
+def test_rows_without_elements_are_refused():
+    """A width of zero is an error on the host (it divides the number of elements there)."""
+    from fourierattention_amd import _lib, ops
+    e = lambda *s: torch.empty(s, device="cuda", dtype=torch.bfloat16)
+    with pytest.raises(AssertionError):
+        ops.add_rmsnorm(e(2, 0), None, e(0), 1e-5)
+    with pytest.raises(AssertionError):
+        _lib.load_host().linear_packed(e(2, 0), e(0), 0, 16)
+    assert ops.silu_mul(e(2, 0), e(2, 0)).shape == (2, 0) and ops.silu_mul(e(0, 8), e(0, 8)).shape == (0, 8)
