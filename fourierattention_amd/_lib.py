@@ -138,7 +138,7 @@ _SIGNATURES = {
 
 EXPORTED = tuple(_SIGNATURES)
 
-# bumped with every change of a prototype or of an argument struct (fa_abi_version in the library)
+# FA_ABI_VERSION of the header
 ABI_VERSION = 7
 
 _lib = None
@@ -185,6 +185,11 @@ def load_host():
         except ImportError as exc:
             raise ImportError(f"{PKG_DIR}/_fa_host.so is missing or does not load ({exc}); run "
                               "`python -m fourierattention_amd.build`") from exc
+        lib = load()
+        there = lib.fa_abi_version(), lib.fa_decode_args_size(), lib.fa_stream_args_size()
+        if _fa_host.layout() != there:
+            raise ImportError(f"{_fa_host.__file__} was built for ABI version and argument sizes {_fa_host.layout()}, the library "
+                              f"beside it has {there}: run `python -m fourierattention_amd.build`")
         from . import ops
         _fa_host.init(ops._raw_stream, check, ops.workspace)
         _host = _fa_host

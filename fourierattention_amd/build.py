@@ -246,6 +246,8 @@ def build(verbose: bool = True, extra_flags=()) -> str:
     srcs = sources()
     with ThreadPoolExecutor(max_workers=min(8, len(srcs))) as ex:
         objs = list(ex.map(lambda s: _compile(s, obj_dir, list(extra_flags)), srcs))
+    if os.path.exists(HOST_PATH):
+        os.remove(HOST_PATH)     # it belongs to the library it was linked with: never beside another one
     cmd = [HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", *objs, "-o", LIB_PATH]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:

@@ -622,6 +622,11 @@ PyObject* operands(PyObject*, PyObject* const* a, Py_ssize_t n) {
   FA_END
 }
 
+// layout() -> (ABI version, sizes of the argument structs) this module was compiled with
+PyObject* layout(PyObject*, PyObject* const*, Py_ssize_t) {
+  return Py_BuildValue("(inn)", FA_ABI_VERSION, (Py_ssize_t)sizeof(fa_decode_args), (Py_ssize_t)sizeof(fa_stream_args));
+}
+
 // init(stream_fn, check_fn, workspace_fn)
 PyObject* init(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (n != 3) {
@@ -638,7 +643,7 @@ PyObject* init(PyObject*, PyObject* const* a, Py_ssize_t n) {
 }
 
 #define FN(name) {#name, (PyCFunction)(void*)name, METH_FASTCALL, nullptr}
-PyMethodDef methods[] = {FN(init), FN(stream_update), FN(decode_attn), FN(add_rmsnorm), FN(linear_packed), FN(silu_mul), FN(rope_qk), FN(operands), FN(append_rows),
+PyMethodDef methods[] = {FN(init), FN(layout), FN(stream_update), FN(decode_attn), FN(add_rmsnorm), FN(linear_packed), FN(silu_mul), FN(rope_qk), FN(operands), FN(append_rows),
                          {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_fa_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 

@@ -41,6 +41,7 @@ enum fa_status {
 enum fa_dtype { FA_BF16 = 0, FA_FP16 = 1, FA_FP32 = 2 };
 
 const char* fa_last_error_string(void);
+#define FA_ABI_VERSION 7 /* of this header; bumped with every change of a prototype or of an argument struct */
 int fa_abi_version(void);
 
 /* ---------------------------------------------------------------------------

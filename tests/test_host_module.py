@@ -20,6 +20,22 @@ def test_cpu_tensors_and_wrong_types_are_refused():
         host.silu_mul(x)
 
 
+def test_a_library_of_another_layout_is_refused(monkeypatch):
+    """The module fills argument structs for the library beside it: another version or struct size is an import error."""
+    from types import SimpleNamespace
+    from fourierattention_amd import _lib
+    lib = _lib.load()
+    own = lib.fa_abi_version(), lib.fa_decode_args_size(), lib.fa_stream_args_size()
+    assert _lib.load_host().layout() == own
+    for i in range(3):
+        other = [v + (i == j) for j, v in enumerate(own)]
+        fake = SimpleNamespace(**{n: (lambda v=v: v) for n, v in zip(("fa_abi_version", "fa_decode_args_size", "fa_stream_args_size"), other)})
+        monkeypatch.setattr(_lib, "load", lambda: fake)
+        monkeypatch.setattr(_lib, "_host", None)
+        with pytest.raises(ImportError, match="was built for"):
+            _lib.load_host()
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("B,q_len", [(1, 1), (5, 1), (1, 7), (3, 4)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
