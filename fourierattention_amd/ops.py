@@ -113,32 +113,36 @@ def mat_fourier_triton(a: torch.Tensor, N: int, T: int, K_start: int = 0) -> tor
 def mat_avg_std(a: torch.Tensor, cols: Optional[torch.Tensor] = None, round_dtype: Optional[torch.dtype] = None):
     """fp32 ``(avg, max_dev)`` of the columns of ``a (B, K, width)``, each rounded through
     ``round_dtype`` when given."""
-    return _avg_std(a, cols, round_dtype).unbind(0)
-
-
-def _avg_std(a, cols, round_dtype) -> torch.Tensor:
-    """Both statistics as one ``(2, B, columns)`` tensor."""
     _require_gpu(a, "a")
     assert a.dim() == 3 and a.stride(2) == 1
     B, K, width = a.shape
     Mc = width if cols is None else cols.numel()
-    both = torch.empty((2, B, Mc), device=a.device, dtype=torch.float32)
-    avg, dev = both.unbind(0)
+    avg = torch.empty((B, Mc), device=a.device, dtype=torch.float32)
+    dev = torch.empty((B, Mc), device=a.device, dtype=torch.float32)
     if Mc == 0 or B == 0:
-        return both
+        return avg, dev
     lib = _lib.load()
     nbytes = lib.fa_stats_workspace_bytes(B, Mc, K)
     ws = workspace(a.device, nbytes)
     rd = FA_FP32 if round_dtype is None else dtype_code(round_dtype)
     check(lib.fa_mat_avg_std(a.data_ptr(), dtype_code(a.dtype), a.stride(0), a.stride(1), _ptr(cols), avg.data_ptr(),
                              dev.data_ptr(), B, K, Mc, rd, ws.data_ptr(), ws.numel(), _stream(a.device)))
-    return both
+    return avg, dev
 
 
 def mat_avg_std_triton(a: torch.Tensor):
     assert a.is_cuda and a.is_contiguous(), "Input tensor must be a contiguous CUDA tensor"  # TRI:438
     assert a.dim() == 3, "Input tensor must be 3-dimensional"
-    return _avg_std(a, None, a.dtype).to(a.dtype).unbind(0)  # TRI:461 (both in one launch)
+    return _cast_pair(mat_avg_std(a, round_dtype=a.dtype), a.dtype)  # TRI:461
+
+
+def _cast_pair(pair, dtype: torch.dtype):
+    """Both tensors in ``dtype``, each in memory of its own, in one launch."""
+    if dtype == torch.float32:
+        return pair
+    out = tuple(torch.empty_like(t, dtype=dtype) for t in pair)
+    torch._foreach_copy_(out, pair)
+    return out
 
 
 # --------------------------------------------------------------------------- K3
@@ -147,18 +151,13 @@ def mat_fourier_avg_std(c: torch.Tensor, K: int, T: int, round_dtype: Optional[t
     """Mean and maximum deviation, per column, of the signal reconstructed from ``c`` at positions 0..K-1.
     Long reconstructions run on the matrix cores (fp16 operands, fp32 accumulation) unless
     ``matrix_cores`` is false."""
-    return _fourier_avg_std(c, K, T, round_dtype, matrix_cores).unbind(0)
-
-
-def _fourier_avg_std(c, K, T, round_dtype, matrix_cores=True) -> torch.Tensor:
-    """Both statistics as one ``(2, B, columns)`` tensor."""
     _require_gpu(c, "c")
     assert c.is_contiguous() and c.dtype == torch.float32 and c.dim() == 3
     B, N2, Mc = c.shape
-    both = torch.empty((2, B, Mc), device=c.device, dtype=torch.float32)
-    avg, dev = both.unbind(0)
+    avg = torch.empty((B, Mc), device=c.device, dtype=torch.float32)
+    dev = torch.empty((B, Mc), device=c.device, dtype=torch.float32)
     if Mc == 0 or B == 0:
-        return both
+        return avg, dev
     lib = _lib.load()
     if matrix_cores:
         nbytes = lib.fa_mat_fourier_avg_std_workspace_bytes(B, N2 // 2, Mc, int(K))
@@ -168,12 +167,12 @@ def _fourier_avg_std(c, K, T, round_dtype, matrix_cores=True) -> torch.Tensor:
     rd = FA_FP32 if round_dtype is None else dtype_code(round_dtype)
     check(lib.fa_mat_fourier_avg_std(c.data_ptr(), avg.data_ptr(), dev.data_ptr(), B, N2 // 2, Mc, int(K), int(T), rd,
                                      ws.data_ptr(), int(nbytes), _stream(c.device)))
-    return both
+    return avg, dev
 
 
 def mat_fourier_avg_std_triton(c: torch.Tensor, K: int, T: int):
     assert c.is_contiguous(), "Matrix C must be contiguous"  # TRI:286
-    return _fourier_avg_std(c.float() if c.dtype != torch.float32 else c, K, T, torch.float16).to(torch.float16).unbind(0)  # TRI:326
+    return _cast_pair(mat_fourier_avg_std(c.float() if c.dtype != torch.float32 else c, K, T, torch.float16), torch.float16)  # TRI:326
 
 
 # ------------------------------------------------------------------ reconstruction

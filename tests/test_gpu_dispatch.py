@@ -543,3 +543,16 @@ def test_operands_when_only_empty_lists_need_a_conversion():
         assert all(a.dtype == torch.int32 and a.tolist() == b.tolist() for a, b in zip(l32, lists))
         assert all(a.dtype == torch.float32 and torch.equal(a, b.float()) for a, b in zip(s32, stats))
         assert paging is None or (paging[0], paging[1], paging[2].tolist(), paging[3].tolist()) == ([0, 1, 2], [0, 1, 1], [0, 32, 64], [0, 16, 16])
+
+
+@pytest.mark.parametrize("rows,C", [(1100, 33), (60, 1)])
+def test_statistics_are_tensors_of_their_own(rows, C):
+    """Mean and deviation share no storage (keeping or saving one keeps one) and start where an allocation does."""
+    from fourierattention_amd import ops
+    a = torch.randn((2, rows, C), device="cuda").bfloat16()
+    c = torch.randn((2, 64, C), device="cuda")
+    for pair in (ops.mat_avg_std(a), ops.mat_avg_std_triton(a), ops.mat_fourier_avg_std(c, rows, 2000), ops.mat_fourier_avg_std_triton(c, rows, 2000)):
+        avg, dev = pair
+        assert avg.untyped_storage().data_ptr() != dev.untyped_storage().data_ptr()
+        assert all(t.storage_offset() == 0 and t.is_contiguous() and t.data_ptr() % 256 == 0 and t.shape == (2, C) for t in pair)
+        assert all(t.untyped_storage().nbytes() < 2 * t.numel() * t.element_size() + 512 and t._base is None for t in pair)
