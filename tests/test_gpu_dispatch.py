@@ -226,6 +226,19 @@ def test_projections_with_the_steps_beside_them(dtype, rows, K, n_out):
     assert torch.equal(ops.linear_packed_step(x, pw, norm, 1e-5, residual=kept), h + got)
 
 
+def _launches(f):
+    """Kernel launches of a call: the nodes of a graph it is captured into (which is never run)."""
+    import ctypes
+    from fourierattention_amd import _lib
+    graph, n = torch.cuda.CUDAGraph(keep_graph=True), ctypes.c_size_t()
+    with torch.cuda.graph(graph):
+        f()
+    get_nodes = _lib.load().hipGraphGetNodes      # (of the runtime the library runs on)
+    get_nodes.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.POINTER(ctypes.c_size_t)]
+    assert get_nodes(graph.raw_cuda_graph(), None, ctypes.byref(n)) == 0
+    return n.value
+
+
 @pytest.mark.parametrize("dtype,B,Hq,Hkv,D,states,init,W,counts,wide", [
     (torch.bfloat16, 1, 8, 2, 128, 256, 4, 100, [64, 64], False),     # matrix cores, merge in the launch, sub-splits
     (torch.bfloat16, 3, 12, 4, 128, 256, 4, 61, [128, 0, 77, 1], True),   # a head without compressed K, tokens as slices of wider rows
@@ -261,6 +274,12 @@ def test_update_in_the_attention_launch(dtype, B, Hq, Hkv, D, states, init, W, c
     for a, b in zip((one.key_cache[0], one.value_cache[0]), (two.key_cache[0], two.value_cache[0])):
         assert all(torch.equal(a[n], b[n]) for n in a)
     assert one.get_seq_length() == two.get_seq_length() == S + W + 5
+    # one launch less than the two calls, except with head dims that have no vectorised window kernel
+    def both():
+        two.update(k, v, 0)
+        two.decode_attention(q, 0, Hq, Hkv, out_dtype=dtype)
+    joined = _launches(lambda: fourier_attention(q, k, v, one, 0, Hq, Hkv))
+    assert joined == _launches(both) - (D != 80)
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
