@@ -681,16 +681,22 @@ def main():
     torch.cuda.synchronize()
     upd_wall = (time.perf_counter() - t0) / 30
     upd_bytes = w["B"] * 2 * w["M"] * (ck + cv) * 4
-    # a decode step in use: the streaming update, then the attention over the updated cache
-    # (--update-inside-attention: the attention applies the rank-1 update of the coefficients while it streams them)
+    # a decode step in use: the attention forward's call of one new token, the streaming update in the attention's first launch
+    # (--update-inside-attention: update and attention as two calls, the second of which applies the rank-1 update of the
+    # coefficients while it streams them)
     cache.defer_coef_update = bool(args.update_inside_attention)
+    if args.update_inside_attention:
+        def step():
+            cache.update(kn, vn, 0)
+            cache.decode_attention(q, 0, Hq, Hkv)
+    else:
+        from fourierattention_amd.attention import fourier_attention
+        step = lambda: fourier_attention(q, kn, vn, cache, 0, Hq, Hkv)
     for _ in range(3):
-        cache.update(kn, vn, 0)
-        cache.decode_attention(q, 0, Hq, Hkv)
+        step()
     start.record()
     for _ in range(50):
-        cache.update(kn, vn, 0)
-        cache.decode_attention(q, 0, Hq, Hkv)
+        step()
     stop.record()
     torch.cuda.synchronize()
     both_ms = start.elapsed_time(stop) / 50

@@ -379,7 +379,7 @@ __device__ __forceinline__ float dot8(const Row8<E>& a, const Row8<E>& b) {
 // workgroup - in the scores lane = token and each wave sums its quarter of the frequencies and of the stored dims, in
 // g = F^T p thread = (frequency, share of the tokens) - so that a short context still gives every compute unit a tile.
 // (One thread per token over all frequencies on tiles of 256 tokens took 137 us for 1532 mid rows of 24 / 8 heads and
-// 128 frequencies in fp32, 48 workgroups; this split KMID_US us.)  Weights and probabilities lie in LDS head by head, so a
+// 128 frequencies in fp32, 48 workgroups; this split 12.8 us.)  Weights and probabilities lie in LDS head by head, so a
 // thread fetches those of all heads with one broadcast read.
 constexpr int kMidTile = 64;   // tokens per tile
 

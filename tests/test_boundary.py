@@ -76,7 +76,7 @@ def test_attention_forward_computes_rotary_tables_from_position_ids():
 
 def test_shapes_off_the_matrix_cores_are_announced_once():
     """Long contexts whose shape only the any-shape vector kernels take (e.g. float32 storage, 384 frequencies) are
-    about 50x slower: the operator says so, once per shape."""
+    several times slower: the operator says so, once per shape."""
     import warnings
     import torch
     from fourierattention_amd import ops
