@@ -2507,7 +2507,7 @@ extern "C" int fa_decode_attn(const fa_decode_args* a, fa_stream_t stream) { ret
 
 // Whether the update `s` can ride in the first launch of the attention `a`: that launch exists (vectorised sink/window rows
 // in front of mid rows), the attention reads the state the update leaves (the sink/window rows are one buffer around the
-// evicted slot, the new token's slot among them), and the token can be read like a row of the window.
+// evicted slot, the new token's slot among them), the token can be read like a row of the window, and it is the quicker way.
 static bool step_joins(const fa_stream_args* s, const fa_decode_args* a, JoinedStep& j) {
   if (!s || !a || s->skip_coef || a->upd_k_row || a->upd_v_row || a->L_m <= 0 || a->B != s->B || a->Hkv != s->Hkv ||
       a->dtype != s->dtype || a->N != s->N || a->D <= 0 || s->width != a->Hkv * a->D || a->q_len != 1)
@@ -2527,6 +2527,15 @@ static bool step_joins(const fa_stream_args* s, const fa_decode_args* a, JoinedS
   const int64_t fresh = at / rs + s->write_slot, evicted = at / rs + s->evict_slot;
   if (evicted != gap || fresh == gap || fresh - (fresh > gap) >= gap + a->il_rows[1]) return false;
   if ((((uintptr_t)s->k_new | (uintptr_t)s->v_new | (uintptr_t)(s->new_batch_stride * es)) & 15) != 0 || !s->k_new || !s->v_new) return false;
+  // Every head's blocks write its own columns of the K coefficients back.  Where heads begin and end inside a line (counts of
+  // compressed dims that differ or are no multiple of 16), two of them write parts of one, and with many coefficients of few
+  // sequences that costs more than the launch: joined / apart, us a layer at 12k tokens, 921 of 1024 dims, 512 frequencies, one
+  // sequence 44.9 / 42.8, four 64.1 / 63.2, eight 89.2 / 90.0; 256 frequencies, one 37.2 / 38.1; 64 dims of every head, 512
+  // frequencies, one 42.3 / 42.2, eight 77.5 / 82.5.  Heads of 64 dims and single precision gain throughout.
+  bool whole_lines = a->Ck % (16 * a->Hkv) == 0;
+  if (a->k_pad_h_host)   // (stored dims, padded: uneven ones show here)
+    for (int h = 0; h < a->Hkv; ++h) whole_lines = whole_lines && a->k_pad_h_host[h + 1] - a->k_pad_h_host[h] == a->k_pad_h_host[1];
+  if (!whole_lines && a->dtype != FA_FP32 && a->D > 64 && a->N >= 512 && a->B < 8) return false;
   if (fa_stream::stream_params(s, true, j.sp) != FA_OK) return false;
   j.k_new = s->k_new; j.v_new = s->v_new; j.new_bs = s->new_batch_stride;
   j.fresh = (int)(fresh - (fresh > gap));
