@@ -372,9 +372,9 @@ int fa_decode_split_plan(int B, int Hq, int Hkv, int D, int N, int il_rows_total
  * `args->workspace_bytes` are ignored; the partial results live in a buffer of FA_DECODE_NOALLOC_SCRATCH_BYTES
  * that is part of the library image on every GPU it runs on (held until the process ends).  Nothing is allocated
  * or freed, by this call or by anything it calls.  k_pad_h_host / v_pad_h_host are ignored as well: every KV head
- * gets the same number of splits, and shapes whose partial results then exceed that size (at most what
- * fa_decode_attn_workspace_bytes(...) reports, which leaves room for uneven shares) are refused with
- * FA_ERR_WORKSPACE.  Every call on one GPU shares that GPU's buffer: calls that may
+ * gets the same number of splits, and shapes whose partial results then exceed that size (on either path, the any-shape
+ * kernels with a split per 256 mid rows or more; at most what fa_decode_attn_workspace_bytes(...) reports, which leaves room for
+ * uneven shares and more splits) are refused with FA_ERR_WORKSPACE.  Every call on one GPU shares that GPU's buffer: calls that may
  * overlap on one GPU (two streams, two threads) race and must be serialised by the caller; consecutive calls on
  * one stream are fine (every kernel writes what it later reads, nothing needs clearing).  The first call on a
  * device looks the buffer's address up (hipGetSymbolAddress): make it outside any stream capture.  This entry
@@ -389,14 +389,16 @@ int fa_decode_attn_noalloc(const fa_decode_args* args, fa_stream_t stream);
  * measurement aid (the reference has no counterpart). */
 int fa_decode_attn_last_fused(void);
 
+/* fa_stream_update(s) followed by fa_decode_attn(a), whose arguments describe the state the update leaves: the same results,
+ * in one launch less where the update can ride in the attention's first launch (16- or 32-bit rows with vectorised
+ * sink/window kernels, the window as one buffer around the evicted slot, a 16-byte aligned token) and that is the quicker
+ * way.  An attention that is refused leaves the update done. */
+int fa_decode_step(const fa_stream_args* s, const fa_decode_args* a, fa_stream_t stream);
+
 /* Same call, bracketed by HIP events on `stream`; synchronises and returns in ms_out[0..3] the
  * milliseconds spent in (0) the coefficient-domain query kernel (plus the operand tables when
  * they are built in the workspace), (1) the mid-row kernel, (2) the sink/window kernel and
  * (3) the merge kernel.  A measurement aid for benchmarks (the reference has no timers). */
-/* fa_stream_update(s) followed by fa_decode_attn(a), whose arguments describe the state the update leaves: the same results,
- * in one launch less where the update can ride in the attention's first launch (16- or 32-bit rows with vectorised
- * sink/window kernels, the window as one buffer around the evicted slot, a 16-byte aligned token). */
-int fa_decode_step(const fa_stream_args* s, const fa_decode_args* a, fa_stream_t stream);
 int fa_decode_attn_timed(const fa_decode_args* args, fa_stream_t stream, float* ms_out);
 
 /* ---------------------------------------------------------------------------
