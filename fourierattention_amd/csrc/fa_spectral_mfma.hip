@@ -48,24 +48,19 @@ __global__ __launch_bounds__(256) void spectral_table_kernel(half2v* __restrict_
 }
 
 // ---- pack: block = 32 tokens x 256 columns; lanes run along the columns for the gather, the transposition to
-// token-contiguous fragments goes through LDS.  grid (ksteps, column blocks, parts * B): part p of the input starts
-// p * a_part elements behind the first and its fragments p * out_part behind the first's ------------------------
+// token-contiguous fragments goes through LDS.  grid (ksteps, column blocks, B) ------------------------------------------
 template <typename E>
 __global__ __launch_bounds__(256) void spectral_pack_kernel(
     const E* __restrict__ a, int64_t a_bs, int64_t a_rs, const int32_t* __restrict__ cols,
-    const float* __restrict__ col_inv_scale, half8* __restrict__ out, int K, int Mc, int CT, int KS32, int B, int64_t a_part,
-    int64_t out_part) {
+    half8* __restrict__ out, int K, int Mc, int CT, int KS32) {
   constexpr int kPitch = 256 + 4;   // f16 elements per LDS row: 8 rows apart = 16 banks apart
   __shared__ _Float16 tile[32][kPitch];
   const int tid = threadIdx.x;
-  const int ks = blockIdx.x, m0 = blockIdx.y * 256, part = blockIdx.z / B, b = blockIdx.z - part * B;
-  a += part * a_part;
-  out += part * out_part;
+  const int ks = blockIdx.x, m0 = blockIdx.y * 256, b = blockIdx.z;
   const int m = m0 + tid;
   const bool mok = m < Mc;
   const int col = mok ? (cols ? cols[m] : m) : 0;
   const E* ab = a + (int64_t)b * a_bs + col;
-  const float mul = (col_inv_scale && mok) ? col_inv_scale[(int64_t)b * Mc + m] : 1.f;
   float v[32];
 #pragma unroll
   for (int kk = 0; kk < 32; ++kk) {
@@ -76,7 +71,7 @@ __global__ __launch_bounds__(256) void spectral_pack_kernel(
   for (int kk = 0; kk < 32; ++kk) {
     const int k = ks * 32 + kk;
     // f16 holds every bf16 / f16 value of magnitude below 65504 exactly (tiny ones as subnormals)
-    const float x = (mok && k < K) ? fminf(fmaxf(v[kk] * mul, -65504.f), 65504.f) : 0.f;
+    const float x = (mok && k < K) ? fminf(fmaxf(v[kk], -65504.f), 65504.f) : 0.f;
     tile[kk][tid] = (_Float16)x;
   }
   __syncthreads();
@@ -219,8 +214,7 @@ __global__ __launch_bounds__(256) void prefill_pack_kernel(const PrefillPackPara
 // ((j, ks) at lds + (4 j + ks) KiB) are requested one kstep ahead of the products that take them, the first ones in
 // front of the rotation, which has 128 vector instructions to cover them: a wave that read and then waited spent longer
 // on LDS latency than on its matrix instructions.  No branch between a request and its wait (accumulators start as
-// zeros, which rotate to zeros).  32768 rows x 512 columns, 512 frequencies: 37.8 -> 34.8 us (990 TFLOP/s), reconstruction
-// statistics of the same size 56 -> 48 us together with the scales kept in LDS.
+// zeros, which rotate to zeros).  32768 rows x 512 columns, 512 frequencies: 37.8 -> 34.8 us (990 TFLOP/s).
 __device__ __forceinline__ void spectral_step(float4v (&acc)[4][4], const half8 (&Ea)[4][kStepK], const float (&rc)[4][2],
                                               const float (&rs)[4][2], unsigned lds) {
   uint4v b0[4], b1[4];
@@ -369,200 +363,363 @@ __global__ __launch_bounds__(256) void spectral_reduce_kernel(const float* __res
 }
 
 // ---------------------------------------------------------------------------------------------------------
-// Statistics of the reconstruction (mat_fourier_avg_std_triton, TRI:285-326) on the same machinery.
-//   r[k, m] = (1/N) sum_n cos(theta k n) c[n, m] + sin(theta k n) c[N + n, m] = (1/N) Re sum_n e^{i theta k n} (c - i s)
-// is the compression GEMM with the roles of position and frequency exchanged: the rows are the positions k,
-// the "tokens" are the N coefficient indices.  A workgroup owns 128 positions, keeps their basis rows in
-// registers, and walks over its blocks of 64 columns: one pass over the cos coefficients (keeps the real part A_k),
-// one over the sin coefficients (keeps the imaginary part B_k), then folds its positions into sum / max / min.
-// Position k gives r[k] = A_k + B_k and, because the period is a whole number of positions, also its mirror image
-// r[T - k] = A_k - B_k: only the positions up to T / 2 are computed, each standing for two where the sequence
-// reaches past T / 2.
-// The column blocks are dealt to the workgroups of a row block so that the launch fills the device (recon_col_share):
-// the matrix cores bound it, and with one workgroup per 128 positions four sequences of 1977 positions kept 64 of 256
-// compute units busy.
-// The coefficients travel as f16 scaled by a power of two per column (their range is not bounded).
+// Statistics of the reconstruction (mat_fourier_avg_std_triton, TRI:285-326):
+//   r[k, m] = (1/N) sum_n cos(theta k n) c[n, m] + sin(theta k n) s[n, m],     s[n] = c[N + n]
+// The roles of position and frequency are those of the compression exchanged: rows are the positions k, and the
+// contraction runs over the coefficient index n, cut into steps of 128.  A step is taken from its centre
+// n_c = 128 t + 63.5: with the coefficients folded, c+ = c[n_c + j] + c[n_c - j] and c- = c[n_c + j] - c[n_c - j] for the 64
+// offsets j = 1/2, 3/2 ..,
+//   sum over the step of cos(theta k n) c[n] = cos(phi) . (E_cos c+) - sin(phi) . (E_sin c-)
+//   sum over the step of sin(theta k n) s[n] = sin(phi) . (E_cos s+) + cos(phi) . (E_sin s-),      phi = theta k n_c
+// so that the matrix cores compute real sums only, half of what two complex ones (basis rows cos and sin for every
+// coefficient, one accumulator of the two used) take, and a step ends in two multiply-adds per sum instead of a complex
+// rotation.  The fold happens in 32 bits ahead of the rounding to f16, scaled by a power of two per column (the range of
+// coefficients is not bounded).  The coefficient of frequency 0 stays out of the products: its basis is one, and the mean of
+// the signal, often its largest part, is added in 32 bits behind them (as c[0] it would meet the rounded basis of offset
+// 63.5).
+// Position k gives r[k] = A_k + B_k (A cosine, B sine part) and, because the period is a whole number of positions, also
+// its mirror image r[T - k] = A_k - B_k: only the positions up to T / 2 are computed, each standing for two where the
+// sequence reaches past T / 2.
+// Bound by the matrix cores and the LDS reads that feed them (a fragment feeds four products).  32768 positions x 512 columns,
+// 512 frequencies, all launches: 72.9 us with complex sums on coefficients packed by launches of their own -> 43.9; eight tensors
+// of 31740 positions 294 -> 165, four of 1977 x 910 56 -> 37.  Against 64 bits the mean is off by 4e-7 .. 4e-5 (1e-4 .. 2e-4
+// before, the rounding of the coefficient of frequency 0), the deviation by as much as before (7e-5).
 // ---------------------------------------------------------------------------------------------------------
-__global__ __launch_bounds__(1024) void coef_colscale_kernel(const float* __restrict__ c, float* __restrict__ scale,
-                                                             float* __restrict__ inv_scale, int N2, int Mc) {
-  // 16 columns x 64 row classes: 64 bytes of a row per access, and four times the blocks of whole waves of columns
+constexpr int kRecPos = 256;      // positions of a workgroup: four waves x four tiles of 16
+constexpr int kRecCols = 32;      // columns of a unit of work: two tiles of 16
+constexpr int kRecStep = 128;     // coefficient indices of a step
+constexpr int kRecFrags = 8;      // fragments of a step and column tile: {c+, c-, s+, s-} x two ksteps of 32 offsets
+constexpr int kMaxColShare = 8;   // units of a workgroup at most
+
+struct ReconPrepParams {
+  const float* c;     // [B][2N][Mc]
+  half8* packed;      // [B][CT][n_steps][kRecFrags][64]
+  float* scale;       // [B][Mc]
+  half2v* tab;        // [position tiles][cos k0, cos k1, sin k0, sin k1][64] x half8
+  float* phi;         // [row blocks][n_steps][cos, sin][kRecPos]
+  int B, N, Mc, CT, T, n_steps;
+};
+
+// Everything the statistics need, in one launch of 1024 threads a block: the first CT * B blocks fold and pack a column tile
+// each (thread = column, offset), the rest evaluate the basis of 32 positions and their phases at the steps.
+__global__ __launch_bounds__(1024) void recon_prep_kernel(const ReconPrepParams p) {
+  constexpr int kHold = 8;   // steps whose coefficients a thread holds between the maximum and the scaling
+  constexpr int kOut = 4;    // steps that leave through LDS at a time
   __shared__ float s_mx[64][16];
-  const int lane = threadIdx.x & 15, g = threadIdx.x >> 4;
-  const int m = blockIdx.x * 16 + lane, b = blockIdx.y;
-  float mx = 0.f;
-  if (m < Mc) {
-    const float* cp = c + (int64_t)b * N2 * Mc + m;
-    for (int n0 = g; n0 < N2; n0 += 64 * 8) {
-      float v[8];
+  __shared__ __attribute__((aligned(16))) _Float16 s_out[kOut * kRecFrags * 512];
+  const int tid = threadIdx.x;
+  int blk = blockIdx.x;
+  if (blk >= p.CT * p.B) {
+    blk -= p.CT * p.B;   // 32 positions: two tiles, thread = (tile, kstep, lane group, position, pair of offsets)
+    const int ep = tid & 3, lc = (tid >> 2) & 15, lg = (tid >> 6) & 3, kk = (tid >> 8) & 1, tile = blk * 2 + (tid >> 9);
+    half2v co2, sn2;
+    float own = 0.f;
 #pragma unroll
-      for (int u = 0; u < 8; ++u) v[u] = cp[(int64_t)min(n0 + 64 * u, N2 - 1) * Mc];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) mx = fmaxf(mx, fabsf(v[u]));
+    for (int e = 0; e < 2; ++e) {
+      float sn, co;
+      fa_sincos_phase(tile * 16 + lc, 2 * (32 * kk + 8 * lg + 2 * ep + e) + 1, 2 * p.T, &sn, &co);
+      co2[e] = (_Float16)co;
+      sn2[e] = (_Float16)sn;
+      own = fmaf((float)co2[e], co, fmaf((float)sn2[e], sn, own));
     }
-  }
-  s_mx[g][lane] = mx;
-  __syncthreads();
-  if (g == 0 && m < Mc) {
+    half2v* out = p.tab + ((int64_t)(tile * 4 + kk) * 64 + lg * 16 + lc) * 4 + ep;
+    out[0] = co2;
+    out[2 * 64 * 4] = sn2;
+    // A rounded basis answers its own position with a sum of squares that is not quite 64: the phases carry the
+    // reciprocal, so that what is coherent with the position - the signal at its extremes - comes out unscaled.
+    float* s_own = &s_mx[0][0];   // [32 positions][32]
+    s_own[((tid >> 9) * 16 + lc) * 32 + (kk * 4 + lg) * 4 + ep] = own;
+    __syncthreads();
+    const int pos = tid & 31;
+    float sum = 0.f;
 #pragma unroll
-    for (int i = 1; i < 64; ++i) mx = fmaxf(mx, s_mx[i][lane]);
-    const float sc = mx > 0.f ? exp2f(ceilf(log2f(mx))) : 1.f;   // power of two: scaling is exact
-    scale[(int64_t)b * Mc + m] = sc;
-    inv_scale[(int64_t)b * Mc + m] = 1.0f / sc;
+    for (int k = 0; k < 32; ++k) sum += s_own[pos * 32 + ((k + pos) & 31)];   // (rotated: no two lanes on one bank)
+    const float unit = 64.0f / sum;
+    const int k = blk * 32 + pos, rb = k / kRecPos;
+    for (int t = tid >> 5; t < p.n_steps; t += 32) {
+      float sn, co;
+      fa_sincos_phase(k, 2 * kRecStep * t + kRecStep - 1, 2 * p.T, &sn, &co);
+      float* o = p.phi + ((int64_t)(rb * p.n_steps + t) * 2) * kRecPos + k % kRecPos;
+      o[0] = co * unit;
+      o[kRecPos] = sn * unit;
+    }
+    return;
+  }
+  const int ct = blk % p.CT, b = blk / p.CT;
+  const int lc = tid & 15, i = tid >> 4, m = ct * 16 + lc;
+  const float* cb = p.c + (int64_t)b * 2 * p.N * p.Mc + min(m, p.Mc - 1);
+  float v[kHold][4];   // cos rows above and below the centre, sin rows likewise
+  auto load = [&](int t0) {
+#pragma unroll
+    for (int u = 0; u < kHold; ++u)
+      if (t0 + u < p.n_steps) {
+        const int hi = (t0 + u) * kRecStep + 64 + i, lo = (t0 + u) * kRecStep + 63 - i;
+        v[u][0] = cb[(int64_t)min(hi, p.N - 1) * p.Mc];
+        v[u][1] = cb[(int64_t)min(lo, p.N - 1) * p.Mc];
+        v[u][2] = cb[(int64_t)(p.N + min(hi, p.N - 1)) * p.Mc];
+        v[u][3] = cb[(int64_t)(p.N + min(lo, p.N - 1)) * p.Mc];
+        if (lo == 0) v[u][1] = v[u][3] = 0.f;   // (frequency 0: added behind the products)
+      }
+  };
+  float mx = 0.f;
+  for (int t0 = 0; t0 < p.n_steps; t0 += kHold) {
+    load(t0);
+#pragma unroll
+    for (int u = 0; u < kHold; ++u)
+      if (t0 + u < p.n_steps)
+        mx = fmaxf(mx, fmaxf(fmaxf(fabsf(v[u][0]), fabsf(v[u][1])), fmaxf(fabsf(v[u][2]), fabsf(v[u][3]))));
+  }
+  s_mx[i][lc] = mx;
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < 64; ++k) mx = fmaxf(mx, s_mx[k][lc]);
+  // power of two: scaling is exact.  (Columns of nothing but tiny values are not scaled into the denormals' reciprocal.)
+  const float sc = mx > 0.f ? exp2f(fmaxf(ceilf(log2f(mx)), -100.f)) : 1.f, inv = 1.0f / sc;
+  if (i == 0 && m < p.Mc) p.scale[(int64_t)b * p.Mc + m] = sc;
+  half8* out = p.packed + ((int64_t)(b * p.CT + ct) * p.n_steps) * kRecFrags * 64;
+  const int at = ((i >> 5) * 64 + ((i >> 3) & 3) * 16 + lc) * 8 + (i & 7);   // of offset i in a pair of fragments
+  for (int t0 = 0; t0 < p.n_steps; t0 += kHold) {
+    if (p.n_steps > kHold) load(t0);
+#pragma unroll
+    for (int u0 = 0; u0 < kHold; u0 += kOut) {
+      if (t0 + u0 >= p.n_steps) break;
+#pragma unroll
+      for (int u = 0; u < kOut; ++u)
+        if (t0 + u0 + u < p.n_steps) {
+          const int hi = (t0 + u0 + u) * kRecStep + 64 + i, lo = (t0 + u0 + u) * kRecStep + 63 - i;
+          const bool ok_h = m < p.Mc && hi < p.N, ok_l = m < p.Mc && lo < p.N;
+          const float ch = ok_h ? v[u0 + u][0] * inv : 0.f, cl = ok_l ? v[u0 + u][1] * inv : 0.f;
+          const float sh = ok_h ? v[u0 + u][2] * inv : 0.f, sl = ok_l ? v[u0 + u][3] * inv : 0.f;
+          _Float16* o = s_out + u * kRecFrags * 512 + at;
+          o[0 * 1024] = (_Float16)(ch + cl);
+          o[1 * 1024] = (_Float16)(ch - cl);
+          o[2 * 1024] = (_Float16)(sh + sl);
+          o[3 * 1024] = (_Float16)(sh - sl);
+        }
+      __syncthreads();
+      const int n = min(kOut, p.n_steps - t0 - u0) * kRecFrags * 64;
+      for (int k = tid; k < n; k += 1024) out[(int64_t)(t0 + u0) * kRecFrags * 64 + k] = ((const half8*)s_out)[k];
+      __syncthreads();
+    }
   }
 }
 
-constexpr int kMaxColShare = 16;   // column blocks of a workgroup at most
-
 struct ReconStatsParams {
-  const half8* tab;        // basis rows of the positions: [ceil(K/8)][kStepK][64]
-  const half8* packed[2];  // cos / sin coefficients, [B][CT][KS32][64] fragments
-  const float* scale;      // [B][Mc]
+  const float* c;
+  const half8* tab;
+  const half8* packed;
+  const float* phi;
+  const float* scale;
   float* psum;
   float* pmax;
-  float* pmin;             // [B][RB][Mc]
-  int B, N, Mc, CT, KS32, K, T, n_steps, RB;
-  int cb_per; // column blocks of a workgroup
-  int Kd;     // positions computed directly: min(K, T / 2 + 1)
-  int half;   // T / 2: mirror images beyond it count as positions of their own (a value no position exceeds
-              // when the sequence is longer than the period and every position is computed directly)
+  float* pmin;   // [B][RB][Mc]
+  int B, N, Mc, CT, K, T, n_steps, RB;
+  int cb_per;    // units (column blocks) of a workgroup
+  int Kd;        // positions computed directly: min(K, T / 2 + 1)
+  int half;      // T / 2: mirror images beyond it count as positions of their own (a value no position exceeds
+                 // when the sequence is longer than the period and every position is computed directly)
 };
 
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void spectral_recon_stats_kernel(
     const ReconStatsParams p) {
-  constexpr int NST = 4;
-  __shared__ __attribute__((aligned(16))) unsigned char s_stage[NST][4][kStepK][1024];
-  __shared__ float s_red[3][4][kWgCols];
-  __shared__ float s_scale[kMaxColShare * kWgCols];   // scale / N of this workgroup's columns
+  constexpr int NST = 3;                                // steps in LDS: the one in use and two on their way
+  constexpr int kStage = 2 * kRecFrags * 1024 + 2048;   // the fragments of two column tiles, the phases of the positions
+  __shared__ __attribute__((aligned(16))) unsigned char s_stage[NST][kStage];
+  __shared__ float s_stat[3][4][kMaxColShare * kRecCols];   // sum / max / min, by wave and column
   const int tid = threadIdx.x, lane = tid & 63, lg = lane >> 4, lc = lane & 15;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int rb = blockIdx.x, b = blockIdx.y;
-  const int rt0 = (rb * 4 + w) * 4;
-  const int n_rt = (p.Kd + 7) / 8;
   const int S = p.n_steps;
   const int cb0 = blockIdx.z * p.cb_per;
-  const int n_cb = min((p.Mc + kWgCols - 1) / kWgCols - cb0, p.cb_per);
-  const int Q = n_cb * 2 * S;   // steps of this workgroup: column block, pass (cos, sin), step (last to first)
+  const int n_cb = min((p.Mc + kRecCols - 1) / kRecCols - cb0, p.cb_per);
+  const int Q = n_cb * S;
 
-  int next_cb = cb0, next_pass = 0, next_s = S - 1;   // the step requested next (walked, not divided out of a step number)
+  int next_cb = cb0, next_s = 0;   // the step requested next
   auto issue = [&](int stage) {
-    const int ct = min(next_cb * 4 + w, p.CT - 1);
-    const half8* frags = next_pass ? p.packed[1] : p.packed[0];
-    const _Float16* src = (const _Float16*)(frags + (((int64_t)b * p.CT + ct) * p.KS32) * 64) + lane * 8;
+    // wave w: four fragments of column tile w / 2 (clamped: a tile past the end repeats the last one); the first two
+    // waves bring the phases as well
+    const int ct = min(next_cb * 2 + (w >> 1), p.CT - 1);
+    const half8* src = p.packed + (((int64_t)(b * p.CT + ct) * S + next_s) * kRecFrags + (w & 1) * 4) * 64 + lane;
 #pragma unroll
-    for (int ks = 0; ks < kStepK; ++ks)
-      load_frag_to_lds(src + (int64_t)(next_s * kStepK + ks) * 512, &s_stage[stage][w][ks][0]);
-    if (--next_s < 0) {
-      next_s = S - 1;
-      next_cb += next_pass;
-      next_pass ^= 1;
+    for (int f = 0; f < 4; ++f) load_frag_to_lds(src + f * 64, &s_stage[stage][(w * 4 + f) * 1024]);
+    if (w < 2) load_frag_to_lds(p.phi + ((int64_t)(rb * S + next_s) * 2 + w) * kRecPos + 4 * lane, &s_stage[stage][(16 + w) * 1024]);
+    if (++next_s == S) {
+      next_s = 0;
+      ++next_cb;
     }
   };
+  half8 Ec[4][2], Es[4][2];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const half8* t = p.tab + ((int64_t)(rb * (kRecPos / 16) + w * 4 + i) * 4) * 64 + lane;
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+      Ec[i][kk] = t[kk * 64];
+      Es[i][kk] = t[(2 + kk) * 64];
+    }
+  }
 #pragma unroll
   for (int i = 0; i < NST - 1; ++i)
     if (i < Q) issue(i);
+  float4v A[4][2], Bs[4][2];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) A[i][j] = Bs[i][j] = float4v{0.f, 0.f, 0.f, 0.f};
+  // (the table must have landed before the loop: inside it the only waits on vector memory are explicit)
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) asm volatile("" ::"v"(Ec[i][kk]), "v"(Es[i][kk]));
 
-  half8 Ea[4][kStepK];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int ks = 0; ks < kStepK; ++ks) Ea[i][ks] = p.tab[((int64_t)min(rt0 + i, n_rt - 1) * kStepK + ks) * 64 + lane];
-  float rc[4][2], rs[4][2];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int f2 = 0; f2 < 2; ++f2) fast_sincos_phase(min(rt0 + i, n_rt - 1) * 8 + lg * 2 + f2, kStepTokens, p.T, &rs[i][f2], &rc[i][f2]);
-  float4v acc[4][4];
-  float re[4][4][2];   // real part left by the cos pass
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = float4v{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int ks = 0; ks < kStepK; ++ks) asm volatile("" ::"v"(Ea[i][ks]));
-
-  // (read here once: a load behind the walk of a column block would wait for every tile on its way)
-  const float inv_n = 1.0f / (float)p.N;
-  for (int i = tid; i < n_cb * kWgCols; i += 256) {
-    const int m = cb0 * kWgCols + i;
-    s_scale[i] = m < p.Mc ? p.scale[(int64_t)b * p.Mc + m] * inv_n : 0.f;
-  }
-  int cb = cb0, pass = 0, it = -1;
+  const int kw = rb * kRecPos + w * 64;   // first position of the wave
+  const bool all_in = kw + 63 < p.Kd;
+  const bool mirror_all = all_in && p.T - (kw + 63) > p.half && p.T - kw < p.K;
+  const bool mirror_none = p.T - kw <= p.half || p.T - (kw + 63) >= p.K;
+  int it = -1, cbl = 0;
   for (int q = 0; q < Q; ++q) {
     if (++it == S) {
       it = 0;
-      cb += pass;
-      pass ^= 1;
+      ++cbl;
     }
     const int stage = q % NST;
-    if (q + NST - 2 < Q) wait_vmcnt<(NST - 2) * kStepK>();
-    else wait_vmcnt<0>();
-    barrier_lds_only();
+    if (q + NST - 2 >= Q) wait_vmcnt<0>();
+    else if (w < 2) wait_vmcnt<(NST - 2) * 5>();
+    else wait_vmcnt<(NST - 2) * 4>();
+    barrier_lds_only();   // every wave's share of the step has landed; nobody still reads the stage refilled next
     if (q + NST - 1 < Q) issue((q + NST - 1) % NST);
-    spectral_step(acc, Ea, rc, rs, lds_addr_of(&s_stage[stage][0][0][lane * 16]));
+    const unsigned st = lds_addr_of(&s_stage[stage][0]), fr = st + lane * 16, ph = st + 16 * 1024 + (w * 64 + 4 * lg) * 4;
+    uint4v pc[4], ps[4], b0[4], b1[4];
+    pc[0] = lds_read_b128_async_at<0>(ph);
+    pc[1] = lds_read_b128_async_at<64>(ph);
+    pc[2] = lds_read_b128_async_at<128>(ph);
+    pc[3] = lds_read_b128_async_at<192>(ph);
+    ps[0] = lds_read_b128_async_at<1024 + 0>(ph);
+    ps[1] = lds_read_b128_async_at<1024 + 64>(ph);
+    ps[2] = lds_read_b128_async_at<1024 + 128>(ph);
+    ps[3] = lds_read_b128_async_at<1024 + 192>(ph);
+#define FA_REC_READ(B, G)                                       \
+  B[0] = lds_read_b128_async_at<((G) * 4 + 0) * 1024>(fr);      \
+  B[1] = lds_read_b128_async_at<((G) * 4 + 1) * 1024>(fr);      \
+  B[2] = lds_read_b128_async_at<((G) * 4 + 2) * 1024>(fr);      \
+  B[3] = lds_read_b128_async_at<((G) * 4 + 3) * 1024>(fr)
+    // one column tile's cosine or sine coefficients: f = {+ k0, + k1, - k0, - k1}
+    auto products = [&](const uint4v (&f)[4], float4v (&acc)[4][2], int j, bool sine) {
+      float4v C[4], D[4];
+#pragma unroll
+      for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          C[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Ec[i][kk], __builtin_bit_cast(half8, f[kk]),
+                                                        kk ? C[i] : float4v{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+      for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          D[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Es[i][kk], __builtin_bit_cast(half8, f[2 + kk]),
+                                                        kk ? D[i] : float4v{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float4v co = __builtin_bit_cast(float4v, pc[i]), sn = __builtin_bit_cast(float4v, ps[i]);
+        acc[i][j] += (sine ? sn : co) * C[i];
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float4v co = __builtin_bit_cast(float4v, pc[i]), sn = __builtin_bit_cast(float4v, ps[i]);
+        if (sine) acc[i][j] += co * D[i];
+        else acc[i][j] -= sn * D[i];
+      }
+    };
+    FA_REC_READ(b0, 0);
+    lds_wait_for4<8>(pc);
+    lds_wait_for4<4>(ps);
+    FA_REC_READ(b1, 1);
+    lds_wait_for4<4>(b0);
+    products(b0, A, 0, false);
+    FA_REC_READ(b0, 2);
+    lds_wait_for4<4>(b1);
+    products(b1, Bs, 0, true);
+    FA_REC_READ(b1, 3);
+    lds_wait_for4<4>(b0);
+    products(b0, A, 1, false);
+    lds_wait_for4<0>(b1);
+    products(b1, Bs, 1, true);
+#undef FA_REC_READ
     if (it != S - 1) continue;
-    if (pass == 0) {
+    // the column block is complete: r = A +- B (the scale follows behind the loop) at this lane's 16 positions per column
+    // and at their mirror images
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          re[i][j][0] = acc[i][j][0];
-          re[i][j][1] = acc[i][j][2];
-          acc[i][j] = float4v{0.f, 0.f, 0.f, 0.f};
-        }
-      continue;
-    }
-    // both passes done for this column block: r = (re +- im) * scale / N at this lane's 8 positions per column and
-    // at their mirror images
-    const int half = p.half;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const float sc = s_scale[((cb - cb0) * 4 + j) * 16 + lc];
+    for (int j = 0; j < 2; ++j) {
       float sum = 0.f, mx = -INFINITY, mn = INFINITY;
+      if (mirror_all) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int f2 = 0; f2 < 2; ++f2) {
-          const int k = (rt0 + i) * 8 + lg * 2 + f2;
-          const float r = (re[i][j][f2] + acc[i][j][2 * f2 + 1]) * sc;
-          if (k < p.Kd) {
+          for (int v = 0; v < 4; ++v) {
+            const float a = A[i][j][v], bb = Bs[i][j][v], hi = a + bb, lo = a - bb;
+            sum += a;
+            mx = fa_fmax(fa_fmax(mx, hi), lo);
+            mn = fa_fmin(fa_fmin(mn, hi), lo);
+          }
+        sum += sum;
+      } else if (all_in && mirror_none) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int v = 0; v < 4; ++v) {
+            const float r = A[i][j][v] + Bs[i][j][v];
             sum += r;
-            mx = fmaxf(mx, r);
-            mn = fminf(mn, r);
+            mx = fa_fmax(mx, r);
+            mn = fa_fmin(mn, r);
           }
-          const int km = p.T - k;   // the mirror image counts where it is a position of its own beyond T / 2
-          const float r2 = (re[i][j][f2] - acc[i][j][2 * f2 + 1]) * sc;
-          if (k < p.Kd && km > half && km < p.K) {
-            sum += r2;
-            mx = fmaxf(mx, r2);
-            mn = fminf(mn, r2);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int v = 0; v < 4; ++v) {
+            const int k = kw + i * 16 + 4 * lg + v;
+            const float r = A[i][j][v] + Bs[i][j][v], r2 = A[i][j][v] - Bs[i][j][v];
+            if (k < p.Kd) {
+              sum += r;
+              mx = fa_fmax(mx, r);
+              mn = fa_fmin(mn, r);
+            }
+            const int km = p.T - k;   // the mirror image counts where it is a position of its own beyond T / 2
+            if (k < p.Kd && km > p.half && km < p.K) {
+              sum += r2;
+              mx = fa_fmax(mx, r2);
+              mn = fa_fmin(mn, r2);
+            }
           }
-        }
+      }
       sum = fa_rows_sum(sum);
       mx = fa_rows_max(mx);
       mn = fa_rows_min(mn);
       if (lg == 0) {
-        s_red[0][w][j * 16 + lc] = sum;
-        s_red[1][w][j * 16 + lc] = mx;
-        s_red[2][w][j * 16 + lc] = mn;
+        // (written past the compiler, which would wait for the tiles on their way first)
+        const unsigned at = lds_addr_of(&s_stat[0][w][cbl * kRecCols + j * 16 + lc]);
+        constexpr int kKind = 4 * kMaxColShare * kRecCols * 4;   // bytes
+        asm volatile("ds_write_b32 %0, %1\n\tds_write_b32 %0, %2 offset:%4\n\tds_write_b32 %0, %3 offset:%5" ::"v"(at), "v"(sum),
+                     "v"(mx), "v"(mn), "n"(kKind), "n"(2 * kKind)
+                     : "memory");
       }
-    }
-    __syncthreads();
-    if (tid < kWgCols) {
-      const int m = cb * kWgCols + tid;
-      if (m < p.Mc) {
-        const int64_t o = ((int64_t)b * p.RB + rb) * p.Mc + m;
-        p.psum[o] = (s_red[0][0][tid] + s_red[0][1][tid]) + (s_red[0][2][tid] + s_red[0][3][tid]);
-        p.pmax[o] = fmaxf(fmaxf(s_red[1][0][tid], s_red[1][1][tid]), fmaxf(s_red[1][2][tid], s_red[1][3][tid]));
-        p.pmin[o] = fminf(fminf(s_red[2][0][tid], s_red[2][1][tid]), fminf(s_red[2][2][tid], s_red[2][3][tid]));
-      }
-    }
-    // the next barrier (top of the loop) orders these reads before s_red is written again
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) acc[i][j] = float4v{0.f, 0.f, 0.f, 0.f};
+      for (int i = 0; i < 4; ++i) A[i][j] = Bs[i][j] = float4v{0.f, 0.f, 0.f, 0.f};
+    }
+  }
+  barrier_lds_only();   // (behind the wait for the writes above)
+  const float inv_n = 1.0f / (float)p.N;
+  // positions and mirror images the workgroup stands for
+  const int k0 = rb * kRecPos, k1 = min(k0 + kRecPos, p.Kd);
+  const int n_pos = k1 - k0 + (p.half < p.T ? max(0, min(k1, p.T - p.half) - max(k0, p.T - p.K + 1)) : 0);
+  for (int c = tid; c < n_cb * kRecCols; c += 256) {
+    const int m = cb0 * kRecCols + c;
+    if (m >= p.Mc) break;
+    const float sc = p.scale[(int64_t)b * p.Mc + m] * inv_n, c0 = p.c[(int64_t)b * 2 * p.N * p.Mc + m] * inv_n;
+    const int64_t o = ((int64_t)b * p.RB + rb) * p.Mc + m;
+    p.psum[o] = ((s_stat[0][0][c] + s_stat[0][1][c]) + (s_stat[0][2][c] + s_stat[0][3][c])) * sc + (float)n_pos * c0;
+    p.pmax[o] = fa_fmax(fa_fmax(s_stat[1][0][c], s_stat[1][1][c]), fa_fmax(s_stat[1][2][c], s_stat[1][3][c])) * sc + c0;
+    p.pmin[o] = fa_fmin(fa_fmin(s_stat[2][0][c], s_stat[2][1][c]), fa_fmin(s_stat[2][2][c], s_stat[2][3][c])) * sc + c0;
   }
 }
 
@@ -616,9 +773,9 @@ int fa_spectral_mfma_launch(const void* a, int a_dtype, int64_t a_bs, int64_t a_
   half8* packed = (half8*)((char*)workspace + pl.off_packed);
   dim3 pgrid(pl.KS32, fa_cdiv(Mc, 256), B);
   if (a_dtype == FA_BF16)
-    spectral_pack_kernel<bf16_t><<<pgrid, 256, 0, st>>>((const bf16_t*)a, a_bs, a_rs, cols, nullptr, packed, K, Mc, pl.CT, pl.KS32, B, 0, 0);
+    spectral_pack_kernel<bf16_t><<<pgrid, 256, 0, st>>>((const bf16_t*)a, a_bs, a_rs, cols, packed, K, Mc, pl.CT, pl.KS32);
   else
-    spectral_pack_kernel<f16_t><<<pgrid, 256, 0, st>>>((const f16_t*)a, a_bs, a_rs, cols, nullptr, packed, K, Mc, pl.CT, pl.KS32, B, 0, 0);
+    spectral_pack_kernel<f16_t><<<pgrid, 256, 0, st>>>((const f16_t*)a, a_bs, a_rs, cols, packed, K, Mc, pl.CT, pl.KS32);
   return spectral_after_pack(pl, c, B, Mc, N, T, k_start, accumulate, workspace, st);
 }
 
@@ -720,23 +877,21 @@ extern "C" int fa_prefill_compress(const void* src, int dtype, int64_t src_bs, i
 
 namespace {
 struct ReconPlan {
-  int CT, KS32, n_steps, RB;
-  size_t off_tab, off_pc, off_ps, off_scale, off_inv, off_sum, off_max, off_min, total;
+  int CT, n_steps, RB;
+  size_t off_tab, off_packed, off_phi, off_scale, off_sum, off_max, off_min, total;
 };
 ReconPlan recon_plan(int B, int N, int Mc, int K) {
   using namespace fa_mfma;
   ReconPlan p{};
   p.CT = fa_cdiv(Mc, 16);
-  p.n_steps = fa_cdiv(N, kStepTokens);
-  p.KS32 = p.n_steps * kStepK;
-  p.RB = fa_cdiv(K, kWgFreqs);
+  p.n_steps = fa_cdiv(N, kRecStep);
+  p.RB = fa_cdiv(K, kRecPos);
   size_t o = 0;
   auto take = [&](size_t bytes) { size_t at = o; o += fa_align_up(bytes, 256); return at; };
-  p.off_tab = take((size_t)fa_cdiv(K, 8) * kStepK * 64 * 16);
-  p.off_pc = take((size_t)B * p.CT * p.KS32 * 1024);
-  p.off_ps = take((size_t)B * p.CT * p.KS32 * 1024);
+  p.off_tab = take((size_t)p.RB * (kRecPos / 16) * 4 * 1024);
+  p.off_packed = take((size_t)B * p.CT * p.n_steps * kRecFrags * 1024);
+  p.off_phi = take((size_t)p.RB * p.n_steps * 2 * kRecPos * 4);
   p.off_scale = take((size_t)B * Mc * 4);
-  p.off_inv = take((size_t)B * Mc * 4);
   p.off_sum = take((size_t)B * p.RB * Mc * 4);
   p.off_max = take((size_t)B * p.RB * Mc * 4);
   p.off_min = take((size_t)B * p.RB * Mc * 4);
@@ -772,30 +927,27 @@ int fa_recon_stats_mfma_launch(const float* c, int B, int N, int Mc, int K, int 
   const ReconPlan pl = recon_plan(B, N, Mc, K);
   char* ws = (char*)workspace;
   half8* tab = (half8*)(ws + pl.off_tab);
-  half8* pc = (half8*)(ws + pl.off_pc);
-  half8* ps = (half8*)(ws + pl.off_ps);
+  half8* packed = (half8*)(ws + pl.off_packed);
+  float* phi = (float*)(ws + pl.off_phi);
   float* scale = (float*)(ws + pl.off_scale);
-  float* inv = (float*)(ws + pl.off_inv);
   *psum = (float*)(ws + pl.off_sum);
   *pmax = (float*)(ws + pl.off_max);
   *pmin = (float*)(ws + pl.off_min);
   // positions 0 .. T / 2 stand for their mirror images as well (unless the sequence is longer than the period)
   const bool mirror = K <= T + 1;
   const int Kd = mirror && T / 2 + 1 < K ? T / 2 + 1 : K;
-  const int RBd = fa_cdiv(Kd, kWgFreqs);
-  const int kp8 = fa_cdiv(Kd, 8) * 8;
-  spectral_table_kernel<<<fa_cdiv((int64_t)(kp8 / 8) * kTableThreads, 256), 256, 0, st>>>((half2v*)tab, kp8, T);
-  coef_colscale_kernel<<<dim3(fa_cdiv(Mc, 16), B), 1024, 0, st>>>(c, scale, inv, 2 * N, Mc);
-  // the cosine rows and, behind them, the sine rows
-  spectral_pack_kernel<float><<<dim3(pl.KS32, fa_cdiv(Mc, 256), 2 * B), 256, 0, st>>>(c, (int64_t)2 * N * Mc, Mc, nullptr, inv, pc, N, Mc,
-                                                                                     pl.CT, pl.KS32, B, (int64_t)N * Mc, ps - pc);
+  const int RBd = fa_cdiv(Kd, kRecPos);
+  ReconPrepParams pp{};
+  pp.c = c; pp.packed = packed; pp.scale = scale; pp.tab = (half2v*)tab; pp.phi = phi;
+  pp.B = B; pp.N = N; pp.Mc = Mc; pp.CT = pl.CT; pp.T = T; pp.n_steps = pl.n_steps;
+  recon_prep_kernel<<<pl.CT * B + RBd * (kRecPos / 32), 1024, 0, st>>>(pp);
   ReconStatsParams rp{};
-  rp.tab = tab; rp.packed[0] = pc; rp.packed[1] = ps; rp.scale = scale;
+  rp.c = c; rp.tab = tab; rp.packed = packed; rp.phi = phi; rp.scale = scale;
   rp.psum = *psum; rp.pmax = *pmax; rp.pmin = *pmin;
-  rp.B = B; rp.N = N; rp.Mc = Mc; rp.CT = pl.CT; rp.KS32 = pl.KS32; rp.K = K; rp.T = T; rp.n_steps = pl.n_steps; rp.RB = RBd;
+  rp.B = B; rp.N = N; rp.Mc = Mc; rp.CT = pl.CT; rp.K = K; rp.T = T; rp.n_steps = pl.n_steps; rp.RB = RBd;
   rp.Kd = Kd;
   rp.half = mirror ? T / 2 : 0x7fffffff;
-  const int n_cb = fa_cdiv(Mc, kWgCols);
+  const int n_cb = fa_cdiv(Mc, kRecCols);
   rp.cb_per = recon_col_share(RBd * B, n_cb);
   spectral_recon_stats_kernel<<<dim3(RBd, B, fa_cdiv(n_cb, rp.cb_per)), 256, 0, st>>>(rp);
   return RBd;

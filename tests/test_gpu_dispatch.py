@@ -26,6 +26,41 @@ def test_reconstruction_statistics_by_shares_of_column_blocks(B, L, C, N, T):
         assert np.max((a - b).abs().cpu().numpy() / size) <= 2e-3
 
 
+@pytest.mark.parametrize("B,L,C,N,T", [
+    (1, 1300, 33, 1100, 2700),   # nine steps of 128 coefficients, the last one short; a column block of one column
+    (2, 2048, 32, 1024, 2048),   # eight whole steps; whole blocks of positions and, with position T / 2, one of a single one
+    (1, 1025, 17, 129, 1400),    # one coefficient past a step
+])
+def test_reconstruction_statistics_of_signals_with_a_mean(B, L, C, N, T):
+    """Folded steps of the coefficients against float64, for signals whose mean outweighs their deviation.  Bound: coefficients
+    and basis carry up to 2^-11 relative rounding each, independent from term to term, so a position is off by at most about
+    five standard deviations (1 / sqrt(3) of the bound each, 4 in all) of 2^-11 times the 2-norm of the column's coefficients
+    over N - without that of frequency 0, which is summed in single precision like the mean: 1e-5 of it.  The deviation is a
+    difference of two such values.  What is not a number stays in its column."""
+    from fourierattention_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(5)
+    t = torch.arange(L, dtype=torch.float64, device="cuda")
+    x = torch.randn((B, L, C), generator=g, device="cuda", dtype=torch.float64) + 40.0
+    n = torch.arange(N, dtype=torch.float64, device="cuda")
+    ph = 2 * np.pi / T * torch.remainder(n[:, None] * t[None], T)
+    c = torch.cat([ph.cos() @ x, ph.sin() @ x], dim=1).float()
+    r = (ph.cos().T @ c[:, :N].double() + ph.sin().T @ c[:, N:].double()) / N
+    avg = r.mean(1)
+    dev = torch.maximum(r.amax(1) - avg, avg - r.amin(1))
+    got = ops.mat_fourier_avg_std(c, L, T, None)
+    rest = c.double()
+    rest[:, [0, N]] = 0.0
+    bound = 4 * 2.0 ** -11 * rest.norm(dim=1) / N + 1e-5 * avg.abs()
+    assert ((got[0].double() - avg).abs() <= bound).all()
+    assert ((got[1].double() - dev).abs() <= 2 * bound).all()
+    c[0, N // 2, 3], c[0, N + 1, 5], c[0, 0, 7] = float("nan"), float("inf"), float("nan")
+    bad = ops.mat_fourier_avg_std(c, L, T, None)
+    whole = torch.ones((B, C), dtype=torch.bool, device="cuda")
+    whole[0, [3, 5, 7]] = False
+    for a, b in zip(bad, got):
+        assert torch.equal(a[whole], b[whole]) and not torch.isfinite(a[~whole]).any()
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
 @pytest.mark.parametrize("B,Hq,Hkv,D,n_il,L,N,k_counts,v_counts", [
     (1, 3, 1, 128, 5, 1, 5, [127], [1]),                        # one mid row; one stored K dim, one compressed V dim
