@@ -10,7 +10,7 @@
 //   G_s[n] = sum_{i<128} E[n, i] a[128 s + i]
 // so the steps are walked from the last to the first, acc <- G_s + e^{i theta n 128} acc, with the
 // accumulators (fp32) never leaving registers.  Three kernels:
-//   pack    gathers the compressed columns of the token-major input, converts them to f16 and writes them
+//   pack    evaluates the basis table, gathers the compressed columns of the token-major input, converts them to f16 and writes them
 //           as ready-made MFMA B operands (column tile of 16, kstep of 32 tokens, 64 lanes x 8 tokens)
 //   gemm    one workgroup = 128 frequencies x 64 columns x one chunk of steps; the operands of a step
 //           travel HBM -> LDS with global_load_lds, one barrier per step
@@ -28,9 +28,12 @@ constexpr int kWgCols = 64;                    // columns per workgroup (four co
 // cos (r even) or sin (r odd); lane l holds row l % 16, tokens 8 * (l / 16) + e of the kstep ----------------
 // A thread takes two tokens of a frequency and writes both rows: one evaluation per phase (a thread per row would
 // evaluate every phase twice), short chains (7.4 -> 5.6 us for 512 frequencies).
+// It needs nothing but N and T: the blocks of the table ride in the launch that packs the columns (as a launch of its own
+// in front of the products: 3.8 - 6 us).
 constexpr int kTableThreads = kStepK * 128;    // per row tile
-__global__ __launch_bounds__(256) void spectral_table_kernel(half2v* __restrict__ tab, int N, int T) {
-  const int idx = blockIdx.x * 256 + threadIdx.x;
+__host__ __device__ inline int table_blocks(int N) { return (N / 8 * kTableThreads + 255) / 256; }
+__device__ __forceinline__ void spectral_table_block(half2v* __restrict__ tab, int N, int T, int block) {
+  const int idx = block * 256 + threadIdx.x;
   if (idx >= (N / 8) * kTableThreads) return;
   const int ep = idx & 3, f = (idx >> 2) & 7, lg = (idx >> 5) & 3, frag = idx >> 7;   // frag = rt * kStepK + ks
   const int n = frag / kStepK * 8 + f, token = frag % kStepK * 32 + 8 * lg + 2 * ep;
@@ -46,15 +49,23 @@ __global__ __launch_bounds__(256) void spectral_table_kernel(half2v* __restrict_
   out[0] = c;
   out[4] = s;
 }
+struct SpectralTable {
+  half2v* tab;
+  int N, T;
+};
 
 // ---- pack: block = 32 tokens x 256 columns; lanes run along the columns for the gather, the transposition to
-// token-contiguous fragments goes through LDS.  grid (ksteps, column blocks, B) ------------------------------------------
+// token-contiguous fragments goes through LDS.  grid (ksteps + blocks of the basis table, column blocks, B) ------------------------------------------
 template <typename E>
 __global__ __launch_bounds__(256) void spectral_pack_kernel(
     const E* __restrict__ a, int64_t a_bs, int64_t a_rs, const int32_t* __restrict__ cols,
-    half8* __restrict__ out, int K, int Mc, int CT, int KS32) {
+    half8* __restrict__ out, int K, int Mc, int CT, int KS32, const SpectralTable st) {
   constexpr int kPitch = 256 + 4;   // f16 elements per LDS row: 8 rows apart = 16 banks apart
   __shared__ _Float16 tile[32][kPitch];
+  if ((int)blockIdx.x >= KS32) {
+    spectral_table_block(st.tab, st.N, st.T, ((int)blockIdx.x - KS32) * gridDim.y * gridDim.z + blockIdx.z * gridDim.y + blockIdx.y);
+    return;
+  }
   const int tid = threadIdx.x;
   const int ks = blockIdx.x, m0 = blockIdx.y * 256, b = blockIdx.z;
   const int m = m0 + tid;
@@ -113,6 +124,7 @@ struct PrefillPackParams {
   half8* packed;                // [B][CT][KS32][64]
   float* psum; float* pmax; float* pmin;   // [B][n_blocks][Mc]
   int Mc, CT, KS32, n_pages, n_blocks, Hkv, D, is_v;
+  SpectralTable table;          // the blocks of x behind n_blocks evaluate the basis of the products
 };
 
 template <typename E>
@@ -124,6 +136,10 @@ __global__ __launch_bounds__(256) void prefill_pack_kernel(const PrefillPackPara
   __shared__ int s_col[kMaxD];                      // dim within the head of every stored position
   __shared__ int s_ccol[kMaxD];                     // ... of every compressed position
   const int h = blockIdx.y, b = blockIdx.z, tid = threadIdx.x, D = p.D;
+  if ((int)blockIdx.x >= p.n_blocks) {
+    spectral_table_block(p.table.tab, p.table.N, p.table.T, ((int)blockIdx.x - p.n_blocks) * gridDim.y * gridDim.z + b * gridDim.y + h);
+    return;
+  }
   const int n0 = p.n_h[h], n_len = p.n_h[h + 1] - n0;
   const int p0 = p.pad_h[h], dp = p.pad_h[h + 1] - p0;
   const int c0 = p.c_h[h], c_len = p.c_h[h + 1] - c0;
@@ -737,11 +753,16 @@ SpectralPlan spectral_plan(int B, int K, int Mc, int N) {
   p.n_steps = fa_cdiv(K, kStepTokens);
   p.KS32 = p.n_steps * kStepK;
   const int64_t tiles = (int64_t)B * fa_cdiv(N, kWgFreqs) * fa_cdiv(Mc, kWgCols);
-  int want = fa_cdiv(512, tiles);                  // two workgroups per CU
-  if (want < 1) want = 1;
-  const int max_chunks = p.n_steps / 4 > 0 ? p.n_steps / 4 : 1;   // at least four steps per chunk
-  if (want > max_chunks) want = max_chunks;
-  p.steps_per_chunk = fa_cdiv(p.n_steps, want);
+  // Chunks of the walk, at least four steps each: two workgroups fit a compute unit, so the launch takes as many rounds as
+  // there are 512s of workgroups, each as long as a chunk and about three steps of prologue and store.  (Always rounded up to
+  // 512 workgroups, 240 tiles of 16 steps ran as 720 workgroups of 6 steps in two rounds: 50.8 us a call against 39.7.)
+  const int max_chunks = p.n_steps / 4 > 0 ? p.n_steps / 4 : 1;
+  int64_t best = INT64_MAX;
+  for (int n = 1; n <= max_chunks && (n == 1 || tiles * n <= 1024); ++n) {
+    const int per = fa_cdiv(p.n_steps, n);
+    const int64_t cost = (int64_t)fa_cdiv(tiles * fa_cdiv(p.n_steps, per), 512) * (per + 3);
+    if (cost < best) { best = cost; p.steps_per_chunk = per; }
+  }
   p.n_chunks = fa_cdiv(p.n_steps, p.steps_per_chunk);
   size_t o = 0;
   auto take = [&](size_t bytes) { size_t at = o; o += fa_align_up(bytes, 256); return at; };
@@ -760,7 +781,7 @@ bool fa_spectral_mfma_ok(int a_dtype, int K, int Mc, int N) {
 size_t fa_spectral_mfma_workspace(int B, int K, int Mc, int N) { return spectral_plan(B, K, Mc, N).total; }
 
 namespace {
-// table, GEMM and chunk reduction on fragments that are already in the workspace
+// GEMM and chunk reduction on the table and the fragments that are already in the workspace
 int spectral_after_pack(const SpectralPlan& pl, float* c, int B, int Mc, int N, int T, int64_t k_start, int accumulate,
                         void* workspace, hipStream_t st);
 }  // namespace
@@ -771,11 +792,12 @@ int fa_spectral_mfma_launch(const void* a, int a_dtype, int64_t a_bs, int64_t a_
   using namespace fa_mfma;
   const SpectralPlan pl = spectral_plan(B, K, Mc, N);
   half8* packed = (half8*)((char*)workspace + pl.off_packed);
-  dim3 pgrid(pl.KS32, fa_cdiv(Mc, 256), B);
+  const SpectralTable table{(half2v*)((char*)workspace + pl.off_tab), N, T};
+  dim3 pgrid(pl.KS32 + fa_cdiv(table_blocks(N), (int64_t)fa_cdiv(Mc, 256) * B), fa_cdiv(Mc, 256), B);
   if (a_dtype == FA_BF16)
-    spectral_pack_kernel<bf16_t><<<pgrid, 256, 0, st>>>((const bf16_t*)a, a_bs, a_rs, cols, packed, K, Mc, pl.CT, pl.KS32);
+    spectral_pack_kernel<bf16_t><<<pgrid, 256, 0, st>>>((const bf16_t*)a, a_bs, a_rs, cols, packed, K, Mc, pl.CT, pl.KS32, table);
   else
-    spectral_pack_kernel<f16_t><<<pgrid, 256, 0, st>>>((const f16_t*)a, a_bs, a_rs, cols, packed, K, Mc, pl.CT, pl.KS32);
+    spectral_pack_kernel<f16_t><<<pgrid, 256, 0, st>>>((const f16_t*)a, a_bs, a_rs, cols, packed, K, Mc, pl.CT, pl.KS32, table);
   return spectral_after_pack(pl, c, B, Mc, N, T, k_start, accumulate, workspace, st);
 }
 
@@ -787,7 +809,6 @@ int spectral_after_pack(const SpectralPlan& pl, float* c, int B, int Mc, int N, 
   half8* tab = (half8*)(ws + pl.off_tab);
   half8* packed = (half8*)(ws + pl.off_packed);
   float* part = (float*)(ws + pl.off_part);
-  spectral_table_kernel<<<fa_cdiv((int64_t)(N / 8) * kTableThreads, 256), 256, 0, st>>>((half2v*)tab, N, T);
   SpectralGemmParams gp{};
   const bool direct = pl.n_chunks == 1;   // nothing to sum: the GEMM writes (or adds to) c itself
   gp.tab = tab; gp.packed = packed; gp.part = direct ? c : part;
@@ -866,7 +887,8 @@ extern "C" int fa_prefill_compress(const void* src, int dtype, int64_t src_bs, i
     pp.psum = psum; pp.pmax = pmax; pp.pmin = pmin;
     pp.Mc = Mc; pp.CT = pl.sp.CT; pp.KS32 = pl.sp.KS32; pp.n_pages = pl.n_pages; pp.n_blocks = pl.n_blocks;
     pp.Hkv = Hkv; pp.D = D; pp.is_v = is_v;
-    prefill_pack_kernel<E><<<dim3(pl.n_blocks, Hkv, B), 256, 0, st>>>(pp);
+    pp.table = SpectralTable{(half2v*)(ws + pl.sp.off_tab), N, T};
+    prefill_pack_kernel<E><<<dim3(pl.n_blocks + fa_cdiv(table_blocks(N), (int64_t)Hkv * B), Hkv, B), 256, 0, st>>>(pp);
   };
   if (dtype == FA_BF16) launch(bf16_t{}); else launch(f16_t{});
   int rc = spectral_after_pack(pl.sp, coef, B, Mc, N, T, 0, 0, workspace, st);
