@@ -94,6 +94,7 @@ _SIGNATURES = {
                                        c_size_t, c_void_p]),
     "fa_stats_workspace_bytes": (c_size_t, [c_int, c_int, c_int]),
     "fa_mat_fourier_avg_std_workspace_bytes": (c_size_t, [c_int, c_int, c_int, c_int]),
+    "fa_recon_scale": (c_int, [c_void_p] * 8 + [c_int] * 6 + [c_void_p, c_size_t, c_void_p]),
     "fa_reconstruct": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int,
                                c_void_p]),
     "fa_coeff_update": (c_int, [c_void_p, c_void_p, c_int, c_int64, c_void_p, c_int, c_int, c_int, c_int64, c_int,
@@ -117,6 +118,8 @@ _SIGNATURES = {
                             c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p]),
     "fa_append_rows": (c_int, [c_void_p, c_void_p, c_int64, c_int64, c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int, c_int,
                                c_int, c_int, c_void_p]),
+    "fa_prompt_rows": (c_int, [c_void_p, c_void_p, c_int64, c_int64, c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_int64]
+                       + [c_int] * 8 + [c_void_p]),
     "fa_convert": (c_int, [c_void_p, c_int, c_void_p]),
     "fa_prefill_compress_ok": (c_int, [c_int, c_int, c_int, c_int, c_int, c_int]),
     "fa_prefill_compress_workspace_bytes": (c_size_t, [c_int, c_int, c_int, c_int, c_int]),

@@ -18,6 +18,7 @@ reference's shapes only when somebody indexes them; the attention forward in
 from __future__ import annotations
 
 import json
+from array import array
 from collections.abc import Mapping
 from typing import Any, Dict, List, Optional, Tuple
 
@@ -99,6 +100,28 @@ class CacheParts(Mapping):
         return self.cache._window_in_order(layer, t)
 
 
+def _device_lists(lists, device):
+    """Lists of integers as int64 and as int32 tensors on ``device``: views of one tensor of each type, which take one copy
+    (asynchronous, from pinned memory) and one conversion whatever their number - a copy and a conversion per list, each
+    waited for, were a fifth of the time of a short prompt.  Every view starts 128 bytes aligned."""
+    flat, spans = array("q"), []
+    try:
+        for lst in lists:
+            spans.append((len(flat), len(lst)))
+            flat.extend(lst)
+            flat.extend([0] * (-len(flat) % 32))
+    except (TypeError, OverflowError):      # entries that are no integers: what torch makes of them
+        wide = [torch.tensor(lst, dtype=torch.int64, device=device) for lst in lists]
+        return wide, [t.to(torch.int32) for t in wide]
+    host = torch.frombuffer(flat, dtype=torch.int64) if len(flat) else torch.empty(0, dtype=torch.int64)
+    if device.type == "cuda":
+        all64 = torch.empty(host.shape, dtype=torch.int64, pin_memory=True).copy_(host).to(device, non_blocking=True)
+    else:
+        all64 = host.clone().to(device)
+    all32 = all64.to(torch.int32)
+    return tuple([t[o: o + n] if n else t.new_empty(0) for o, n in spans] for t in (all64, all32))
+
+
 class Cache(torch.nn.Module):
     """Base class of every cache object, as in cache_utils_fourier.py:39-125 (a ``torch.nn.Module`` there too).
     The modified LLaMA imports this name next to ``DynamicCache`` and ``StaticCache``
@@ -178,30 +201,34 @@ class DynamicCache(Cache):
         self.v_non_critical_dims, self.v_non_critical_head_dims = [], []
         self.v_critical_dims, self.v_critical_head_dims = [], []
         self._lists32: List[Tuple[torch.Tensor, ...]] = []
-        dev = self.device
-        for layer_idx in range(len(masks)):
+        self._pads32: List[Tuple[torch.Tensor, ...]] = []
+        self._num_layers = len(masks)
+        self._head_lists, every = [], []
+        for layer_idx in range(self._num_layers):
             self.curr_tokennum.append(0)
             key = f"Layer_{layer_idx}"
             if key not in masks:
                 raise ValueError(f"Layer index {layer_idx} not found in non-critical dimensions JSON file.")
             m = masks[key]
-            t64 = lambda lst: torch.tensor(lst, dtype=torch.int64, device=dev)
-            self.k_non_critical_dims.append(t64(m["kc_list"]))
-            self.k_critical_dims.append(t64(m["kn_list"]))
-            self.v_non_critical_dims.append(t64(m["vc_list"]))
-            self.v_critical_dims.append(t64(m["vn_list"]))
-            self.k_non_critical_head_dims.append(t64([0] + list(m["kc_h_list"])))
-            self.k_critical_head_dims.append(t64([0] + list(m["kn_h_list"])))
-            self.v_non_critical_head_dims.append(t64([0] + list(m["vc_h_list"])))
-            self.v_critical_head_dims.append(t64([0] + list(m["vn_h_list"])))
-            self._lists32.append(tuple(t.to(torch.int32) for t in (
-                self.k_non_critical_dims[-1], self.k_non_critical_head_dims[-1],
-                self.k_critical_dims[-1], self.k_critical_head_dims[-1],
-                self.v_non_critical_dims[-1], self.v_non_critical_head_dims[-1],
-                self.v_critical_dims[-1], self.v_critical_head_dims[-1])))
-        self._num_layers = len(masks)
-        self._head_lists = [([0] + list(masks[f"Layer_{i}"]["kn_h_list"]), [0] + list(masks[f"Layer_{i}"]["vn_h_list"]))
-                            for i in range(self._num_layers)]
+            kn_h, vn_h = [0] + list(m["kn_h_list"]), [0] + list(m["vn_h_list"])
+            self._head_lists.append((kn_h, vn_h))
+            every += [m["kc_list"], [0] + list(m["kc_h_list"]), m["kn_list"], kn_h,
+                      m["vc_list"], [0] + list(m["vc_h_list"]), m["vn_list"], vn_h]
+            # the padded offsets of the page stores (other head counts than the masks': MidStore makes its own)
+            every += [MidStore.padded(n, len(n) - 1, is_v) for n, is_v in ((kn_h, False), (vn_h, True))]
+        wide, narrow = _device_lists(every, self.device)
+        for at in range(0, len(every), 10):
+            kc, kc_h, kn, kn_h, vc, vc_h, vn, vn_h = wide[at: at + 8]
+            self.k_non_critical_dims.append(kc)
+            self.k_non_critical_head_dims.append(kc_h)
+            self.k_critical_dims.append(kn)
+            self.k_critical_head_dims.append(kn_h)
+            self.v_non_critical_dims.append(vc)
+            self.v_non_critical_head_dims.append(vc_h)
+            self.v_critical_dims.append(vn)
+            self.v_critical_head_dims.append(vn_h)
+            self._lists32.append(tuple(narrow[at: at + 8]))
+            self._pads32.append(tuple(narrow[at + 8: at + 10]))
         self._tables: Optional[torch.Tensor] = None   # constant operands of the MFMA decode kernels
         self.force_generic = False                     # testing: keep decode attention off the MFMA kernels
         self.balance_heads = True                      # mid rows: more splits for heads that store more dims
@@ -286,17 +313,15 @@ class DynamicCache(Cache):
         return (layer.k.il, layer.v.il, self.numinittokens + layer.spare)
 
     def _compress_tensor(self, t: _Tensor, states: torch.Tensor, c32: torch.Tensor, ch32: torch.Tensor, n32: torch.Tensor,
-                         nh32: torch.Tensor, nh_host, is_v: bool, L: int, fft_rows: int, n_f: int):
+                         nh32: torch.Tensor, nh_host, pad32: torch.Tensor, is_v: bool, L: int, fft_rows: int, n_f: int):
         I, W = self.numinittokens, self.maxlocallen
         B, S, HD = states.shape
         mid = states[:, I: S - W, :]
-        t.il = torch.empty((B, I + W + 1, HD), dtype=states.dtype, device=states.device)
-        t.init, t.ring = t.il[:, :I, :], t.il[:, I:, :]
-        t.init.copy_(states[:, :I, :])
-        t.ring[:, :W, :].copy_(states[:, S - W:, :])
-        t.ring[:, W, :].zero_()
+        if pad32.numel() != self.heads + 1:
+            pad32 = None
         cap = max(self._book.t_x, L + int(self.maxnewtokens)) + 1     # room for every row the decode will evict
-        t.mid = MidStore(B, n32, nh32, nh_host, self.heads, self.head_dim, cap, states.dtype, states.device, is_v)
+        t.mid = MidStore(B, n32, nh32, nh_host, self.heads, self.head_dim, cap, states.dtype, states.device, is_v,
+                         pad_h32=pad32)
         fused = t.mid.pack_and_compress(states, I, L, fft_rows, c32, ch32, n_f, self._book.t_c, states.dtype) \
             if self.fuse_prefill else None
         if fused is not None:   # pages, coefficients and column statistics from one read of the rows
@@ -306,13 +331,27 @@ class DynamicCache(Cache):
             # spectral compression of the selected columns (gather fused into the kernel)
             t.coef = ops.mat_fourier(mid, n_f, self._book.t_c, 0, cols=c32, K=fft_rows)
             u_avg, u_std = ops.mat_avg_std(mid, cols=c32, round_dtype=states.dtype)
-        i_avg, i_std = ops.mat_fourier_avg_std(t.coef, L, self._book.t_x, torch.float16)
         # dtypes as the reference leaves them: u_* in the model dtype, i_* in fp16, quotient promoted
-        u_avg_m, u_std_m = u_avg.to(states.dtype), u_std.to(states.dtype)
-        i_avg_h, i_std_h = i_avg.to(torch.float16), i_std.to(torch.float16)
-        scale = u_std_m / i_std_h
-        t.stats32 = (u_avg.contiguous(), i_avg.contiguous(), scale.float().contiguous())
+        scale, u_avg_m, i_avg_h, t.stats32 = ops.recon_scale(t.coef, L, self._book.t_x, u_avg, u_std, states.dtype)
         return scale, u_avg_m, i_avg_h
+
+    def _prompt_rows(self, layer: _Layer, key_states: torch.Tensor, value_states: torch.Tensor, slots: int, first: int, last: int,
+                     spare: int):
+        """K and V of a prompt token-major, and its first and last rows (and ``spare`` rows of zeros) in new buffers of
+        ``slots`` rows, which become the layer's ``il``."""
+        bsz, heads, q_len, head_dim = key_states.shape
+        width = heads * head_dim
+        layer.k.il, layer.v.il = near = tuple(torch.empty((bsz, slots, width), dtype=s.dtype, device=s.device)
+                                              for s in (key_states, value_states))
+        rows = ops.prompt_rows(key_states, value_states, near, first, last, spare)
+        if rows is None:
+            rows = tuple(s.permute(0, 2, 1, 3).reshape(bsz, q_len, width) for s in (key_states, value_states))
+            for dst, s in zip(near, rows):
+                dst[:, :first, :].copy_(s[:, :first, :])
+                dst[:, first: first + last, :].copy_(s[:, q_len - last:, :])
+                if spare:
+                    dst[:, first + last: first + last + spare, :].zero_()
+        return rows
 
     # -- update ------------------------------------------------------------------
     def update(self, key_states: torch.Tensor, value_states: torch.Tensor, layer_idx: int,
@@ -339,8 +378,6 @@ class DynamicCache(Cache):
         bsz, heads, q_len, head_dim = key_states.shape
         if step.action is Action.STREAM:
             return self._stream(key_states, value_states, layer_idx, step)
-        k = key_states.permute(0, 2, 1, 3).reshape(bsz, q_len, heads * head_dim)
-        v = value_states.permute(0, 2, 1, 3).reshape(bsz, q_len, heads * head_dim)
         layer = self._layers[layer_idx]
         lb = self._book.layers[layer_idx]
         if step.action in (Action.PREFILL_COMPRESS, Action.PREFILL_LOCAL):
@@ -360,13 +397,15 @@ class DynamicCache(Cache):
                 self.value_cache.append([])
             layer.version += 1
             if step.action is Action.PREFILL_COMPRESS:
-                l32 = self._lists32[layer_idx]
+                l32, pads = self._lists32[layer_idx], self._pads32[layer_idx]
                 n_f = self.maxmidstates // 2
                 hl = self._head_lists[layer_idx]
-                ks, ku, kd = self._compress_tensor(layer.k, k, l32[0], l32[1], l32[2], l32[3], hl[0], False, step.mid_rows,
-                                                   step.fft_rows, n_f)
-                vs, vu, vd = self._compress_tensor(layer.v, v, l32[4], l32[5], l32[6], l32[7], hl[1], True, step.mid_rows,
-                                                   step.fft_rows, n_f)
+                I, W = self.numinittokens, self.maxlocallen
+                k, v = self._prompt_rows(layer, key_states, value_states, I + W + 1, I, W, 1)
+                for t in (layer.k, layer.v):
+                    t.init, t.ring = t.il[:, :I, :], t.il[:, I:, :]
+                ks, ku, kd = self._compress_tensor(layer.k, k, *l32[0:4], hl[0], pads[0], False, step.mid_rows, step.fft_rows, n_f)
+                vs, vu, vd = self._compress_tensor(layer.v, v, *l32[4:8], hl[1], pads[1], True, step.mid_rows, step.fft_rows, n_f)
                 if self._tables is None and layer_idx == 0:
                     self._tables = ops.decode_tables(n_f, self.period_reconstruct, self.device)
                 layer.compressed, layer.window_only, layer.growing, layer.spare = True, False, False, self.maxlocallen
@@ -377,9 +416,9 @@ class DynamicCache(Cache):
                 layer.compressed, layer.window_only, layer.growing, layer.spare = False, True, True, 0
                 layer.n_local, layer.n_mid = q_len, 0
                 cap = q_len + max(int(self.maxnewtokens), 16)
-                for t, s in ((layer.k, k), (layer.v, v)):
-                    t.ring = torch.empty((bsz, cap, s.shape[2]), dtype=s.dtype, device=s.device)
-                    t.ring[:, :q_len, :].copy_(s)
+                k, v = self._prompt_rows(layer, key_states, value_states, cap, q_len, 0, 0)
+                for t in (layer.k, layer.v):
+                    t.ring = t.il
                     t.il, t.init, t.coef, t.mid, t.stats32 = None, None, None, None, None
                 kview, vview = self._placeholder_parts(layer_idx, bsz, heads * head_dim)
             if len(self.key_cache) <= layer_idx:
@@ -391,6 +430,8 @@ class DynamicCache(Cache):
             return local_only(k, v)
 
         if step.action is Action.APPEND_LOCAL:
+            k = key_states.permute(0, 2, 1, 3).reshape(bsz, q_len, heads * head_dim)
+            v = value_states.permute(0, 2, 1, 3).reshape(bsz, q_len, heads * head_dim)
             layer.version += 1
             if not layer.growing:
                 # a compressed layer whose mid is short: the reference concatenates onto k_local and

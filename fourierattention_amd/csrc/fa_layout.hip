@@ -225,6 +225,60 @@ __global__ __launch_bounds__(256) void append_rows_kernel(const U* __restrict__ 
   (is_v ? v_dst : k_dst)[b * dst_bs + t * dst_rs + i] = (is_v ? v : k)[b * src_bs + t * src_rs + i];
 }
 
+// The rows of a prompt: token-major copies and the near rows (sink, window, spare slot) in one pass.  A block takes 16 rows of
+// K or V; a thread moves 16 bytes at a time, neighbouring threads along a row of the copy, four loads ahead of their
+// stores.  Bound by HBM: 4 x 3001 rows of 1024 16-bit values, K and V, head-major: 22 us (4.5 TB/s) where a copy of each
+// and six small ones took 18 + 18 + 25.
+constexpr int kPromptRows = 16;
+struct PromptRowsParams {
+  const uint4 *k, *v;      // strides in pieces of 16 bytes
+  int64_t bs, hs, rs;
+  uint4 *k_tok, *v_tok, *k_near, *v_near;
+  int64_t near_bs;
+  int n_first, n_last, spare, S, heads, ppd;   // ppd: pieces of a head's row
+};
+
+__global__ __launch_bounds__(256) void prompt_rows_kernel(const PromptRowsParams p) {
+  const bool is_v = blockIdx.y != 0;
+  const int64_t b = blockIdx.z;
+  const uint4* src = (is_v ? p.v : p.k) + b * p.bs;
+  uint4* tok = is_v ? p.v_tok : p.k_tok;
+  uint4* near_rows = is_v ? p.v_near : p.k_near;
+  if (near_rows) near_rows += b * p.near_bs;
+  const int ppr = p.heads * p.ppd;   // pieces of a row
+  const int n_near = p.n_first + p.n_last;
+  // rows of the launch: with copies every row of the prompt, otherwise the near ones; behind them the row of zeros
+  const int rows = tok ? p.S : n_near;
+  const int r0 = blockIdx.x * kPromptRows, r1 = min(rows + (near_rows ? p.spare : 0), r0 + kPromptRows);
+  const int n = (r1 - r0) * ppr;
+  for (int i0 = threadIdx.x; i0 < n; i0 += 4 * 256) {
+    uint4 x[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int i = min(i0 + u * 256, n - 1), r = r0 + i / ppr, c = i % ppr, h = c / p.ppd;
+      const int s = tok ? min(r, p.S - 1) : r < p.n_first ? r : min(p.S - p.n_last + (r - p.n_first), p.S - 1);
+      x[u] = src[h * p.hs + s * p.rs + (c - h * p.ppd)];
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int i = i0 + u * 256;
+      if (i >= n) break;
+      const int r = r0 + i / ppr, c = i % ppr;
+      int slot = -1;
+      if (r >= rows) {
+        slot = n_near;
+        x[u] = uint4{0, 0, 0, 0};
+      } else if (!tok) {
+        slot = r;
+      } else {
+        tok[(b * p.S + r) * ppr + c] = x[u];
+        slot = r < p.n_first ? r : r >= p.S - p.n_last ? p.n_first + r - (p.S - p.n_last) : -1;
+      }
+      if (near_rows && slot >= 0) near_rows[(int64_t)slot * ppr + c] = x[u];
+    }
+  }
+}
+
 // Operands of a call in the types the kernels take, all in one launch: a grid row per item, items in the argument block.
 constexpr int kMaxConvert = 16;
 struct ConvertArgs { fa_convert_item item[kMaxConvert]; };
@@ -360,6 +414,33 @@ extern "C" int fa_append_rows(const void* k, const void* v, int64_t src_bs, int6
   else if (es == 4) go(uint32_t{});
   else go(uint16_t{});
   return fa_check_launch("fa_append_rows");
+}
+
+extern "C" int fa_prompt_rows(const void* k, const void* v, int64_t bs, int64_t hs, int64_t rs, void* k_tok, void* v_tok,
+                              void* k_near, void* v_near, int64_t near_bs, int n_first, int n_last, int spare, int dtype, int B,
+                              int S, int heads, int D, fa_stream_t stream) {
+  FA_REQUIRE(k && v && (!k_tok == !v_tok) && (!k_near == !v_near) && (k_tok || k_near), FA_ERR_NULL_POINTER,
+             "fa_prompt_rows: null pointer");
+  FA_REQUIRE(B > 0 && B <= 65535 && S > 0 && heads > 0 && D > 0 && n_first >= 0 && n_last >= 0 && (int64_t)n_first + n_last <= S &&
+                 (spare == 0 || spare == 1), FA_ERR_BAD_SHAPE,
+             "fa_prompt_rows: B=%d S=%d heads=%d D=%d near rows %d + %d + %d", B, S, heads, D, n_first, n_last, spare);
+  FA_REQUIRE(dtype == FA_BF16 || dtype == FA_FP16 || dtype == FA_FP32, FA_ERR_BAD_DTYPE, "fa_prompt_rows: dtype %d", dtype);
+  const int64_t es = dtype == FA_FP32 ? 4 : 2;
+  const uintptr_t ptrs = (uintptr_t)k | (uintptr_t)v | (uintptr_t)k_tok | (uintptr_t)v_tok | (uintptr_t)k_near | (uintptr_t)v_near;
+  FA_REQUIRE(((ptrs | (uint64_t)((bs | hs | rs | near_bs | D) * es)) & 15) == 0, FA_ERR_MISALIGNED,
+             "fa_prompt_rows: rows, strides and pointers must be multiples of 16 bytes");
+  const int64_t row = (int64_t)heads * D;
+  FA_REQUIRE(!k_near || near_bs >= (n_first + n_last + spare) * row, FA_ERR_BAD_SHAPE, "fa_prompt_rows: near rows overlap");
+  FA_REQUIRE(row * es / 16 * kPromptRows <= INT32_MAX - 1024, FA_ERR_UNSUPPORTED, "fa_prompt_rows: rows of %lld elements", (long long)row);
+  const int per = (int)(16 / es);
+  PromptRowsParams p{};
+  p.k = (const uint4*)k; p.v = (const uint4*)v; p.bs = bs / per; p.hs = hs / per; p.rs = rs / per;
+  p.k_tok = (uint4*)k_tok; p.v_tok = (uint4*)v_tok; p.k_near = (uint4*)k_near; p.v_near = (uint4*)v_near; p.near_bs = near_bs / per;
+  p.n_first = n_first; p.n_last = n_last; p.spare = spare; p.S = S; p.heads = heads; p.ppd = D / per;
+  const int rows = (k_tok ? S : n_first + n_last) + (k_near ? spare : 0);
+  if (rows == 0) return FA_OK;
+  prompt_rows_kernel<<<dim3(fa_cdiv(rows, kPromptRows), 2, B), 256, 0, fa_hip_stream(stream)>>>(p);
+  return fa_check_launch("fa_prompt_rows");
 }
 
 extern "C" int fa_convert(const fa_convert_item* items, int n, fa_stream_t stream) {

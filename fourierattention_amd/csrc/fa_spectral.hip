@@ -136,9 +136,19 @@ __global__ __launch_bounds__(256) void col_stats_partial_kernel(
 // block = 64 columns; sixteen waves bring in 128 splits at a time (32768 rows of column statistics are one round of loads),
 // four of them add the sums up, each a class of splits in ascending order (6.2 -> 5.0 us against four waves that load and add)
 constexpr int kFinalizeWaves = 16;
+// what else the last launch leaves where the statistics are those of a cache's reconstruction (fa_recon_scale)
+struct ScaleOut {
+  const float* u_avg;   // null: nothing
+  const float* u_dev;
+  float* scale;
+  f16_t* avg_f16;
+  void* u_avg_model;
+  f16_t* scale_model;
+  int model_dtype;
+};
 __global__ __launch_bounds__(64 * kFinalizeWaves) void stats_finalize_kernel(
     const float* __restrict__ psum, const float* __restrict__ pmax, const float* __restrict__ pmin,
-    float* __restrict__ avg, float* __restrict__ dev, int K, int Mc, int nsplit, int round_dtype) {
+    float* __restrict__ avg, float* __restrict__ dev, int K, int Mc, int nsplit, int round_dtype, const ScaleOut ex) {
   __shared__ float s_sum[kFinalizeWaves * 8][64];
   __shared__ float s_red[3][kFinalizeWaves][64];
   const int lane = threadIdx.x & 63, g = threadIdx.x >> 6;
@@ -178,8 +188,25 @@ __global__ __launch_bounds__(64 * kFinalizeWaves) void stats_finalize_kernel(
   }
   float av = sum / (float)K;
   float dv = fmaxf(mx - av, av - mn);
-  avg[(int64_t)b * Mc + m] = fa_round_through(av, round_dtype);
-  dev[(int64_t)b * Mc + m] = fa_round_through(dv, round_dtype);
+  const int64_t o = (int64_t)b * Mc + m;
+  av = fa_round_through(av, round_dtype);
+  dv = fa_round_through(dv, round_dtype);
+  avg[o] = av;
+  if (dev) dev[o] = dv;
+  if (ex.u_avg) {
+    const float ua = ex.u_avg[o];
+    float sc = ex.u_dev[o] / dv;
+    ex.avg_f16[o] = f16_t{(_Float16)av};
+    if (ex.model_dtype == FA_FP16) {   // fp16 / fp16 stays fp16
+      const _Float16 h = (_Float16)sc;
+      ex.scale_model[o] = f16_t{h};
+      sc = (float)h;
+      ((f16_t*)ex.u_avg_model)[o] = f16_t{(_Float16)ua};
+    } else if (ex.model_dtype == FA_BF16) {
+      ((bf16_t*)ex.u_avg_model)[o] = bf16_t{fa_f32_to_bf16_bits(ua)};
+    }
+    ex.scale[o] = sc;
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -328,7 +355,7 @@ int stats_splits(int K) { return K <= 0 ? 1 : fa_cdiv(K, 256); }
 
 void fa_stats_finalize_launch(const float* psum, const float* pmax, const float* pmin, float* avg, float* dev, int B, int K,
                               int Mc, int nsplit, int round_dtype, hipStream_t st) {
-  stats_finalize_kernel<<<dim3(fa_cdiv(Mc, 64), B), 64 * kFinalizeWaves, 0, st>>>(psum, pmax, pmin, avg, dev, K, Mc, nsplit, round_dtype);
+  stats_finalize_kernel<<<dim3(fa_cdiv(Mc, 64), B), 64 * kFinalizeWaves, 0, st>>>(psum, pmax, pmin, avg, dev, K, Mc, nsplit, round_dtype, ScaleOut{});
 }
 
 // ---------------------------------------------------------------------------
@@ -403,7 +430,7 @@ extern "C" int fa_mat_avg_std(const void* a, int a_dtype, int64_t a_bs, int64_t 
     default:
       FA_REQUIRE(false, FA_ERR_BAD_DTYPE, "fa_mat_avg_std: dtype %d", a_dtype);
   }
-  stats_finalize_kernel<<<dim3(fa_cdiv(Mc, 64), B), 64 * kFinalizeWaves, 0, s>>>(psum, pmax, pmin, avg, max_dev, K, Mc, nsplit, round_dtype);
+  stats_finalize_kernel<<<dim3(fa_cdiv(Mc, 64), B), 64 * kFinalizeWaves, 0, s>>>(psum, pmax, pmin, avg, max_dev, K, Mc, nsplit, round_dtype, ScaleOut{});
   return fa_check_launch("fa_mat_avg_std");
 }
 
@@ -417,10 +444,8 @@ extern "C" size_t fa_mat_fourier_avg_std_workspace_bytes(int B, int N, int Mc, i
   return a;
 }
 
-extern "C" int fa_mat_fourier_avg_std(const float* c, float* avg, float* max_dev, int B, int N, int Mc, int K,
-                                      int T, int round_dtype, void* workspace, size_t workspace_bytes,
-                                      fa_stream_t stream) {
-  FA_REQUIRE(c && avg && max_dev, FA_ERR_NULL_POINTER, "fa_mat_fourier_avg_std: null pointer");
+static int recon_stats(const float* c, float* avg, float* max_dev, int B, int N, int Mc, int K, int T, int round_dtype,
+                       const ScaleOut& ex, void* workspace, size_t workspace_bytes, fa_stream_t stream) {
   FA_REQUIRE(B > 0 && N > 0 && Mc > 0 && K > 0 && T > 0, FA_ERR_BAD_SHAPE,
              "fa_mat_fourier_avg_std: bad shape B=%d N=%d Mc=%d K=%d T=%d", B, N, Mc, K, T);
   FA_REQUIRE(workspace && workspace_bytes >= fa_stats_workspace_bytes(B, Mc, K), FA_ERR_WORKSPACE,
@@ -430,7 +455,7 @@ extern "C" int fa_mat_fourier_avg_std(const float* c, float* avg, float* max_dev
     FA_REQUIRE(((uintptr_t)workspace & 255) == 0, FA_ERR_MISALIGNED, "fa_mat_fourier_avg_std: workspace not 256-byte aligned");
     float *ps, *px, *pn;
     const int rb = fa_recon_stats_mfma_launch(c, B, N, Mc, K, T, workspace, &ps, &px, &pn, s);
-    stats_finalize_kernel<<<dim3(fa_cdiv(Mc, 64), B), 64 * kFinalizeWaves, 0, s>>>(ps, px, pn, avg, max_dev, K, Mc, rb, round_dtype);
+    stats_finalize_kernel<<<dim3(fa_cdiv(Mc, 64), B), 64 * kFinalizeWaves, 0, s>>>(ps, px, pn, avg, max_dev, K, Mc, rb, round_dtype, ex);
     return fa_check_launch("fa_mat_fourier_avg_std");
   }
   const int nsplit = stats_splits(K);
@@ -440,8 +465,26 @@ extern "C" int fa_mat_fourier_avg_std(const float* c, float* avg, float* max_dev
   constexpr int MB = 32;
   reconstruct_kernel<true, MB><<<dim3(fa_cdiv(Mc, MB), nsplit, B), 256, 0, s>>>(
       c, N, Mc, K, T, psum, pmax, pmin, nsplit, nullptr, nullptr, nullptr, nullptr);
-  stats_finalize_kernel<<<dim3(fa_cdiv(Mc, 64), B), 64 * kFinalizeWaves, 0, s>>>(psum, pmax, pmin, avg, max_dev, K, Mc, nsplit, round_dtype);
+  stats_finalize_kernel<<<dim3(fa_cdiv(Mc, 64), B), 64 * kFinalizeWaves, 0, s>>>(psum, pmax, pmin, avg, max_dev, K, Mc, nsplit, round_dtype, ex);
   return fa_check_launch("fa_mat_fourier_avg_std");
+}
+
+extern "C" int fa_mat_fourier_avg_std(const float* c, float* avg, float* max_dev, int B, int N, int Mc, int K,
+                                      int T, int round_dtype, void* workspace, size_t workspace_bytes,
+                                      fa_stream_t stream) {
+  FA_REQUIRE(c && avg && max_dev, FA_ERR_NULL_POINTER, "fa_mat_fourier_avg_std: null pointer");
+  return recon_stats(c, avg, max_dev, B, N, Mc, K, T, round_dtype, ScaleOut{}, workspace, workspace_bytes, stream);
+}
+
+extern "C" int fa_recon_scale(const float* c, const float* u_avg, const float* u_dev, float* avg, float* scale, void* avg_f16,
+                              void* u_avg_model, void* scale_model, int model_dtype, int B, int N, int Mc, int K, int T,
+                              void* workspace, size_t workspace_bytes, fa_stream_t stream) {
+  FA_REQUIRE(model_dtype == FA_BF16 || model_dtype == FA_FP16 || model_dtype == FA_FP32, FA_ERR_BAD_DTYPE, "fa_recon_scale: dtype %d",
+             model_dtype);
+  FA_REQUIRE(c && u_avg && u_dev && avg && scale && avg_f16 && (u_avg_model || model_dtype == FA_FP32) &&
+                 (scale_model || model_dtype != FA_FP16), FA_ERR_NULL_POINTER, "fa_recon_scale: null pointer");
+  const ScaleOut ex{u_avg, u_dev, scale, (f16_t*)avg_f16, u_avg_model, (f16_t*)scale_model, model_dtype};
+  return recon_stats(c, avg, nullptr, B, N, Mc, K, T, FA_FP16, ex, workspace, workspace_bytes, stream);
 }
 
 extern "C" int fa_reconstruct(const float* c, const float* avg_u, const float* avg_d, const float* scale, float* r,

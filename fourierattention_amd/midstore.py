@@ -22,16 +22,21 @@ class MidStore:
         self.B, self.Hkv, self.D, self.is_v = batch, num_kv_heads, head_dim, bool(is_v)
         self.n_list32, self.n_h32 = n_list32, n_h32
         self.Cn = int(n_h_host[-1])
+        self.pad_h_host = pad = self.padded(n_h_host, num_kv_heads, is_v)
+        self.max_pad = max([pad[h + 1] - pad[h] for h in range(num_kv_heads)] + [0])
+        self.pad_h32 = torch.tensor(pad, dtype=torch.int32, device=device) if pad_h32 is None else pad_h32
+        self.dtype, self.device = dtype, torch.device(device)
+        self._alloc(cap_tokens, zeroed)
+
+    @staticmethod
+    def padded(n_h_host: List[int], num_kv_heads: int, is_v: bool) -> List[int]:
+        """Per-head offsets of the stored dims with every head's count rounded up to whole fragments."""
         unit = V_DIM_PAD if is_v else K_DIM_PAD
         pad = [0]
         for h in range(num_kv_heads):
             n = n_h_host[h + 1] - n_h_host[h]
             pad.append(pad[-1] + (n + unit - 1) // unit * unit)
-        self.pad_h_host = pad
-        self.max_pad = max([pad[h + 1] - pad[h] for h in range(num_kv_heads)] + [0])
-        self.pad_h32 = torch.tensor(pad, dtype=torch.int32, device=device) if pad_h32 is None else pad_h32
-        self.dtype, self.device = dtype, torch.device(device)
-        self._alloc(cap_tokens, zeroed)
+        return pad
 
     def _alloc(self, cap_tokens: int, zeroed: bool = True):
         self.cap_pages = max(1, (int(cap_tokens) + PAGE_TOKENS - 1) // PAGE_TOKENS)

@@ -175,6 +175,29 @@ def mat_fourier_avg_std_triton(c: torch.Tensor, K: int, T: int):
     return _cast_pair(mat_fourier_avg_std(c.float() if c.dtype != torch.float32 else c, K, T, torch.float16), torch.float16)  # TRI:326
 
 
+def recon_scale(c: torch.Tensor, K: int, T: int, u_avg: torch.Tensor, u_dev: torch.Tensor, dtype: torch.dtype):
+    """What a cache of a ``dtype`` model keeps of a compressed tensor's statistics (cache_utils_fourier.py:567, 590), without
+    launches of its own: ``(scale, u_avg, avg_d)`` in the types the reference leaves them in - the quotient of the two
+    deviations promoted, the mean of the original in ``dtype``, that of the reconstruction in float16 - and the same three as
+    the kernels take them, float32 ``(u_avg, avg_d, scale)``.  ``u_avg, u_dev``: ``mat_avg_std(..., round_dtype=dtype)``."""
+    _require_gpu(c, "c")
+    assert c.is_contiguous() and c.dtype == torch.float32 and c.dim() == 3
+    B, N2, Mc = c.shape
+    assert all(t.is_contiguous() and t.dtype == torch.float32 and tuple(t.shape) == (B, Mc) for t in (u_avg, u_dev))
+    new = lambda dt: torch.empty((B, Mc), device=c.device, dtype=dt)
+    avg, scale, avg_h = new(torch.float32), new(torch.float32), new(torch.float16)
+    u_avg_m = u_avg if dtype == torch.float32 else new(dtype)
+    scale_m = new(torch.float16) if dtype == torch.float16 else scale
+    if Mc and B:
+        lib = _lib.load()
+        nbytes = lib.fa_mat_fourier_avg_std_workspace_bytes(B, N2 // 2, Mc, int(K))
+        ws = workspace(c.device, nbytes, "spectral")
+        check(lib.fa_recon_scale(c.data_ptr(), u_avg.data_ptr(), u_dev.data_ptr(), avg.data_ptr(), scale.data_ptr(), avg_h.data_ptr(),
+                                 u_avg_m.data_ptr(), scale_m.data_ptr(), dtype_code(dtype), B, N2 // 2, Mc, int(K), int(T),
+                                 ws.data_ptr(), int(nbytes), _stream(c.device)))
+    return scale_m, u_avg_m, avg_h, (u_avg, avg, scale)
+
+
 # ------------------------------------------------------------------ reconstruction
 def mat_fourier_inv(c: torch.Tensor, K: int, T: int, avg_u=None, avg_d=None, scale=None) -> torch.Tensor:
     """``(B, K, Mc)`` fp32 reconstruction (TRI:782-791), optionally through the affine statistics."""
@@ -223,6 +246,37 @@ def stream_update(k_new: torch.Tensor, v_new: torch.Tensor, k_ring: torch.Tensor
 def append_rows(k: torch.Tensor, v: torch.Tensor, k_dst: torch.Tensor, v_dst: torch.Tensor, pos: int) -> None:
     """Rows of K and V ``(B, rows, width)`` to rows ``pos ..`` of two buffers, in one launch."""
     _lib.load_host().append_rows(k, v, k_dst, v_dst, pos)
+
+
+def prompt_rows(k: torch.Tensor, v: torch.Tensor, near: Optional[Tuple[torch.Tensor, torch.Tensor]] = None, first: int = 0,
+                last: int = 0, spare: int = 0):
+    """The rows of a prompt, ``k, v (B, heads, S, D)``, as token-major ``(B, S, heads*D)`` tensors (the source's own memory
+    where its heads lie side by side, else copies) and, in the same launch, into ``near = (k, v)``, ``(B, slots, heads*D)``:
+    the first ``first`` rows, the last ``last``, then ``spare`` rows of zeros.  ``None`` where the layout is for tensor
+    operations: rows that are no multiples of 16 bytes, other devices, tensors that take part in a graph of gradients."""
+    B, heads, S, D = k.shape
+    es = k.element_size()
+    if (not k.is_cuda or k.device != v.device or k.shape != v.shape or k.dtype != v.dtype or k.dtype not in _DTYPE_CODE
+            or k.stride() != v.stride() or k.stride(3) != 1 or k.requires_grad or v.requires_grad or not 0 < B <= 65535 or S == 0
+            or any((s * es) % 16 for s in (*k.stride()[:3], D)) or k.data_ptr() % 16 or v.data_ptr() % 16
+            or first + last > S):
+        return None
+    if near is not None and any(t.dtype != k.dtype or t.device != k.device or t.stride(2) != 1 or t.stride(1) != heads * D
+                                or t.stride(0) != near[0].stride(0) or t.shape[1] < first + last + spare or t.data_ptr() % 16
+                                for t in near):
+        return None
+    out, tok = (k, v), (None, None)
+    if heads == 1 or k.stride(1) == D:
+        out = tuple(t.permute(0, 2, 1, 3).reshape(B, S, heads * D) for t in (k, v))
+        if near is None:
+            return out
+    else:
+        out = tok = tuple(torch.empty((B, S, heads * D), dtype=k.dtype, device=k.device) for _ in (k, v))
+    n = (None, None) if near is None else near
+    check(_lib.load().fa_prompt_rows(k.data_ptr(), v.data_ptr(), k.stride(0), k.stride(1), k.stride(2), _ptr(tok[0]), _ptr(tok[1]),
+                                     _ptr(n[0]), _ptr(n[1]), 0 if near is None else near[0].stride(0), first, last, spare,
+                                     dtype_code(k.dtype), B, S, heads, D, _stream(k.device)))
+    return out
 
 
 def add_rmsnorm(h: torch.Tensor, delta: Optional[torch.Tensor], weight: torch.Tensor, eps: float) -> torch.Tensor:

@@ -93,6 +93,16 @@ int fa_mat_fourier_avg_std(const float* c, float* avg, float* max_dev, int B, in
 size_t fa_stats_workspace_bytes(int B, int Mc, int K);
 size_t fa_mat_fourier_avg_std_workspace_bytes(int B, int N, int Mc, int K);
 
+/* What a cache keeps of a compressed tensor's statistics (CACHE:567, 590), in the launches of fa_mat_fourier_avg_std: given
+ * mean and maximum deviation of the original columns (u_avg, u_dev, fp32 holding values of model_dtype), those of the
+ * reconstruction rounded through fp16 (avg) and the quotient scale = u_dev / deviation in the type the two promote to
+ * (fp16 for an fp16 model, fp32 otherwise).  avg and scale: fp32 (B, Mc); avg_f16: avg as fp16; u_avg_model, scale_model: the
+ * same as u_avg and scale in model_dtype resp. fp16, written for 16-bit models resp. fp16 models only (may be null
+ * otherwise).  workspace as for fa_mat_fourier_avg_std. */
+int fa_recon_scale(const float* c, const float* u_avg, const float* u_dev, float* avg, float* scale, void* avg_f16,
+                   void* u_avg_model, void* scale_model, int model_dtype, int B, int N, int Mc, int K, int T, void* workspace,
+                   size_t workspace_bytes, fa_stream_t stream);
+
 /* Reconstruction r (B, K, Mc) fp32 from coefficients (mat_fourier_inv_torch,
  * TRI:782-791); with stats pointers non-NULL also applies
  * (r - avg_d) * scale + avg_u (TRI:813).  Used for validation and for
@@ -293,6 +303,15 @@ int fa_mid_pack(const void* src, int dtype, int64_t src_batch_stride, int64_t sr
 int fa_append_rows(const void* k, const void* v, int64_t src_batch_stride, int64_t src_row_stride, void* k_dst, void* v_dst,
                    int64_t dst_batch_stride, int64_t dst_row_stride, int64_t pos, int B, int rows, int width, int dtype,
                    fa_stream_t stream);
+
+/* The rows of a prompt, all in one launch: K and V (B, heads, S, D) with common strides in elements (D contiguous) to
+ * token-major rows (B, S, heads * D), dense (k_tok, v_tok; both null where the caller reads the source rows in place), and
+ * to the buffers of the rows a decode step reads at full width (k_near, v_near; both null for none), (B, slots, heads * D)
+ * dense: the first n_first rows, behind them the last n_last, then, with spare != 0, one row of zeros (slots = n_first +
+ * n_last + spare; n_first + n_last <= S).  Rows, strides and pointers must be multiples of 16 bytes. */
+int fa_prompt_rows(const void* k, const void* v, int64_t batch_stride, int64_t head_stride, int64_t row_stride, void* k_tok,
+                   void* v_tok, void* k_near, void* v_near, int64_t near_batch_stride, int n_first, int n_last, int spare,
+                   int dtype, int B, int S, int heads, int D, fa_stream_t stream);
 
 /* Small operands of a call (index lists, statistics) in the types the kernels take, all in one launch of at most 16
  * items: dst[i] = src[i] converted, for i < count; with the FA_CONVERT_PAD kinds src holds per-head offsets with the

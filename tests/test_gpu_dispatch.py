@@ -61,6 +61,47 @@ def test_reconstruction_statistics_of_signals_with_a_mean(B, L, C, N, T):
         assert torch.equal(a[whole], b[whole]) and not torch.isfinite(a[~whole]).any()
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("B,H,S,D,first,last,spare,tokens_first", [
+    (1, 1, 1, 8, 0, 1, 0, False),        # one row of one piece or two
+    (2, 8, 517, 128, 4, 500, 1, False),  # the last block of rows holds six, among them the row of zeros
+    (3, 2, 31, 64, 31, 0, 0, False),     # every row is a near one
+    (2, 8, 300, 128, 4, 64, 1, True),    # token-major already: the rows are read in place
+    (1, 5, 64, 24, 0, 0, 1, False),      # no near rows but the zeros; rows of odd widths
+])
+def test_rows_of_a_prompt(dtype, B, H, S, D, first, last, spare, tokens_first):
+    """Copies are exact: token-major rows and near rows against the tensor operations they stand for."""
+    from fourierattention_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(1)
+    make = lambda: torch.randn((B, S, H, D) if tokens_first else (B, H, S, D), generator=g, device="cuda").to(dtype)
+    k, v = ((t.transpose(1, 2) if tokens_first else t) for t in (make(), make()))
+    near = tuple(torch.full((B, first + last + spare + 3, H * D), 7.0, device="cuda", dtype=dtype) for _ in range(2))
+    got = ops.prompt_rows(k, v, near, first, last, spare)
+    for t, rows, n in zip((k, v), got, near):
+        want = t.permute(0, 2, 1, 3).reshape(B, S, H * D)
+        assert torch.equal(rows, want) and (not tokens_first or rows.data_ptr() == t.data_ptr())
+        assert torch.equal(n[:, :first], want[:, :first]) and torch.equal(n[:, first:first + last], want[:, S - last:])
+        assert (n[:, first + last:first + last + spare] == 0).all() and (n[:, first + last + spare:] == 7).all()
+    assert ops.prompt_rows(k[..., :-1], v[..., :-1]) is None                          # rows that are no multiples of 16 bytes
+    assert ops.prompt_rows(k, v.transpose(2, 3).contiguous().transpose(2, 3)) is None or S == 1 or D == 1   # strides of their own
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("B,L,C,N,T", [(2, 300, 5, 16, 400), (1, 1100, 70, 64, 1500)])   # vector kernels / matrix cores
+def test_statistics_a_cache_keeps(dtype, B, L, C, N, T):
+    """The same values, bit for bit, as the conversions and the division as tensor operations."""
+    from fourierattention_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(2)
+    x = (torch.randn((B, L, C), generator=g, device="cuda") * 3 + 1).to(dtype)
+    c = ops.mat_fourier(x, N, T)
+    u_avg, u_dev = ops.mat_avg_std(x, round_dtype=dtype)
+    i_avg, i_dev = ops.mat_fourier_avg_std(c, L, T, torch.float16)
+    scale = u_dev.to(dtype) / i_dev.to(torch.float16)
+    got = ops.recon_scale(c, L, T, u_avg, u_dev, dtype)
+    for a, b in zip((*got[:3], *got[3]), (scale, u_avg.to(dtype), i_avg.to(torch.float16), u_avg, i_avg, scale.float())):
+        assert a.dtype == b.dtype and torch.equal(a, b)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
 @pytest.mark.parametrize("B,Hq,Hkv,D,n_il,L,N,k_counts,v_counts", [
     (1, 3, 1, 128, 5, 1, 5, [127], [1]),                        # one mid row; one stored K dim, one compressed V dim

@@ -123,3 +123,15 @@ def test_rows_without_elements_are_refused():
     with pytest.raises(AssertionError):
         _lib.load_host().linear_packed(e(2, 0), e(0), 0, 16)
     assert ops.silu_mul(e(2, 0), e(2, 0)).shape == (2, 0) and ops.silu_mul(e(0, 8), e(0, 8)).shape == (0, 8)
+
+
+def test_lists_of_a_cache_in_one_tensor():
+    """Every list of the masks comes back whole, in both types, whatever its length or the type of its entries."""
+    import numpy as np
+    import torch
+    from fourierattention_amd.cache import _device_lists
+    lists = [[], [3], list(range(40)), [np.int64(5), 2 ** 31 - 1], (1, 2), [True, -4]]
+    for got, want in ((_device_lists(lists, torch.device("cpu")), lists), (_device_lists([[1.5, 2]], torch.device("cpu")), [[1, 2]])):
+        for tensors, dt in zip(got, (torch.int64, torch.int32)):
+            assert [t.tolist() for t in tensors] == [[int(x) for x in lst] for lst in want]
+            assert all(t.dtype == dt and t.is_contiguous() and t.storage_offset() % 32 == 0 for t in tensors)
