@@ -5,6 +5,7 @@
 // except where a reduction order or an exponential differs in the last place.
 #include "fa_common.h"
 #include "fa_mfma_util.h"
+#include <type_traits>
 
 namespace {
 
@@ -186,19 +187,23 @@ __global__ __launch_bounds__(256) void linear_pack_kernel(const E* __restrict__ 
 
 // The elementwise steps either side of a projection ride in its launch, with the values rounded where the launches of their
 // own round them:
-//   NORM       x is the residual stream: every workgroup normalises its rows for itself, behind the requests for its first
-//              weights (RMSNorm, modeling_llama_fourier.py:87-92).  The rows then come from LDS.
+//   NORM       x is the residual stream: every workgroup normalises its rows for itself (RMSNorm,
+//              modeling_llama_fourier.py:87-92), NORM pieces of eight elements a thread, while its first weights are on
+//              their way.  The rows and the norm's weight are requested in front of those: loads return in order, and behind
+//              them the rows arrived with the last of two thirds of the weights, the memory then idle through the norm.
+//              The rows then come from LDS.
 //   EPI_ADD    out is the residual stream: out += product, in place (735-750); every element has one owner.
 //   EPI_GATE   the weight holds the gate rows and, behind them, the up rows: a workgroup owns a tile of both and stores
 //              silu(gate) * up (277).
-// A launch of their own took 5 us each for a row or two, a chain of one load, one reduction and one store, and the weights
-// wait meanwhile.  One layer of the 8B decoder at one row: 90 -> 84 us of kernels and three
-// launches less (1371 -> 1337 us for a step of eight layers at 32k tokens).
+// A launch of their own takes 5 us each for a row or two, a chain of one load, one reduction and one store, and the weights
+// wait meanwhile.  Bound by HBM: gate / up of the 8B decoder at one row 39.0 us (6.0 TB/s), of the 3B one at two rows 19.1
+// (5.3 TB/s); 43.8 and 23.3 while the rows were requested behind the weights and the gated instances took 136 registers, one
+// workgroup per compute unit instead of the two that four waves per SIMD allow.
 enum LinearEpilogue { EPI_STORE = 0, EPI_ADD = 1, EPI_GATE = 2 };
 constexpr int kLinNormElems = 16384;    // elements of the normalised rows a workgroup keeps (32 KB: four workgroups fit a CU)
 
-template <typename E, bool NORM, int EPI>
-__global__ __launch_bounds__(64 * kLinWaves) void linear_packed_kernel(const E* x, int64_t x_rs, const E* __restrict__ norm_w,
+template <typename E, int NORM, int EPI>
+__global__ __launch_bounds__(64 * kLinWaves, NORM > 0 ? 4 : 2) void linear_packed_kernel(const E* x, int64_t x_rs, const E* __restrict__ norm_w,
                                                                         float eps, const E* __restrict__ wp, E* out,
                                                                         int rows, int K, int n_out) {
   using M = fa_mfma::Mma<E>;
@@ -211,7 +216,7 @@ __global__ __launch_bounds__(64 * kLinWaves) void linear_packed_kernel(const E* 
   extern __shared__ float4v s_dyn[];
   E* s_x = (E*)s_dyn;
   auto s_part = (float4v(*)[T][64])s_dyn;
-  __shared__ float s_sq[NORM ? 16 : 1][kLinWaves];
+  __shared__ float s_sq[NORM ? NORM * kLinWaves : 1];   // sums of squares of 64 pieces, one after the other
   const int tid = threadIdx.x, lane = tid & 63, lg = lane >> 4, lc = lane & 15;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int tile = blockIdx.x, tiles = gridDim.x;              // the up tile of a gate tile lies `tiles` further on
@@ -248,44 +253,52 @@ __global__ __launch_bounds__(64 * kLinWaves) void linear_packed_kernel(const E* 
       }
     }
   };
-  load_w(0, A0);
-  if constexpr (NORM) {
+  if constexpr (NORM > 0) {
+    const int packs = K >> 3, total = rows * packs;            // packs is a multiple of 128: a wave's pieces lie in one row
+    Pack v[NORM], nw[NORM];
+    int row[NORM];
+#pragma unroll
+    for (int j = 0; j < NORM; ++j) {
+      const int i0 = (w + j * kLinWaves) * 64;                 // the wave's first piece (uniform)
+      row[j] = i0 < total ? i0 / packs : 0;
+      const int i = i0 < total ? i0 - row[j] * packs + lane : lane;
+      v[j] = *(const Pack*)(x + row[j] * x_rs + i * 8);
+      nw[j] = *(const Pack*)(norm_w + i * 8);
+    }
+    asm volatile("" ::: "memory");   // (in this order)
+    load_w(0, A0);
     if (n_groups > 1) load_w(1, A1);
-    const int packs = K >> 3;
-    for (int r = 0; r < rows; ++r) {
-      float ss = 0.f;
-      for (int i = tid; i < packs; i += 64 * kLinWaves) {
-        const Pack v = *(const Pack*)(x + r * x_rs + i * 8);
-        *(Pack*)&s_x[r * pitch + i * 8] = v;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const float f = fa_to_float(v.e[e]);
-          ss += f * f;
-        }
+    for (int j = 0; j < NORM; ++j) {
+      float ss = 0.f;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float f = fa_to_float(v[j].e[e]);
+        ss += f * f;
       }
-      ss = fa_wave_sum(ss);
-      if (lane == 0) s_sq[r][w] = ss;
+      ss = fa_rows_sum(fa_group_sum<16>(ss));
+      if (lane == 0) s_sq[j * kLinWaves + w] = ss;
     }
     __syncthreads();
-    for (int r = 0; r < rows; ++r) {
-      float ss = 0.f;
+    const int per_row = packs >> 6;
 #pragma unroll
-      for (int i = 0; i < kLinWaves; ++i) ss += s_sq[r][i];
+    for (int j = 0; j < NORM; ++j) {
+      if (tid + j * 64 * kLinWaves >= total) break;
+      float ss = 0.f;
+      for (int i = 0; i < per_row; ++i) ss += s_sq[row[j] * per_row + i];
       const float inv = rsqrtf(ss / (float)K + eps);
-      for (int i = tid; i < packs; i += 64 * kLinWaves) {   // the pieces this thread put there
-        Pack v = *(Pack*)&s_x[r * pitch + i * 8];
-        const Pack g = *(const Pack*)(norm_w + i * 8);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) v.e[e] = Rounder<E>::put(fa_to_float(g.e[e]) * rnd<E>(fa_to_float(v.e[e]) * inv));
-        *(Pack*)&s_x[r * pitch + i * 8] = v;
-      }
+      for (int e = 0; e < 8; ++e) v[j].e[e] = Rounder<E>::put(fa_to_float(nw[j].e[e]) * rnd<E>(fa_to_float(v[j].e[e]) * inv));
+      *(Pack*)&s_x[row[j] * pitch + (tid + j * 64 * kLinWaves - row[j] * packs) * 8] = v[j];
     }
     __syncthreads();
+  } else {
+    load_w(0, A0);
   }
   load_x(0, B0);
   for (int g = 0; g < n_groups; g += 2) {
     if (g + 1 < n_groups) {
-      if (!NORM || g > 0) load_w(g + 1, A1);
+      if (NORM == 0 || g > 0) load_w(g + 1, A1);
       load_x(g + 1, B1);
     }
     compute(A0, B0);
@@ -295,7 +308,7 @@ __global__ __launch_bounds__(64 * kLinWaves) void linear_packed_kernel(const E* 
     }
     if (g + 1 < n_groups) compute(A1, B1);
   }
-  if (NORM) __syncthreads();
+  if (NORM > 0) __syncthreads();
 #pragma unroll
   for (int t = 0; t < T; ++t) s_part[w][t][lane] = acc0[t] + acc1[t];
   __syncthreads();
@@ -452,15 +465,18 @@ extern "C" int fa_linear_packed_step(const void* x, int64_t x_row_stride, const 
         kernel<<<grid, 64 * kLinWaves, sums > x_bytes ? sums : x_bytes, st>>>((const E*)x, x_row_stride, (const E*)norm_weight, eps, (const E*)w_packed, (E*)out,
                                                 rows, K, n_out);
       };
-      if (norm_weight) {
-        if (epilogue == EPI_GATE) go(linear_packed_kernel<E, true, EPI_GATE>);
-        else if (epilogue == EPI_ADD) go(linear_packed_kernel<E, true, EPI_ADD>);
-        else go(linear_packed_kernel<E, true, EPI_STORE>);
-      } else {
-        if (epilogue == EPI_GATE) go(linear_packed_kernel<E, false, EPI_GATE>);
-        else if (epilogue == EPI_ADD) go(linear_packed_kernel<E, false, EPI_ADD>);
-        else go(linear_packed_kernel<E, false, EPI_STORE>);
-      }
+      auto by_epilogue = [&](auto pieces) {   // pieces of the rows a thread normalises
+        constexpr int P = decltype(pieces)::value;
+        if (epilogue == EPI_GATE) go(linear_packed_kernel<E, P, EPI_GATE>);
+        else if (epilogue == EPI_ADD) go(linear_packed_kernel<E, P, EPI_ADD>);
+        else go(linear_packed_kernel<E, P, EPI_STORE>);
+      };
+      const int64_t per_piece = 8 * 64 * kLinWaves;
+      static_assert(kLinNormElems == 4 * 8 * 64 * kLinWaves, "at most four pieces a thread");
+      if (!norm_weight) by_epilogue(std::integral_constant<int, 0>{});
+      else if ((int64_t)rows * K <= per_piece) by_epilogue(std::integral_constant<int, 1>{});
+      else if ((int64_t)rows * K <= 2 * per_piece) by_epilogue(std::integral_constant<int, 2>{});
+      else by_epilogue(std::integral_constant<int, 4>{});
     }
   });
   return fa_check_launch("fa_linear_packed");

@@ -78,11 +78,11 @@ class LlamaMLP(nn.Module):
         return self.down_proj(F.silu(self.gate_proj(x)) * self.up_proj(x))
 
 
-# Elements of a decode step's rows up to which the RMSNorm rides in the projection behind it.  Every workgroup of that launch
-# normalises all rows, one after the other; a launch of its own does them side by side.  A step of four layers at 2200 tokens,
-# in the projections / apart, us: 4096 wide 1 row 742 / 757, 2 rows 810 / 794, 4 rows 883 / 813; 3072 wide 1 row 562 / 578,
-# 2 rows 606 / 610, 3 rows 619 / 598, 5 rows 669 / 616.
-_NORM_IN_PROJECTION = 6144
+# Rows of a decode step, and elements of them, up to which the RMSNorm rides in the projection behind it.  Every workgroup of
+# that launch normalises all rows; a launch of its own does them once.  q/k/v, gate/up and down of a layer, in the projections /
+# apart, us: 4096 wide 1 row 70.1 / 75.9, 2 rows 71.6 / 76.0, 3 rows 75.6 / 75.8, 4 rows 75.7 / 75.8; 3072 wide 1 row
+# 39.0 / 44.7, 3 rows 42.1 / 45.2, 4 rows 43.6 / 43.7, 5 rows 45.3 / 44.2.
+_NORM_ROWS, _NORM_IN_PROJECTION = 3, 12288
 
 
 class LlamaDecoderLayer(nn.Module):
@@ -166,7 +166,7 @@ class LlamaDecoderLayer(nn.Module):
         Returns this layer's MLP output, to be added by whoever normalises next (``None``: ``h`` has it already)."""
         at = self.self_attn
         bsz, q_len, width = h.shape
-        norm_rides = bsz * q_len * width <= _NORM_IN_PROJECTION
+        norm_rides = bsz * q_len <= _NORM_ROWS and bsz * q_len * width <= _NORM_IN_PROJECTION
         nq, nk = at.num_heads * at.head_dim, at.num_key_value_heads * at.head_dim
         pk = self._packed_weight("qkv")
         norm = self.input_layernorm
