@@ -111,6 +111,7 @@ _SIGNATURES = {
     "fa_linear_packed_norm_ok": (c_int, [c_int, c_int]),
     "fa_linear_packed_step": (c_int, [c_void_p, c_int64, c_void_p, c_float, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int,
                                       c_void_p]),
+    "fa_linear_packed_qkv": (c_int, [c_void_p, c_int64, c_void_p, c_float] + [c_void_p] * 5 + [c_int] * 6 + [c_void_p]),
     "fa_decode_split_plan": (c_int, [c_int] * 7 + [c_void_p, c_void_p, c_void_p, c_void_p]),
     "fa_decode_tables_bytes": (c_size_t, [c_int]),
     "fa_decode_tables_build": (c_int, [c_void_p, c_size_t, c_int, c_int, c_void_p]),

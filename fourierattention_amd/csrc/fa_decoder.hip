@@ -195,17 +195,28 @@ __global__ __launch_bounds__(256) void linear_pack_kernel(const E* __restrict__ 
 //   EPI_ADD    out is the residual stream: out += product, in place (735-750); every element has one owner.
 //   EPI_GATE   the weight holds the gate rows and, behind them, the up rows: a workgroup owns a tile of both and stores
 //              silu(gate) * up (277).
+//   EPI_ROPE   the weight holds the q, k and v rows of an attention layer, those of q and k so that the sixteen of a tile are
+//              eight of the first half of a head and the eight they turn with, D / 2 further on: the rotary embedding
+//              (213-244) is an exchange between the two halves of the wave that adds the sums up.  Columns go out in their
+//              natural order.  As a launch of its own it took 2.7 - 3.9 us and the gap in front of it.
 // A launch of their own takes 5 us each for a row or two, a chain of one load, one reduction and one store, and the weights
 // wait meanwhile.  Bound by HBM: gate / up of the 8B decoder at one row 39.0 us (6.0 TB/s), of the 3B one at two rows 19.1
 // (5.3 TB/s); 43.8 and 23.3 while the rows were requested behind the weights and the gated instances took 136 registers, one
 // workgroup per compute unit instead of the two that four waves per SIMD allow.
-enum LinearEpilogue { EPI_STORE = 0, EPI_ADD = 1, EPI_GATE = 2 };
+enum LinearEpilogue { EPI_STORE = 0, EPI_ADD = 1, EPI_GATE = 2, EPI_ROPE = 3 };
+template <typename E>
+struct RopeOut {   // EPI_ROPE: q goes to out, dense
+  const E* cos;    // one row of D per row of x
+  const E* sin;
+  E* kv;           // (rows, k then v)
+  int nq, nqk, D;  // columns of q, of q and k
+};
 constexpr int kLinNormElems = 16384;    // elements of the normalised rows a workgroup keeps (32 KB: four workgroups fit a CU)
 
 template <typename E, int NORM, int EPI>
 __global__ __launch_bounds__(64 * kLinWaves, NORM > 0 ? 4 : 2) void linear_packed_kernel(const E* x, int64_t x_rs, const E* __restrict__ norm_w,
                                                                         float eps, const E* __restrict__ wp, E* out,
-                                                                        int rows, int K, int n_out) {
+                                                                        int rows, int K, int n_out, const RopeOut<E> ro) {
   using M = fa_mfma::Mma<E>;
   using vec8 = typename M::vec8;
   using fa_mfma::float4v;
@@ -322,6 +333,29 @@ __global__ __launch_bounds__(64 * kLinWaves, NORM > 0 ? 4 : 2) void linear_packe
     }
     // lane (lg, lc) holds the output features 4 lg .. 4 lg + 3 of the tile for row lc
     struct alignas(sizeof(E) * 4) Quad { E e[4]; } o;
+    if constexpr (EPI == EPI_ROPE) {
+      const int f0 = tile * 16;
+      int f = f0 + 4 * lg;   // this lane's first column
+      if (f0 < ro.nqk) {
+        const int head = f0 / ro.D, half = ro.D >> 1;
+        const int d = ((f0 - head * ro.D) >> 1) + 4 * (lg & 1) + (lg >> 1) * half;
+        f = head * ro.D + d;
+        const Quad c = *(const Quad*)(ro.cos + (int64_t)lc * ro.D + d), sn = *(const Quad*)(ro.sin + (int64_t)lc * ro.D + d);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          float x1, x2;   // of the first half, of the second
+          fa_swap32(rnd<E>(s[0][e]), &x1, &x2);
+          const float own = lg < 2 ? x1 : x2, other = lg < 2 ? -x2 : x1;
+          o.e[e] = Rounder<E>::put(rnd<E>(own * fa_to_float(c.e[e])) + rnd<E>(other * fa_to_float(sn.e[e])));
+        }
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o.e[e] = Rounder<E>::put(s[0][e]);
+      }
+      if (f < ro.nq) *(Quad*)(out + (int64_t)lc * ro.nq + f) = o;
+      else *(Quad*)(ro.kv + (int64_t)lc * (n_out - ro.nq) + f - ro.nq) = o;
+      return;
+    }
     const int width = EPI == EPI_GATE ? n_out >> 1 : n_out;
     Quad* dst = (Quad*)(out + (int64_t)lc * width + tile * 16 + 4 * lg);
     if constexpr (EPI == EPI_ADD) o = *dst;
@@ -438,9 +472,10 @@ extern "C" int fa_linear_packed_ok(int rows, int K, int n_out) {
 
 extern "C" int fa_linear_packed_norm_ok(int rows, int K) { return rows >= 1 && rows <= 16 && (int64_t)rows * K <= kLinNormElems; }
 
-extern "C" int fa_linear_packed_step(const void* x, int64_t x_row_stride, const void* norm_weight, float eps,
-                                     const void* w_packed, void* out, int rows, int K, int n_out, int epilogue, int dtype,
-                                     fa_stream_t stream) {
+namespace {
+struct RopeCall { const void *cos, *sin; void* kv; int nq, nqk, D; };
+int linear_packed(const void* x, int64_t x_row_stride, const void* norm_weight, float eps, const void* w_packed, void* out,
+                  int rows, int K, int n_out, int epilogue, int dtype, const RopeCall& rc, fa_stream_t stream) {
   FA_REQUIRE(x && w_packed && out, FA_ERR_NULL_POINTER, "fa_linear_packed: null pointer");
   FA_REQUIRE(fa_linear_packed_ok(rows, K, n_out), FA_ERR_UNSUPPORTED,
              "fa_linear_packed: rows=%d (1..16) K=%d (multiple of %d) n_out=%d (multiple of 16)", rows, K,
@@ -449,8 +484,7 @@ extern "C" int fa_linear_packed_step(const void* x, int64_t x_row_stride, const 
   FA_REQUIRE(x_row_stride >= K && x_row_stride % 8 == 0 &&
                  (((uintptr_t)x | (uintptr_t)w_packed | (uintptr_t)out | (uintptr_t)norm_weight) & 15) == 0,
              FA_ERR_MISALIGNED, "fa_linear_packed: rows of x / pointers not 16-byte aligned");
-  FA_REQUIRE(epilogue >= EPI_STORE && epilogue <= EPI_GATE && (epilogue != EPI_GATE || n_out % 32 == 0), FA_ERR_UNSUPPORTED,
-             "fa_linear_packed: epilogue %d, n_out=%d", epilogue, n_out);
+  FA_REQUIRE(epilogue != EPI_GATE || n_out % 32 == 0, FA_ERR_UNSUPPORTED, "fa_linear_packed: epilogue %d, n_out=%d", epilogue, n_out);
   FA_REQUIRE(!norm_weight || fa_linear_packed_norm_ok(rows, K), FA_ERR_UNSUPPORTED,
              "fa_linear_packed: %d rows of %d are more than a workgroup normalises for itself", rows, K);
   FA_REQUIRE(epilogue != EPI_ADD || x != out, FA_ERR_BAD_SHAPE, "fa_linear_packed: the rows added to are the input");
@@ -463,11 +497,12 @@ extern "C" int fa_linear_packed_step(const void* x, int64_t x_row_stride, const 
       const size_t x_bytes = norm_weight ? (size_t)rows * (K + 8) * 2 : 0;
       auto go = [&](auto kernel) {
         kernel<<<grid, 64 * kLinWaves, sums > x_bytes ? sums : x_bytes, st>>>((const E*)x, x_row_stride, (const E*)norm_weight, eps, (const E*)w_packed, (E*)out,
-                                                rows, K, n_out);
+                                                rows, K, n_out, RopeOut<E>{(const E*)rc.cos, (const E*)rc.sin, (E*)rc.kv, rc.nq, rc.nqk, rc.D});
       };
       auto by_epilogue = [&](auto pieces) {   // pieces of the rows a thread normalises
         constexpr int P = decltype(pieces)::value;
-        if (epilogue == EPI_GATE) go(linear_packed_kernel<E, P, EPI_GATE>);
+        if (epilogue == EPI_ROPE) go(linear_packed_kernel<E, P, EPI_ROPE>);
+        else if (epilogue == EPI_GATE) go(linear_packed_kernel<E, P, EPI_GATE>);
         else if (epilogue == EPI_ADD) go(linear_packed_kernel<E, P, EPI_ADD>);
         else go(linear_packed_kernel<E, P, EPI_STORE>);
       };
@@ -480,6 +515,26 @@ extern "C" int fa_linear_packed_step(const void* x, int64_t x_row_stride, const 
     }
   });
   return fa_check_launch("fa_linear_packed");
+}
+}  // namespace
+
+extern "C" int fa_linear_packed_step(const void* x, int64_t x_row_stride, const void* norm_weight, float eps,
+                                     const void* w_packed, void* out, int rows, int K, int n_out, int epilogue, int dtype,
+                                     fa_stream_t stream) {
+  FA_REQUIRE(epilogue >= EPI_STORE && epilogue <= EPI_GATE, FA_ERR_UNSUPPORTED, "fa_linear_packed: epilogue %d, n_out=%d", epilogue, n_out);
+  return linear_packed(x, x_row_stride, norm_weight, eps, w_packed, out, rows, K, n_out, epilogue, dtype, RopeCall{}, stream);
+}
+
+extern "C" int fa_linear_packed_qkv(const void* x, int64_t x_row_stride, const void* norm_weight, float eps, const void* w_packed,
+                                    const void* cos, const void* sin, void* q, void* kv, int rows, int K, int Hq, int Hkv, int D,
+                                    int dtype, fa_stream_t stream) {
+  FA_REQUIRE(cos && sin && q && kv, FA_ERR_NULL_POINTER, "fa_linear_packed_qkv: null pointer");
+  FA_REQUIRE(Hq > 0 && Hkv > 0 && D > 0 && D % 16 == 0 && ((int64_t)Hq + 2 * Hkv) * D <= INT32_MAX, FA_ERR_BAD_SHAPE,
+             "fa_linear_packed_qkv: Hq=%d Hkv=%d D=%d (a multiple of 16)", Hq, Hkv, D);
+  FA_REQUIRE((((uintptr_t)cos | (uintptr_t)sin | (uintptr_t)q | (uintptr_t)kv) & 15) == 0, FA_ERR_MISALIGNED,
+             "fa_linear_packed_qkv: pointers not 16-byte aligned");
+  return linear_packed(x, x_row_stride, norm_weight, eps, w_packed, q, rows, K, (Hq + 2 * Hkv) * D, EPI_ROPE, dtype,
+                       RopeCall{cos, sin, kv, Hq * D, (Hq + Hkv) * D, D}, stream);
 }
 
 extern "C" int fa_linear_packed(const void* x, int64_t x_row_stride, const void* w_packed, void* out, int rows, int K,

@@ -454,6 +454,46 @@ PyObject* linear_packed(PyObject*, PyObject* const* a, Py_ssize_t n) {
   FA_END
 }
 
+// linear_packed_qkv(x (B, q_len, k), packed weight, norm weight or None, eps, cos, sin, Hq, Hkv, D) -> q, k, v (B, heads, q_len, D)
+PyObject* linear_packed_qkv(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  FA_BEGIN
+  CHECK(n == 9, "linear_packed_qkv takes 9 arguments");
+  const at::Tensor &x = gpu_tensor(a[0], "x"), &w = gpu_tensor(a[1], "weight"), &cos = gpu_tensor(a[4], "cos"), &sin = gpu_tensor(a[5], "sin");
+  const int64_t Hq = integer(a[6]), Hkv = integer(a[7]), D = integer(a[8]);
+  CHECK(x.dim() == 3 && x.scalar_type() == w.scalar_type() && x.size(2) > 0 && Hq > 0 && Hkv > 0 && D > 0 && w.numel() == x.size(2) * (Hq + 2 * Hkv) * D,
+        "linear_packed_qkv: x (B, q_len, k) does not fit the weight");
+  const int64_t B = x.size(0), q_len = x.size(1), k = x.size(2), rows = B * q_len;
+  for (const at::Tensor* t : {&cos, &sin})
+    CHECK(t->is_contiguous() && t->scalar_type() == x.scalar_type() && (B == 1 ? t->numel() >= rows * D : t->numel() == rows * D), "linear_packed_qkv: one row of cos and sin per token, of the type of x");
+  const void* norm = nullptr;
+  if (a[2] != Py_None) {
+    const at::Tensor& nw = gpu_tensor(a[2], "norm weight");
+    CHECK(nw.scalar_type() == x.scalar_type() && nw.is_contiguous() && nw.numel() == k, "linear_packed_qkv: the norm weight must match the rows of x");
+    norm = nw.data_ptr();
+  }
+  const float eps = (float)real(a[3]);
+  const int64_t stride = row_stride(x);
+  const int dtype = dtype_code(x);
+  const fa_stream_t st = stream_of(x);
+  at::Tensor q, kv;
+  unlocked([&] {
+    q = at::empty({B, q_len, Hq, D}, x.options());
+    kv = at::empty({B, q_len, 2 * Hkv, D}, x.options());
+    return 0;
+  });
+  LAUNCH(fa_linear_packed_qkv(x.data_ptr(), stride, norm, eps, w.data_ptr(), cos.data_ptr(), sin.data_ptr(), q.data_ptr(), kv.data_ptr(),
+                              (int)rows, (int)k, (int)Hq, (int)Hkv, (int)D, dtype, st));
+  const auto heads = kv.transpose(1, 2);
+  PyObject* out[3] = {THPVariable_Wrap(q.transpose(1, 2)), THPVariable_Wrap(heads.narrow(1, 0, Hkv)), THPVariable_Wrap(heads.narrow(1, Hkv, Hkv))};
+  PyObject* t = PyTuple_New(3);
+  for (int i = 0; i < 3; ++i) {
+    if (t && out[i]) PyTuple_SET_ITEM(t, i, out[i]);
+    else { Py_CLEAR(t); Py_XDECREF(out[i]); }
+  }
+  return t;
+  FA_END
+}
+
 // silu_mul(gate, up) -> dense
 PyObject* silu_mul(PyObject*, PyObject* const* a, Py_ssize_t n) {
   FA_BEGIN
@@ -643,7 +683,7 @@ PyObject* init(PyObject*, PyObject* const* a, Py_ssize_t n) {
 }
 
 #define FN(name) {#name, (PyCFunction)(void*)name, METH_FASTCALL, nullptr}
-PyMethodDef methods[] = {FN(init), FN(layout), FN(stream_update), FN(decode_attn), FN(add_rmsnorm), FN(linear_packed), FN(silu_mul), FN(rope_qk), FN(operands), FN(append_rows),
+PyMethodDef methods[] = {FN(init), FN(layout), FN(stream_update), FN(decode_attn), FN(add_rmsnorm), FN(linear_packed), FN(linear_packed_qkv), FN(silu_mul), FN(rope_qk), FN(operands), FN(append_rows),
                          {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_fa_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 

@@ -93,6 +93,7 @@ class LlamaDecoderLayer(nn.Module):
         self.input_layernorm = LlamaRMSNorm(config.hidden_size, config.rms_norm_eps)
         self.post_attention_layernorm = LlamaRMSNorm(config.hidden_size, config.rms_norm_eps)
         self._qkv_weight = self._gate_up_weight = None
+        self._rotary_rides = False
         self._packed = {}   # "qkv", "o", "gate_up", "down" -> ops.PackedLinearWeight (decode steps of at most 16 rows)
 
     def pack_projections(self):
@@ -110,6 +111,10 @@ class LlamaDecoderLayer(nn.Module):
             if n_out % 16 or k % 1024:
                 continue
             fused = mods[0].weight.data if len(mods) == 1 else torch.cat([m.weight.data for m in mods], dim=0)
+            # (the rotary embedding rides in the launch of q/k/v, sixteen dims of a head at a time)
+            self._rotary_rides = at.head_dim % 16 == 0
+            if name == "qkv" and self._rotary_rides:
+                fused = fused[ops.rotary_pairs(n_out, at.num_heads + at.num_key_value_heads, at.head_dim, fused.device)]
             self._packed[name] = ops.PackedLinearWeight(fused.contiguous(), sources=[m.weight for m in mods])
 
     def _packed_weight(self, name):
@@ -170,21 +175,25 @@ class LlamaDecoderLayer(nn.Module):
         nq, nk = at.num_heads * at.head_dim, at.num_key_value_heads * at.head_dim
         pk = self._packed_weight("qkv")
         norm = self.input_layernorm
-        if norm_rides and delta is None and pk is not None and pk.covers(h) and pk.normalises(h, norm.weight):
-            q, k, v = ops.linear_packed_step(h, pk, norm.weight, norm.variance_epsilon).split((nq, nk, nk), dim=-1)
+        cos, sin = position_embeddings
+        rides = norm_rides and delta is None and pk is not None and pk.covers(h) and pk.normalises(h, norm.weight)
+        y = h if rides else ops.add_rmsnorm(h, delta, norm.weight, norm.variance_epsilon)
+        if pk is not None and pk.covers(y) and self._rotary_rides:
+            q, k, v = ops.linear_packed_qkv(y, pk, norm.weight if rides else None, norm.variance_epsilon, cos, sin, at.num_heads,
+                                            at.num_key_value_heads, at.head_dim)
         else:
-            y = ops.add_rmsnorm(h, delta, norm.weight, norm.variance_epsilon)
-            if pk is not None and pk.covers(y):
+            if rides:
+                q, k, v = ops.linear_packed_step(h, pk, norm.weight, norm.variance_epsilon).split((nq, nk, nk), dim=-1)
+            elif pk is not None and pk.covers(y):
                 q, k, v = ops.linear_packed(y, pk).split((nq, nk, nk), dim=-1)
             elif self._qkv_weight is not None:
                 q, k, v = F.linear(y, self._qkv_weight).split((nq, nk, nk), dim=-1)
             else:
                 q, k, v = at.q_proj(y), at.k_proj(y), at.v_proj(y)
-        cos, sin = position_embeddings
-        q = ops.rope_qk(q, k, cos, sin, at.head_dim)
-        split = lambda t, n: t.view(bsz, q_len, n, at.head_dim).transpose(1, 2)
-        o = fourier_attention(split(q, at.num_heads), split(k, at.num_key_value_heads), split(v, at.num_key_value_heads),
-                              past_key_value, at.layer_idx, at.num_heads, at.num_key_value_heads,
+            q = ops.rope_qk(q, k, cos, sin, at.head_dim)
+            split = lambda t, n: t.view(bsz, q_len, n, at.head_dim).transpose(1, 2)
+            q, k, v = split(q, at.num_heads), split(k, at.num_key_value_heads), split(v, at.num_key_value_heads)
+        o = fourier_attention(q, k, v, past_key_value, at.layer_idx, at.num_heads, at.num_key_value_heads,
                               {"sin": sin, "cos": cos, "cache_position": cache_position})
         delta = self._linear("o", o, at.o_proj, onto=h)
         pk = self._packed_weight("gate_up")

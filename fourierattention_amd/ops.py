@@ -285,14 +285,19 @@ def add_rmsnorm(h: torch.Tensor, delta: Optional[torch.Tensor], weight: torch.Te
     return _lib.load_host().add_rmsnorm(h, delta, weight, eps)
 
 
+def _rotary_tables(cos: torch.Tensor, sin: torch.Tensor, x: torch.Tensor):
+    if cos.shape[0] != x.shape[0]:
+        cos, sin = cos.expand(x.shape[0], -1, -1), sin.expand(x.shape[0], -1, -1)
+    if cos.dtype != x.dtype or sin.dtype != x.dtype or not (cos.is_contiguous() and sin.is_contiguous()):
+        cos, sin = cos.to(x.dtype).contiguous(), sin.to(x.dtype).contiguous()
+    return cos, sin
+
+
 def rope_qk(q: torch.Tensor, k: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, head_dim: int) -> torch.Tensor:
     """Rotary embedding of ``q (B, q_len, Hq*D)`` and ``k (B, q_len, Hkv*D)`` (the projection outputs, possibly
     column slices of one fused projection output); ``cos, sin (B or 1, q_len, D)`` (modeling_llama_fourier.py:213-244).
     ``k`` is rotated in place; the rotated ``q`` is returned densely packed (``q`` itself when it was dense)."""
-    if cos.shape[0] != q.shape[0]:
-        cos, sin = cos.expand(q.shape[0], -1, -1), sin.expand(q.shape[0], -1, -1)
-    if cos.dtype != q.dtype or sin.dtype != q.dtype or not (cos.is_contiguous() and sin.is_contiguous()):
-        cos, sin = cos.to(q.dtype).contiguous(), sin.to(q.dtype).contiguous()
+    cos, sin = _rotary_tables(cos, sin, q)
     return _lib.load_host().rope_qk(q, k, cos, sin, head_dim)
 
 
@@ -368,6 +373,22 @@ def linear_packed_step(x: torch.Tensor, w: PackedLinearWeight, norm: Optional[to
     ``residual (..., n_out)``, which the product is added to in place (and which is returned); ``gated``, a weight of gate
     and then up rows (``n_out`` a multiple of 32), ``silu(gate) * up`` is returned (modeling_llama_fourier.py:87-92, 277, 735-750)."""
     return _lib.load_host().linear_packed(x, w.data, w.k, w.n_out, norm, eps, residual, gated)
+
+
+def rotary_pairs(rows: int, heads: int, head_dim: int, device) -> torch.Tensor:
+    """The order of a q/k/v weight's rows that ``linear_packed_qkv`` takes: in the first ``heads`` heads (q and k) eight rows of
+    the first half of the head and the eight they turn with side by side, the rest as they are."""
+    turned = torch.arange(heads * head_dim, device=device).view(heads, 2, head_dim // 16, 8).transpose(1, 2).reshape(-1)
+    return torch.cat([turned, torch.arange(heads * head_dim, rows, device=device)])
+
+
+def linear_packed_qkv(x: torch.Tensor, w: PackedLinearWeight, norm: Optional[torch.Tensor], eps: float, cos: torch.Tensor,
+                      sin: torch.Tensor, num_heads: int, num_kv_heads: int, head_dim: int):
+    """q, k and v of a decode step, ``(B, heads, q_len, head_dim)`` views, from ``x (B, q_len, hidden)``: RMSNorm in front
+    (``norm``, if given), one pass over the weight (its rows in the order of ``rotary_pairs``), rotary embedding of q and k - what
+    ``linear_packed_step`` and ``rope_qk`` do in two launches, with the same results.  ``cos, sin``: as for ``rope_qk``."""
+    cos, sin = _rotary_tables(cos, sin, x)
+    return _lib.load_host().linear_packed_qkv(x, w.data, norm, eps, cos, sin, num_heads, num_kv_heads, head_dim)
 
 
 def linear_packed(x: torch.Tensor, w: PackedLinearWeight) -> torch.Tensor:

@@ -489,6 +489,13 @@ int fa_linear_packed(const void* x, int64_t x_row_stride, const void* w_packed, 
 int fa_linear_packed_norm_ok(int rows, int K);
 int fa_linear_packed_step(const void* x, int64_t x_row_stride, const void* norm_weight, float eps, const void* w_packed,
                           void* out, int rows, int K, int n_out, int epilogue, int dtype, fa_stream_t stream);
+/* q/k/v of a decode step with the rotary embedding (MODEL:597-601, 213-244) in the launch, rounded where fa_rope_qk rounds.  The
+ * weight has (Hq + 2 Hkv) * D rows, D a multiple of 16, packed by fa_linear_pack with the rows of every q and k head in the order
+ * 0 .. 7, D/2 .. D/2 + 7, 8 .. 15, D/2 + 8 ..: the eight rows of a tile beside the eight they turn with.  cos, sin (rows, D);
+ * q (rows, Hq * D), kv (rows, 2 Hkv * D: k, then v), all dense, columns in their natural order. */
+int fa_linear_packed_qkv(const void* x, int64_t x_row_stride, const void* norm_weight, float eps, const void* w_packed,
+                         const void* cos, const void* sin, void* q, void* kv, int rows, int K, int Hq, int Hkv, int D, int dtype,
+                         fa_stream_t stream);
 
 #ifdef __cplusplus
 }

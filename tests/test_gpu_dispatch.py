@@ -302,6 +302,27 @@ def test_projections_with_the_steps_beside_them(dtype, rows, K, n_out):
     assert torch.equal(ops.linear_packed_step(x, pw, norm, 1e-5, residual=kept), h + got)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,q_len,K,Hq,Hkv,D", [(1, 1, 1024, 1, 1, 16), (2, 1, 3072, 6, 2, 128), (3, 5, 1024, 4, 2, 64), (1, 4, 4096, 2, 1, 48)])
+def test_rotary_embedding_in_the_projection(dtype, B, q_len, K, Hq, Hkv, D):
+    """q, k and v of one launch against the projection on the weight in its natural order and the rotary embedding as launches
+    of their own: the same bits (same sums, same rounding), with and without the norm in front."""
+    from fourierattention_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(K + D)
+    rn = lambda *s: torch.randn(s, generator=g, device="cuda")
+    n_out = (Hq + 2 * Hkv) * D
+    w = (rn(n_out, K) * 0.05).to(dtype)
+    plain, pairs = ops.PackedLinearWeight(w), ops.PackedLinearWeight(w[ops.rotary_pairs(n_out, Hq + Hkv, D, "cuda")].contiguous())
+    x, norm = (rn(B, q_len, K) * 3).to(dtype), (1 + 0.1 * rn(K)).to(dtype)
+    cos, sin = rn(B, q_len, D).to(dtype), rn(B, q_len, D).to(dtype)
+    for nw in (None, norm) if B * q_len * K <= 16384 else (None,):
+        row = ops.linear_packed(x, plain) if nw is None else ops.linear_packed_step(x, plain, nw, 1e-5)
+        q, k, v = (t.contiguous() for t in row.split((Hq * D, Hkv * D, Hkv * D), dim=-1))
+        q = ops.rope_qk(q, k, cos, sin, D)
+        for got, want in zip(ops.linear_packed_qkv(x, pairs, nw, 1e-5, cos, sin, Hq, Hkv, D), (q, k, v)):
+            assert torch.equal(got, want.view(B, q_len, -1, D).transpose(1, 2))
+
+
 def _launches(f):
     """Kernel launches of a call: the nodes of a graph it is captured into (which is never run)."""
     import ctypes
