@@ -405,14 +405,43 @@ __global__ __launch_bounds__(256) void decode_mid_kernel(
   const int kn0 = kn_h[h], kn_len = kn_h[h + 1] - kn0;
   const int vn0 = vn_h[h], vn_len = vn_h[h + 1] - vn0;
 
-  for (int e = tid; e < GM * 2 * N; e += 256) {
-    const int g = e / (2 * N), n = e - g * 2 * N;
-    const float x = g < G ? W[((int64_t)b * Hq + h * G + g) * 2 * N + n] : 0.f;
-    s_w[n < N ? 2 * n : 2 * (n - N) + 1].v[g] = x;
-  }
-  for (int e = tid; e < GM * 128; e += 256) {
-    const int g = e >> 7, j = e & 127;
-    s_qn[j].v[g] = g < G && j < kn_len ? fa_to_float(q[((int64_t)b * Hq + h * G + g) * D + (kn_list[kn0 + j] - h * D)]) * sm_log2e : 0.f;
+  // Weights and stored query dims: every load goes out before the first is used (one after the other they were six round
+  // trips to memory, half of the kernel's time on a short context), heads past the group read the last one
+  {
+    const int j = tid & 127, g0 = tid >> 7;
+    const int col = kn_len > 0 ? kn_list[kn0 + min(j, kn_len - 1)] - h * D : 0;
+    const float* w0 = W + ((int64_t)b * Hq + h * G) * 2 * N;
+    constexpr int kRows = 4;   // coefficient rows of a thread and batch
+    float x[kRows][GM];
+    auto load_rows = [&](int n0) {
+#pragma unroll
+      for (int u = 0; u < kRows; ++u)
+        if (n0 + u * 256 < 2 * N)
+#pragma unroll
+          for (int g = 0; g < GM; ++g) x[u][g] = w0[(int64_t)min(g, G - 1) * 2 * N + min(n0 + u * 256 + tid, 2 * N - 1)];
+    };
+    load_rows(0);
+    E qv[GM / 2];
+#pragma unroll
+    for (int i = 0; i < GM / 2; ++i) qv[i] = q[((int64_t)b * Hq + h * G + min(g0 + 2 * i, G - 1)) * D + col];
+    for (int n0 = 0; n0 < 2 * N; n0 += kRows * 256) {
+      if (n0 > 0) load_rows(n0);
+#pragma unroll
+      for (int u = 0; u < kRows; ++u) {
+        const int n = n0 + u * 256 + tid;
+        if (n < 2 * N) {
+          Heads o;
+#pragma unroll
+          for (int g = 0; g < GM; ++g) o.v[g] = g < G ? x[u][g] : 0.f;
+          s_w[n < N ? 2 * n : 2 * (n - N) + 1] = o;
+        }
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < GM / 2; ++i) {
+      const int g = g0 + 2 * i;
+      s_qn[j].v[g] = g < G && j < kn_len ? fa_to_float(qv[i]) * sm_log2e : 0.f;
+    }
   }
   const int l_beg = split * tiles_per_split * kMidTile;
   const int l_end = min(L_m, l_beg + tiles_per_split * kMidTile);
