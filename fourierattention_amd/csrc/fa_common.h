@@ -28,8 +28,9 @@ int fa_check_launch(const char* what);
 bool fa_spectral_mfma_ok(int a_dtype, int K, int Mc, int N);
 bool fa_recon_stats_mfma_ok(int N, int Mc, int K);
 size_t fa_recon_stats_mfma_workspace(int B, int N, int Mc, int K);
-// partial sums / maxima / minima of the reconstruction, [B][row blocks][Mc] each; returns the number of row blocks
-int fa_recon_stats_mfma_launch(const float* c, int B, int N, int Mc, int K, int T, void* workspace, float** psum,
+// partial sums / maxima / minima of the reconstruction, [B][row blocks][Mc] each; returns the number of row blocks.
+// single: the statistics are a single-precision cache's
+int fa_recon_stats_mfma_launch(const float* c, int B, int N, int Mc, int K, int T, bool single, void* workspace, float** psum,
                                float** pmax, float** pmin, hipStream_t st);
 // the last launch of the column statistics (fa_spectral.hip): partials [B][nsplit][Mc] -> mean and maximum deviation
 void fa_stats_finalize_launch(const float* psum, const float* pmax, const float* pmin, float* avg, float* dev, int B, int K,

@@ -454,7 +454,7 @@ static int recon_stats(const float* c, float* avg, float* max_dev, int B, int N,
   if (fa_recon_stats_mfma_ok(N, Mc, K) && workspace_bytes >= fa_recon_stats_mfma_workspace(B, N, Mc, K)) {
     FA_REQUIRE(((uintptr_t)workspace & 255) == 0, FA_ERR_MISALIGNED, "fa_mat_fourier_avg_std: workspace not 256-byte aligned");
     float *ps, *px, *pn;
-    const int rb = fa_recon_stats_mfma_launch(c, B, N, Mc, K, T, workspace, &ps, &px, &pn, s);
+    const int rb = fa_recon_stats_mfma_launch(c, B, N, Mc, K, T, ex.u_avg && ex.model_dtype == FA_FP32, workspace, &ps, &px, &pn, s);
     stats_finalize_kernel<<<dim3(fa_cdiv(Mc, 64), B), 64 * kFinalizeWaves, 0, s>>>(ps, px, pn, avg, max_dev, K, Mc, rb, round_dtype, ex);
     return fa_check_launch("fa_mat_fourier_avg_std");
   }

@@ -55,11 +55,13 @@ struct SpectralTable {
 };
 
 // ---- pack: block = 32 tokens x 256 columns; lanes run along the columns for the gather, the transposition to
-// token-contiguous fragments goes through LDS.  grid (ksteps + blocks of the basis table, column blocks, B) ------------------------------------------
+// token-contiguous fragments goes through LDS.  grid (ksteps + blocks of the basis table, column blocks, parts * B): part p of the input starts p * a_part
+// elements behind the first and its fragments p * out_part behind the first's; with col_inv_scale the columns are scaled ------
 template <typename E>
 __global__ __launch_bounds__(256) void spectral_pack_kernel(
     const E* __restrict__ a, int64_t a_bs, int64_t a_rs, const int32_t* __restrict__ cols,
-    half8* __restrict__ out, int K, int Mc, int CT, int KS32, const SpectralTable st) {
+    const float* __restrict__ col_inv_scale, half8* __restrict__ out, int K, int Mc, int CT, int KS32, int B, int64_t a_part,
+    int64_t out_part, const SpectralTable st) {
   constexpr int kPitch = 256 + 4;   // f16 elements per LDS row: 8 rows apart = 16 banks apart
   __shared__ _Float16 tile[32][kPitch];
   if ((int)blockIdx.x >= KS32) {
@@ -67,11 +69,14 @@ __global__ __launch_bounds__(256) void spectral_pack_kernel(
     return;
   }
   const int tid = threadIdx.x;
-  const int ks = blockIdx.x, m0 = blockIdx.y * 256, b = blockIdx.z;
+  const int ks = blockIdx.x, m0 = blockIdx.y * 256, part = blockIdx.z / B, b = blockIdx.z - part * B;
+  a += part * a_part;
+  out += part * out_part;
   const int m = m0 + tid;
   const bool mok = m < Mc;
   const int col = mok ? (cols ? cols[m] : m) : 0;
   const E* ab = a + (int64_t)b * a_bs + col;
+  const float mul = (col_inv_scale && mok) ? col_inv_scale[(int64_t)b * Mc + m] : 1.f;
   float v[32];
 #pragma unroll
   for (int kk = 0; kk < 32; ++kk) {
@@ -82,7 +87,7 @@ __global__ __launch_bounds__(256) void spectral_pack_kernel(
   for (int kk = 0; kk < 32; ++kk) {
     const int k = ks * 32 + kk;
     // f16 holds every bf16 / f16 value of magnitude below 65504 exactly (tiny ones as subnormals)
-    const float x = (mok && k < K) ? fminf(fmaxf(v[kk], -65504.f), 65504.f) : 0.f;
+    const float x = (mok && k < K) ? fminf(fmaxf(v[kk] * mul, -65504.f), 65504.f) : 0.f;
     tile[kk][tid] = (_Float16)x;
   }
   __syncthreads();
@@ -739,6 +744,195 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   }
 }
 
+// The statistics of a cache in single precision: complex sums, one pass over the cosine and one over the sine coefficients
+// on the walk of the compression, from which the real and the imaginary part are taken.  Twice the work of the kernel above,
+// with errors of the same size (deviations 5e-5, means 1e-4) in other places.  The statistics are rounded to fp16, where a
+// place is up to 1e-3 of a value: with either kernel some columns of a tensor round the other way, and the attention over
+// it moves by 5e-4 - nothing beside the roundings of a 16-bit model, but fifty times the 1e-5 that single precision holds its
+// results to.
+__global__ __launch_bounds__(1024) void coef_colscale_kernel(const float* __restrict__ c, float* __restrict__ scale,
+                                                             float* __restrict__ inv_scale, int N2, int Mc) {
+  // 16 columns x 64 row classes: 64 bytes of a row per access, and four times the blocks of whole waves of columns
+  __shared__ float s_mx[64][16];
+  const int lane = threadIdx.x & 15, g = threadIdx.x >> 4;
+  const int m = blockIdx.x * 16 + lane, b = blockIdx.y;
+  float mx = 0.f;
+  if (m < Mc) {
+    const float* cp = c + (int64_t)b * N2 * Mc + m;
+    for (int n0 = g; n0 < N2; n0 += 64 * 8) {
+      float v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = cp[(int64_t)min(n0 + 64 * u, N2 - 1) * Mc];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) mx = fmaxf(mx, fabsf(v[u]));
+    }
+  }
+  s_mx[g][lane] = mx;
+  __syncthreads();
+  if (g == 0 && m < Mc) {
+#pragma unroll
+    for (int i = 1; i < 64; ++i) mx = fmaxf(mx, s_mx[i][lane]);
+    const float sc = mx > 0.f ? exp2f(ceilf(log2f(mx))) : 1.f;   // power of two: scaling is exact
+    scale[(int64_t)b * Mc + m] = sc;
+    inv_scale[(int64_t)b * Mc + m] = 1.0f / sc;
+  }
+}
+
+constexpr int kWalkColShare = 16;   // column blocks of a workgroup at most
+
+struct ReconWalkParams {
+  const half8* tab;        // basis rows of the positions: [ceil(K/8)][kStepK][64]
+  const half8* packed[2];  // cos / sin coefficients, [B][CT][KS32][64] fragments
+  const float* scale;      // [B][Mc]
+  float* psum;
+  float* pmax;
+  float* pmin;             // [B][RB][Mc]
+  int B, N, Mc, CT, KS32, K, T, n_steps, RB;
+  int cb_per; // column blocks of a workgroup
+  int Kd;     // positions computed directly: min(K, T / 2 + 1)
+  int half;   // T / 2: mirror images beyond it count as positions of their own (a value no position exceeds
+              // when the sequence is longer than the period and every position is computed directly)
+};
+
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void spectral_recon_walk_kernel(
+    const ReconWalkParams p) {
+  constexpr int NST = 4;
+  __shared__ __attribute__((aligned(16))) unsigned char s_stage[NST][4][kStepK][1024];
+  __shared__ float s_red[3][4][kWgCols];
+  __shared__ float s_scale[kWalkColShare * kWgCols];   // scale / N of this workgroup's columns
+  const int tid = threadIdx.x, lane = tid & 63, lg = lane >> 4, lc = lane & 15;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int rb = blockIdx.x, b = blockIdx.y;
+  const int rt0 = (rb * 4 + w) * 4;
+  const int n_rt = (p.Kd + 7) / 8;
+  const int S = p.n_steps;
+  const int cb0 = blockIdx.z * p.cb_per;
+  const int n_cb = min((p.Mc + kWgCols - 1) / kWgCols - cb0, p.cb_per);
+  const int Q = n_cb * 2 * S;   // steps of this workgroup: column block, pass (cos, sin), step (last to first)
+
+  int next_cb = cb0, next_pass = 0, next_s = S - 1;   // the step requested next (walked, not divided out of a step number)
+  auto issue = [&](int stage) {
+    const int ct = min(next_cb * 4 + w, p.CT - 1);
+    const half8* frags = next_pass ? p.packed[1] : p.packed[0];
+    const _Float16* src = (const _Float16*)(frags + (((int64_t)b * p.CT + ct) * p.KS32) * 64) + lane * 8;
+#pragma unroll
+    for (int ks = 0; ks < kStepK; ++ks)
+      load_frag_to_lds(src + (int64_t)(next_s * kStepK + ks) * 512, &s_stage[stage][w][ks][0]);
+    if (--next_s < 0) {
+      next_s = S - 1;
+      next_cb += next_pass;
+      next_pass ^= 1;
+    }
+  };
+#pragma unroll
+  for (int i = 0; i < NST - 1; ++i)
+    if (i < Q) issue(i);
+
+  half8 Ea[4][kStepK];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int ks = 0; ks < kStepK; ++ks) Ea[i][ks] = p.tab[((int64_t)min(rt0 + i, n_rt - 1) * kStepK + ks) * 64 + lane];
+  float rc[4][2], rs[4][2];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int f2 = 0; f2 < 2; ++f2) fast_sincos_phase(min(rt0 + i, n_rt - 1) * 8 + lg * 2 + f2, kStepTokens, p.T, &rs[i][f2], &rc[i][f2]);
+  float4v acc[4][4];
+  float re[4][4][2];   // real part left by the cos pass
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[i][j] = float4v{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int ks = 0; ks < kStepK; ++ks) asm volatile("" ::"v"(Ea[i][ks]));
+
+  // (read here once: a load behind the walk of a column block would wait for every tile on its way)
+  const float inv_n = 1.0f / (float)p.N;
+  for (int i = tid; i < n_cb * kWgCols; i += 256) {
+    const int m = cb0 * kWgCols + i;
+    s_scale[i] = m < p.Mc ? p.scale[(int64_t)b * p.Mc + m] * inv_n : 0.f;
+  }
+  int cb = cb0, pass = 0, it = -1;
+  for (int q = 0; q < Q; ++q) {
+    if (++it == S) {
+      it = 0;
+      cb += pass;
+      pass ^= 1;
+    }
+    const int stage = q % NST;
+    if (q + NST - 2 < Q) wait_vmcnt<(NST - 2) * kStepK>();
+    else wait_vmcnt<0>();
+    barrier_lds_only();
+    if (q + NST - 1 < Q) issue((q + NST - 1) % NST);
+    spectral_step(acc, Ea, rc, rs, lds_addr_of(&s_stage[stage][0][0][lane * 16]));
+    if (it != S - 1) continue;
+    if (pass == 0) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          re[i][j][0] = acc[i][j][0];
+          re[i][j][1] = acc[i][j][2];
+          acc[i][j] = float4v{0.f, 0.f, 0.f, 0.f};
+        }
+      continue;
+    }
+    // both passes done for this column block: r = (re +- im) * scale / N at this lane's 8 positions per column and
+    // at their mirror images
+    const int half = p.half;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float sc = s_scale[((cb - cb0) * 4 + j) * 16 + lc];
+      float sum = 0.f, mx = -INFINITY, mn = INFINITY;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int f2 = 0; f2 < 2; ++f2) {
+          const int k = (rt0 + i) * 8 + lg * 2 + f2;
+          const float r = (re[i][j][f2] + acc[i][j][2 * f2 + 1]) * sc;
+          if (k < p.Kd) {
+            sum += r;
+            mx = fmaxf(mx, r);
+            mn = fminf(mn, r);
+          }
+          const int km = p.T - k;   // the mirror image counts where it is a position of its own beyond T / 2
+          const float r2 = (re[i][j][f2] - acc[i][j][2 * f2 + 1]) * sc;
+          if (k < p.Kd && km > half && km < p.K) {
+            sum += r2;
+            mx = fmaxf(mx, r2);
+            mn = fminf(mn, r2);
+          }
+        }
+      sum = fa_rows_sum(sum);
+      mx = fa_rows_max(mx);
+      mn = fa_rows_min(mn);
+      if (lg == 0) {
+        s_red[0][w][j * 16 + lc] = sum;
+        s_red[1][w][j * 16 + lc] = mx;
+        s_red[2][w][j * 16 + lc] = mn;
+      }
+    }
+    __syncthreads();
+    if (tid < kWgCols) {
+      const int m = cb * kWgCols + tid;
+      if (m < p.Mc) {
+        const int64_t o = ((int64_t)b * p.RB + rb) * p.Mc + m;
+        p.psum[o] = (s_red[0][0][tid] + s_red[0][1][tid]) + (s_red[0][2][tid] + s_red[0][3][tid]);
+        p.pmax[o] = fmaxf(fmaxf(s_red[1][0][tid], s_red[1][1][tid]), fmaxf(s_red[1][2][tid], s_red[1][3][tid]));
+        p.pmin[o] = fminf(fminf(s_red[2][0][tid], s_red[2][1][tid]), fminf(s_red[2][2][tid], s_red[2][3][tid]));
+      }
+    }
+    // the next barrier (top of the loop) orders these reads before s_red is written again
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc[i][j] = float4v{0.f, 0.f, 0.f, 0.f};
+  }
+}
+
 }  // namespace fa_mfma
 
 namespace {
@@ -795,9 +989,9 @@ int fa_spectral_mfma_launch(const void* a, int a_dtype, int64_t a_bs, int64_t a_
   const SpectralTable table{(half2v*)((char*)workspace + pl.off_tab), N, T};
   dim3 pgrid(pl.KS32 + fa_cdiv(table_blocks(N), (int64_t)fa_cdiv(Mc, 256) * B), fa_cdiv(Mc, 256), B);
   if (a_dtype == FA_BF16)
-    spectral_pack_kernel<bf16_t><<<pgrid, 256, 0, st>>>((const bf16_t*)a, a_bs, a_rs, cols, packed, K, Mc, pl.CT, pl.KS32, table);
+    spectral_pack_kernel<bf16_t><<<pgrid, 256, 0, st>>>((const bf16_t*)a, a_bs, a_rs, cols, nullptr, packed, K, Mc, pl.CT, pl.KS32, B, 0, 0, table);
   else
-    spectral_pack_kernel<f16_t><<<pgrid, 256, 0, st>>>((const f16_t*)a, a_bs, a_rs, cols, packed, K, Mc, pl.CT, pl.KS32, table);
+    spectral_pack_kernel<f16_t><<<pgrid, 256, 0, st>>>((const f16_t*)a, a_bs, a_rs, cols, nullptr, packed, K, Mc, pl.CT, pl.KS32, B, 0, 0, table);
   return spectral_after_pack(pl, c, B, Mc, N, T, k_start, accumulate, workspace, st);
 }
 
@@ -926,12 +1120,12 @@ namespace {
 // Column blocks per workgroup of the reconstruction statistics.  Two workgroups fit a compute unit, and a workgroup
 // pays about half a column block for its basis rows before the first product: take the share whose rounds over the
 // device, times the length of a round, come out shortest.
-int recon_col_share(int row_groups, int n_cb) {
-  int best = n_cb < fa_mfma::kMaxColShare ? n_cb : fa_mfma::kMaxColShare;
+int recon_col_share(int row_groups, int n_cb, int most) {
+  int best = n_cb < most ? n_cb : most;
   float best_cost = 1e30f;
   for (int cs = 1; cs <= n_cb; ++cs) {
     const int per = fa_cdiv(n_cb, cs);
-    if (per > fa_mfma::kMaxColShare) continue;
+    if (per > most) continue;
     const float cost = (float)fa_cdiv((int64_t)row_groups * fa_cdiv(n_cb, per), 512) * ((float)per + 0.5f);
     if (cost < best_cost) { best_cost = cost; best = per; }
   }
@@ -939,13 +1133,81 @@ int recon_col_share(int row_groups, int n_cb) {
 }
 }  // namespace
 
+namespace {
+struct ReconWalkPlan {
+  int CT, KS32, n_steps, RB;
+  size_t off_tab, off_pc, off_ps, off_scale, off_inv, off_sum, off_max, off_min, total;
+};
+ReconWalkPlan recon_walk_plan(int B, int N, int Mc, int K) {
+  using namespace fa_mfma;
+  ReconWalkPlan p{};
+  p.CT = fa_cdiv(Mc, 16);
+  p.n_steps = fa_cdiv(N, kStepTokens);
+  p.KS32 = p.n_steps * kStepK;
+  p.RB = fa_cdiv(K, kWgFreqs);
+  size_t o = 0;
+  auto take = [&](size_t bytes) { size_t at = o; o += fa_align_up(bytes, 256); return at; };
+  p.off_tab = take((size_t)fa_cdiv(K, 8) * kStepK * 64 * 16);
+  p.off_pc = take((size_t)B * p.CT * p.KS32 * 1024);
+  p.off_ps = take((size_t)B * p.CT * p.KS32 * 1024);
+  p.off_scale = take((size_t)B * Mc * 4);
+  p.off_inv = take((size_t)B * Mc * 4);
+  p.off_sum = take((size_t)B * p.RB * Mc * 4);
+  p.off_max = take((size_t)B * p.RB * Mc * 4);
+  p.off_min = take((size_t)B * p.RB * Mc * 4);
+  p.total = o;
+  return p;
+}
+}  // namespace
+
+namespace {
+int recon_walk_launch(const float* c, int B, int N, int Mc, int K, int T, void* workspace, float** psum, float** pmax, float** pmin,
+                      hipStream_t st) {
+  using namespace fa_mfma;
+  const ReconWalkPlan pl = recon_walk_plan(B, N, Mc, K);
+  char* ws = (char*)workspace;
+  half8* tab = (half8*)(ws + pl.off_tab);
+  half8* pc = (half8*)(ws + pl.off_pc);
+  half8* ps = (half8*)(ws + pl.off_ps);
+  float* scale = (float*)(ws + pl.off_scale);
+  float* inv = (float*)(ws + pl.off_inv);
+  *psum = (float*)(ws + pl.off_sum);
+  *pmax = (float*)(ws + pl.off_max);
+  *pmin = (float*)(ws + pl.off_min);
+  // positions 0 .. T / 2 stand for their mirror images as well (unless the sequence is longer than the period)
+  const bool mirror = K <= T + 1;
+  const int Kd = mirror && T / 2 + 1 < K ? T / 2 + 1 : K;
+  const int RBd = fa_cdiv(Kd, kWgFreqs);
+  const int kp8 = fa_cdiv(Kd, 8) * 8;
+  coef_colscale_kernel<<<dim3(fa_cdiv(Mc, 16), B), 1024, 0, st>>>(c, scale, inv, 2 * N, Mc);
+  // the cosine rows and, behind them, the sine rows; the basis of the positions beside them
+  const int pack_rows = fa_cdiv(Mc, 256) * 2 * B;
+  spectral_pack_kernel<float><<<dim3(pl.KS32 + fa_cdiv(table_blocks(kp8), pack_rows), fa_cdiv(Mc, 256), 2 * B), 256, 0, st>>>(c, (int64_t)2 * N * Mc, Mc, nullptr, inv, pc, N, Mc,
+                                                                                     pl.CT, pl.KS32, B, (int64_t)N * Mc, ps - pc, SpectralTable{(half2v*)tab, kp8, T});
+  ReconWalkParams rp{};
+  rp.tab = tab; rp.packed[0] = pc; rp.packed[1] = ps; rp.scale = scale;
+  rp.psum = *psum; rp.pmax = *pmax; rp.pmin = *pmin;
+  rp.B = B; rp.N = N; rp.Mc = Mc; rp.CT = pl.CT; rp.KS32 = pl.KS32; rp.K = K; rp.T = T; rp.n_steps = pl.n_steps; rp.RB = RBd;
+  rp.Kd = Kd;
+  rp.half = mirror ? T / 2 : 0x7fffffff;
+  const int n_cb = fa_cdiv(Mc, kWgCols);
+  rp.cb_per = recon_col_share(RBd * B, n_cb, kWalkColShare);
+  spectral_recon_walk_kernel<<<dim3(RBd, B, fa_cdiv(n_cb, rp.cb_per)), 256, 0, st>>>(rp);
+  return RBd;
+}
+}  // namespace
+
 bool fa_recon_stats_mfma_ok(int N, int Mc, int K) { return N >= 32 && Mc >= 16 && K >= 1024; }
 
-size_t fa_recon_stats_mfma_workspace(int B, int N, int Mc, int K) { return recon_plan(B, N, Mc, K).total; }
+size_t fa_recon_stats_mfma_workspace(int B, int N, int Mc, int K) {
+  const size_t a = recon_plan(B, N, Mc, K).total, b = recon_walk_plan(B, N, Mc, K).total;
+  return a > b ? a : b;
+}
 
-int fa_recon_stats_mfma_launch(const float* c, int B, int N, int Mc, int K, int T, void* workspace, float** psum,
+int fa_recon_stats_mfma_launch(const float* c, int B, int N, int Mc, int K, int T, bool single, void* workspace, float** psum,
                                float** pmax, float** pmin, hipStream_t st) {
   using namespace fa_mfma;
+  if (single) return recon_walk_launch(c, B, N, Mc, K, T, workspace, psum, pmax, pmin, st);
   const ReconPlan pl = recon_plan(B, N, Mc, K);
   char* ws = (char*)workspace;
   half8* tab = (half8*)(ws + pl.off_tab);
@@ -970,7 +1232,7 @@ int fa_recon_stats_mfma_launch(const float* c, int B, int N, int Mc, int K, int 
   rp.Kd = Kd;
   rp.half = mirror ? T / 2 : 0x7fffffff;
   const int n_cb = fa_cdiv(Mc, kRecCols);
-  rp.cb_per = recon_col_share(RBd * B, n_cb);
+  rp.cb_per = recon_col_share(RBd * B, n_cb, kMaxColShare);
   spectral_recon_stats_kernel<<<dim3(RBd, B, fa_cdiv(n_cb, rp.cb_per)), 256, 0, st>>>(rp);
   return RBd;
 }
