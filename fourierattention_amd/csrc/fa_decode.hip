@@ -110,21 +110,65 @@ __device__ __forceinline__ void decode_prep_body(const PrepArgs<E>& pa, int bx, 
   const int h = blockIdx.y, b = blockIdx.z;
   const int G = Hq / Hkv;
   const int kc0 = kc_h[h], kc_len = kc_h[h + 1] - kc0;
-  for (int e = tid; e < kGMax * 128; e += 256) {
-    const int g = e >> 7, j = e & 127;
-    float qs = 0.f, qa = 0.f;
-    if (g < G && j < kc_len) {
-      const int d = kc_list[kc0 + j] - h * D;
-      const float sc = scale[(int64_t)b * Ck + kc0 + j];
-      const float a = avg_u[(int64_t)b * Ck + kc0 + j] - avg_d[(int64_t)b * Ck + kc0 + j] * sc;
-      const float qv = fa_to_float(q[((int64_t)b * Hq + h * G + g) * D + d]);
-      qs = qv * sc;
-      qa = qv * a;
+  // The query's compressed dims (thread = dim, every other head) and, in one block, its stored dims as the mid-row kernel's
+  // operands: lists and statistics first, then every query element, so that the chain is two round trips to memory however
+  // many heads and sub-splits there are.  (A list entry and a query element at a time, head by head and sub-split by
+  // sub-split, the launch took 8.5 us where it takes 6.9 at one sequence of 32k, 13.4 against 11.1 with the update.)
+  const int j = tid & 127, g0 = tid >> 7;
+  const bool on = j < kc_len;
+  int col = h * D;
+  float sc = 0.f, mean = 0.f;
+  if (on) {
+    const int64_t o = (int64_t)b * Ck + kc0 + j;
+    col = kc_list[kc0 + j];
+    sc = scale[o];
+    mean = avg_u[o] - avg_d[o] * sc;
+  }
+  const bool stores_q = sizeof(E) == 2 && bx == 1 && pa.q_stored;
+  // kstep, lane group and column of this thread's eight stored dims
+  const int qks = tid >> 6, qlane = tid & 63, qlc = qlane & 15, qj0 = qks * 32 + 8 * (qlane >> 4);
+  const int qgrp = b / pa.nbpg, qbb = b - qgrp * pa.nbpg;
+  int kn_len = 0, ncol[8];
+  if (stores_q) {
+    const int kn0 = pa.kn_h[h];
+    kn_len = pa.kn_h[h + 1] - kn0;
+    // (a head that stores no K dims has no entries in the list and nobody reads its operands)
+    if (kn_len > 0)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) ncol[e] = pa.kn_list[kn0 + min(qj0 + e, kn_len - 1)];   // clamped: no load under a per-lane condition
+  }
+  E qv[kGMax / 2];
+#pragma unroll
+  for (int i = 0; i < kGMax / 2; ++i)
+    if (2 * i < G) qv[i] = q[((int64_t)b * Hq + h * G + min(g0 + 2 * i, G - 1)) * D + (col - h * D)];
+  // the column's query head and the slot it belongs to: a batch element of the group, or (one sequence) a sub-split
+  const int qslot = qlc / G, qg = qlc - qslot * G;
+  E qn[8];
+  if (kn_len > 0) {
+    const E* qr = q + ((int64_t)b * Hq + h * G + qg) * D - h * D;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) qn[e] = qr[ncol[e]];
+  }
+  float ue = 0.f;
+  if constexpr (UPD)
+    if (on && g0 == 0) ue = fa_to_float(pa.upd_row[(int64_t)b * pa.upd_bs + col]);
+#pragma unroll
+  for (int i = 0; i < kGMax / 2; ++i) {
+    const int g = g0 + 2 * i;
+    const bool live = on && g < G;
+    const float x = live ? fa_to_float(qv[i]) : 0.f;
+    s_qs[g][j] = x * sc;
+    s_qa[g][j] = x * mean;
+  }
+  if constexpr (UPD)
+    if (g0 == 0) s_ue[j] = ue;
+  if (kn_len > 0) {
+    for (int sl = pa.sub ? 0 : qbb, last = pa.sub ? 3 : qbb; sl <= last; ++sl) {
+      union { E e[8]; uint4 raw; } o;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) o.e[e] = qslot == sl && qj0 + e < kn_len ? qn[e] : E();
+      *(uint4*)(pa.q_stored + ((((int64_t)(qgrp * Hkv + h) * 4 + sl) * 4 + qks) * 64 + qlane) * 8) = o.raw;
     }
-    s_qs[g][j] = qs;
-    s_qa[g][j] = qa;
-    if constexpr (UPD)
-      if (g == 0) s_ue[j] = j < kc_len ? fa_to_float(pa.upd_row[(int64_t)b * pa.upd_bs + kc_list[kc0 + j]]) : 0.f;
   }
   if constexpr (UPD) {
     if (tid < kPrepRows) {
@@ -140,25 +184,6 @@ __device__ __forceinline__ void decode_prep_body(const PrepArgs<E>& pa, int bx, 
     for (int g = 0; g < G; ++g) {
       float v = fa_wave_sum(s_qa[g][tid] + s_qa[g][tid + 64]);
       if (tid == 0) c0[(int64_t)b * Hq + h * G + g] = v * sm_log2e;
-    }
-  }
-  if constexpr (sizeof(E) == 2) if (bx == 1 && pa.q_stored) {
-    const int kn0 = pa.kn_h[h], kn_len = pa.kn_h[h + 1] - kn0;
-    const int s = tid >> 6, lane = tid & 63, lg = lane >> 4, lc = lane & 15;
-    const int grp = b / pa.nbpg;
-    // (a head that stores no K dims has no entries in the list and nobody reads its operands)
-    for (int sl = pa.sub ? 0 : b - grp * pa.nbpg, last = pa.sub ? 3 : sl; sl <= last && kn_len > 0; ++sl) {
-      const int g = lc - sl * G;   // the column's query head if the column is this batch element's (this sub-split's)
-      const bool mine = g >= 0 && g < G;
-      const E* qr = q + ((int64_t)b * Hq + h * G + (mine ? g : 0)) * D - h * D;
-      union { E e[8]; uint4 raw; } o;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int j = s * 32 + 8 * lg + e;
-        const E qv = qr[pa.kn_list[kn0 + min(j, kn_len - 1)]];   // clamped: no load under a per-lane condition
-        o.e[e] = (mine && j < kn_len) ? qv : E();
-      }
-      *(uint4*)(pa.q_stored + ((((int64_t)(grp * Hkv + h) * 4 + sl) * 4 + s) * 64 + lane) * 8) = o.raw;
     }
   }
   // sixteen lanes share a row (64 bytes of it per access), a thread four rows.  (Requested ahead of the query's list and gather instead: 17.3 us where this takes

@@ -889,8 +889,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       // g of this split, back from its last frame (rotation by +phi of the frame centre), in the layout the merge
       // reads: [batch group][KV head][split][slice][row tile rt][column][lane group lg'] x {cos f, sin f, cos f+1,
       // sin f+1} with f = 8 rt + 2 lg' (the layout of the weights W).  This lane holds the frequencies
-      // 16 j + 4 lg + v, v = 0 .. 3, of tile pair j: rt = 2 j + lg / 2, lg' = 2 (lg % 2) + v / 2.  Lanes of columns
-      // past the group store values that nobody reads.
+      // 16 j + 4 lg + v, v = 0 .. 3, of tile pair j: rt = 2 j + lg / 2, lg' = 2 (lg % 2) + v / 2.  (Columns past
+      // the group store nothing: a batch of three leaves seven of the sixteen idle.)
       float4v* gl = (float4v*)p.pg + ((((int64_t)(grp * p.Hkv + h) * p.n_split + split) * NSL + sl) * 2 * KS) * 64 + lc * 4;
       // twice the centre of the last frame, in half tokens
       const int64_t c2 = (int64_t)64 * (t_beg + c_beg + (n_it > 0 ? ((n_it - 1) & ~1) : 0) + 1) - 1;
@@ -911,7 +911,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             o[2 * f2 + 1] = sn[v] * x + co[v] * y;
           }
           if (c_none) o = float4v{0.f, 0.f, 0.f, 0.f};
-          gl[(2 * j + (lg >> 1)) * 64 + 2 * (lg & 1) + h2] = o;
+          if (valid_r) gl[(2 * j + (lg >> 1)) * 64 + 2 * (lg & 1) + h2] = o;
         }
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
