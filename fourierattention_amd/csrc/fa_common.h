@@ -108,6 +108,7 @@ __device__ __forceinline__ float fa_dpp(float v) {
 #define FA_DPP_XOR2 0x4E
 #define FA_DPP_HALF_MIRROR 0x141
 #define FA_DPP_MIRROR 0x140
+#define FA_DPP_ROR4 0x124
 #define FA_DPP_ROR8 0x128
 
 // sum over the LANES consecutive lanes (4, 8 or 16, aligned) that contain this lane; every lane gets it

@@ -142,7 +142,8 @@ __device__ __forceinline__ void decode_prep_body(const PrepArgs<E>& pa, int bx, 
   for (int i = 0; i < kGMax / 2; ++i)
     if (2 * i < G) qv[i] = q[((int64_t)b * Hq + h * G + min(g0 + 2 * i, G - 1)) * D + (col - h * D)];
   // the column's query head and the slot it belongs to: a batch element of the group, or (one sequence) a sub-split
-  const int qslot = qlc / G, qg = qlc - qslot * G;
+  // (sub-splits keep four columns each, however many heads there are)
+  const int qslot = pa.sub ? qlc >> 2 : qlc / G, qcol = pa.sub ? qlc & 3 : qlc - qslot * G, qg = min(qcol, G - 1);
   E qn[8];
   if (kn_len > 0) {
     const E* qr = q + ((int64_t)b * Hq + h * G + qg) * D - h * D;
@@ -166,7 +167,7 @@ __device__ __forceinline__ void decode_prep_body(const PrepArgs<E>& pa, int bx, 
     for (int sl = pa.sub ? 0 : qbb, last = pa.sub ? 3 : qbb; sl <= last; ++sl) {
       union { E e[8]; uint4 raw; } o;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) o.e[e] = qslot == sl && qj0 + e < kn_len ? qn[e] : E();
+      for (int e = 0; e < 8; ++e) o.e[e] = qslot == sl && qcol < G && qj0 + e < kn_len ? qn[e] : E();
       *(uint4*)(pa.q_stored + ((((int64_t)(qgrp * Hkv + h) * 4 + sl) * 4 + qks) * 64 + qlane) * 8) = o.raw;
     }
   }

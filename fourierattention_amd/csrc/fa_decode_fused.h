@@ -151,9 +151,9 @@ struct FusedShare {
 __host__ __device__ __forceinline__ int fused_tail_lds_floats(int n_parts) { return 2 * 16 * n_parts + 32 + 2048 + 8192 + 128 + 384; }
 
 // SUB: the team belongs to one batch element whose mid rows were cut into four sub-splits per workgroup (see the
-// mid-row kernel): the sixteen column slots are (sub-split, query head), all of them multiply with the V coefficients
-// of that one batch element, so the product first adds the four sub-splits of a head and the threads that would
-// have taken the other batch elements take further row classes instead.
+// mid-row kernel).  The sub-splits of a head have met before they were stored, all but the outputs of the stored dims, which
+// share the head's reference: four columns, the query heads, and the threads that would have taken the other batch elements
+// take further row classes instead.
 template <bool SUB, typename P>
 __device__ __forceinline__ FusedShare fused_share(const P& p, int vc0, int vc_len, int split, int n_s, int b0, int nb, int KS,
                                                   int tid) {
@@ -221,11 +221,11 @@ __device__ __forceinline__ void fused_merge_tail(const P& p, float* sm, float* s
   float* s_stat = (float*)(s_src + 128);   // [3][128] scale, avg_u, avg_d of the compressed dims of the column share
   unsigned* cnt = p.fz.cnt + (int64_t)(grp * p.Hkv + h) * 2;
   const int vn0 = p.vn_h[h], vn_len = p.vn_h[h + 1] - vn0;
-  // column slot c16 = 4 * batch element of the group + query head; SUB: 4 * sub-split + query head, the partials of
-  // sub-split j being those of the virtual batch element 4 b0 + j and the sink/window tiles belonging to slot j = 0
-  auto slot_ok = [&](int c16) { return (SUB || (c16 >> 2) < nb) && (c16 & 3) < G; };
-  auto qrow_of = [&](int c16) { return (int64_t)(b0 + (SUB ? 0 : c16 >> 2)) * p.Hq + h * G + (c16 & 3); };   // the query row
-  auto prow_of = [&](int c16) { return (int64_t)((SUB ? 4 * b0 : b0) + (c16 >> 2)) * p.Hq + h * G + (c16 & 3); };   // its mid partials
+  // column slot c16 = 4 * batch element of the group + query head (SUB: one batch element; the outputs of the stored dims of
+  // sub-split j are those of the virtual batch element 4 b0 + j)
+  constexpr int kSlots = SUB ? 4 : 16, kTile = kSlots * 16;   // column slots; floats of a g tile
+  auto slot_ok = [&](int c16) { return (c16 >> 2) < nb && (c16 & 3) < G; };
+  auto qrow_of = [&](int c16) { return (int64_t)(b0 + (c16 >> 2)) * p.Hq + h * G + (c16 & 3); };
   // column share: the columns are query heads g_lo .. g_lo + ncol - 1 of batch element cbb (the host only fuses when
   // the columns of a workgroup belong to one batch element)
   const int ncol = f.u_hi - f.u_lo, cbb = f.u_lo / G, g_lo = f.u_lo - cbb * G;
@@ -307,7 +307,7 @@ __device__ __forceinline__ void fused_merge_tail(const P& p, float* sm, float* s
   }
 
   // ---- requests: everything the shares need goes out before the first result is used -----------------------------
-  const int64_t g_split_floats = (int64_t)16 * 2 * N;
+  const int64_t g_split_floats = (int64_t)kSlots * 2 * N;
   const float* g_team = p.pg + (int64_t)(grp * p.Hkv + h) * NS * g_split_floats;
   // maxima and denominators of the parts (requested first: the weights are computed while the rest arrives)
   float m_raw[4], d_raw[4];
@@ -317,11 +317,11 @@ __device__ __forceinline__ void fused_merge_tail(const P& p, float* sm, float* s
     const int c16 = idx / WS, e = idx - c16 * WS;
     m_raw[u] = -INFINITY;
     d_raw[u] = 0.f;
-    if (idx < 16 * WS && slot_ok(c16)) {
+    if (idx < kSlots * WS && slot_ok(c16)) {
       if (e < n_s) {
-        m_raw[u] = p.pm[prow_of(c16) * NS + e];
-        d_raw[u] = p.pd[prow_of(c16) * NS + e];
-      } else if (e >= NS && (!SUB || c16 < 4)) {
+        m_raw[u] = p.pm[qrow_of(c16) * NS + e];
+        d_raw[u] = p.pd[qrow_of(c16) * NS + e];
+      } else if (e >= NS) {
         m_raw[u] = p.fz.il_m[qrow_of(c16) * n_il + (e - NS)];
         d_raw[u] = p.fz.il_d[qrow_of(c16) * n_il + (e - NS)];
       }
@@ -332,17 +332,18 @@ __device__ __forceinline__ void fused_merge_tail(const P& p, float* sm, float* s
   float4v gv[kFusedGPre];
   if (has_coef) {
     const int ntb = min(kFusedTileBlock, f.t1 - f.t0);
-    const int n_items = 64 * ntb, n_cls = 512 / n_items;
+    const int n_items = kSlots * 4 * ntb, n_cls = 512 / n_items;
     const int item = tid % n_items, cls = tid / n_items;
-    if (cls < n_cls && ((item & 63) >> 2) < (SUB ? 4 : nb) * G) {
-      const float* gp = g_team + (f.t0 + (item >> 6)) * 256 + (item & 63) * 4;
+    if (cls < n_cls && (item % (kSlots * 4)) / 4 < nb * G) {
+      const float* gp = g_team + (f.t0 + item / (kSlots * 4)) * kTile + (item % (kSlots * 4)) * 4;
 #pragma unroll
-      for (int u = 0; u < kFusedGPre; ++u) gv[u] = *(const float4v*)(gp + (int64_t)min(cls + u * n_cls, n_s - 1) * g_split_floats);
+      for (int u = 0; u < kFusedGPre; ++u)
+        if (u * n_cls < n_s) gv[u] = *(const float4v*)(gp + (int64_t)min(cls + u * n_cls, n_s - 1) * g_split_floats);
     }
   }
 #pragma unroll
   for (int u = 0; u < 4; ++u)
-    if (tid + 512 * u < 16 * WS) {
+    if (tid + 512 * u < kSlots * WS) {
       s_w[tid + 512 * u] = m_raw[u];
       s_d[tid + 512 * u] = d_raw[u];
     }
@@ -364,14 +365,7 @@ __device__ __forceinline__ void fused_merge_tail(const P& p, float* sm, float* s
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       const int e = e0 + 32 * u;
-      if (e < WS) {
-        if constexpr (SUB) {   // one reference for the four sub-splits of the query head
-#pragma unroll
-          for (int j = 0; j < 4; ++j) mstar = fa_fmax(mstar, s_w[(4 * j + (c16 & 3)) * WS + e]);
-        } else {
-          mstar = fa_fmax(mstar, mrow[e]);
-        }
-      }
+      if (e < WS) mstar = fa_fmax(mstar, mrow[e]);   // (SUB: the waves of the slots past the heads compute nothing of use)
     }
     mstar = fa_fmax(mstar, fa_dpp<FA_DPP_XOR1>(mstar));
     mstar = fa_fmax(mstar, fa_dpp<FA_DPP_XOR2>(mstar));
@@ -434,8 +428,7 @@ __device__ __forceinline__ void fused_merge_tail(const P& p, float* sm, float* s
   const int on_col = on_h > 1 ? x_cl % ncol : x_cl, on_hlp = on_h > 1 ? x_cl / ncol : 0;
   const bool on_on = on_col < ncol && 4 * x_d4 < vn_len;
   const int on_first = SUB ? on_hlp : x_cls, on_step = SUB ? on_h : 4;
-  const int on_slot = SUB ? 4 * x_cls + c16_0 + on_col : c16_0 + on_col;
-  const float* on_src = p.pon + (SUB ? prow_of(on_slot) : qrow0 + on_col) * NS * D + 4 * x_d4;
+  const float* on_src = p.pon + (SUB ? (int64_t)(4 * b0 + x_cls) * p.Hq + h * G + g_lo + on_col : qrow0 + on_col) * NS * D + 4 * x_d4;
   if (on_on) {
 #pragma unroll
     for (int u = 0; u < kPre; ++u) on_pre[u] = *(const float4v*)(on_src + (int64_t)min(on_first + on_step * u, n_s - 1) * D);
@@ -450,12 +443,12 @@ __device__ __forceinline__ void fused_merge_tail(const P& p, float* sm, float* s
     if (upd && f.v_on) ue = *(const float4v*)(s_own + 4 * tid);
     for (int tb = f.t0; tb < f.t1; tb += kFusedTileBlock) {
       const int ntb = min(kFusedTileBlock, f.t1 - tb);
-      const int n_items = 64 * ntb, n_cls = 512 / n_items;
+      const int n_items = kSlots * 4 * ntb, n_cls = 512 / n_items;
       const int item = tid % n_items, cls = tid / n_items;
-      const int tl = item >> 6, rem = item & 63, lc = rem >> 2, lgp = rem & 3;
-      const int c16 = (lc / G) * 4 + (lc % G);
+      const int tl = item / (kSlots * 4), rem = item % (kSlots * 4), lc = rem >> 2, lgp = rem & 3;
+      const int c16 = SUB ? lc : (lc / G) * 4 + (lc % G);
       if (tb > f.t0) __syncthreads();   // the block before is done with s_g and s_red
-      const bool col_ok = lc < (SUB ? 4 : nb) * G;   // (columns past the group hold nothing; their slots of s_g are never read)
+      const bool col_ok = lc < nb * G;   // (columns past the group hold nothing; their slots of s_g are never read)
       auto put_g = [&](const float4v& a4) {
         const int rb = tl * 16 + 2 * lgp;
         s_g[rb * 16 + c16] = a4[0]; s_g[(rb + 8) * 16 + c16] = a4[1];
@@ -463,7 +456,7 @@ __device__ __forceinline__ void fused_merge_tail(const P& p, float* sm, float* s
       };
       if (cls < n_cls && col_ok) {
         const float* wg = s_w + c16 * WS;
-        const float* gp = g_team + (tb + tl) * 256 + rem * 4;
+        const float* gp = g_team + (tb + tl) * kTile + rem * 4;
         float4v a4 = float4v{0.f, 0.f, 0.f, 0.f};
         int s0 = cls;
         if (tb == f.t0) {
@@ -487,7 +480,14 @@ __device__ __forceinline__ void fused_merge_tail(const P& p, float* sm, float* s
         __syncthreads();
         if (cls == 0 && col_ok) {
           float4v a4 = *(const float4v*)(s_red + item * 4);
-          for (int c = 1; c < n_cls; ++c) a4 += *(const float4v*)(s_red + (c * n_items + item) * 4);
+          for (int c = 1; c < n_cls; c += 4) {   // four reads in flight
+            float4v t[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) t[u] = *(const float4v*)(s_red + (min(c + u, n_cls - 1) * n_items + item) * 4);
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+              if (c + u < n_cls) a4 += t[u];
+          }
           put_g(a4);
         }
       }
@@ -496,9 +496,7 @@ __device__ __forceinline__ void fused_merge_tail(const P& p, float* sm, float* s
         const int rows = 16 * ntb;
         auto fma_row = [&](int r, float4v v) {
           if (ragged) v = fused_v_place(v, f.v_back);
-          float4v gq = *(const float4v*)(s_g + r * 16 + f.bbslot * 4);
-          if constexpr (SUB)   // the four sub-splits of a query head meet here
-            gq = (gq + *(const float4v*)(s_g + r * 16 + 4)) + (*(const float4v*)(s_g + r * 16 + 8) + *(const float4v*)(s_g + r * 16 + 12));
+          const float4v gq = *(const float4v*)(s_g + r * 16 + f.bbslot * 4);
 #pragma unroll
           for (int g = 0; g < GS; ++g) acc[g] += v * gq[g];
         };
@@ -547,7 +545,7 @@ __device__ __forceinline__ void fused_merge_tail(const P& p, float* sm, float* s
     *(float4v*)(s_red + ((x_cls * 4 + x_cl) * 32 + x_d4) * 4) = a4;
     a4 = float4v{0.f, 0.f, 0.f, 0.f};
     if (on_on) {
-      const float* wg = s_w + on_slot * WS;
+      const float* wg = s_w + (c16_0 + on_col) * WS;
 #pragma unroll
       for (int u = 0; u < kPre; ++u)
         if (on_first + on_step * u < n_s) a4 += on_pre[u] * wg[on_first + on_step * u];
@@ -579,8 +577,6 @@ __device__ __forceinline__ void fused_merge_tail(const P& p, float* sm, float* s
     }
     __syncthreads();
     float* pc = pc_team + (int64_t)split * 16 * 128;
-    // (SUB: the row classes hold four slots each, those of the query heads)
-    constexpr int kSlots = SUB ? 4 : 16;
     const int n_out = kSlots * f.nqp;
     // the row classes [r0, r1) of one output (column slot, four dims) added up: four reads in flight, fixed order
     // (the number of classes is a power of two, at least four)
@@ -641,13 +637,10 @@ __device__ __forceinline__ void fused_merge_tail(const P& p, float* sm, float* s
         for (int u = 0; u < 16; ++u)
           if (z0 + u < n_blocks) sum += t[u];
       }
-      float pmid = s_sc[16 + c16_0 + o_cl];
-      if constexpr (SUB) pmid = (pmid + s_sc[20 + c16_0 + o_cl]) + (s_sc[24 + c16_0 + o_cl] + s_sc[28 + c16_0 + o_cl]);
+      const float pmid = s_sc[16 + c16_0 + o_cl];
       o_val += s_stat[o_src] * (sum * (1.0f / (float)N) - s_stat[256 + o_src] * pmid) + s_stat[128 + o_src] * pmid;
     }
-    float den = s_sc[c16_0 + o_cl];
-    if constexpr (SUB) den = (den + s_sc[4 + c16_0 + o_cl]) + (s_sc[8 + c16_0 + o_cl] + s_sc[12 + c16_0 + o_cl]);
-    o_val *= 1.0f / den;
+    o_val *= 1.0f / s_sc[c16_0 + o_cl];
     const int64_t at = (qrow0 + o_cl) * D + o_d;
     if (p.fz.out) p.fz.out[at] = o_val;
     if constexpr (sizeof(E) == 2) {

@@ -278,10 +278,10 @@ struct MidParams {
 // SUB (FUSE only, a batch of one sequence, at most four query heads per KV head): a single batch element would
 // leave twelve of the sixteen matrix-core columns and three of the four page streams of a workgroup idle.  The
 // workgroup's pages are cut into four sub-splits instead, which take the places of four batch elements: wave i
-// streams the pages of sub-split i, column 4 j' + g (j' = sub-split, as a batch element would be) holds query head g
-// with its weights W' rotated to the first frame of sub-split j', and every column keeps its own softmax reference,
-// g history and outputs, i.e. each sub-split ends as a partial result of its own ("virtual batch element" j' of the
-// partial buffers).  The page loop has a quarter of the trips.  Pages past the end of a sub-split are fetched from a
+// streams the pages of sub-split i, column 4 j' + g (j' = sub-split) holds query head g with its weights W' rotated to the
+// first frame of sub-split j', and every column keeps its own softmax reference, g history and outputs.  Behind the loop the
+// columns of a head are brought to one reference and added up (the outputs of the stored dims leave one by one, as
+// "virtual batch elements" j' of the partial buffers).  The page loop has a quarter of the trips.  Pages past the end of a sub-split are fetched from a
 // valid page and masked.
 // UPD (FUSE only): the tail also applies a pending rank-1 update to the V coefficients of its row share.
 template <typename E, int KS, int KMAX, int VMAX, int NST, int MODE = 0, bool FUSE = false, bool SUB = false, bool UPD = false>
@@ -336,10 +336,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int b0 = grp * p.nbpg;
   const int nb_real = min(p.nbpg, p.B - b0);
   const int nb = SUB ? 4 : nb_real;   // SUB: four sub-splits of the one batch element in the places of batch elements
-  const int R = nb * G;
-  const bool valid_r = lc < R;
-  const int bb_r = lc / G, g_r = lc - bb_r * G;
-  // the query row of this lane's column; the row of its partial results (SUB: virtual batch element 4 b + sub-split)
+  // this lane's column: batch element of the group (SUB: sub-split, four columns each) and query head
+  const int bb_r = SUB ? lc >> 2 : lc / G, g_r = SUB ? lc & 3 : lc - bb_r * G;
+  const bool valid_r = SUB ? g_r < G : lc < nb * G;
+  // the query row of this lane's column; the row of its stored-dim outputs (SUB: virtual batch element 4 b + sub-split)
   const int64_t qrow = valid_r ? ((int64_t)(b0 + (SUB ? 0 : bb_r)) * p.Hq + h * G + g_r) : 0;
   const int64_t prow = !SUB ? qrow : valid_r ? ((int64_t)(b0 * 4 + bb_r) * p.Hq + h * G + g_r) : 0;
   if (MODE != 1 && split == 0 && tid < nb_real && p.merge_count) p.merge_count[(b0 + tid) * p.Hkv + h] = 0u;
@@ -875,14 +875,26 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
 
     // ---- partials of this split ------------------------------------------------------
-    const float dsum = fa_rows_sum(d_run);
-    // SUB: a column whose sub-split has no page has seen masked scores only; what it accumulated is not a number
+    float dsum = fa_rows_sum(d_run);
+    // SUB: a column whose sub-split has no page has seen masked scores only; what it accumulated is not a number.  The four
+    // sub-splits of a head are brought to one reference and added up here, by lane exchanges: a quarter of the partials to
+    // store, to wait for and to read back (one sequence of 32k tokens: 36.5 - 38.2 us a launch -> 34.2 - 35.2).
     const bool c_none = SUB && c_n == 0;
-    if (valid_r) {
-      const int64_t base = prow * p.n_split + split;
+    float m_out = m_run, wgt = 1.f;
+    if constexpr (SUB) {
+      m_out = c_none ? -INFINITY : m_run;
+      m_out = fa_fmax(m_out, fa_dpp<FA_DPP_ROR8>(m_out));
+      m_out = fa_fmax(m_out, fa_dpp<FA_DPP_ROR4>(m_out));
+      wgt = c_none || m_run == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_run - m_out);
+      dsum = c_none ? 0.f : dsum * wgt;
+      dsum += fa_dpp<FA_DPP_ROR8>(dsum);
+      dsum += fa_dpp<FA_DPP_ROR4>(dsum);
+    }
+    if (valid_r && (!SUB || bb_r == 0)) {
+      const int64_t base = qrow * p.n_split + split;
       if (sl == 0 && lg == 0) {
-        p.pm[base] = c_none ? -INFINITY : m_run;
-        p.pd[base] = c_none ? 0.f : dsum;
+        p.pm[base] = m_out;
+        p.pd[base] = dsum;
       }
     }
     {
@@ -890,14 +902,18 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       // reads: [batch group][KV head][split][slice][row tile rt][column][lane group lg'] x {cos f, sin f, cos f+1,
       // sin f+1} with f = 8 rt + 2 lg' (the layout of the weights W).  This lane holds the frequencies
       // 16 j + 4 lg + v, v = 0 .. 3, of tile pair j: rt = 2 j + lg / 2, lg' = 2 (lg % 2) + v / 2.  (Columns past
-      // the group store nothing: a batch of three leaves seven of the sixteen idle.)
-      float4v* gl = (float4v*)p.pg + ((((int64_t)(grp * p.Hkv + h) * p.n_split + split) * NSL + sl) * 2 * KS) * 64 + lc * 4;
+      // the group store nothing: a batch of three leaves seven of the sixteen idle.)  SUB: four columns, the query heads;
+      // every lane of a head holds the sums of its sub-splits and stores one of four neighbouring pieces.
+      constexpr int kCols = SUB ? 4 : 16;
+      float4v* gl = (float4v*)p.pg + ((((int64_t)(grp * p.Hkv + h) * p.n_split + split) * NSL + sl) * 2 * KS) * kCols * 4 +
+                    (SUB ? g_r : lc) * 4;
       // twice the centre of the last frame, in half tokens
       const int64_t c2 = (int64_t)64 * (t_beg + c_beg + (n_it > 0 ? ((n_it - 1) & ~1) : 0) + 1) - 1;
       float sn[4], co[4], s16, c16;   // stepped phases, as for the first frame of the score waves
       fast_sincos_phase(16, c2, 2 * p.T, &s16, &c16);
 #pragma unroll
       for (int v = 0; v < 4; ++v) fast_sincos_phase(fbase + 4 * lg + v, c2, 2 * p.T, &sn[v], &co[v]);
+      float4v piece;
 #pragma unroll
       for (int j = 0; j < KS; ++j) {
 #pragma unroll
@@ -910,8 +926,22 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             o[2 * f2] = co[v] * x - sn[v] * y;
             o[2 * f2 + 1] = sn[v] * x + co[v] * y;
           }
-          if (c_none) o = float4v{0.f, 0.f, 0.f, 0.f};
-          if (valid_r) gl[(2 * j + (lg >> 1)) * 64 + 2 * (lg & 1) + h2] = o;
+          if constexpr (SUB) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              float x = c_none ? 0.f : o[e] * wgt;
+              x += fa_dpp<FA_DPP_ROR8>(x);
+              x += fa_dpp<FA_DPP_ROR4>(x);
+              o[e] = x;
+            }
+            constexpr int kPieces = 4;   // (j, h2), two tile pairs at a time
+            const int at = (2 * j + h2) % kPieces;
+            piece = at == 0 || bb_r == at ? o : piece;
+            if (at == kPieces - 1 && valid_r)
+              gl[(2 * (j - 1 + (bb_r >> 1)) + (lg >> 1)) * kCols * 4 + 2 * (lg & 1) + (bb_r & 1)] = piece;
+          } else {
+            if (valid_r) gl[(2 * j + (lg >> 1)) * kCols * 4 + 2 * (lg & 1) + h2] = o;
+          }
         }
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
@@ -928,7 +958,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         float* on = p.pon + base * p.D;
 #pragma unroll
         for (int f = 0; f < VMAX; ++f)
-          if (f < ndg) *(float4v*)&on[f * 16 + 4 * lg] = c_none ? float4v{0.f, 0.f, 0.f, 0.f} : oacc[f];
+          if (f < ndg) *(float4v*)&on[f * 16 + 4 * lg] = c_none ? float4v{0.f, 0.f, 0.f, 0.f} : SUB ? oacc[f] * wgt : oacc[f];
       }
     }
   }
