@@ -71,8 +71,8 @@ struct PrepArgs {
   const int32_t* kn_h;
   // fused step: the two meeting counters of every (batch group, KV head), cleared here for the launch behind
   unsigned* team_cnt;
-  // a batch of one sequence whose mid rows run as four sub-splits per workgroup (SUB instances of the mid-row kernel):
-  // the stored query dims go out four times, once for the columns of each sub-split
+  // sub-splits a workgroup of the mid rows runs per batch element (SUB instances of the mid-row kernel: four for one sequence,
+  // two for two; otherwise 1): the stored query dims go out once for the columns of each of them
   int sub;
   // A rank-1 update the K coefficients are still owed (the row that left the window, see fa_decode_args.upd_*): every
   // coefficient is read here by exactly one thread, which adds the row's term, writes the coefficient back and goes
@@ -141,9 +141,9 @@ __device__ __forceinline__ void decode_prep_body(const PrepArgs<E>& pa, int bx, 
 #pragma unroll
   for (int i = 0; i < kGMax / 2; ++i)
     if (2 * i < G) qv[i] = q[((int64_t)b * Hq + h * G + min(g0 + 2 * i, G - 1)) * D + (col - h * D)];
-  // the column's query head and the slot it belongs to: a batch element of the group, or (one sequence) a sub-split
-  // (sub-splits keep four columns each, however many heads there are)
-  const int qslot = pa.sub ? qlc >> 2 : qlc / G, qcol = pa.sub ? qlc & 3 : qlc - qslot * G, qg = min(qcol, G - 1);
+  // the column's query head and the slot it belongs to: a batch element of the group, or a sub-split of one (slots of
+  // sub-splits keep four columns each, however many heads there are; 4 / sub batch elements, then their next sub-splits)
+  const int qslot = pa.sub > 1 ? qlc >> 2 : qlc / G, qcol = pa.sub > 1 ? qlc & 3 : qlc - qslot * G, qg = min(qcol, G - 1);
   E qn[8];
   if (kn_len > 0) {
     const E* qr = q + ((int64_t)b * Hq + h * G + qg) * D - h * D;
@@ -164,7 +164,7 @@ __device__ __forceinline__ void decode_prep_body(const PrepArgs<E>& pa, int bx, 
   if constexpr (UPD)
     if (g0 == 0) s_ue[j] = ue;
   if (kn_len > 0) {
-    for (int sl = pa.sub ? 0 : qbb, last = pa.sub ? 3 : qbb; sl <= last; ++sl) {
+    for (int sl = qbb; sl < 4; sl += 4 / pa.sub) {
       union { E e[8]; uint4 raw; } o;
 #pragma unroll
       for (int e = 0; e < 8; ++e) o.e[e] = qslot == sl && qcol < G && qj0 + e < kn_len ? qn[e] : E();
@@ -2244,10 +2244,12 @@ int launch_all(const fa_decode_args& a, const Plan& p, bool p_il_fast, float sm_
   uint16_t wg_map[fa_mfma::kFusedMaxWgs] = {};
   // (the sink/window tiles must be in front of the mid rows for the merge to run inside that launch)
   const bool fused = sizeof(E) == 2 && (fuse_il || p.n_il_split == 0) && fused_merge_plan(a, p, wg_map, st);
-  // one sequence: its mid rows as four sub-splits per workgroup in the places of four batch elements
+  // one sequence: its mid rows as four sub-splits per workgroup in the places of four batch elements; two: two of each
+  // (a layer's step, update and all, with one sub-split each / two: two sequences of 32k 68.5 / 59.5 us, of 100k with 100 of 128
+  // dims compressed 114 / 89.5, of 3k 34.4 / 33.7; three and four fill the columns as they are)
   const bool one_pass = p.path == Path::Mfma && fa_mfma::table_slices(a.N) == 4;
-  const bool sub = fused && one_pass && a.B == 1 && !(a.no_fuse & 2);
-  g_last_call_fused = fused ? (sub ? 2 : 1) : 0;
+  const int nsub = fused && one_pass && a.B <= 2 && !(a.no_fuse & 2) ? 4 / a.B : 1;
+  g_last_call_fused = fused ? (nsub == 4 ? 2 : 1) : 0;
   // A rank-1 update the coefficients are still owed: the query preparation applies it to the K coefficients it streams,
   // the merge inside the mid-row launch to the V coefficients; where those do not run it gets a launch of its own
   if (a.upd_k_row && a.Ck > 0 && p.n_mid_split <= 0) {
@@ -2267,7 +2269,7 @@ int launch_all(const fa_decode_args& a, const Plan& p, bool p_il_fast, float sm_
                    a.Hq, a.Hkv, a.D, a.N, a.Ck, sm_log2e,
                    p.path == Path::Mfma ? W : nullptr, p.nbpg, p.path == Path::Mfma ? fa_mfma::table_slices(a.N) : 0, p.ks,
                    p.path == Path::Mfma ? (E*)(ws + p.off_qn) : nullptr, a.kn_list, a.kn_h_list,
-                   fused ? (unsigned*)(ws + p.off_cnt) + (size_t)a.B * a.Hkv : nullptr, sub ? 1 : 0,
+                   fused ? (unsigned*)(ws + p.off_cnt) + (size_t)a.B * a.Hkv : nullptr, nsub,
                    a.Ck > 0 ? (const E*)a.upd_k_row : nullptr, a.upd_batch_stride, a.upd_phase, a.upd_T};
     const int n_prep = fa_cdiv(2 * a.N, kPrepRows);
     if (fuse_il) {
@@ -2305,7 +2307,10 @@ int launch_all(const fa_decode_args& a, const Plan& p, bool p_il_fast, float sm_
         const int NSL = table_slices(a.N);
         mp.tabET = mp.tabE + NSL * 2 * KS * 64;
         mp.rot = (const float2v*)(mp.tabET + NSL * 2 * KS * 64);
-        mp.pm = mm; mp.pd = md; mp.pg = mg; mp.pon = mon;
+        mp.pm = mm; mp.pd = md; mp.pg = mg;
+        // (two sequences: the outputs of four slots lie in the half of the g partials that the folded columns leave free -
+        // 4 Hq rows of D against Hkv * 8 columns of 2 N, N >= 128 and at most four heads of 128 dims to a KV head)
+        mp.pon = nsub == 2 ? mg + (size_t)a.Hkv * 8 * p.n_mid_split * 2 * a.N : mon;
         mp.scores = (float*)(ws + p.off_scores);
         mp.merge_count = fused ? nullptr : (unsigned*)(ws + p.off_cnt);
         if (fused) {
@@ -2328,7 +2333,7 @@ int launch_all(const fa_decode_args& a, const Plan& p, bool p_il_fast, float sm_
         mp.sm_log2e = sm_log2e;
         if (ev) hipEventRecord(ev[1], st);
         const bool wide = a.mid_max_k_pad > 64 || a.mid_max_v_pad > 64;
-        launch_mid_rows<E>(mp, MidLaunch{p.n_wg, p.n_groups, KS, wide, NSL > 4, fused, sub}, st);
+        launch_mid_rows<E>(mp, MidLaunch{p.n_wg, p.n_groups, KS, wide, NSL > 4, fused, nsub}, st);
       }
     } else {
       const bool paged = a.mid_layout == FA_MID_PAGED;

@@ -150,11 +150,11 @@ struct FusedShare {
 // split classes of the g sums and the sink/window sums), where each dim comes from, statistics of the compressed dims
 __host__ __device__ __forceinline__ int fused_tail_lds_floats(int n_parts) { return 2 * 16 * n_parts + 32 + 2048 + 8192 + 128 + 384; }
 
-// SUB: the team belongs to one batch element whose mid rows were cut into four sub-splits per workgroup (see the
+// NSUB: the team belongs to 4 / NSUB batch elements whose mid rows were cut into NSUB sub-splits per workgroup (see the
 // mid-row kernel).  The sub-splits of a head have met before they were stored, all but the outputs of the stored dims, which
-// share the head's reference: four columns, the query heads, and the threads that would have taken the other batch elements
+// share the head's reference: four columns a batch element, and the threads that would have taken the other batch elements
 // take further row classes instead.
-template <bool SUB, typename P>
+template <int NSUB, typename P>
 __device__ __forceinline__ FusedShare fused_share(const P& p, int vc0, int vc_len, int split, int n_s, int b0, int nb, int KS,
                                                   int tid) {
   FusedShare f;
@@ -173,9 +173,10 @@ __device__ __forceinline__ FusedShare fused_share(const P& p, int vc0, int vc_le
   f.nqp = nqp;
   f.lq = lq;
   f.q = tid & (nqp - 1);
-  f.bbslot = SUB ? 0 : (tid >> lq) & 3;
-  f.rc = SUB ? tid >> lq : tid >> (lq + 2);
-  f.n_rc = (SUB ? 512 : 128) >> lq;
+  constexpr int kBat = 4 / NSUB, kBatLog = NSUB == 1 ? 2 : NSUB == 2 ? 1 : 0;
+  f.bbslot = (tid >> lq) & (kBat - 1);
+  f.rc = tid >> (lq + kBatLog);
+  f.n_rc = 512 >> (lq + kBatLog);
   f.v_on = f.vc_len > 0 && f.bbslot < nb && 4 * f.q < f.vc_len && f.t1 > f.t0;
   // every thread reads 16 bytes per row (4-byte aligned: the head's columns start anywhere); the group that would
   // reach past the head's columns starts early instead and its values are moved down when they are used
@@ -204,7 +205,7 @@ __device__ __forceinline__ float4v fused_v_place(float4v v, int back) {
 // waited for.  P: the mid-row kernel's parameter block (pm, pd, pg, pon, n_split, shape) with the FusedParams in
 // P::fz.  sm: LDS of at least fused_tail_lds_floats(n_split + n_il) floats that no wave uses any more.  KS: ksteps per
 // frequency slice.  s_own: four more floats of LDS per thread (free behind the page loops as well).
-template <typename E, bool SUB, bool UPD, typename P>
+template <typename E, int NSUB, bool UPD, typename P>
 __device__ __forceinline__ void fused_merge_tail(const P& p, float* sm, float* s_own, int* s_flag, const FusedShare& f, int grp,
                                                  int h, int split, int n_s, int b0, int nb, int KS) {
   constexpr int D = kFusedD, GS = kFusedG;
@@ -221,9 +222,10 @@ __device__ __forceinline__ void fused_merge_tail(const P& p, float* sm, float* s
   float* s_stat = (float*)(s_src + 128);   // [3][128] scale, avg_u, avg_d of the compressed dims of the column share
   unsigned* cnt = p.fz.cnt + (int64_t)(grp * p.Hkv + h) * 2;
   const int vn0 = p.vn_h[h], vn_len = p.vn_h[h + 1] - vn0;
-  // column slot c16 = 4 * batch element of the group + query head (SUB: one batch element; the outputs of the stored dims of
-  // sub-split j are those of the virtual batch element 4 b0 + j)
-  constexpr int kSlots = SUB ? 4 : 16, kTile = kSlots * 16;   // column slots; floats of a g tile
+  // column slot c16 = 4 * batch element of the group + query head (NSUB > 1: the outputs of the stored dims of sub-split j are
+  // those of the virtual batch element 4 / NSUB * j + batch element)
+  constexpr bool SUB = NSUB > 1;
+  constexpr int kBat = 4 / NSUB, kSlots = 4 * kBat, kTile = kSlots * 16;   // batch elements, column slots; floats of a g tile
   auto slot_ok = [&](int c16) { return (c16 >> 2) < nb && (c16 & 3) < G; };
   auto qrow_of = [&](int c16) { return (int64_t)(b0 + (c16 >> 2)) * p.Hq + h * G + (c16 & 3); };
   // column share: the columns are query heads g_lo .. g_lo + ncol - 1 of batch element cbb (the host only fuses when
@@ -334,7 +336,8 @@ __device__ __forceinline__ void fused_merge_tail(const P& p, float* sm, float* s
     const int ntb = min(kFusedTileBlock, f.t1 - f.t0);
     const int n_items = kSlots * 4 * ntb, n_cls = 512 / n_items;
     const int item = tid % n_items, cls = tid / n_items;
-    if (cls < n_cls && (item % (kSlots * 4)) / 4 < nb * G) {
+    const int col = (item % (kSlots * 4)) / 4;
+    if (cls < n_cls && (SUB ? slot_ok(col) : col < nb * G)) {
       const float* gp = g_team + (f.t0 + item / (kSlots * 4)) * kTile + (item % (kSlots * 4)) * 4;
 #pragma unroll
       for (int u = 0; u < kFusedGPre; ++u)
@@ -421,14 +424,15 @@ __device__ __forceinline__ void fused_merge_tail(const P& p, float* sm, float* s
 #pragma unroll
     for (int u = 0; u < kPre; ++u) il_pre[u] = *(const float4v*)(il_src + (int64_t)min(x_cls + 4 * u, n_il - 1) * D);
   }
-  // (SUB: class j takes all splits of sub-split j, whose partials are those of virtual batch element 4 b0 + j - up to
-  // 32 of them, a chain of dependent loads if one thread walks them all.  A workgroup with one or two columns has
+  // (SUB: a sub-split's classes take all its splits - up to 32 of them, a chain of dependent loads if one thread walks
+  // them all.  A workgroup with one or two columns has
   // threads for four: the spare ones help, thread column x_cl working for column x_cl % ncol on every on_h-th split.)
   const int on_h = (SUB && (ncol == 1 || ncol == 2)) ? 4 / ncol : 1;
   const int on_col = on_h > 1 ? x_cl % ncol : x_cl, on_hlp = on_h > 1 ? x_cl / ncol : 0;
   const bool on_on = on_col < ncol && 4 * x_d4 < vn_len;
-  const int on_first = SUB ? on_hlp : x_cls, on_step = SUB ? on_h : 4;
-  const float* on_src = p.pon + (SUB ? (int64_t)(4 * b0 + x_cls) * p.Hq + h * G + g_lo + on_col : qrow0 + on_col) * NS * D + 4 * x_d4;
+  constexpr int kPerSub = 4 / NSUB;   // classes of a sub-split
+  const int on_first = x_cls / NSUB + kPerSub * on_hlp, on_step = kPerSub * on_h;
+  const float* on_src = p.pon + (SUB ? (int64_t)(kBat * (x_cls % NSUB) + cbb) * p.Hq + h * G + g_lo + on_col : qrow0 + on_col) * NS * D + 4 * x_d4;
   if (on_on) {
 #pragma unroll
     for (int u = 0; u < kPre; ++u) on_pre[u] = *(const float4v*)(on_src + (int64_t)min(on_first + on_step * u, n_s - 1) * D);
@@ -448,7 +452,7 @@ __device__ __forceinline__ void fused_merge_tail(const P& p, float* sm, float* s
       const int tl = item / (kSlots * 4), rem = item % (kSlots * 4), lc = rem >> 2, lgp = rem & 3;
       const int c16 = SUB ? lc : (lc / G) * 4 + (lc % G);
       if (tb > f.t0) __syncthreads();   // the block before is done with s_g and s_red
-      const bool col_ok = lc < nb * G;   // (columns past the group hold nothing; their slots of s_g are never read)
+      const bool col_ok = SUB ? slot_ok(lc) : lc < nb * G;   // (columns past the group hold nothing; their slots of s_g are never read)
       auto put_g = [&](const float4v& a4) {
         const int rb = tl * 16 + 2 * lgp;
         s_g[rb * 16 + c16] = a4[0]; s_g[(rb + 8) * 16 + c16] = a4[1];
@@ -573,7 +577,7 @@ __device__ __forceinline__ void fused_merge_tail(const P& p, float* sm, float* s
   if (has_coef) {
     if (f.v_on) {
 #pragma unroll
-      for (int g = 0; g < GS; ++g) *(float4v*)(s_red + ((f.rc * (SUB ? 1 : 4) + f.bbslot) * GS + g) * 4 * f.nqp + 4 * f.q) = acc[g];
+      for (int g = 0; g < GS; ++g) *(float4v*)(s_red + ((f.rc * kBat + f.bbslot) * GS + g) * 4 * f.nqp + 4 * f.q) = acc[g];
     }
     __syncthreads();
     float* pc = pc_team + (int64_t)split * 16 * 128;

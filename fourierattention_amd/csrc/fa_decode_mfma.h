@@ -275,22 +275,26 @@ struct MidParams {
 //         per frame.
 // FUSE (MODE 0 and the value pass, MODE 2): the launch merges its own partials and writes the output rows, see fa_decode_fused.h; the
 // workgroups are then numbered through p.fz.wg_map so that the splits of a (batch group, KV head) share one die.
-// SUB (FUSE only, a batch of one sequence, at most four query heads per KV head): a single batch element would
-// leave twelve of the sixteen matrix-core columns and three of the four page streams of a workgroup idle.  The
-// workgroup's pages are cut into four sub-splits instead, which take the places of four batch elements: wave i
-// streams the pages of sub-split i, column 4 j' + g (j' = sub-split) holds query head g with its weights W' rotated to the
-// first frame of sub-split j', and every column keeps its own softmax reference, g history and outputs.  Behind the loop the
-// columns of a head are brought to one reference and added up (the outputs of the stored dims leave one by one, as
-// "virtual batch elements" j' of the partial buffers).  The page loop has a quarter of the trips.  Pages past the end of a sub-split are fetched from a
+// SUB (FUSE only, a batch of one or two sequences, at most four query heads per KV head): a single batch element would
+// leave twelve of the sixteen matrix-core columns and three of the four page streams of a workgroup idle, two of them half.
+// The workgroup's pages are cut into NSUB = 4 resp. 2 sub-splits instead, so that four slots take the places of four batch
+// elements: slot s = batch element s % (4 / NSUB), sub-split s / (4 / NSUB).  Wave i streams the pages of slot i, column
+// 4 s + g holds query head g with its weights W' rotated to the first frame of its sub-split, and every column keeps its own
+// softmax reference, g history and outputs.  Behind the loop the columns of a head are brought to one reference and added up
+// (the outputs of the stored dims leave one by one, as "virtual batch elements" s of the partial buffers).  The page loop has
+// 1 / NSUB of the trips.  Pages past the end of a sub-split are fetched from a
 // valid page and masked.
 // UPD (FUSE only): the tail also applies a pending rank-1 update to the V coefficients of its row share.
-template <typename E, int KS, int KMAX, int VMAX, int NST, int MODE = 0, bool FUSE = false, bool SUB = false, bool UPD = false>
+template <typename E, int KS, int KMAX, int VMAX, int NST, int MODE = 0, int NSUB = 1, bool FUSE = false, bool SUB = false,
+          bool UPD = false>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void decode_mid_mfma_kernel(
     const MidParams<E> p) {
   static_assert(!FUSE || MODE == 0 || MODE == 2, "the fused merge runs behind the one-pass pipeline or behind the value pass");
   static_assert(!SUB || MODE == 0, "sub-splits belong to the one-pass pipeline");
   static_assert(!UPD || MODE == 0, "the pending update keeps its row in the LDS of the score partials");
   static_assert(!SUB || FUSE, "sub-splits end in the fused merge");
+  static_assert(SUB ? NSUB == 2 || NSUB == 4 : NSUB == 1, "two or four sub-splits");
+  constexpr int kBat = 4 / NSUB;   // SUB: batch elements of the group
   static_assert(!UPD || FUSE, "the pending update rides in the fused merge");
   constexpr int NSL = MODE == 0 ? kFreqWaves : 2 * kFreqWaves;   // frequency slices
   using M = Mma<E>;
@@ -335,17 +339,17 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int G = p.G, N = p.N;
   const int b0 = grp * p.nbpg;
   const int nb_real = min(p.nbpg, p.B - b0);
-  const int nb = SUB ? 4 : nb_real;   // SUB: four sub-splits of the one batch element in the places of batch elements
-  // this lane's column: batch element of the group (SUB: sub-split, four columns each) and query head
+  const int nb = SUB ? 4 : nb_real;   // SUB: slots in the places of batch elements
+  // this lane's column: batch element of the group (SUB: slot, four columns each) and query head
   const int bb_r = SUB ? lc >> 2 : lc / G, g_r = SUB ? lc & 3 : lc - bb_r * G;
   const bool valid_r = SUB ? g_r < G : lc < nb * G;
-  // the query row of this lane's column; the row of its stored-dim outputs (SUB: virtual batch element 4 b + sub-split)
-  const int64_t qrow = valid_r ? ((int64_t)(b0 + (SUB ? 0 : bb_r)) * p.Hq + h * G + g_r) : 0;
-  const int64_t prow = !SUB ? qrow : valid_r ? ((int64_t)(b0 * 4 + bb_r) * p.Hq + h * G + g_r) : 0;
+  // the query row of this lane's column; the row of its stored-dim outputs (SUB: virtual batch element = slot)
+  const int64_t qrow = valid_r ? ((int64_t)(b0 + (SUB ? bb_r % kBat : bb_r)) * p.Hq + h * G + g_r) : 0;
+  const int64_t prow = !SUB ? qrow : valid_r ? ((int64_t)bb_r * p.Hq + h * G + g_r) : 0;
   if (MODE != 1 && split == 0 && tid < nb_real && p.merge_count) p.merge_count[(b0 + tid) * p.Hkv + h] = 0u;
   const int fbase = sl * 16 * KS;
   const bool has_mn = sl < nb && sl < kFreqWaves;
-  const int my_b = b0 + (has_mn && !SUB ? sl : 0);
+  const int my_b = b0 + (!has_mn ? 0 : SUB ? sl % kBat : sl);
   const int stw = has_mn ? w & 3 : 0;   // page stage of this wave
 
   const int n_tiles = (p.L_m + 31) >> 5;
@@ -353,11 +357,11 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int t_beg = split * tiles_per_split;
   const int t_end = min(n_tiles, t_beg + tiles_per_split);
   const int n_pages = t_end > t_beg ? t_end - t_beg : 0;
-  // trips of the page loop; SUB: a quarter of the pages per sub-split, the sub-split of this wave (wave-uniform) and
+  // trips of the page loop; SUB: the pages of a sub-split, the sub-split of this wave (wave-uniform) and
   // of this lane's column start at page w_beg / c_beg of the split, and the column's has c_n pages
-  const int n_it = SUB ? (n_pages + 3) >> 2 : n_pages;
-  const int w_beg = SUB ? min(n_pages, (w & 3) * n_it) : 0;
-  const int c_beg = SUB ? min(n_pages, min(bb_r, 3) * n_it) : 0;
+  const int n_it = SUB ? (n_pages + NSUB - 1) / NSUB : n_pages;
+  const int w_beg = SUB ? min(n_pages, (w & 3) / kBat * n_it) : 0;
+  const int c_beg = SUB ? min(n_pages, bb_r / kBat * n_it) : 0;
   const int c_n = SUB ? min(n_pages, c_beg + n_it) - c_beg : n_pages;
   const int t_beg_w = t_beg + w_beg;
   // fused merge: the head's compressed V dims (offset into the lists, count), needed behind the page loop
@@ -421,8 +425,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     // the lanes of other batch elements and past the head's count): requested behind the weights
     vec8 Qb[KMAX];
     {
-      // (SUB: every sub-split starts from the weights of its query head, column g of the one batch element)
-      const float2v* wl = (const float2v*)p.W + ((int64_t)((grp * p.Hkv + h) * NSL + sl) * 2 * KS * 2) * 64 + ((SUB ? g_r : lc) * 4 + lg);
+      // (SUB: every sub-split starts from the weights of its query head, column g of its batch element)
+      const float2v* wl = (const float2v*)p.W + ((int64_t)((grp * p.Hkv + h) * NSL + sl) * 2 * KS * 2) * 64 + ((SUB ? bb_r % kBat * G + min(g_r, G - 1) : lc) * 4 + lg);
       float2v wc2[2 * KS], ws2[2 * KS];
 #pragma unroll
       for (int rt = 0; rt < 2 * KS; ++rt) {
@@ -876,21 +880,21 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 
     // ---- partials of this split ------------------------------------------------------
     float dsum = fa_rows_sum(d_run);
-    // SUB: a column whose sub-split has no page has seen masked scores only; what it accumulated is not a number.  The four
-    // sub-splits of a head are brought to one reference and added up here, by lane exchanges: a quarter of the partials to
-    // store, to wait for and to read back (one sequence of 32k tokens: 36.5 - 38.2 us a launch -> 34.2 - 35.2).
+    // SUB: a column whose sub-split has no page has seen masked scores only; what it accumulated is not a number.  The
+    // sub-splits of a head are brought to one reference and added up here, by lane exchanges: a half or a quarter of the
+    // partials to store, to wait for and to read back (one sequence of 32k tokens: 36.5 - 38.2 us a launch -> 34.2 - 35.2).
     const bool c_none = SUB && c_n == 0;
     float m_out = m_run, wgt = 1.f;
     if constexpr (SUB) {
       m_out = c_none ? -INFINITY : m_run;
-      m_out = fa_fmax(m_out, fa_dpp<FA_DPP_ROR8>(m_out));
-      m_out = fa_fmax(m_out, fa_dpp<FA_DPP_ROR4>(m_out));
+      m_out = fa_fmax(m_out, fa_dpp<FA_DPP_ROR8>(m_out));   // slots s and s + 2
+      if (NSUB == 4) m_out = fa_fmax(m_out, fa_dpp<FA_DPP_ROR4>(m_out));
       wgt = c_none || m_run == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_run - m_out);
       dsum = c_none ? 0.f : dsum * wgt;
       dsum += fa_dpp<FA_DPP_ROR8>(dsum);
-      dsum += fa_dpp<FA_DPP_ROR4>(dsum);
+      if (NSUB == 4) dsum += fa_dpp<FA_DPP_ROR4>(dsum);
     }
-    if (valid_r && (!SUB || bb_r == 0)) {
+    if (valid_r && (!SUB || bb_r < kBat)) {
       const int64_t base = qrow * p.n_split + split;
       if (sl == 0 && lg == 0) {
         p.pm[base] = m_out;
@@ -902,11 +906,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       // reads: [batch group][KV head][split][slice][row tile rt][column][lane group lg'] x {cos f, sin f, cos f+1,
       // sin f+1} with f = 8 rt + 2 lg' (the layout of the weights W).  This lane holds the frequencies
       // 16 j + 4 lg + v, v = 0 .. 3, of tile pair j: rt = 2 j + lg / 2, lg' = 2 (lg % 2) + v / 2.  (Columns past
-      // the group store nothing: a batch of three leaves seven of the sixteen idle.)  SUB: four columns, the query heads;
-      // every lane of a head holds the sums of its sub-splits and stores one of four neighbouring pieces.
-      constexpr int kCols = SUB ? 4 : 16;
+      // the group store nothing: a batch of three leaves seven of the sixteen idle.)  SUB: four columns a
+      // batch element; every lane of a head holds the sums of its sub-splits and stores one of NSUB neighbouring pieces.
+      constexpr int kCols = 16 / NSUB;
+      const int sub = bb_r / kBat;
       float4v* gl = (float4v*)p.pg + ((((int64_t)(grp * p.Hkv + h) * p.n_split + split) * NSL + sl) * 2 * KS) * kCols * 4 +
-                    (SUB ? g_r : lc) * 4;
+                    (SUB ? 4 * (bb_r % kBat) + g_r : lc) * 4;
       // twice the centre of the last frame, in half tokens
       const int64_t c2 = (int64_t)64 * (t_beg + c_beg + (n_it > 0 ? ((n_it - 1) & ~1) : 0) + 1) - 1;
       float sn[4], co[4], s16, c16;   // stepped phases, as for the first frame of the score waves
@@ -931,14 +936,13 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             for (int e = 0; e < 4; ++e) {
               float x = c_none ? 0.f : o[e] * wgt;
               x += fa_dpp<FA_DPP_ROR8>(x);
-              x += fa_dpp<FA_DPP_ROR4>(x);
+              if (NSUB == 4) x += fa_dpp<FA_DPP_ROR4>(x);
               o[e] = x;
             }
-            constexpr int kPieces = 4;   // (j, h2), two tile pairs at a time
-            const int at = (2 * j + h2) % kPieces;
-            piece = at == 0 || bb_r == at ? o : piece;
-            if (at == kPieces - 1 && valid_r)
-              gl[(2 * (j - 1 + (bb_r >> 1)) + (lg >> 1)) * kCols * 4 + 2 * (lg & 1) + (bb_r & 1)] = piece;
+            const int at = (2 * j + h2) % NSUB;   // pieces are (j, h2), two or one tile pairs at a time
+            piece = at == 0 || sub == at ? o : piece;
+            if (at == NSUB - 1 && valid_r)
+              gl[(2 * (j - (NSUB / 2 - 1) + (sub >> 1)) + (lg >> 1)) * kCols * 4 + 2 * (lg & 1) + (sub & 1)] = piece;
           } else {
             if (valid_r) gl[(2 * j + (lg >> 1)) * kCols * 4 + 2 * (lg & 1) + h2] = o;
           }
@@ -963,8 +967,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
   }
   if constexpr (FUSE) {
-    const FusedShare fs = fused_share<SUB>(p, fz_vc0, fz_vc_len, split, p.st.n[h], b0, nb_real, KS, tid);
-    fused_merge_tail<E, SUB, UPD>(p, (float*)&s_stage[0][0][0], &s_part[0][0][0], &s_team_flag, fs, grp, h, split, p.st.n[h], b0, nb_real, KS);
+    const FusedShare fs = fused_share<NSUB>(p, fz_vc0, fz_vc_len, split, p.st.n[h], b0, nb_real, KS, tid);
+    fused_merge_tail<E, NSUB, UPD>(p, (float*)&s_stage[0][0][0], &s_part[0][0][0], &s_team_flag, fs, grp, h, split, p.st.n[h], b0, nb_real, KS);
   }
 }
 

@@ -14,7 +14,7 @@ struct MidLaunch {
   bool wide;            // a head stores more than 64 K or V dims
   bool two_pass;        // 1024 frequencies: a score pass, then a value pass over the same pages
   bool fused;           // the (last) launch merges its own partials; its workgroups are numbered through mp.fz.wg_map
-  bool sub;             // ... and runs four sub-splits per workgroup (a batch of one sequence)
+  int nsub;             // ... and runs as many sub-splits per workgroup (four for one sequence, two for two, else one)
 };
 
 template <typename E>
@@ -29,11 +29,11 @@ void launch_mid_mfma_two_pass(const MidParams<E>& mp, const MidLaunch& ml, hipSt
   dim3 grid(ml.n_wg, ml.n_groups), flat(ml.n_wg * ml.n_groups);
   if (ml.wide) {
     decode_mid_mfma_kernel<E, 8, 4, 8, 3, 1><<<grid, 512, 0, st>>>(mp);
-    if (ml.fused) decode_mid_mfma_kernel<E, 8, 4, 8, 3, 2, true><<<flat, 512, 0, st>>>(mp);
+    if (ml.fused) decode_mid_mfma_kernel<E, 8, 4, 8, 3, 2, 1, true><<<flat, 512, 0, st>>>(mp);
     else decode_mid_mfma_kernel<E, 8, 4, 8, 3, 2><<<grid, 512, 0, st>>>(mp);
   } else {
     decode_mid_mfma_kernel<E, 8, 2, 4, 4, 1><<<grid, 512, 0, st>>>(mp);
-    if (ml.fused) decode_mid_mfma_kernel<E, 8, 2, 4, 4, 2, true><<<flat, 512, 0, st>>>(mp);
+    if (ml.fused) decode_mid_mfma_kernel<E, 8, 2, 4, 4, 2, 1, true><<<flat, 512, 0, st>>>(mp);
     else decode_mid_mfma_kernel<E, 8, 2, 4, 4, 2><<<grid, 512, 0, st>>>(mp);
   }
 }
@@ -45,16 +45,20 @@ void launch_mid_mfma_ks(const MidParams<E>& mp, const MidLaunch& ml, hipStream_t
     grid = dim3(ml.n_wg * ml.n_groups);   // numbered through wg_map
     const bool upd = mp.fz.upd_row != nullptr;   // (instances of their own, like the query preparation's)
     auto go = [&](auto sub_tag, auto upd_tag) {
-      constexpr bool S = decltype(sub_tag)::value, U = decltype(upd_tag)::value;
+      constexpr int S = decltype(sub_tag)::value;
+      constexpr bool U = decltype(upd_tag)::value;
       if (ml.wide)
-        decode_mid_mfma_kernel<E, KS, 4, 8, 2, 0, true, S, U><<<grid, 512, 0, st>>>(mp);
+        decode_mid_mfma_kernel<E, KS, 4, 8, 2, 0, S, true, (S > 1), U><<<grid, 512, 0, st>>>(mp);
       else
-        decode_mid_mfma_kernel<E, KS, 2, 4, 2, 0, true, S, U><<<grid, 512, 0, st>>>(mp);
+        decode_mid_mfma_kernel<E, KS, 2, 4, 2, 0, S, true, (S > 1), U><<<grid, 512, 0, st>>>(mp);
     };
-    if (ml.sub && upd) go(std::true_type{}, std::true_type{});
-    else if (ml.sub) go(std::true_type{}, std::false_type{});
-    else if (upd) go(std::false_type{}, std::true_type{});
-    else go(std::false_type{}, std::false_type{});
+    auto by_subs = [&](auto upd_tag) {
+      if (ml.nsub == 4) go(std::integral_constant<int, 4>{}, upd_tag);
+      else if (ml.nsub == 2) go(std::integral_constant<int, 2>{}, upd_tag);
+      else go(std::integral_constant<int, 1>{}, upd_tag);
+    };
+    if (upd) by_subs(std::true_type{});
+    else by_subs(std::false_type{});
   } else if (ml.wide) {
     decode_mid_mfma_kernel<E, KS, 4, 8, 2><<<grid, 512, 0, st>>>(mp);
   } else {

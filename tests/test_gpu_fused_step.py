@@ -38,6 +38,13 @@ CASES = [
     (torch.bfloat16, 4, 24, 4, 40, 2048, 6000, U, U, 1),
     (torch.float16, 2, 32, 4, 64, 2048, 5000, [64, 0, 128, 30, 64, 64, 100, 64], [1, 64, 2, 3, 128, 64, 0, 64], 1),
     (torch.bfloat16, 1, 32, 4, 64, 2048, 7000, U, U, 1),                                   # one sequence there: no sub-splits either
+    # two sequences: two sub-splits of each (reported as 1, like every launch that merges; the way without them runs as well)
+    (torch.bfloat16, 2, 32, 4, 64, 1024, 9000, U, U, 1),
+    (torch.bfloat16, 2, 32, 4, 60, 1024, 5000, [0, 128, 64, 3, 125, 127, 64, 96], [128, 0, 61, 64, 2, 64, 127, 1], 1),
+    (torch.float16, 2, 24, 4, 48, 512, 3011, U, [40] * 8, 1),                              # three query heads per KV head
+    (torch.bfloat16, 2, 32, 4, 33, 256, 4000, U, [120, 125, 128, 112, 64, 127, 100, 116], 1),   # 128 frequencies: the smallest g
+    (torch.bfloat16, 2, 8, 4, 32, 256, 700, U, U, 1),                                      # one query head; splits of a few pages
+    (torch.float16, 2, 32, 4, 32, 256, 330, U, U, 1),                                      # two pages of mid rows: empty sub-splits
 ]
 
 
