@@ -114,7 +114,15 @@ __global__ __launch_bounds__(256) void spectral_pack_kernel(
 //              column tile that two heads share is written by both, each its own 16-byte pieces),
 //   partials   sum / max / min of every compressed column over the block's tokens (what col_stats_partial_kernel
 //              leaves, finished by the same final launch).
-constexpr int kPackPages = 4;   // pages per block
+// Blocks take up to four pages one after the other; a prompt too short to fill the chip that way - four blocks for every
+// compute unit - takes fewer a block.  Packing and compressing, us, four pages -> by this rule: 3001 tokens x 4 sequences
+// x 8 heads 55.6 -> 50.8, 3000 x 1 x 8 32.7 -> 27.3, 1800 x 1 x 8 29.5 -> 24.4; from 1024 blocks on (5000 x 8 x 8,
+// 32768 x 1 x 8 and 12000 x 2 x 8) the rule is the same as before: 57, 77.6 and 102.6 both.
+inline int pack_pages_per_block(int n_pages, int heads_x_batch) {
+  int per = 4;
+  while (per > 1 && (int64_t)fa_cdiv(n_pages, per) * heads_x_batch < 1024) per >>= 1;
+  return per;
+}
 
 template <typename E>
 struct PrefillPackParams {
@@ -128,7 +136,7 @@ struct PrefillPackParams {
   const int32_t* c_list; const int32_t* c_h;                         // compressed dims, likewise
   half8* packed;                // [B][CT][KS32][64]
   float* psum; float* pmax; float* pmin;   // [B][n_blocks][Mc]
-  int Mc, CT, KS32, n_pages, n_blocks, Hkv, D, is_v;
+  int Mc, CT, KS32, n_pages, per_block, n_blocks, Hkv, D, is_v;
   SpectralTable table;          // the blocks of x behind n_blocks evaluate the basis of the products
 };
 
@@ -156,8 +164,8 @@ __global__ __launch_bounds__(256) void prefill_pack_kernel(const PrefillPackPara
   // columns past the last compressed dim in the last column tile belong to nobody: the last head clears them
   const int c_extra = h == p.Hkv - 1 ? p.CT * 16 - p.Mc : 0;
   float sum = 0.f, mx = -INFINITY, mn = INFINITY;   // thread j < c_len: statistics of its column
-  for (int pp = 0; pp < kPackPages; ++pp) {
-    const int page = blockIdx.x * kPackPages + pp;
+  for (int pp = 0; pp < p.per_block; ++pp) {
+    const int page = blockIdx.x * p.per_block + pp;
     if (page >= p.n_pages) break;
     __syncthreads();                                // the tile of the page before has been read (and the lists stored)
     if (page < pages_of_rows) {
@@ -1019,7 +1027,7 @@ int spectral_after_pack(const SpectralPlan& pl, float* c, int B, int Mc, int N, 
 
 struct PrefillPlan {
   SpectralPlan sp;
-  int n_pages, n_blocks;
+  int n_pages;
   size_t off_sum, off_max, off_min, total;
 };
 PrefillPlan prefill_plan(int B, int L, int K_fft, int Mc, int N) {
@@ -1027,12 +1035,13 @@ PrefillPlan prefill_plan(int B, int L, int K_fft, int Mc, int N) {
   p.sp = spectral_plan(B, K_fft, Mc, N);
   const int pages_of_rows = fa_cdiv(L, 32);
   p.n_pages = pages_of_rows > p.sp.KS32 ? pages_of_rows : p.sp.KS32;
-  p.n_blocks = fa_cdiv(p.n_pages, fa_mfma::kPackPages);
+  // (room for as many blocks as the smallest number of KV heads, one, could ask for)
+  const size_t blocks = fa_cdiv(p.n_pages, fa_mfma::pack_pages_per_block(p.n_pages, B));
   size_t o = p.sp.total;
   auto take = [&](size_t bytes) { size_t at = o; o += fa_align_up(bytes, 256); return at; };
-  p.off_sum = take((size_t)B * p.n_blocks * Mc * 4);
-  p.off_max = take((size_t)B * p.n_blocks * Mc * 4);
-  p.off_min = take((size_t)B * p.n_blocks * Mc * 4);
+  p.off_sum = take((size_t)B * blocks * Mc * 4);
+  p.off_max = take((size_t)B * blocks * Mc * 4);
+  p.off_min = take((size_t)B * blocks * Mc * 4);
   p.total = o;
   return p;
 }
@@ -1071,6 +1080,7 @@ extern "C" int fa_prefill_compress(const void* src, int dtype, int64_t src_bs, i
   float* psum = (float*)(ws + pl.off_sum);
   float* pmax = (float*)(ws + pl.off_max);
   float* pmin = (float*)(ws + pl.off_min);
+  const int per_block = pack_pages_per_block(pl.n_pages, Hkv * B), n_blocks = fa_cdiv(pl.n_pages, per_block);
   auto launch = [&](auto tag) {
     using E = decltype(tag);
     PrefillPackParams<E> pp{};
@@ -1079,15 +1089,15 @@ extern "C" int fa_prefill_compress(const void* src, int dtype, int64_t src_bs, i
     pp.n_list = n_list; pp.n_h = n_h; pp.pad_h = pad_h; pp.c_list = c_list; pp.c_h = c_h;
     pp.packed = (half8*)(ws + pl.sp.off_packed);
     pp.psum = psum; pp.pmax = pmax; pp.pmin = pmin;
-    pp.Mc = Mc; pp.CT = pl.sp.CT; pp.KS32 = pl.sp.KS32; pp.n_pages = pl.n_pages; pp.n_blocks = pl.n_blocks;
+    pp.Mc = Mc; pp.CT = pl.sp.CT; pp.KS32 = pl.sp.KS32; pp.n_pages = pl.n_pages; pp.per_block = per_block; pp.n_blocks = n_blocks;
     pp.Hkv = Hkv; pp.D = D; pp.is_v = is_v;
     pp.table = SpectralTable{(half2v*)(ws + pl.sp.off_tab), N, T};
-    prefill_pack_kernel<E><<<dim3(pl.n_blocks + fa_cdiv(table_blocks(N), (int64_t)Hkv * B), Hkv, B), 256, 0, st>>>(pp);
+    prefill_pack_kernel<E><<<dim3(n_blocks + fa_cdiv(table_blocks(N), (int64_t)Hkv * B), Hkv, B), 256, 0, st>>>(pp);
   };
   if (dtype == FA_BF16) launch(bf16_t{}); else launch(f16_t{});
   int rc = spectral_after_pack(pl.sp, coef, B, Mc, N, T, 0, 0, workspace, st);
   if (rc != FA_OK) return rc;
-  fa_stats_finalize_launch(psum, pmax, pmin, avg, max_dev, B, L, Mc, pl.n_blocks, stats_round_dtype, st);
+  fa_stats_finalize_launch(psum, pmax, pmin, avg, max_dev, B, L, Mc, n_blocks, stats_round_dtype, st);
   return fa_check_launch("fa_prefill_compress");
 }
 

@@ -276,6 +276,8 @@ def test_one_full_length_sequence_against_the_oracle(mask, dtype, Hq, S, states,
     (torch.bfloat16, 1, 8, 128, 64, 256, 5000, 1 << 17, [64] * 8, [64] * 8),   # several chunks of the transform
     (torch.bfloat16, 2, 8, 128, 64, 128, 3000, 1 << 17, [83, 116, 117, 96, 122, 88, 116, 81],
      [120, 128, 110, 111, 8, 122, 128, 92]),                                   # head counts of a searched mask: odd totals
+    (torch.float16, 4, 8, 64, 32, 64, 2990, 1 << 17, [30] * 8, [64] * 7 + [2]),      # two pages a block, the last has one
+    (torch.bfloat16, 8, 8, 64, 32, 64, 2500, 1 << 17, [30] * 8, [64, 0] * 4),        # four pages a block, the last has one
 ])
 def test_prefill_in_one_pass_matches_the_separate_calls(dtype, B, Hkv, D, W, M, prompt, t_c, kcounts, vcounts):
     """The cache's prefill reads the prompt's mid rows once for pages, coefficients and column statistics
