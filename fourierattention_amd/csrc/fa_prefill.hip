@@ -54,36 +54,52 @@ struct PrefillParams {
 // slot e of lane group lg in a 32-key tile
 __device__ __forceinline__ int slot_key(int lg, int e) { return e < 4 ? 4 * lg + e : 16 + 4 * lg + (e - 4); }
 
+// A wave transposes kVtTiles key tiles on its own: a lane holds eight keys (its slots of a tile) of eight dims, so that the
+// 16-bit values change places inside the lane, and LDS only turns the lanes' 128-byte runs into whole rows of fragments
+// (the pieces of a run are permuted so that neither side meets a bank twice).  All eight loads are on their way at once.
+// Before, a block of 256 threads turned the tile with 2-byte reads of LDS behind two loads in a row.  us, before -> now: two
+// sequences of 700 rows x 8 heads of 128 16.5 -> 6.5, four of 3001 19.2 -> 10.4 (4.7 TB/s), one of 8192 18.9 -> 9.6, eight of
+// 1000 x 4 heads of 64 16.8 -> 6.4, one of 65 x 2 heads of 64 3.4 -> 3.6.
+template <int D>
+constexpr int kVtTiles = 128 / D;
+
 template <typename E, int D>
-__global__ __launch_bounds__(256) void prefill_vt_kernel(const E* __restrict__ v, int64_t v_bs, int64_t v_rs,
-                                                         f16_t* __restrict__ vt, int S, int Hkv, int n_tiles) {
+__global__ __launch_bounds__(64) void prefill_vt_kernel(const E* __restrict__ v, int64_t v_bs, int64_t v_rs,
+                                                        f16_t* __restrict__ vt, int S, int Hkv, int n_tiles) {
   // The second product runs in f16 whatever the storage type: the reference computes this attention as
   // flash_attn_func(q.half(), k.half(), v.half()) (MODEL:633), with probabilities of 11 significant bits; a bf16
   // operand would keep 8.  bf16 -> f16 is exact between 2^-14 and 65504 (larger magnitudes are clamped there).
   struct alignas(sizeof(E) * 8) Piece { E e[8]; };
   struct alignas(16) PieceOut { f16_t e[8]; };
-  __shared__ __attribute__((aligned(16))) E tile[kTileKeys][D + 8];
-  const int t = blockIdx.x, h = blockIdx.y, b = blockIdx.z, tid = threadIdx.x;
-  const E* src = v + (int64_t)b * v_bs + (int64_t)h * D;
-  constexpr int PPR = D / 8;
-  for (int pidx = tid; pidx < kTileKeys * PPR; pidx += 256) {
-    const int r = pidx / PPR, c = pidx - r * PPR;
-    const int key = t * kTileKeys + r;
-    Piece pc{};
-    if (key < S) pc = *(const Piece*)(src + (int64_t)key * v_rs + c * 8);
-    *(Piece*)&tile[r][c * 8] = pc;
-  }
-  __syncthreads();
-  PieceOut* dst = (PieceOut*)(vt + (((int64_t)b * Hkv + h) * n_tiles + t) * (int64_t)(kTileKeys * D));
-  for (int pidx = tid; pidx < (D / 16) * 64; pidx += 256) {
-    const int dg = pidx >> 6, lane = pidx & 63, lg = lane >> 4, ld = lane & 15;
+  __shared__ PieceOut s_out[8 * 64];
+  constexpr int C = D / 8;                        // pieces of a row
+  const int lane = threadIdx.x, c = lane % C, lg = lane / C & 3, tl = lane / (4 * C);
+  const int t0 = blockIdx.x * kVtTiles<D>, h = blockIdx.y, b = blockIdx.z;
+  const E* src = v + (int64_t)b * v_bs + (int64_t)h * D + c * 8;
+  const int key0 = (t0 + tl) * kTileKeys;
+  Piece pc[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) pc[e] = *(const Piece*)(src + (int64_t)min(key0 + slot_key(lg, e), S - 1) * v_rs);
+  // piece x of the tiles (16 bytes of f16): eight to a run, run k = x / 8, kept at place (x ^ swz(k)) of the run
+  auto swz = [](int k) { return (k ^ (k >> 3)) & 7; };
+  const int run = ((tl * (D / 16) + (c >> 1)) * 4 + lg) * 2 + (c & 1);
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
     PieceOut o;
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-      const float x = fa_to_float(tile[slot_key(lg, e)][16 * dg + ld]);
+      const float x = key0 + slot_key(lg, e) < S ? fa_to_float(pc[e].e[j]) : 0.f;
       o.e[e] = f16_t{(_Float16)fminf(fmaxf(x, -65504.f), 65504.f)};
     }
-    dst[pidx] = o;
+    s_out[run * 8 + (j ^ swz(run))] = o;
+  }
+  __syncthreads();
+  PieceOut* dst = (PieceOut*)(vt + (((int64_t)b * Hkv + h) * n_tiles + t0) * (int64_t)(kTileKeys * D));
+  const int here = min(kVtTiles<D>, n_tiles - t0) * (kTileKeys * D / 8);   // pieces of the tiles that there are
+#pragma unroll
+  for (int it = 0; it < 8; ++it) {
+    const int x = it * 64 + lane;
+    if (x < here) dst[x] = s_out[(x & ~7) | ((x & 7) ^ swz(x >> 3))];
   }
 }
 
@@ -312,7 +328,7 @@ int launch_prefill(const void* q, int64_t q_bs, int64_t q_hs, int64_t q_rs, cons
                    int q_len, float sm_scale, hipStream_t st) {
   const int n_tiles = fa_cdiv(S, kTileKeys);
   f16_t* vt = (f16_t*)workspace;
-  prefill_vt_kernel<E, D><<<dim3(n_tiles, Hkv, B), 256, 0, st>>>((const E*)v, v_bs, v_rs, vt, S, Hkv, n_tiles);
+  prefill_vt_kernel<E, D><<<dim3(fa_cdiv(n_tiles, kVtTiles<D>), Hkv, B), 64, 0, st>>>((const E*)v, v_bs, v_rs, vt, S, Hkv, n_tiles);
   const int G = Hq / Hkv;
   PrefillParams<E> p{};
   p.q = (const E*)q; p.q_bs = q_bs; p.q_hs = q_hs; p.q_rs = q_rs;

@@ -57,6 +57,7 @@ def _case(seed, B, Hq, Hkv, D, S, q_len, dtype, rope=True):
     (1, 16, 2, 64, 75, 75),       # eight query heads per KV head
     (2, 4, 2, 128, 150, 37),      # fewer query rows than keys: the mask is aligned to the last key
     (1, 8, 2, 128, 33, 1),        # a single query row
+    (3, 2, 2, 64, 20, 20),        # one key tile where a wave could take two
 ])
 def test_every_row_of_small_shapes(dtype, B, Hq, Hkv, D, S, q_len):
     from fourierattention_amd import ops
