@@ -228,8 +228,8 @@ typedef struct fa_decode_args {
   void* workspace;
   size_t workspace_bytes;
   /* bit 0: never run the merge inside the mid-row launch (see fa_decode_attn); the mid rows and the merge then run as
-   * launches of their own.  bit 1: with a batch of one sequence, keep one page stream per workgroup instead of four
-   * sub-splits.  (Both for testing and comparison.) */
+   * launches of their own.  bit 1: with one or two sequences, keep a page stream per sequence and workgroup instead of
+   * four resp. two sub-splits of each.  (Both for testing and comparison.) */
   int32_t no_fuse;
   /* A rank-1 update that the coefficients are still owed (fa_stream_update with skip_coef), applied by this call
    * before it uses them: k_mc[b, n, j] += cos(2 pi n p / upd_T) x_k[b, kc_list[j]] and k_mc[b, N + n, j] += sin(...),
@@ -369,9 +369,9 @@ int fa_decode_tables_build(void* tables, size_t tables_bytes, int N, int T, fa_s
  * Launches: query preparation + sink/window tiles, mid rows (two passes with 1024 frequencies), merge.  On the
  * matrix-core path with 16-bit storage, head_dim 128 and at most four query heads per KV head the workgroups of the
  * last mid-row launch merge their own partials and write the output rows (one launch fewer); args->no_fuse bit 0
- * keeps the merge launch.  With a batch of one sequence and up to 512 frequencies every workgroup of that launch then
- * runs four sub-splits of its pages side by side (in the matrix-core columns and page streams that further batch
- * elements would use).
+ * keeps the merge launch.  With one or two sequences and up to 512 frequencies every workgroup of that launch then
+ * runs four resp. two sub-splits of each sequence's pages side by side (in the matrix-core columns and page streams that
+ * further batch elements would use).
  * That needs the device to deal the workgroups of a launch out to its dies in turn, which the first call on a device
  * checks with a tiny launch and ONE synchronisation of `stream` (skipped, and asked again by the next call, while
  * the stream is being captured). */

@@ -601,8 +601,8 @@ def test_a_refused_update_leaves_the_layer():
 
 @pytest.mark.parametrize("rows,launches", [(1, 1), (3, 1), (4, 3), (16, 3)])
 def test_where_the_norms_of_a_decoder_step_run(rows, launches, monkeypatch):
-    """Up to 6144 elements the two norms of a layer ride in its projections and only the final one is a launch; above, all
-    three are.  The logits against the chain of tensor ops, which rounds between them: bf16 through one layer, 2^-8 of the
+    """Up to three rows of 12288 elements together the two norms of a layer ride in its projections and only the final one is a
+    launch; above, all three are.  The logits against the chain of tensor ops, which rounds between them: bf16 through one layer, 2^-8 of the
     largest, a few times over."""
     from fourierattention_amd import DynamicCache, ExtraConfig, masks, ops
     from fourierattention_amd.llama import LlamaConfig, random_init

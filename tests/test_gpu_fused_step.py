@@ -1,7 +1,7 @@
 """The three ways ``fa_decode_attn`` runs a step on the one-pass matrix-core path must agree: mid rows and merge as
 launches of their own, the merge inside the mid-row launch (teams of workgroups that meet through the L2 of their
-die), and, for a batch of one sequence, the same with four sub-splits per workgroup in the places of four batch
-elements.  Every case is also held against the CPU restatement (bound 2e-2 for 16-bit storage, as everywhere).
+die), and, for one or two sequences, the same with four resp. two sub-splits of each per workgroup in the places of
+four batch elements.  Every case is also held against the CPU restatement (bound 2e-2 for 16-bit storage, as everywhere).
 
 Geometries: eight KV heads so that the teams of a launch fill the eight dies (what the fused merge needs), one to
 four query heads per KV head, batches that fill a group of four, leave it ragged or consist of one sequence, heads
