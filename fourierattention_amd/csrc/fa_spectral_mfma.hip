@@ -395,29 +395,39 @@ __global__ __launch_bounds__(256) void spectral_reduce_kernel(const float* __res
 // Statistics of the reconstruction (mat_fourier_avg_std_triton, TRI:285-326):
 //   r[k, m] = (1/N) sum_n cos(theta k n) c[n, m] + sin(theta k n) s[n, m],     s[n] = c[N + n]
 // The roles of position and frequency are those of the compression exchanged: rows are the positions k, and the
-// contraction runs over the coefficient index n, cut into steps of 128.  A step is taken from its centre
-// n_c = 128 t + 63.5: with the coefficients folded, c+ = c[n_c + j] + c[n_c - j] and c- = c[n_c + j] - c[n_c - j] for the 64
-// offsets j = 1/2, 3/2 ..,
+// contraction runs over the coefficient index n, cut into steps of 127.  A step is taken from its centre n_c = 127 t:
+// with the coefficients folded, c+ = c[n_c + j] + c[n_c - j] and c- = c[n_c + j] - c[n_c - j] for the 64 offsets j = 0 .. 63
+// (c+ = c- = c[n_c] for j = 0),
 //   sum over the step of cos(theta k n) c[n] = cos(phi) . (E_cos c+) - sin(phi) . (E_sin c-)
 //   sum over the step of sin(theta k n) s[n] = sin(phi) . (E_cos s+) + cos(phi) . (E_sin s-),      phi = theta k n_c
 // so that the matrix cores compute real sums only, half of what two complex ones (basis rows cos and sin for every
 // coefficient, one accumulator of the two used) take, and a step ends in two multiply-adds per sum instead of a complex
 // rotation.  The fold happens in 32 bits ahead of the rounding to f16, scaled by a power of two per column (the range of
-// coefficients is not bounded).  The coefficient of frequency 0 stays out of the products: its basis is one, and the mean of
-// the signal, often its largest part, is added in 32 bits behind them (as c[0] it would meet the rounded basis of offset
-// 63.5).
+// coefficients is not bounded).
+// The lowest frequencies carry the mean, the drift and the slow oscillations of a signal, often its largest part, and theirs
+// are the largest errors.  Step 0 has no lower half, so cosines meet c and sines meet s, and the fragments that
+// c- and s+ would take hold what the rounding of c and s leaves over; the extremes of a slow column fall on a basis of one.
+// The coefficient of frequency 0 stays out of the products altogether and is added in 32 bits.  (Steps of 128 from
+// their centres 63.5, .. need one step less, but there c[1] meets the rounded basis of offset 62.5: columns with a drift
+// had their deviation off by 1.07e-4 instead of the 7.6e-5 of a basis that is not folded.)
 // Position k gives r[k] = A_k + B_k (A cosine, B sine part) and, because the period is a whole number of positions, also
 // its mirror image r[T - k] = A_k - B_k: only the positions up to T / 2 are computed, each standing for two where the
 // sequence reaches past T / 2.
-// Bound by the matrix cores and the LDS reads that feed them (a fragment feeds four products).  32768 positions x 512 columns,
-// 512 frequencies, all launches: 72.9 us with complex sums on coefficients packed by launches of their own -> 43.9; eight tensors
-// of 31740 positions 294 -> 165, four of 1977 x 910 56 -> 37.  Against 64 bits the mean is off by 4e-7 .. 4e-5 (1e-4 .. 2e-4
-// before, the rounding of the coefficient of frequency 0), the deviation by as much as before (7e-5).
+// Bound by the matrix cores and the LDS reads that feed them (a fragment feeds four products).
+// us, all launches (complex sums on coefficients packed by launches of their own -> now; steps of 128 without the second
+// term of step 0 in brackets): 32768 positions x 512 columns, 512 frequencies 73.1 -> 48.9 (44.3); eight tensors of 31740 positions
+// 296 -> 190 (164), four of 1977 x 910 54.7 -> 39.9 (36.4), two of 9000 x 300 with 128 frequencies 26.2 -> 18.5 (17.1).  Relative
+// error of the deviation against 64 bits, rms over the columns, same three: 31740 x 512 of a period of 130044, noise
+// 4.04e-5 -> 3.77e-5 (4.03e-5), mean of twice the noise 1.67e-4 -> 8.4e-5 (1.87e-4), drift 7.6e-5 -> 4.3e-5 (1.07e-4); 32768 of 32768,
+// drift 5.3e-5 -> 4.3e-5 (7.9e-5).  The mean, over the deviation: 2.1e-4 -> 1.8e-6 (1.1e-4) with a mean, 2.8e-6 -> 1.9e-7 (1.7e-6)
+// without.
 // ---------------------------------------------------------------------------------------------------------
 constexpr int kRecPos = 256;      // positions of a workgroup: four waves x four tiles of 16
 constexpr int kRecCols = 32;      // columns of a unit of work: two tiles of 16
-constexpr int kRecStep = 128;     // coefficient indices of a step
+constexpr int kRecStep = 127;     // coefficient indices of a step: its centre and 63 to either side (step 0: above it only)
+constexpr int kRecHalf = 64;      // offsets of a step
 constexpr int kRecFrags = 8;      // fragments of a step and column tile: {c+, c-, s+, s-} x two ksteps of 32 offsets
+__host__ __device__ inline int recon_steps(int N) { return N <= kRecHalf ? 1 : 1 + (N - kRecHalf + kRecStep - 1) / kRecStep; }
 constexpr int kMaxColShare = 8;   // units of a workgroup at most
 
 struct ReconPrepParams {
@@ -446,7 +456,7 @@ __global__ __launch_bounds__(1024) void recon_prep_kernel(const ReconPrepParams 
 #pragma unroll
     for (int e = 0; e < 2; ++e) {
       float sn, co;
-      fa_sincos_phase(tile * 16 + lc, 2 * (32 * kk + 8 * lg + 2 * ep + e) + 1, 2 * p.T, &sn, &co);
+      fa_sincos_phase(tile * 16 + lc, 32 * kk + 8 * lg + 2 * ep + e, p.T, &sn, &co);
       co2[e] = (_Float16)co;
       sn2[e] = (_Float16)sn;
       own = fmaf((float)co2[e], co, fmaf((float)sn2[e], sn, own));
@@ -455,7 +465,8 @@ __global__ __launch_bounds__(1024) void recon_prep_kernel(const ReconPrepParams 
     out[0] = co2;
     out[2 * 64 * 4] = sn2;
     // A rounded basis answers its own position with a sum of squares that is not quite 64: the phases carry the
-    // reciprocal, so that what is coherent with the position - the signal at its extremes - comes out unscaled.
+    // reciprocal, so that what is coherent with the position - the signal at its extremes - comes out unscaled.  (Step 0
+    // takes no phases.)
     float* s_own = &s_mx[0][0];   // [32 positions][32]
     s_own[((tid >> 9) * 16 + lc) * 32 + (kk * 4 + lg) * 4 + ep] = own;
     __syncthreads();
@@ -467,7 +478,7 @@ __global__ __launch_bounds__(1024) void recon_prep_kernel(const ReconPrepParams 
     const int k = blk * 32 + pos, rb = k / kRecPos;
     for (int t = tid >> 5; t < p.n_steps; t += 32) {
       float sn, co;
-      fa_sincos_phase(k, 2 * kRecStep * t + kRecStep - 1, 2 * p.T, &sn, &co);
+      fa_sincos_phase(k, kRecStep * t, p.T, &sn, &co);
       float* o = p.phi + ((int64_t)(rb * p.n_steps + t) * 2) * kRecPos + k % kRecPos;
       o[0] = co * unit;
       o[kRecPos] = sn * unit;
@@ -477,17 +488,20 @@ __global__ __launch_bounds__(1024) void recon_prep_kernel(const ReconPrepParams 
   const int ct = blk % p.CT, b = blk / p.CT;
   const int lc = tid & 15, i = tid >> 4, m = ct * 16 + lc;
   const float* cb = p.c + (int64_t)b * 2 * p.N * p.Mc + min(m, p.Mc - 1);
-  float v[kHold][4];   // cos rows above and below the centre, sin rows likewise
+  float v[kHold][4];   // cos rows above and below the centre, sin rows likewise; zeros where there are none
   auto load = [&](int t0) {
 #pragma unroll
     for (int u = 0; u < kHold; ++u)
       if (t0 + u < p.n_steps) {
-        const int hi = (t0 + u) * kRecStep + 64 + i, lo = (t0 + u) * kRecStep + 63 - i;
-        v[u][0] = cb[(int64_t)min(hi, p.N - 1) * p.Mc];
-        v[u][1] = cb[(int64_t)min(lo, p.N - 1) * p.Mc];
-        v[u][2] = cb[(int64_t)(p.N + min(hi, p.N - 1)) * p.Mc];
-        v[u][3] = cb[(int64_t)(p.N + min(lo, p.N - 1)) * p.Mc];
-        if (lo == 0) v[u][1] = v[u][3] = 0.f;   // (frequency 0: added behind the products)
+        const int hi = (t0 + u) * kRecStep + i, lo = (t0 + u) * kRecStep - i;
+        const int hc = min(hi, p.N - 1), lc0 = min(max(lo, 0), p.N - 1);
+        v[u][0] = cb[(int64_t)hc * p.Mc];
+        v[u][1] = cb[(int64_t)lc0 * p.Mc];
+        v[u][2] = cb[(int64_t)(p.N + hc) * p.Mc];
+        v[u][3] = cb[(int64_t)(p.N + lc0) * p.Mc];
+        // (frequency 0 is added behind the products; step 0 has nothing below its centre, and the centre counts once)
+        if (hi == 0 || hi >= p.N) v[u][0] = v[u][2] = 0.f;
+        if (lo <= 0 || lo >= p.N || i == 0) v[u][1] = v[u][3] = 0.f;
       }
   };
   float mx = 0.f;
@@ -515,15 +529,15 @@ __global__ __launch_bounds__(1024) void recon_prep_kernel(const ReconPrepParams 
 #pragma unroll
       for (int u = 0; u < kOut; ++u)
         if (t0 + u0 + u < p.n_steps) {
-          const int hi = (t0 + u0 + u) * kRecStep + 64 + i, lo = (t0 + u0 + u) * kRecStep + 63 - i;
-          const bool ok_h = m < p.Mc && hi < p.N, ok_l = m < p.Mc && lo < p.N;
-          const float ch = ok_h ? v[u0 + u][0] * inv : 0.f, cl = ok_l ? v[u0 + u][1] * inv : 0.f;
-          const float sh = ok_h ? v[u0 + u][2] * inv : 0.f, sl = ok_l ? v[u0 + u][3] * inv : 0.f;
+          const float own = m < p.Mc ? inv : 0.f;
+          const float ch = v[u0 + u][0] * own, cl = v[u0 + u][1] * own, sh = v[u0 + u][2] * own, sl = v[u0 + u][3] * own;
+          const bool first = t0 + u0 + u == 0;
+          const _Float16 cp = (_Float16)(ch + cl), sp = (_Float16)(sh + sl);
           _Float16* o = s_out + u * kRecFrags * 512 + at;
-          o[0 * 1024] = (_Float16)(ch + cl);
-          o[1 * 1024] = (_Float16)(ch - cl);
-          o[2 * 1024] = (_Float16)(sh + sl);
-          o[3 * 1024] = (_Float16)(sh - sl);
+          o[0 * 1024] = cp;
+          o[1 * 1024] = (_Float16)(ch - (first ? (float)cp : cl));   // step 0: what the rounding leaves over
+          o[2 * 1024] = sp;
+          o[3 * 1024] = (_Float16)(sh - (first ? (float)sp : sl));
         }
       __syncthreads();
       const int n = min(kOut, p.n_steps - t0 - u0) * kRecFrags * 64;
@@ -590,11 +604,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
   for (int i = 0; i < NST - 1; ++i)
     if (i < Q) issue(i);
-  float4v A[4][2], Bs[4][2];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) A[i][j] = Bs[i][j] = float4v{0.f, 0.f, 0.f, 0.f};
+  float4v A[4][2], Bs[4][2];   // (step 0 of a column block starts them)
   // (the table must have landed before the loop: inside it the only waits on vector memory are explicit)
 #pragma unroll
   for (int i = 0; i < 4; ++i)
@@ -632,9 +642,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   B[1] = lds_read_b128_async_at<((G) * 4 + 1) * 1024>(fr);      \
   B[2] = lds_read_b128_async_at<((G) * 4 + 2) * 1024>(fr);      \
   B[3] = lds_read_b128_async_at<((G) * 4 + 3) * 1024>(fr)
-    // one column tile's cosine or sine coefficients: f = {+ k0, + k1, - k0, - k1}
+    // one column tile's cosine or sine coefficients: f = {+ k0, + k1, - k0, - k1}; step 0: {c k0, c k1, rest k0, rest k1}
     auto products = [&](const uint4v (&f)[4], float4v (&acc)[4][2], int j, bool sine) {
       float4v C[4], D[4];
+      if (it == 0) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(sine ? Es[i][k & 1] : Ec[i][k & 1], __builtin_bit_cast(half8, f[k]),
+                                                               k ? acc[i][j] : float4v{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+        return;
+      }
 #pragma unroll
       for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
@@ -732,8 +751,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                      "v"(mx), "v"(mn), "n"(kKind), "n"(2 * kKind)
                      : "memory");
       }
-#pragma unroll
-      for (int i = 0; i < 4; ++i) A[i][j] = Bs[i][j] = float4v{0.f, 0.f, 0.f, 0.f};
     }
   }
   barrier_lds_only();   // (behind the wait for the writes above)
@@ -753,11 +770,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 }
 
 // The statistics of a cache in single precision: complex sums, one pass over the cosine and one over the sine coefficients
-// on the walk of the compression, from which the real and the imaginary part are taken.  Twice the work of the kernel above,
-// with errors of the same size (deviations 5e-5, means 1e-4) in other places.  The statistics are rounded to fp16, where a
-// place is up to 1e-3 of a value: with either kernel some columns of a tensor round the other way, and the attention over
-// it moves by 5e-4 - nothing beside the roundings of a 16-bit model, but fifty times the 1e-5 that single precision holds its
-// results to.
+// on the walk of the compression, from which the real and the imaginary part are taken.  Twice the work of the kernel above and
+// further from 64 bits (deviations 4e-5 .. 2e-4, means 1e-4 of the deviation): it is kept for unchanged results, not for its
+// accuracy.  The statistics are rounded to fp16, where a place is up to 1e-3 of a value, and with any other order of roundings some
+// columns round the other way: the attention over them moves by 5e-4, nothing beside the roundings of a 16-bit model, but
+// fifty times the 1e-5 to which results in single precision are to stay what they are.
 __global__ __launch_bounds__(1024) void coef_colscale_kernel(const float* __restrict__ c, float* __restrict__ scale,
                                                              float* __restrict__ inv_scale, int N2, int Mc) {
   // 16 columns x 64 row classes: 64 bytes of a row per access, and four times the blocks of whole waves of columns
@@ -1110,7 +1127,7 @@ ReconPlan recon_plan(int B, int N, int Mc, int K) {
   using namespace fa_mfma;
   ReconPlan p{};
   p.CT = fa_cdiv(Mc, 16);
-  p.n_steps = fa_cdiv(N, kRecStep);
+  p.n_steps = recon_steps(N);
   p.RB = fa_cdiv(K, kRecPos);
   size_t o = 0;
   auto take = [&](size_t bytes) { size_t at = o; o += fa_align_up(bytes, 256); return at; };

@@ -61,6 +61,25 @@ def test_reconstruction_statistics_of_signals_with_a_mean(B, L, C, N, T):
         assert torch.equal(a[whole], b[whole]) and not torch.isfinite(a[~whole]).any()
 
 
+@pytest.mark.parametrize("N", [64, 65, 191, 192, 512])   # one step of the coefficients, one past it, two, one past those, five
+def test_reconstruction_statistics_of_slow_columns(N):
+    """Columns of a single low frequency, which is what a drift or a slow oscillation is made of: their extremes fall on
+    positions where the basis is one, so nothing of the basis' rounding reaches the deviation (the period is a power of two and
+    the whole of it is covered: the errors of the mean cancel).  Bound: a coefficient travels as two f16 terms, 2^-22 of it is
+    lost, and single precision adds a few 2^-24."""
+    from fourierattention_amd import ops
+    T, low = 4096, 63
+    g = torch.Generator(device="cuda").manual_seed(6)
+    c = torch.zeros((1, 2 * N, 2 * low), device="cuda")
+    n = torch.arange(1, low + 1, device="cuda")
+    amp = (0.5 + torch.rand(2 * low, generator=g, device="cuda")) * 10.0 ** torch.randint(-3, 4, (2 * low,), generator=g, device="cuda")
+    c[0, n, n - 1] = amp[:low]
+    c[0, N + n, low + n - 1] = -amp[low:]
+    avg, dev = ops.mat_fourier_avg_std(c, T, T, None)
+    assert (avg[0].abs() * N <= 2.0 ** -20 * amp).all()
+    assert ((dev[0] * N - amp).abs() <= 2.0 ** -20 * amp).all()
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("B,H,S,D,first,last,spare,tokens_first", [
     (1, 1, 1, 8, 0, 1, 0, False),        # one row of one piece or two
