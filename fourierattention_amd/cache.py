@@ -119,7 +119,8 @@ def _device_lists(lists, device):
         wide = [torch.tensor(lst, dtype=torch.int64, device=device) for lst in lists]
         return wide, [t.to(torch.int32) for t in wide]
     n = len(flat)
-    host = torch.empty(12 * n, dtype=torch.uint8, pin_memory=device.type == "cuda")
+    # (device by name: a default device that the program has set must not take it)
+    host = torch.empty(12 * n, dtype=torch.uint8, device="cpu", pin_memory=device.type == "cuda")
     if n:
         wide = torch.frombuffer(flat, dtype=torch.int64)
         host[: 8 * n].view(torch.int64).copy_(wide)

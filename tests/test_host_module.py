@@ -135,3 +135,13 @@ def test_lists_of_a_cache_in_one_tensor():
         for tensors, dt in zip(got, (torch.int64, torch.int32)):
             assert [t.tolist() for t in tensors] == [[int(x) for x in lst] for lst in want]
             assert all(t.dtype == dt and t.is_contiguous() and t.storage_offset() % 32 == 0 for t in tensors)
+
+
+def test_lists_of_a_cache_under_another_default_device():
+    """A cache made where the program has set a default device (``torch.device(..)`` as a context) gets its lists on its own."""
+    import torch
+    from fourierattention_amd.cache import _device_lists
+    with torch.device("meta"):
+        got = _device_lists([[3, 1], [7]], torch.device("cpu"))
+    for tensors, dt in zip(got, (torch.int64, torch.int32)):
+        assert [(t.device.type, t.dtype, t.tolist()) for t in tensors] == [("cpu", dt, [3, 1]), ("cpu", dt, [7])]
