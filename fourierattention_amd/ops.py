@@ -387,7 +387,8 @@ def linear_packed_qkv(x: torch.Tensor, w: PackedLinearWeight, norm: Optional[tor
     """q, k and v of a decode step, ``(B, heads, q_len, head_dim)`` views, from ``x (B, q_len, hidden)``: RMSNorm in front
     (``norm``, if given), one pass over the weight (its rows in the order of ``rotary_pairs``), rotary embedding of q and k - what
     ``linear_packed_step`` and ``rope_qk`` do in two launches, with the same results.  ``cos, sin``: as for ``rope_qk``."""
-    cos, sin = _rotary_tables(cos, sin, x)
+    # (the launch reads the tables in vectors; ``rope_qk`` takes them wherever they lie)
+    cos, sin = (t if t.data_ptr() % 16 == 0 else t.clone() for t in _rotary_tables(cos, sin, x))
     return _lib.load_host().linear_packed_qkv(x, w.data, norm, eps, cos, sin, num_heads, num_kv_heads, head_dim)
 
 

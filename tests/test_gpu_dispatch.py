@@ -347,6 +347,22 @@ def test_rotary_embedding_in_the_projection(dtype, B, q_len, K, Hq, Hkv, D):
             assert torch.equal(got, want.view(B, q_len, -1, D).transpose(1, 2))
 
 
+@pytest.mark.parametrize("at", [1, 4])     # elements past an aligned address
+def test_rotary_tables_anywhere(at):
+    """Tables that start off a vector's alignment - a slice of a longer buffer - are taken as ``rope_qk`` takes them."""
+    from fourierattention_amd import ops
+    K, Hq, Hkv, D = 1024, 2, 1, 16
+    g = torch.Generator(device="cuda").manual_seed(at)
+    rn = lambda *s: torch.randn(s, generator=g, device="cuda").bfloat16()
+    w = ops.PackedLinearWeight(rn((Hq + 2 * Hkv) * D, K))
+    x, table = rn(1, 1, K), rn(128)
+    cos, sin = (table[i + at: i + at + D].view(1, 1, D) for i in (0, 64))
+    assert cos.data_ptr() % 16 and sin.data_ptr() % 16
+    want = ops.linear_packed_qkv(x, w, None, 0.0, cos.clone(), sin.clone(), Hq, Hkv, D)
+    for got, t in zip(ops.linear_packed_qkv(x, w, None, 0.0, cos, sin, Hq, Hkv, D), want):
+        assert torch.equal(got, t)
+
+
 def _launches(f):
     """Kernel launches of a call: the nodes of a graph it is captured into (which is never run)."""
     import ctypes
