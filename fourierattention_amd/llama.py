@@ -78,11 +78,17 @@ class LlamaMLP(nn.Module):
         return self.down_proj(F.silu(self.gate_proj(x)) * self.up_proj(x))
 
 
-# Rows of a decode step, and elements of them, up to which the RMSNorm rides in the projection behind it.  Every workgroup of
-# that launch normalises all rows; a launch of its own does them once.  q/k/v, gate/up and down of a layer, in the projections /
-# apart, us: 4096 wide 1 row 70.1 / 75.9, 2 rows 71.6 / 76.0, 3 rows 75.6 / 75.8, 4 rows 75.7 / 75.8; 3072 wide 1 row
-# 39.0 / 44.7, 3 rows 42.1 / 45.2, 4 rows 43.6 / 43.7, 5 rows 45.3 / 44.2.
-_NORM_ROWS, _NORM_IN_PROJECTION = 3, 12288
+# Where the RMSNorms of a decode step ride in the projections behind them: up to 6144 elements of rows, or three rows of up to 12288.
+# Every workgroup of such a launch normalises all rows; a launch of its own does them once.  q/k/v and gate/up of a layer, in
+# launches of their own / in the projections, us: 4096 wide 1 row 59.8 / 53.5, 2 rows 59.9 / 53.2, 3 rows 58.3 / 57.6, 4 rows 58.3 /
+# 60.0; 3072 wide 2 rows 34.0 / 29.7, 3 rows 33.7 / 32.0, 4 rows 33.8 / 33.4, 5 rows 33.9 / 34.8; 2048 wide 3 rows 23.0 / 21.6, 4 rows
+# 23.1 / 22.4, 5 rows 23.2 / 23.9; 1024 wide 4 rows 13.9 / 11.1, 6 rows 14.1 / 12.7, 8 rows 14.2 / 13.1, 12 rows 14.6 / 15.1.
+_NORM_ELEMENTS = 6144
+_NORM_ROWS, _NORM_ELEMENTS_OF_FEW_ROWS = 3, 12288
+
+
+def _norm_rides(rows, width):
+    return rows * width <= (_NORM_ELEMENTS_OF_FEW_ROWS if rows <= _NORM_ROWS else _NORM_ELEMENTS)
 
 
 class LlamaDecoderLayer(nn.Module):
@@ -171,7 +177,7 @@ class LlamaDecoderLayer(nn.Module):
         Returns this layer's MLP output, to be added by whoever normalises next (``None``: ``h`` has it already)."""
         at = self.self_attn
         bsz, q_len, width = h.shape
-        norm_rides = bsz * q_len <= _NORM_ROWS and bsz * q_len * width <= _NORM_IN_PROJECTION
+        norm_rides = _norm_rides(bsz * q_len, width)
         nq, nk = at.num_heads * at.head_dim, at.num_key_value_heads * at.head_dim
         pk = self._packed_weight("qkv")
         norm = self.input_layernorm

@@ -661,6 +661,31 @@ def test_where_the_norms_of_a_decoder_step_run(rows, launches, monkeypatch):
     assert float((logits[0] - logits[1]).abs().max()) <= 4 * 2.0 ** -8 * float(logits[1].abs().max())
 
 
+@pytest.mark.parametrize("rows,launches", [(4, 1), (6, 1), (7, 3)])
+def test_where_the_norms_of_a_narrow_decoder_step_run(rows, launches, monkeypatch):
+    """Rows of 6144 elements together ride however many they are (1024 wide: 5 rows 14.3 us a layer apart, 12.3 riding)."""
+    from fourierattention_amd import DynamicCache, ExtraConfig, masks, ops
+    from fourierattention_amd.llama import LlamaConfig, random_init
+    llama = LlamaConfig(hidden_size=1024, intermediate_size=1024, num_hidden_layers=1, num_attention_heads=8, num_key_value_heads=8,
+                        head_dim=128, vocab_size=512)
+    model = random_init(llama, torch.bfloat16, "cuda:0", seed=1)
+    model.model.pack_projections()
+    cfg = ExtraConfig(numinittokens=4, maxlocallen=64, maxmidstates=64, non_critical_dims=masks.synthetic_masks(1, 8, 128, [64] * 8, [64] * 8, seed=1),
+                      non_critical_dims_path=None, max_position_embeddings=4096, num_key_value_heads=8, max_new_tokens=8, model_type="llama")
+    ids = torch.randint(0, 512, (rows, 21), device="cuda")
+    own, calls, logits = ops.add_rmsnorm, [], []
+    monkeypatch.setattr(ops, "add_rmsnorm", lambda *a: (calls.append(1), own(*a))[1])
+    with torch.no_grad():
+        for fused in (True, False):
+            model.model.fused_elementwise = fused
+            cache = DynamicCache(cfg)
+            model(ids[:, :20], cache)
+            calls.clear()
+            logits.append(model(ids[:, 20:], cache).logits)
+            assert len(calls) == (launches if fused else 0)
+    assert float((logits[0] - logits[1]).abs().max()) <= 4 * 2.0 ** -8 * float(logits[1].abs().max())
+
+
 def test_argument_forms_of_the_decode_call():
     """Lists instead of tuples, whole numbers that are not ints, timings in any mutable sequence; the sine table alone in another
     type, tables with rows to spare."""
