@@ -327,6 +327,24 @@ def test_projections_with_the_steps_beside_them(dtype, rows, K, n_out):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("K", [5120, 14336, 16384])     # two pieces of a row for some threads, the last of four for some, four for all
+def test_norm_of_a_long_row_in_the_projection(dtype, K):
+    """One row whose pieces share their sum of squares, against the norm as tensor operations.  Bound as above: the scale of the
+    row moves by a place of float32, single operands by a place of ``dtype``."""
+    from fourierattention_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(K)
+    rn = lambda *s: torch.randn(s, generator=g, device="cuda")
+    pw = ops.PackedLinearWeight((rn(64, K) * 0.05).to(dtype))
+    x, norm = (rn(1, 1, K) * 3).to(dtype), (1 + 0.1 * rn(K)).to(dtype)
+    f = x.float()
+    y = norm * (f * torch.rsqrt(f.pow(2).mean(-1, keepdim=True) + 1e-5)).to(dtype)
+    want, got = ops.linear_packed(y, pw), ops.linear_packed_step(x, pw, norm, 1e-5)
+    ulp = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    assert float((got.float() - want.float()).abs().max()) <= 2 * ulp * float(want.abs().max()) + ulp * float(y.abs().max()) * 0.2 * 4
+    assert torch.equal(ops.linear_packed_step(x, pw, norm, 1e-5, gated=True), ops.silu_mul(*got.chunk(2, dim=-1)))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("B,q_len,K,Hq,Hkv,D", [(1, 1, 1024, 1, 1, 16), (2, 1, 3072, 6, 2, 128), (3, 5, 1024, 4, 2, 64), (1, 4, 4096, 2, 1, 48)])
 def test_rotary_embedding_in_the_projection(dtype, B, q_len, K, Hq, Hkv, D):
     """q, k and v of one launch against the projection on the weight in its natural order and the rotary embedding as launches
