@@ -19,6 +19,7 @@ from __future__ import annotations
 from typing import Dict, Optional, Tuple
 
 import torch
+from torch.autograd.forward_ad import unpack_dual
 
 from . import _lib
 from ._lib import FA_BF16, FA_FP16, FA_FP32, check
@@ -253,13 +254,14 @@ def prompt_rows(k: torch.Tensor, v: torch.Tensor, near: Optional[Tuple[torch.Ten
     """The rows of a prompt, ``k, v (B, heads, S, D)``, as token-major ``(B, S, heads*D)`` tensors (the source's own memory
     where its heads lie side by side, else copies) and, in the same launch, into ``near = (k, v)``, ``(B, slots, heads*D)``:
     the first ``first`` rows, the last ``last``, then ``spare`` rows of zeros.  ``None`` where the layout is for tensor
-    operations: rows that are no multiples of 16 bytes, other devices, tensors that take part in a graph of gradients."""
+    operations: rows that are no multiples of 16 bytes, other devices, tensors that take part in a graph of gradients or carry a
+    tangent."""
     B, heads, S, D = k.shape
     es = k.element_size()
     if (not k.is_cuda or k.device != v.device or k.shape != v.shape or k.dtype != v.dtype or k.dtype not in _DTYPE_CODE
             or k.stride() != v.stride() or k.stride(3) != 1 or k.requires_grad or v.requires_grad or not 0 < B <= 65535 or S == 0
             or any((s * es) % 16 for s in (*k.stride()[:3], D)) or k.data_ptr() % 16 or v.data_ptr() % 16
-            or first + last > S):
+            or first + last > S or any(unpack_dual(t).tangent is not None for t in (k, v))):
         return None
     if near is not None and any(t.dtype != k.dtype or t.device != k.device or t.stride(2) != 1 or t.stride(1) != heads * D
                                 or t.stride(0) != near[0].stride(0) or t.shape[1] < first + last + spare or t.data_ptr() % 16

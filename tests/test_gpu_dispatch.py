@@ -105,6 +105,20 @@ def test_rows_of_a_prompt(dtype, B, H, S, D, first, last, spare, tokens_first):
     assert ops.prompt_rows(k, v.transpose(2, 3).contiguous().transpose(2, 3)) is None or S == 1 or D == 1   # strides of their own
 
 
+def test_prompt_of_a_window_keeps_its_tangent():
+    """A prompt that fits the window comes back as tensor operations return it: with its gradient, or its tangent."""
+    import torch.autograd.forward_ad as fwd
+    from fourierattention_amd import DynamicCache, ExtraConfig, masks
+    cache = DynamicCache(ExtraConfig(numinittokens=4, maxlocallen=40, maxmidstates=64, non_critical_dims=masks.synthetic_masks(1, 2, 128, [64] * 2, [64] * 2, seed=1),
+                                     non_critical_dims_path=None, max_position_embeddings=4096, num_key_value_heads=2, max_new_tokens=8, model_type="llama"))
+    k, v, dk = torch.randn((3, 1, 2, 20, 128), device="cuda").unbind(0)
+    with fwd.dual_level():
+        parts, _ = cache.update(fwd.make_dual(k, dk), v, 0)
+        rows = fwd.unpack_dual(parts["k_local"])
+        assert torch.equal(rows.primal, k.transpose(1, 2).reshape(1, 20, 256))
+        assert rows.tangent is not None and torch.equal(rows.tangent, dk.transpose(1, 2).reshape(1, 20, 256))
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("B,L,C,N,T", [(2, 300, 5, 16, 400), (1, 1100, 70, 64, 1500)])   # vector kernels / matrix cores
 def test_statistics_a_cache_keeps(dtype, B, L, C, N, T):
