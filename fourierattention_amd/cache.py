@@ -110,12 +110,15 @@ def _device_lists(lists, device):
     stand still until that is done (four prompts of 3001 tokens through two layers 1342 us, so 1203).  Every view starts 128 bytes
     aligned."""
     flat, spans = array("q"), []
+    one_by_one = ops.recorded()
     try:
         for lst in lists:
             spans.append((len(flat), len(lst)))
             flat.extend(lst)
             flat.extend([0] * (-len(flat) % 32))
     except (TypeError, OverflowError):      # entries that are no integers: what torch makes of them
+        one_by_one = True
+    if one_by_one:
         wide = [torch.tensor(lst, dtype=torch.int64, device=device) for lst in lists]
         return wide, [t.to(torch.int32) for t in wide]
     n = len(flat)

@@ -249,16 +249,23 @@ def append_rows(k: torch.Tensor, v: torch.Tensor, k_dst: torch.Tensor, v_dst: to
     _lib.load_host().append_rows(k, v, k_dst, v_dst, pos)
 
 
+def recorded() -> bool:
+    """Whether the operations of this thread are recorded or transformed: tracing, a dispatch mode (``make_fx``, fake tensors), a
+    ``torch.func`` transform.  What a kernel reads and writes by address is not seen there."""
+    return (torch.jit.is_tracing() or torch._C._len_torch_dispatch_stack() > 0
+            or torch._C._functorch.peek_interpreter_stack() is not None)
+
+
 def prompt_rows(k: torch.Tensor, v: torch.Tensor, near: Optional[Tuple[torch.Tensor, torch.Tensor]] = None, first: int = 0,
                 last: int = 0, spare: int = 0):
     """The rows of a prompt, ``k, v (B, heads, S, D)``, as token-major ``(B, S, heads*D)`` tensors (the source's own memory
     where its heads lie side by side, else copies) and, in the same launch, into ``near = (k, v)``, ``(B, slots, heads*D)``:
     the first ``first`` rows, the last ``last``, then ``spare`` rows of zeros.  ``None`` where the layout is for tensor
     operations: rows that are no multiples of 16 bytes, other devices, tensors that take part in a graph of gradients or carry a
-    tangent."""
+    tangent, calls that are recorded."""
     B, heads, S, D = k.shape
     es = k.element_size()
-    if (not k.is_cuda or k.device != v.device or k.shape != v.shape or k.dtype != v.dtype or k.dtype not in _DTYPE_CODE
+    if (recorded() or type(k) is not torch.Tensor or type(v) is not torch.Tensor or not k.is_cuda or k.device != v.device or k.shape != v.shape or k.dtype != v.dtype or k.dtype not in _DTYPE_CODE
             or k.stride() != v.stride() or k.stride(3) != 1 or k.requires_grad or v.requires_grad or not 0 < B <= 65535 or S == 0
             or any((s * es) % 16 for s in (*k.stride()[:3], D)) or k.data_ptr() % 16 or v.data_ptr() % 16
             or first + last > S or any(unpack_dual(t).tangent is not None for t in (k, v))):

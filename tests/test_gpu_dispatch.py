@@ -119,6 +119,29 @@ def test_prompt_of_a_window_keeps_its_tangent():
         assert rows.tangent is not None and torch.equal(rows.tangent, dk.transpose(1, 2).reshape(1, 20, 256))
 
 
+@pytest.mark.parametrize("how", ["jvp", "make_fx", "trace", "fake"])
+def test_prompt_of_a_window_where_operations_are_recorded(how):
+    """A new cache and a prompt that fits its window, under a transform, a tracer and fake tensors: tensor operations throughout."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from torch.fx.experimental.proxy_tensor import make_fx
+    from fourierattention_amd import DynamicCache, ExtraConfig, masks
+    cfg = ExtraConfig(numinittokens=4, maxlocallen=40, maxmidstates=64, non_critical_dims=masks.synthetic_masks(1, 2, 128, [64] * 2, [64] * 2, seed=1),
+                      non_critical_dims_path=None, max_position_embeddings=4096, num_key_value_heads=2, max_new_tokens=8, model_type="llama")
+    rows = lambda k, v: DynamicCache(cfg).update(k, v, 0)[0]["k_local"]
+    want = lambda k: k.transpose(1, 2).reshape(1, 20, 256)
+    k, v, other = torch.randn((3, 1, 2, 20, 128), device="cuda").unbind(0)
+    if how == "jvp":
+        got, tangent = torch.func.jvp(lambda k: rows(k, v), (k,), (other,))
+        assert torch.equal(got, want(k)) and torch.equal(tangent, want(other))
+    elif how == "make_fx":
+        assert torch.equal(make_fx(rows)(k, v)(other, v), want(other))
+    elif how == "trace":
+        assert torch.equal(torch.jit.trace(rows, (k, v), check_trace=False)(other, v), want(other))
+    else:
+        with FakeTensorMode(allow_non_fake_inputs=True) as mode:
+            assert rows(mode.from_tensor(k), mode.from_tensor(v)).shape == (1, 20, 256)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("B,L,C,N,T", [(2, 300, 5, 16, 400), (1, 1100, 70, 64, 1500)])   # vector kernels / matrix cores
 def test_statistics_a_cache_keeps(dtype, B, L, C, N, T):

@@ -145,3 +145,15 @@ def test_lists_of_a_cache_under_another_default_device():
         got = _device_lists([[3, 1], [7]], torch.device("cpu"))
     for tensors, dt in zip(got, (torch.int64, torch.int32)):
         assert [(t.device.type, t.dtype, t.tolist()) for t in tensors] == [("cpu", dt, [3, 1]), ("cpu", dt, [7])]
+
+
+def test_lists_of_a_cache_where_operations_are_recorded():
+    """A cache made inside a traced or transformed function."""
+    import torch
+    from torch.fx.experimental.proxy_tensor import make_fx
+    from fourierattention_amd.cache import _device_lists
+    pick = lambda x: x[_device_lists([[3, 1], [2]], torch.device("cpu"))[0][0]]
+    x, y = torch.arange(8.0).view(2, 4)
+    assert make_fx(pick)(x)(y).tolist() == [7.0, 5.0]
+    assert torch.jit.trace(pick, x, check_trace=False)(y).tolist() == [7.0, 5.0]
+    assert torch.func.vmap(pick)(torch.stack([x, y])).tolist() == [[3.0, 1.0], [7.0, 5.0]]
