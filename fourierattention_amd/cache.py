@@ -255,7 +255,7 @@ class DynamicCache(Cache):
         self.balance_heads = True                      # mid rows: more splits for heads that store more dims
         self.fuse_prefill = True                       # prefill: pages, coefficients and statistics from one read
         self.fuse_decode = True                        # decode: the merge inside the mid-row launch where it applies
-        self.sub_splits = True                         # ... and a batch of one as four sub-splits per workgroup
+        self.sub_splits = True                         # ... and one sequence as four sub-splits per workgroup, two as two each
         # streaming: leave the rank-1 update of the coefficients to the next decode_attention of the layer, which
         # streams them anyway.  Off: measured, it is no faster than the update launch (whose reads mostly hit the
         # last-level cache behind the attention of the step before), and two launches where the merge has its own

@@ -2136,7 +2136,8 @@ bool fused_layout_ok(hipStream_t st) {
   return ok;
 }
 
-thread_local int g_last_call_fused = 0;   // what the last fa_decode_attn call of this thread did (a measurement aid)
+thread_local int g_last_call_fused = 0;   // what the last fa_decode_attn call of this thread did (measurement aids)
+thread_local int g_last_call_sub_splits = 0;
 
 // Whether the merge can run inside the mid-row launch (fa_decode_fused.h): the one-pass matrix-core pipeline, heads
 // of 128 dims with at most four query heads per KV head, every workgroup of the launch resident at once (the
@@ -2250,6 +2251,7 @@ int launch_all(const fa_decode_args& a, const Plan& p, bool p_il_fast, float sm_
   const bool one_pass = p.path == Path::Mfma && fa_mfma::table_slices(a.N) == 4;
   const int nsub = fused && one_pass && a.B <= 2 && !(a.no_fuse & 2) ? 4 / a.B : 1;
   g_last_call_fused = fused ? (nsub == 4 ? 2 : 1) : 0;
+  g_last_call_sub_splits = fused ? nsub : 0;
   // A rank-1 update the coefficients are still owed: the query preparation applies it to the K coefficients it streams,
   // the merge inside the mid-row launch to the V coefficients; where those do not run it gets a launch of its own
   if (a.upd_k_row && a.Ck > 0 && p.n_mid_split <= 0) {
@@ -2675,6 +2677,7 @@ extern "C" int fa_decode_attn_noalloc(const fa_decode_args* a, fa_stream_t strea
 }
 
 extern "C" int fa_decode_attn_last_fused(void) { return g_last_call_fused; }
+extern "C" int fa_decode_attn_last_sub_splits(void) { return g_last_call_sub_splits; }
 
 extern "C" int fa_decode_attn_timed(const fa_decode_args* a, fa_stream_t stream, float* ms_out) {
   FA_REQUIRE(ms_out, FA_ERR_NULL_POINTER, "fa_decode_attn_timed: ms_out null");

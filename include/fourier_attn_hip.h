@@ -407,6 +407,9 @@ int fa_decode_attn_noalloc(const fa_decode_args* args, fa_stream_t stream);
  * launch (1; 2: with the four sub-splits per workgroup of a batch of one) or as a launch of its own (0).  A
  * measurement aid (the reference has no counterpart). */
 int fa_decode_attn_last_fused(void);
+/* ... and how many sub-splits of each sequence a workgroup of that launch ran: 4 or 2, 1 for none; 0 where the merge was a
+ * launch of its own. */
+int fa_decode_attn_last_sub_splits(void);
 
 /* fa_stream_update(s) followed by fa_decode_attn(a), whose arguments describe the state the update leaves: the same results,
  * in one launch less where the update can ride in the attention's first launch (16- or 32-bit rows with vectorised

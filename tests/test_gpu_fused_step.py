@@ -30,7 +30,7 @@ CASES = [
     (torch.bfloat16, 1, 32, 4, 32, 512, 1100 + 19, U, U, 2),                               # ragged last page
     (torch.bfloat16, 4, 32, 4, 64, 1024, 3000, U, U, 1),                                   # a full group of four
     (torch.bfloat16, 8, 32, 4, 64, 512, 1500, [64, 0, 128, 30, 64, 64, 100, 64], [1, 64, 2, 3, 128, 64, 0, 64], 1),
-    (torch.float16, 2, 16, 4, 40, 512, 2500, U, U, 1),                                     # two sequences: no sub-splits
+    (torch.float16, 2, 16, 4, 40, 512, 2500, U, U, 1),                                     # two sequences
     # heads with few compressed V dims (8, 3, 0, 16, 64, 1, 28, 12): few outputs and many row classes in the tail's product
     (torch.bfloat16, 4, 32, 4, 64, 512, 2500, U, [120, 125, 128, 112, 64, 127, 100, 116], 1),
     (torch.bfloat16, 1, 32, 4, 64, 1024, 6000, U, [120, 125, 128, 112, 64, 127, 100, 116], 2),
@@ -98,6 +98,26 @@ def test_the_ways_a_step_runs_agree(case):
     # and with them the rounding of the 16-bit probabilities
     assert np.abs(got["merged"] - got["launches"]).max() <= 2e-3
     assert np.abs(got["default"] - got["launches"]).max() <= 2e-3
+
+
+@pytest.mark.parametrize("B,M,sub_splits", [(1, 512, 4), (2, 512, 2), (3, 512, 1), (2, 2048, 1)])
+def test_how_many_sub_splits_a_launch_runs(B, M, sub_splits):
+    """One sequence in four sub-splits, two in two each, more and two passes in none; none where they are switched off."""
+    from fourierattention_amd import DynamicCache, _lib
+    lib, g = _lib.load(), torch.Generator(device="cuda").manual_seed(B)
+    rn = lambda *s: torch.randn(s, generator=g, device="cuda").bfloat16()
+    gpu = DynamicCache(_cfg(_masks(1, 8, 128, U, U, seed=1), numinittokens=4, maxlocallen=40, maxmidstates=M, num_key_value_heads=8, max_new_tokens=16))
+    prompt = M + 44 + 1500
+    gpu.update(rn(B, 8, prompt, 128), rn(B, 8, prompt, 128), 0)
+    gpu.update(rn(B, 8, 1, 128), rn(B, 8, 1, 128), 0)
+    q = rn(B, 32, 1, 128)
+    for on, want in ((True, sub_splits), (False, 1)):
+        gpu.sub_splits = on
+        gpu.decode_attention(q, 0, 32, 8)
+        assert (lib.fa_decode_attn_last_sub_splits(), lib.fa_decode_attn_last_fused()) == (want, 2 if want == 4 else 1)
+    gpu.fuse_decode = False
+    gpu.decode_attention(q, 0, 32, 8)
+    assert (lib.fa_decode_attn_last_sub_splits(), lib.fa_decode_attn_last_fused()) == (0, 0)
 
 
 def test_fused_step_with_converted_output_rows():
