@@ -96,8 +96,8 @@ def audit_async_lds_reads(asm_text: str):
 
 # kernels in which one workgroup hands data to another inside a launch: it stores, waits for the stores, then counts
 # itself in with an atomic (decode_merge_rows_kernel; the instances of decode_mid_mfma_kernel that merge their own
-# partials: the third from last of their template arguments, FUSE, is `true`)
-HANDOVER_KERNELS = (re.compile(r"decode_merge_rows_kernel"), re.compile(r"decode_mid_mfma_kernel\S*Lb1ELb[01]ELb[01]EEEv"))
+# partials: FUSE, the first of the flags that end their template arguments, is `true`)
+HANDOVER_KERNELS = (re.compile(r"decode_merge_rows_kernel"), re.compile(r"decode_mid_mfma_kernel\S*Lb1E(?:Lb[01]E)?Lb[01]EEEv"))
 _STORE_OPS = ("global_store", "buffer_store", "flat_store")
 
 

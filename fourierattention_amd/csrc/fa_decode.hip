@@ -187,8 +187,9 @@ __device__ __forceinline__ void decode_prep_body(const PrepArgs<E>& pa, int bx, 
       if (tid == 0) c0[(int64_t)b * Hq + h * G + g] = v * sm_log2e;
     }
   }
-  // sixteen lanes share a row (64 bytes of it per access), a thread four rows.  (Requested ahead of the query's list and gather instead: 17.3 us where this takes
-  // 14.6 at one sequence of 32k tokens, 27.9 against 26.9 at eight: the loads the rest of the chain waits for queue behind them.)
+  // sixteen lanes share a row (64 bytes of it per access), a thread four rows.  (Requested ahead of the query's list and gather
+  // instead: 17.3 us where this takes 14.6 at one sequence of 32k tokens, 27.9 against 26.9 at eight: the loads the rest of the
+  // chain waits for queue behind them.)
   const int lr = tid & 15, r0 = tid >> 4;
   const float* rows = k_mc + ((int64_t)b * 2 * N + bx * kPrepRows) * Ck + kc0;
   const int n_left = 2 * N - bx * kPrepRows;      // rows from here to the end
@@ -2051,13 +2052,13 @@ Plan make_plan(int B, int Hq, int Hkv, int D, int N, int n_il, int L_m, bool mfm
   p.off_ilm = take(rows * p.n_il_split * 4);
   p.off_ild = take(rows * p.n_il_split * 4);
   p.off_ilo = take(rows * p.n_il_split * D * 4);
-  // (a single sequence on the matrix-core path may run as four sub-splits per workgroup, each with partials of its own)
-  const size_t prows = mfma && B == 1 ? 4 * rows : rows;
-  p.off_mm = take(prows * p.n_mid_split * 4);
-  p.off_md = take(prows * p.n_mid_split * 4);
+  p.off_mm = take(rows * p.n_mid_split * 4);
+  p.off_md = take(rows * p.n_mid_split * 4);
   // g partials: a row of 2N per (query head, split); the matrix-core path stores 16 columns per (batch group, KV head, split)
   p.off_mg = take((mfma ? (size_t)p.n_groups * Hkv * 16 : rows) * p.n_mid_split * 2 * N * 4);
-  p.off_mon = take(prows * p.n_mid_split * D * 4);
+  // (a single sequence on the matrix-core path may run as four sub-splits per workgroup, whose outputs of the stored dims leave
+  // one by one; two sequences in two each keep theirs in the g partials, see launch_all)
+  p.off_mon = take((mfma && B == 1 ? 4 * rows : rows) * p.n_mid_split * D * 4);
   p.off_tab = take(mfma ? fa_mfma::tables_bytes(N) : 0);
   // merge: as many blocks per (b, KV head) as still run side by side on the device (a block fills one compute unit)
   p.n_merge_chunks = kMergeChunksMax;

@@ -275,25 +275,24 @@ struct MidParams {
 //         per frame.
 // FUSE (MODE 0 and the value pass, MODE 2): the launch merges its own partials and writes the output rows, see fa_decode_fused.h; the
 // workgroups are then numbered through p.fz.wg_map so that the splits of a (batch group, KV head) share one die.
-// SUB (FUSE only, a batch of one or two sequences, at most four query heads per KV head): a single batch element would
+// SUB, NSUB > 1 (FUSE only, a batch of one or two sequences, at most four query heads per KV head): a single batch element would
 // leave twelve of the sixteen matrix-core columns and three of the four page streams of a workgroup idle, two of them half.
 // The workgroup's pages are cut into NSUB = 4 resp. 2 sub-splits instead, so that four slots take the places of four batch
 // elements: slot s = batch element s % (4 / NSUB), sub-split s / (4 / NSUB).  Wave i streams the pages of slot i, column
 // 4 s + g holds query head g with its weights W' rotated to the first frame of its sub-split, and every column keeps its own
 // softmax reference, g history and outputs.  Behind the loop the columns of a head are brought to one reference and added up
 // (the outputs of the stored dims leave one by one, as "virtual batch elements" s of the partial buffers).  The page loop has
-// 1 / NSUB of the trips.  Pages past the end of a sub-split are fetched from a
-// valid page and masked.
+// 1 / NSUB of the trips.  Pages past the end of a sub-split are fetched from a valid page and masked.
 // UPD (FUSE only): the tail also applies a pending rank-1 update to the V coefficients of its row share.
-template <typename E, int KS, int KMAX, int VMAX, int NST, int MODE = 0, int NSUB = 1, bool FUSE = false, bool SUB = false,
-          bool UPD = false>
+template <typename E, int KS, int KMAX, int VMAX, int NST, int MODE = 0, int NSUB = 1, bool FUSE = false, bool UPD = false>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void decode_mid_mfma_kernel(
     const MidParams<E> p) {
   static_assert(!FUSE || MODE == 0 || MODE == 2, "the fused merge runs behind the one-pass pipeline or behind the value pass");
+  static_assert(NSUB == 1 || NSUB == 2 || NSUB == 4, "none, two or four sub-splits");
+  constexpr bool SUB = NSUB > 1;
   static_assert(!SUB || MODE == 0, "sub-splits belong to the one-pass pipeline");
   static_assert(!UPD || MODE == 0, "the pending update keeps its row in the LDS of the score partials");
   static_assert(!SUB || FUSE, "sub-splits end in the fused merge");
-  static_assert(SUB ? NSUB == 2 || NSUB == 4 : NSUB == 1, "two or four sub-splits");
   constexpr int kBat = 4 / NSUB;   // SUB: batch elements of the group
   static_assert(!UPD || FUSE, "the pending update rides in the fused merge");
   constexpr int NSL = MODE == 0 ? kFreqWaves : 2 * kFreqWaves;   // frequency slices
@@ -426,7 +425,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     vec8 Qb[KMAX];
     {
       // (SUB: every sub-split starts from the weights of its query head, column g of its batch element)
-      const float2v* wl = (const float2v*)p.W + ((int64_t)((grp * p.Hkv + h) * NSL + sl) * 2 * KS * 2) * 64 + ((SUB ? bb_r % kBat * G + min(g_r, G - 1) : lc) * 4 + lg);
+      const int w_col = SUB ? bb_r % kBat * G + min(g_r, G - 1) : lc;
+      const float2v* wl = (const float2v*)p.W + ((int64_t)((grp * p.Hkv + h) * NSL + sl) * 2 * KS * 2) * 64 + (w_col * 4 + lg);
       float2v wc2[2 * KS], ws2[2 * KS];
 #pragma unroll
       for (int rt = 0; rt < 2 * KS; ++rt) {

@@ -48,9 +48,9 @@ void launch_mid_mfma_ks(const MidParams<E>& mp, const MidLaunch& ml, hipStream_t
       constexpr int S = decltype(sub_tag)::value;
       constexpr bool U = decltype(upd_tag)::value;
       if (ml.wide)
-        decode_mid_mfma_kernel<E, KS, 4, 8, 2, 0, S, true, (S > 1), U><<<grid, 512, 0, st>>>(mp);
+        decode_mid_mfma_kernel<E, KS, 4, 8, 2, 0, S, true, U><<<grid, 512, 0, st>>>(mp);
       else
-        decode_mid_mfma_kernel<E, KS, 2, 4, 2, 0, S, true, (S > 1), U><<<grid, 512, 0, st>>>(mp);
+        decode_mid_mfma_kernel<E, KS, 2, 4, 2, 0, S, true, U><<<grid, 512, 0, st>>>(mp);
     };
     auto by_subs = [&](auto upd_tag) {
       if (ml.nsub == 4) go(std::integral_constant<int, 4>{}, upd_tag);

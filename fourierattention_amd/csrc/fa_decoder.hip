@@ -501,8 +501,9 @@ int linear_packed(const void* x, int64_t x_row_stride, const void* norm_weight, 
       const size_t sums = (size_t)kLinWaves * 64 * 16 * (epilogue == EPI_GATE ? 2 : 1);
       const size_t x_bytes = norm_weight ? (size_t)rows * (K + 8) * 2 : 0;
       auto go = [&](auto kernel) {
-        kernel<<<grid, 64 * kLinWaves, sums > x_bytes ? sums : x_bytes, st>>>((const E*)x, x_row_stride, (const E*)norm_weight, eps, (const E*)w_packed, (E*)out,
-                                                rows, K, n_out, RopeOut<E>{(const E*)rc.cos, (const E*)rc.sin, (E*)rc.kv, rc.nq, rc.nqk, rc.D});
+        kernel<<<grid, 64 * kLinWaves, sums > x_bytes ? sums : x_bytes, st>>>(
+            (const E*)x, x_row_stride, (const E*)norm_weight, eps, (const E*)w_packed, (E*)out, rows, K, n_out,
+            RopeOut<E>{(const E*)rc.cos, (const E*)rc.sin, (E*)rc.kv, rc.nq, rc.nqk, rc.D});
       };
       auto by_epilogue = [&](auto pieces) {   // pieces of the rows a thread normalises
         constexpr int P = decltype(pieces)::value;

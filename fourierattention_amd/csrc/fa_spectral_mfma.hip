@@ -10,8 +10,8 @@
 //   G_s[n] = sum_{i<128} E[n, i] a[128 s + i]
 // so the steps are walked from the last to the first, acc <- G_s + e^{i theta n 128} acc, with the
 // accumulators (fp32) never leaving registers.  Three kernels:
-//   pack    evaluates the basis table, gathers the compressed columns of the token-major input, converts them to f16 and writes them
-//           as ready-made MFMA B operands (column tile of 16, kstep of 32 tokens, 64 lanes x 8 tokens)
+//   pack    evaluates the basis table, gathers the compressed columns of the token-major input, converts them to f16 and
+//           writes them as ready-made MFMA B operands (column tile of 16, kstep of 32 tokens, 64 lanes x 8 tokens)
 //   gemm    one workgroup = 128 frequencies x 64 columns x one chunk of steps; the operands of a step
 //           travel HBM -> LDS with global_load_lds, one barrier per step
 //   reduce  sums the chunks into c
@@ -55,8 +55,9 @@ struct SpectralTable {
 };
 
 // ---- pack: block = 32 tokens x 256 columns; lanes run along the columns for the gather, the transposition to
-// token-contiguous fragments goes through LDS.  grid (ksteps + blocks of the basis table, column blocks, parts * B): part p of the input starts p * a_part
-// elements behind the first and its fragments p * out_part behind the first's; with col_inv_scale the columns are scaled ------
+// token-contiguous fragments goes through LDS.  grid (ksteps + blocks of the basis table, column blocks, parts * B): part p of
+// the input starts p * a_part elements behind the first and its fragments p * out_part behind the first's; with
+// col_inv_scale the columns are scaled ------
 template <typename E>
 __global__ __launch_bounds__(256) void spectral_pack_kernel(
     const E* __restrict__ a, int64_t a_bs, int64_t a_rs, const int32_t* __restrict__ cols,
@@ -1208,9 +1209,10 @@ int recon_walk_launch(const float* c, int B, int N, int Mc, int K, int T, void* 
   const int kp8 = fa_cdiv(Kd, 8) * 8;
   coef_colscale_kernel<<<dim3(fa_cdiv(Mc, 16), B), 1024, 0, st>>>(c, scale, inv, 2 * N, Mc);
   // the cosine rows and, behind them, the sine rows; the basis of the positions beside them
-  const int pack_rows = fa_cdiv(Mc, 256) * 2 * B;
-  spectral_pack_kernel<float><<<dim3(pl.KS32 + fa_cdiv(table_blocks(kp8), pack_rows), fa_cdiv(Mc, 256), 2 * B), 256, 0, st>>>(c, (int64_t)2 * N * Mc, Mc, nullptr, inv, pc, N, Mc,
-                                                                                     pl.CT, pl.KS32, B, (int64_t)N * Mc, ps - pc, SpectralTable{(half2v*)tab, kp8, T});
+  const int col_blocks = fa_cdiv(Mc, 256);
+  const dim3 pgrid(pl.KS32 + fa_cdiv(table_blocks(kp8), col_blocks * 2 * B), col_blocks, 2 * B);
+  spectral_pack_kernel<float><<<pgrid, 256, 0, st>>>(c, (int64_t)2 * N * Mc, Mc, nullptr, inv, pc, N, Mc, pl.CT, pl.KS32, B,
+                                                     (int64_t)N * Mc, ps - pc, SpectralTable{(half2v*)tab, kp8, T});
   ReconWalkParams rp{};
   rp.tab = tab; rp.packed[0] = pc; rp.packed[1] = ps; rp.scale = scale;
   rp.psum = *psum; rp.pmax = *pmax; rp.pmin = *pmin;

@@ -460,11 +460,12 @@ PyObject* linear_packed_qkv(PyObject*, PyObject* const* a, Py_ssize_t n) {
   CHECK(n == 9, "linear_packed_qkv takes 9 arguments");
   const at::Tensor &x = gpu_tensor(a[0], "x"), &w = gpu_tensor(a[1], "weight"), &cos = gpu_tensor(a[4], "cos"), &sin = gpu_tensor(a[5], "sin");
   const int64_t Hq = integer(a[6]), Hkv = integer(a[7]), D = integer(a[8]);
-  CHECK(x.dim() == 3 && x.scalar_type() == w.scalar_type() && x.size(2) > 0 && Hq > 0 && Hkv > 0 && D > 0 && w.numel() == x.size(2) * (Hq + 2 * Hkv) * D,
-        "linear_packed_qkv: x (B, q_len, k) does not fit the weight");
+  CHECK(x.dim() == 3 && x.scalar_type() == w.scalar_type() && x.size(2) > 0 && Hq > 0 && Hkv > 0 && D > 0 &&
+        w.numel() == x.size(2) * (Hq + 2 * Hkv) * D, "linear_packed_qkv: x (B, q_len, k) does not fit the weight");
   const int64_t B = x.size(0), q_len = x.size(1), k = x.size(2), rows = B * q_len;
   for (const at::Tensor* t : {&cos, &sin})
-    CHECK(t->is_contiguous() && t->scalar_type() == x.scalar_type() && (B == 1 ? t->numel() >= rows * D : t->numel() == rows * D), "linear_packed_qkv: one row of cos and sin per token, of the type of x");
+    CHECK(t->is_contiguous() && t->scalar_type() == x.scalar_type() && (B == 1 ? t->numel() >= rows * D : t->numel() == rows * D),
+          "linear_packed_qkv: one row of cos and sin per token, of the type of x");
   const void* norm = nullptr;
   if (a[2] != Py_None) {
     const at::Tensor& nw = gpu_tensor(a[2], "norm weight");

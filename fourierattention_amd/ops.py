@@ -265,7 +265,9 @@ def prompt_rows(k: torch.Tensor, v: torch.Tensor, near: Optional[Tuple[torch.Ten
     tangent, calls that are recorded."""
     B, heads, S, D = k.shape
     es = k.element_size()
-    if (recorded() or type(k) is not torch.Tensor or type(v) is not torch.Tensor or not k.is_cuda or k.device != v.device or k.shape != v.shape or k.dtype != v.dtype or k.dtype not in _DTYPE_CODE
+    if recorded() or type(k) is not torch.Tensor or type(v) is not torch.Tensor:
+        return None
+    if (not k.is_cuda or k.device != v.device or k.shape != v.shape or k.dtype != v.dtype or k.dtype not in _DTYPE_CODE
             or k.stride() != v.stride() or k.stride(3) != 1 or k.requires_grad or v.requires_grad or not 0 < B <= 65535 or S == 0
             or any((s * es) % 16 for s in (*k.stride()[:3], D)) or k.data_ptr() % 16 or v.data_ptr() % 16
             or first + last > S or any(unpack_dual(t).tangent is not None for t in (k, v))):
