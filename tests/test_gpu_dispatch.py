@@ -27,9 +27,9 @@ def test_reconstruction_statistics_by_shares_of_column_blocks(B, L, C, N, T):
 
 
 @pytest.mark.parametrize("B,L,C,N,T", [
-    (1, 1300, 33, 1100, 2700),   # nine steps of 128 coefficients, the last one short; a column block of one column
-    (2, 2048, 32, 1024, 2048),   # eight whole steps; whole blocks of positions and, with position T / 2, one of a single one
-    (1, 1025, 17, 129, 1400),    # one coefficient past a step
+    (1, 1300, 33, 1100, 2700),   # ten steps of the coefficients, the last one short; a column block of one column
+    (2, 2048, 32, 1024, 2048),   # nine steps; whole blocks of positions and, with position T / 2, one of a single one
+    (1, 1025, 17, 129, 1400),    # two steps, the second half full
 ])
 def test_reconstruction_statistics_of_signals_with_a_mean(B, L, C, N, T):
     """Folded steps of the coefficients against float64, for signals whose mean outweighs their deviation.  Bound: coefficients
@@ -142,10 +142,50 @@ def test_prompt_of_a_window_where_operations_are_recorded(how):
             assert rows(mode.from_tensor(k), mode.from_tensor(v)).shape == (1, 20, 256)
 
 
+def _reconstruction64(c, L, T):
+    """Mean and largest deviation of the reconstruction in 64 bits, and the 2-norm of every column's coefficients over N."""
+    N = c.shape[1] // 2
+    ph = 2 * np.pi / T * (torch.arange(L, device="cuda")[:, None] * torch.arange(N, device="cuda")[None] % T).double()
+    r = (ph.cos() @ c[:, :N].double() + ph.sin() @ c[:, N:].double()) / N
+    avg = r.mean(1)
+    return avg, torch.maximum(r.amax(1) - avg, avg - r.amin(1)), c.double().norm(dim=1) / N
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])    # the two kernels of the matrix cores
+@pytest.mark.parametrize("B,L,C,N,T", [
+    (1, 1024, 16, 32, 1100),     # one row group, one column block of one tile
+    (1, 1500, 130, 64, 2999),    # three column blocks of 64, the last two columns wide; odd period; one whole step above its centre
+    (1, 1977, 905, 128, 6073),   # fifteen column blocks, one per workgroup
+    (3, 9000, 833, 128, 9100),   # shares of several column blocks, the last share shorter; mirrored positions
+    (1, 1300, 33, 1100, 2700),   # nine steps of 128 or ten of 127, the last one short
+    (2, 2048, 32, 1024, 2048),   # whole blocks of positions, and position T / 2 in one of its own
+    (1, 1025, 17, 129, 1400),    # one coefficient past a step of 128
+    (1, 1200, 40, 65, 1201),     # one past the first 64; every position but one mirrored
+    (2, 1100, 64, 191, 1100),    # two whole steps of 127 (the first from its centre)
+    (1, 2600, 100, 192, 1280),   # one past those; a sequence of two periods, nothing mirrored
+    (1, 1500, 48, 318, 1499),    # three whole steps; as long as the period and one position more
+])
+def test_both_kernels_of_the_statistics_a_cache_keeps(dtype, B, L, C, N, T):
+    """Mean and deviation as ``recon_scale`` leaves them, against float64.  Bound: coefficients and basis carry up to 2^-11
+    relative rounding each, independent from term to term: a position is off by at most about five standard deviations (1 / sqrt(3) of
+    the bound each, 4 in all) of 2^-11 times the 2-norm of the column's coefficients over N, a deviation by twice that;
+    mean, deviation and an fp16 quotient are rounded to fp16 on top, 2^-11 each."""
+    from fourierattention_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(L + N)
+    c = torch.randn((B, 2 * N, C), generator=g, device="cuda") * (N ** 0.5 * (0.2 + 3 * torch.rand((1, 1, C), generator=g, device="cuda")))
+    c[:, 0] += 2 * N * torch.randn((1, C), generator=g, device="cuda")       # means of the size of the deviation
+    one = torch.ones((B, C), device="cuda")
+    scale, _, _, (_, avg, _) = ops.recon_scale(c, L, T, one, one, dtype)
+    avg64, dev64, norm = _reconstruction64(c, L, T)
+    assert ((avg.double() - avg64).abs() <= 4 * 2.0 ** -11 * norm + 2.0 ** -11 * avg64.abs()).all()
+    assert ((1 / scale.double() - dev64).abs() <= 8 * 2.0 ** -11 * norm + 2 * 2.0 ** -11 * dev64).all()
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("B,L,C,N,T", [(2, 300, 5, 16, 400), (1, 1100, 70, 64, 1500)])   # vector kernels / matrix cores
 def test_statistics_a_cache_keeps(dtype, B, L, C, N, T):
-    """The same values, bit for bit, as the conversions and the division as tensor operations."""
+    """The same values, bit for bit, as the conversions and the division as tensor operations; in single precision on the matrix
+    cores those of the kernel such a cache has for itself."""
     from fourierattention_amd import ops
     g = torch.Generator(device="cuda").manual_seed(2)
     x = (torch.randn((B, L, C), generator=g, device="cuda") * 3 + 1).to(dtype)
@@ -154,13 +194,24 @@ def test_statistics_a_cache_keeps(dtype, B, L, C, N, T):
     i_avg, i_dev = ops.mat_fourier_avg_std(c, L, T, torch.float16)
     scale = u_dev.to(dtype) / i_dev.to(torch.float16)
     got = ops.recon_scale(c, L, T, u_avg, u_dev, dtype)
-    for a, b in zip((*got[:3], *got[3]), (scale, u_avg.to(dtype), i_avg.to(torch.float16), u_avg, i_avg, scale.float())):
-        assert a.dtype == b.dtype
-        if dtype == torch.float32 and L > 1024:   # a single-precision cache has a kernel of its own: a place of fp16, 2^-10, either way
-            size = i_avg.abs() + i_dev if a.shape == i_avg.shape and a.dtype != torch.float32 else b.abs().float() + i_dev
-            assert ((a.float() - b.float()).abs() <= 2.0 ** -9 * size).all()
-        else:
-            assert torch.equal(a, b)
+    want = (scale, u_avg.to(dtype), i_avg.to(torch.float16), u_avg, i_avg, scale.float())
+    have = (*got[:3], *got[3])
+    assert all(a.dtype == b.dtype for a, b in zip(have, want))
+    # a single-precision cache has a kernel of its own on the matrix cores: what comes of the reconstruction may round the other way
+    own = dtype == torch.float32 and L > 1024
+    for at in (1, 3) if own else range(6):
+        assert torch.equal(have[at], want[at])
+    if own:
+        # (the same mean in both types, the same quotient twice, and the quotient of the deviation as fp16 holds it)
+        assert torch.equal(have[2].float(), have[4]) and torch.equal(have[0], have[5])
+        dev = u_dev.double() / have[0].double()
+        dev16 = dev.to(torch.float16).double()
+        assert ((dev - dev16).abs() <= 2.0 ** -22 * dev16).all()
+        # mean and deviation against float64: at most 4 * 2^-11 of the 2-norm of a column's coefficients over N, as for the kernels
+        # themselves (twice that for the deviation), and half a place of fp16
+        avg64, dev64, norm = _reconstruction64(c, L, T)
+        assert ((have[4].double() - avg64).abs() <= 4 * 2.0 ** -11 * norm + 2.0 ** -11 * avg64.abs()).all()
+        assert ((dev16 - dev64).abs() <= 8 * 2.0 ** -11 * norm + 2.0 ** -11 * dev64).all()
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
