@@ -2247,8 +2247,9 @@ int launch_all(const fa_decode_args& a, const Plan& p, bool p_il_fast, float sm_
   // (the sink/window tiles must be in front of the mid rows for the merge to run inside that launch)
   const bool fused = sizeof(E) == 2 && (fuse_il || p.n_il_split == 0) && fused_merge_plan(a, p, wg_map, st);
   // one sequence: its mid rows as four sub-splits per workgroup in the places of four batch elements; two: two of each
-  // (a layer's step, update and all, with one sub-split each / two: two sequences of 32k 68.5 / 59.5 us, of 100k with 100 of 128
-  // dims compressed 114 / 89.5, of 3k 34.4 / 33.7; three and four fill the columns as they are)
+  // (a layer's step, update and all, without / with them, half of the dims compressed: two sequences of 32k 65.3 / 59.0 us, of 12k
+  // 49.2 / 46.8, of 3k 39.3 / 38.1, of 100k with 100 of 128 dims compressed 114 / 91; one of 32k 53.7 / 41.6; three and four
+  // fill the columns as they are)
   const bool one_pass = p.path == Path::Mfma && fa_mfma::table_slices(a.N) == 4;
   const int nsub = fused && one_pass && a.B <= 2 && !(a.no_fuse & 2) ? 4 / a.B : 1;
   g_last_call_fused = fused ? (nsub == 4 ? 2 : 1) : 0;
@@ -2592,9 +2593,11 @@ static bool step_joins(const fa_stream_args* s, const fa_decode_args* a, JoinedS
   if ((((uintptr_t)s->k_new | (uintptr_t)s->v_new | (uintptr_t)(s->new_batch_stride * es)) & 15) != 0 || !s->k_new || !s->v_new) return false;
   // Every head's blocks write its own columns of the K coefficients back.  Where heads begin and end inside a line (counts of
   // compressed dims that differ or are no multiple of 16), two of them write parts of one, and with many coefficients of few
-  // sequences that costs more than the launch: joined / apart, us a layer at 12k tokens, 921 of 1024 dims, 512 frequencies, one
-  // sequence 44.9 / 42.8, four 64.1 / 63.2, eight 89.2 / 90.0; 256 frequencies, one 37.2 / 38.1; 64 dims of every head, 512
-  // frequencies, one 42.3 / 42.2, eight 77.5 / 82.5.  Heads of 64 dims and single precision gain throughout.
+  // sequences that costs as much as the launch: joined / apart, us a layer at 12k tokens, 921 of 1024 dims, 512 frequencies, one
+  // sequence 39.3 / 39.3, two 50.4 / 50.6, four 62.9 / 62.7, six 77.2 / 76.4, eight 86.3 / 88.5; 1024 frequencies, one 68.7 / 68.1;
+  // with 512 of 1024 dims, uneven, it would gain 1 - 3% (one 38.6 / 39.7, four 61.7 / 62.3).  256 frequencies, one 34.3 / 35.8, four
+  // 51.1 / 54.5; 64 dims of every head, 512 frequencies, one 35.6 / 38.2, eight 72.5 / 78.7.  Heads of 64 dims and single
+  // precision gain throughout.
   bool whole_lines = a->Ck % (16 * a->Hkv) == 0;
   if (a->k_pad_h_host)   // (stored dims, padded: uneven ones show here)
     for (int h = 0; h < a->Hkv; ++h) whole_lines = whole_lines && a->k_pad_h_host[h + 1] - a->k_pad_h_host[h] == a->k_pad_h_host[1];
